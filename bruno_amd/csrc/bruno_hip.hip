@@ -330,6 +330,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter_spilled(Slot<KT>* T, const Spi
   }
 }
 
+#include "chains.h"
+
 /* ================================================================== */
 /* chain extraction                                                     */
 /* ================================================================== */
@@ -371,12 +373,13 @@ __device__ uint32_t resolve(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, ui
  * neighbour's facing end points back at k (a chain neighbour) or gets
  * marked terminal by k_termini (a branch neighbour).  Each end that fails
  * (neighbour absent, no edge back, or an end pointing at itself) adds one
- * to ill. */
+ * to ill.  in_branch / out_branch: the neighbour is a branch that answers
+ * the edge, so k_termini marks this end terminal. */
 template <typename KT>
 __device__ void resolve_pair(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, uint32_t rbits, const kops<KT>& ops,
                              KT k, uint32_t self, bool has_in, KT nin, bool has_out, KT nout, uint64_t n_chain,
                              KT* vkmer, uint64_t vcap, Counters* ctr, uint32_t& pin, uint32_t& pout,
-                             unsigned long long& ill) {
+                             bool& in_branch, bool& out_branch, unsigned long long& ill) {
   const KT ri = ops.rc(nin), ro = ops.rc(nout);
   const bool fi = !(nin < ri), fo = !(nout < ro);
   const KT cin = fi ? ri : nin, cout = fo ? ro : nout;
@@ -413,11 +416,13 @@ __device__ void resolve_pair(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, u
     const bool back = si != ~0ULL && (fi ? ni->c[4 + 3 - lb] : ni->c[lb]) > 0;
     const bool loop = si != ~0ULL && cls_i == CLS_CHAIN && idx_i == self && ein == 0u;
     ill += (!back || loop) ? 1 : 0;
+    in_branch = back && cls_i == CLS_BRANCH;
   }
   if (has_out) {
     const bool back = so != ~0ULL && (fo ? no->c[3 - fb] : no->c[4 + fb]) > 0;
     const bool loop = so != ~0ULL && cls_o == CLS_CHAIN && idx_o == self && eout == END_OUT;
     ill += (!back || loop) ? 1 : 0;
+    out_branch = back && cls_o == CLS_BRANCH;
   }
   auto finish = [&](bool found, uint8_t cls, uint32_t idx, KT cn, uint32_t end) -> uint32_t {
     if (found && cls == CLS_CHAIN) return end | idx;
@@ -434,13 +439,20 @@ __device__ void resolve_pair(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, u
 }
 
 /* to_simple_biedge (debruijn_chain_node.hpp:84-141): one neighbour per side
- * at dist 1, else term_mask. */
+ * at dist 1, else term_mask; an end at a branch that answers it is terminal
+ * at once (k_termini writes the same).  So every chain end is known here,
+ * and the rulers of the list ranking (chain ends and sampled nodes) are
+ * marked in a bitmap, a word per wave, instead of by a pass over the 32-byte
+ * records (0.85 ms for 40 M chain nodes).  The node's k-mer goes into its
+ * mailboxes, beside the pointers, for the placing walk (chains.h); the
+ * round-by-round ranking empties them first. */
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_t cap, uint32_t rbits, int K,
                                                       const uint64_t* chain_slot,
                                                       const uint32_t* chain_job, const uint64_t* seg, uint32_t n_jobs,
                                                       uint64_t n_chain, KT* ckmer, const uint8_t* cedge, LRNode* lr,
-                                                      KT* vkmer, uint64_t vcap, Counters* ctr) {
+                                                      KT* vkmer, uint64_t vcap, uint64_t ruler_mask,
+                                                      uint64_t* ruler_bits, uint8_t* alive, Counters* ctr) {
   kops<KT> ops(K);
   const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
   unsigned long long ill = 0;
@@ -472,15 +484,23 @@ __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_
     LRNode st;
     st.p[0] = st.p[1] = IDX_MASK;
     st.d[0] = st.d[1] = TERM_MASK;
-    st.mail[0] = st.mail[1] = 0ULL;
+    st.mail[0] = (uint64_t)k;
+    st.mail[1] = (uint64_t)((u128)k >> 64);
     /* in neighbour c.k[0..K-2]: when canonical its OUT end faces k; out
      * neighbour k[1..].c: when canonical its IN end faces k */
+    bool in_branch = false, out_branch = false;
     resolve_pair<KT>(T, tbase, tcap, rbits, ops, k, (uint32_t)i, ci >= 0, ops.in_nbr(k, ci < 0 ? 0 : ci), co >= 0,
-                     ops.out_nbr(k, co < 0 ? 0 : co), n_chain, vkmer, vcap, ctr, st.p[0], st.p[1], ill);
-    if (ci >= 0) st.d[0] = 1;
-    if (co >= 0) st.d[1] = 1;
+                     ops.out_nbr(k, co < 0 ? 0 : co), n_chain, vkmer, vcap, ctr, st.p[0], st.p[1], in_branch, out_branch,
+                     ill);
+    if (ci >= 0) st.d[0] = in_branch ? 0 : 1;
+    if (co >= 0) st.d[1] = out_branch ? 0 : 1;
     if (!cedge) ckmer[i] = k;
     lr[i] = st;
+    alive[i] = 1;
+    /* a wave covers 64 aligned nodes; lane 0's node is the lowest */
+    const uint64_t word =
+        __ballot(is_terminal(st.d[0]) || is_terminal(st.d[1]) || sampled_ruler(i, ruler_mask));
+    if ((threadIdx.x & 63) == 0) ruler_bits[i >> 6] = word;
   }
   block_add(ill, &ctr->lr_ill);
 }
@@ -651,279 +671,6 @@ __global__ __launch_bounds__(BLOCK) void k_lr_recv(LRNode* lr, const uint32_t* l
   block_add(cyc, &ctr->lr_cycle);
 }
 
-/* ================================================================== */
-/* list ranking by ruler contraction (well-formed chain graphs)         */
-/* ================================================================== */
-/* On a chain graph where every end pointing at a chain node is pointed back
- * at, the chain nodes form disjoint paths and cycles, and the end state of
- * bruno's pointer jumping is fixed: every non-terminal end points at the
- * chain end it leads to, at its exact distance, marked as pointing to a
- * terminal; cycle nodes end with both distances 2^T.  The number of rounds
- * T is the largest ceil(log2 L) over paths of L >= 2 nodes, at least 1 when
- * a cycle exists.  This computes that state without the rounds: rulers
- * (chain ends plus sampled nodes) walk to the next ruler, heads walk the
- * ruler graph, then every node reads its two chain ends off its rulers. */
-constexpr uint32_t NONE32 = 0xFFFFFFFFu;
-constexpr uint32_t WALK_MAX = 1u << 16;
-constexpr uint32_t ERR_NOT_WELL_FORMED = 16;
-constexpr uint32_t ERR_WALK = 32;
-constexpr uint32_t ERR_NO_NODE = 64; /* an output k-mer without its filtered-graph record */
-
-__device__ __forceinline__ uint32_t end_bit(int e) { return e ? END_OUT : 0u; }
-
-constexpr int RULER_LDS = 2048; /* rulers staged per block before an append */
-
-/* ruler_mask + 1 = sampling period of the rulers (a power of two).  Marks
- * the rulers (chain ends and sampled nodes) and lists them (LDS-staged
- * appends).  (Whether the chain graph is well formed was counted by
- * k_chain_init, which read every neighbour's record anyway.) */
-__global__ __launch_bounds__(BLOCK) void k_lr_rulers(const LRNode* lr, uint64_t n_chain, uint64_t* ruler,
-                                                     uint64_t ruler_mask, uint32_t* rlist, uint64_t rlist_cap,
-                                                     Counters* ctr) {
-  __shared__ LdsList<RULER_LDS, uint32_t> Lr;
-  if (threadIdx.x == 0) Lr.n = 0;
-  __syncthreads();
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  for (uint64_t base = (uint64_t)blockIdx.x * BLOCK; base < n_chain; base += stride) {
-    const uint64_t t = base + threadIdx.x;
-    bool is_ruler = false;
-    if (t < n_chain) {
-      const LRNode st = lr[t];
-      const bool head = is_terminal(st.d[0]) || is_terminal(st.d[1]);
-      const bool sampled = (fmix64(t * 0x9e3779b97f4a7c15ULL + 0x1234567ULL) & ruler_mask) == 0;
-      is_ruler = head || sampled;
-    }
-    /* the ruler bitmap, one word per wave (a wave covers 64 aligned nodes) */
-    const uint64_t word = __ballot(is_ruler);
-    if ((threadIdx.x & 63) == 0 && t < n_chain) ruler[t >> 6] = word;
-    if (is_ruler) Lr.v[atomicAdd(&Lr.n, 1u)] = (uint32_t)t;
-    /* all threads read the count between two barriers, then keep room for
-     * one more tile */
-    __syncthreads();
-    const uint32_t nr = Lr.n;
-    __syncthreads();
-    if (nr > RULER_LDS - BLOCK) lds_flush(Lr, rlist, rlist_cap, &ctr->lr_next, &ctr->err);
-  }
-  lds_flush(Lr, rlist, rlist_cap, &ctr->lr_next, &ctr->err);
-}
-
-struct WalkRec {
-  uint32_t who;   /* ruler (node walk) or chain end (ruler walk) */
-  uint32_t edist; /* bit 31: end, low 31 bits: distance */
-};
-/* A node walk's record kept in the node's own mailbox word of the end it
- * was entered through (the mailboxes serve only the round-by-round path,
- * which finds them zero): (end | distance) << 32 | ruler number; zero = no
- * walk reached it (a real walk has distance >= 1). */
-__device__ __forceinline__ unsigned long long walk_word(uint32_t rid, uint32_t edist) {
-  return ((unsigned long long)edist << 32) | rid;
-}
-
-/* From every ruler (number rid in the ruler list), along each non-terminal
- * end, to the next ruler.  Each visited node records, in its mailbox of
- * the end it was entered through, the ruler number, the ruler's end the
- * walk left from and the distance: the node's next pointer is read first,
- * so the record goes into a line the walk has just brought in. */
-__global__ __launch_bounds__(BLOCK) void k_lr_walk_nodes(LRNode* lr, const uint64_t* ruler, const uint32_t* rlist,
-                                                         uint64_t n_rulers, WalkRec* link, Counters* ctr) {
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < 2 * n_rulers; i += stride) {
-    const uint32_t rid = (uint32_t)(i >> 1), r = rlist[rid];
-    const int E = (int)(i & 1);
-    if (is_terminal(lr[r].d[E])) continue;
-    uint32_t ptr = lr[r].p[E];
-    uint32_t dist = 0;
-    for (;;) {
-      const uint32_t j = ptr & IDX_MASK;
-      const int e = (ptr & END_OUT) ? 1 : 0;
-      ++dist;
-      if ((ruler[j >> 6] >> (j & 63)) & 1) {
-        link[2 * (uint64_t)r + E] = WalkRec{j, end_bit(e) | dist};
-        break;
-      }
-      ptr = lr[j].p[1 - e];
-      lr[j].mail[e] = walk_word(rid, end_bit(E) | dist);
-      if (dist >= WALK_MAX) {
-        atomicOr(&ctr->err, ERR_WALK);
-        break;
-      }
-    }
-  }
-}
-
-/* Per ruler number and end Er: what lies past the ruler when a walk left
- * it through Er, i.e. through its other end: the ruler itself when that
- * end is terminal (distance 0 more), else the chain end the ruler walk
- * found that way (NONE32: a cycle).  Dense by ruler number, so the finish
- * pass reads one small table instead of two scattered records. */
-__global__ __launch_bounds__(BLOCK) void k_lr_ruler_ends(const LRNode* lr, const uint32_t* rlist, uint64_t n_rulers,
-                                                         const WalkRec* info, WalkRec* rend) {
-  const uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (i >= 2 * n_rulers) return;
-  const uint32_t r = rlist[i >> 1];
-  const int Er = (int)(i & 1);
-  rend[i] = is_terminal(lr[r].d[1 - Er]) ? WalkRec{r, end_bit(Er)} : info[2 * (uint64_t)r + (1 - Er)];
-}
-
-/* The mailboxes back to empty, for the round-by-round path after a walk
- * that ran past its bound. */
-__global__ __launch_bounds__(BLOCK) void k_lr_zero_mail(LRNode* lr, uint64_t n_chain) {
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  for (uint64_t t = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; t < n_chain; t += stride) {
-    lr[t].mail[0] = 0ULL;
-    lr[t].mail[1] = 0ULL;
-  }
-}
-
-__global__ __launch_bounds__(BLOCK) void k_lr_list_heads(const LRNode* lr, const uint32_t* rlist, uint64_t n_rulers,
-                                                         uint32_t* heads, Counters* ctr) {
-  __shared__ ReserveSmem sm;
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  for (uint64_t base = (uint64_t)blockIdx.x * BLOCK; base < 2 * n_rulers; base += stride) {
-    const uint64_t i = base + threadIdx.x;
-    bool h = false;
-    uint32_t r = 0;
-    int E = (int)(i & 1);
-    if (i < 2 * n_rulers) {
-      r = rlist[i >> 1];
-      /* a head end: this end leads into the chain, the other is terminal */
-      h = !is_terminal(lr[r].d[E]) && is_terminal(lr[r].d[1 - E]);
-    }
-    unsigned long long pos = block_reserve(h, &ctr->lr_next, sm);
-    if (h) heads[pos] = r | end_bit(E);
-  }
-}
-
-/* From every head along the ruler graph: each ruler learns, for the end
- * facing the head, which chain end lies that way and how far. */
-__global__ __launch_bounds__(BLOCK) void k_lr_walk_rulers(const LRNode* lr, const WalkRec* link, const uint32_t* heads,
-                                                          uint64_t n_heads, uint64_t n_rulers, WalkRec* info,
-                                                          Counters* ctr) {
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n_heads; i += stride) {
-    const uint32_t h = heads[i] & IDX_MASK;
-    const int E = (heads[i] & END_OUT) ? 1 : 0;
-    uint32_t cur = h;
-    int leave = E;
-    uint32_t D = 0;
-    uint64_t steps = 0;
-    for (;;) {
-      WalkRec l = link[2 * (uint64_t)cur + leave];
-      if (l.who == NONE32) {
-        atomicOr(&ctr->err, ERR_WALK);
-        break;
-      }
-      uint32_t r = l.who;
-      int e = (l.edist & END_OUT) ? 1 : 0;
-      D += l.edist & DIST_MASK;
-      /* from r through e lies head h, entered through its end E */
-      info[2 * (uint64_t)r + e] = WalkRec{h, end_bit(E) | D};
-      if (is_terminal(lr[r].d[1 - e])) {
-        info[2 * (uint64_t)h + E] = WalkRec{r, end_bit(e) | D};
-        break;
-      }
-      if (++steps > n_rulers) {
-        atomicOr(&ctr->err, ERR_WALK);
-        break;
-      }
-      cur = r;
-      leave = 1 - e;
-    }
-  }
-}
-
-__device__ __forceinline__ uint32_t ceil_log2(uint32_t L) { return L <= 1 ? 0 : 32 - __clz(L - 1); }
-
-/* Final state of every chain node; cycle nodes get both distances 2^T
- * (written in a second pass once T is known). */
-/* jT[job]: largest ceil(log2 L) over the job's paths; jcyc[job] = 1 when
- * the job has a cycle. */
-__global__ __launch_bounds__(BLOCK) void k_lr_finish(LRNode* lr, uint64_t n_chain, const uint64_t* ruler,
-                                                     const WalkRec* rend, const WalkRec* info, uint8_t* cyc,
-                                                     const uint32_t* cjob, uint32_t n_jobs, uint32_t* jT,
-                                                     uint32_t* jcyc, Counters* ctr) {
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  unsigned long long ncyc = 0, maxr = 0;
-  for (uint64_t t = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; t < n_chain; t += stride) {
-    LRNode st = lr[t];
-    bool is_cycle = false;
-    uint32_t np[2], nd[2];
-    for (int E = 0; E < 2; ++E) {
-      np[E] = st.p[E];
-      nd[E] = st.d[E];
-      if (is_terminal(st.d[E])) continue;
-      uint32_t Z, f, D;
-      if ((ruler[t >> 6] >> (t & 63)) & 1) {
-        WalkRec w = info[2 * t + E];
-        if (w.who == NONE32) {
-          is_cycle = true;
-          break;
-        }
-        Z = w.who;
-        f = w.edist & END_OUT;
-        D = w.edist & DIST_MASK;
-      } else {
-        /* the walk that reached this end: ruler number, its end, distance */
-        const uint32_t rid = (uint32_t)st.mail[E], edist = (uint32_t)(st.mail[E] >> 32);
-        const uint32_t d = edist & DIST_MASK;
-        if (d == 0) {
-          is_cycle = true;
-          break;
-        }
-        /* continue past that ruler, leaving through its other end */
-        const WalkRec v = rend[2 * (uint64_t)rid + ((edist & END_OUT) ? 1 : 0)];
-        if (v.who == NONE32) {
-          is_cycle = true;
-          break;
-        }
-        Z = v.who;
-        f = v.edist & END_OUT;
-        D = d + (v.edist & DIST_MASK);
-      }
-      np[E] = Z | f;
-      nd[E] = D | TERM_MASK;
-    }
-    const uint32_t job = n_jobs > 1 ? cjob[t] : 0u;
-    if (is_cycle) {
-      cyc[t] = 1;
-      ++ncyc;
-      if (!jcyc[job]) jcyc[job] = 1;
-      continue;
-    }
-    cyc[t] = 0;
-    /* path length from a head's point of view: L = 1 + dist to the far end */
-    if (is_terminal(st.d[0]) != is_terminal(st.d[1])) {
-      uint32_t L = 1 + cdist(is_terminal(st.d[0]) ? nd[1] : nd[0]);
-      uint32_t R = ceil_log2(L);
-      if (R > maxr) maxr = R;
-      if (n_jobs > 1 && R > jT[job]) atomicMax(&jT[job], R);
-    }
-    st.p[0] = np[0];
-    st.p[1] = np[1];
-    st.d[0] = nd[0];
-    st.d[1] = nd[1];
-    lr[t] = st;
-  }
-  block_add(ncyc, &ctr->lr_cycle);
-  typedef hipcub::BlockReduce<unsigned long long, BLOCK> BR;
-  __shared__ typename BR::TempStorage tmp;
-  __syncthreads();
-  unsigned long long m = BR(tmp).Reduce(maxr, hipcub::Max());
-  if (n_jobs == 1 && threadIdx.x == 0 && m) atomicMax(&jT[0], (uint32_t)m);
-}
-
-/* cycle nodes end with both distances 2^T of their job: jcm[job] */
-__global__ __launch_bounds__(BLOCK) void k_lr_cycles(LRNode* lr, uint64_t n_chain, const uint8_t* cyc,
-                                                     const uint32_t* cjob, uint32_t n_jobs, const uint32_t* jcm) {
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  for (uint64_t t = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; t < n_chain; t += stride)
-    if (cyc[t]) {
-      const uint32_t maxd = jcm[n_jobs > 1 ? cjob[t] : 0u];
-      lr[t].d[0] = maxd;
-      lr[t].d[1] = maxd;
-    }
-}
-
 /* separate_cycles (when unfinished nodes remain) and separate_isolated.
  * jcm[job] = 2^T of the job when its cycles are separated, else 0 (2^T >= 2
  * whenever cycles are separated).  jsep[2 * job + {0, 1}] counts cycle and
@@ -975,14 +722,12 @@ __device__ __forceinline__ KT ptr_kmer(const kops<KT>& ops, uint32_t ptr, const 
 template <typename KT>
 struct RankedRec {
   KT k, rep;
-  uint32_t dist, head, len, job;
+  uint32_t dist, job;
 };
 
 /* to_listranked_chain_node (debruijn_chain_operations.hpp:261-310) for
  * chain node i: the node on the rep's strand, the rep (the smaller end
- * k-mer), the distance from the rep end, plus the chain node at the rep end
- * (NONE32 when that end is not a chain node) and 1 + the distance to the
- * far end (the chain's length when the node is the head). */
+ * k-mer), the distance from the rep end. */
 template <typename KT>
 __device__ __forceinline__ RankedRec<KT> ranked_one(const kops<KT>& ops, const LRNode* lr, const KT* ckmer,
                                                     uint64_t n_chain, const KT* vkmer, uint64_t i) {
@@ -996,21 +741,19 @@ __device__ __forceinline__ RankedRec<KT> ranked_one(const kops<KT>& ops, const L
   r.rep = sense ? L : R;
   const int rs = sense ? 0 : 1;
   r.dist = cdist(st.d[rs]);
-  const uint32_t z = st.p[rs] & IDX_MASK;
-  r.head = is_terminal(st.d[rs]) ? (uint32_t)i : (z < n_chain ? z : NONE32);
-  r.len = cdist(st.d[1 - rs]) + 1;
   return r;
 }
 
 /* Every alive chain node, compacted; RANKED_ITEMS nodes per thread share one
- * output reservation (one global atomic per block tile).  out_job,
- * out_head and out_len are optional. */
+ * output reservation (one global atomic per block tile).  out_job is
+ * optional.  (After the round-by-round ranking; the contraction places its
+ * nodes by k_place, chains.h.) */
 constexpr int RANKED_ITEMS = 4;
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_ranked(const LRNode* lr, const KT* ckmer, uint64_t n_chain, const KT* vkmer,
                                                   const uint8_t* alive, int K, const uint32_t* cjob, KT* out_k,
                                                   KT* out_rep, uint32_t* out_dist, uint32_t* out_job,
-                                                  uint32_t* out_head, uint32_t* out_len, Counters* ctr) {
+                                                  Counters* ctr) {
   __shared__ ReserveSmem sm;
   kops<KT> ops(K);
   const uint64_t tile = (uint64_t)BLOCK * RANKED_ITEMS;
@@ -1036,126 +779,9 @@ __global__ __launch_bounds__(BLOCK) void k_ranked(const LRNode* lr, const KT* ck
         out_rep[pos] = r[q].rep;
         out_dist[pos] = r[q].dist;
         if (out_job) out_job[pos] = r[q].job;
-        if (out_head) {
-          out_head[pos] = r[q].head;
-          out_len[pos] = r[q].len;
-        }
         ++pos;
       }
   }
-}
-
-/* positions of the chain heads (dist 0) among the listranked nodes;
- * HEAD_ITEMS positions per thread share one reservation */
-constexpr int HEAD_ITEMS = 16;
-__global__ __launch_bounds__(BLOCK) void k_list_heads_out(const uint32_t* out_dist, uint64_t n, uint32_t* heads,
-                                                          Counters* ctr) {
-  __shared__ ReserveSmem sm;
-  const uint64_t tile = (uint64_t)BLOCK * HEAD_ITEMS;
-  for (uint64_t base = (uint64_t)blockIdx.x * tile; base < n; base += (uint64_t)gridDim.x * tile) {
-    uint32_t hm = 0, m = 0;
-#pragma unroll
-    for (int q = 0; q < HEAD_ITEMS; ++q) {
-      const uint64_t p = base + (uint64_t)q * BLOCK + threadIdx.x;
-      const bool h = p < n && out_dist[p] == 0;
-      hm |= (uint32_t)h << q;
-      m += h;
-    }
-    unsigned long long at = block_reserve(m, &ctr->n_cand, sm);
-#pragma unroll
-    for (int q = 0; q < HEAD_ITEMS; ++q)
-      if (hm >> q & 1u) heads[at++] = (uint32_t)(base + (uint64_t)q * BLOCK + threadIdx.x);
-  }
-}
-
-/* per chain, by the node at its rep end */
-template <typename KT>
-struct HeadMeta {
-  KT rep;
-  uint32_t off, len, job, pad;
-};
-
-/* for the heads in (job, rep) order (hs[r] = position of the r-th head):
- * each chain's range [coff[r], coff[r] + len) and key, stored by head
- * node; two heads with one key count as bad */
-template <typename KT>
-__global__ void k_head_meta(const uint32_t* hs, const uint64_t* coff, const uint32_t* out_head,
-                            const uint32_t* out_len, const KT* out_rep, const uint32_t* out_job, uint64_t nh,
-                            uint64_t n_chain, HeadMeta<KT>* meta, unsigned long long* bad) {
-  const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nh) return;
-  const uint32_t p = hs[r];
-  const uint32_t node = out_head[p];
-  const uint32_t job = out_job ? out_job[p] : 0u;
-  const KT rep = out_rep[p];
-  bool ok = node < n_chain;
-  if (r > 0) {
-    const uint32_t q = hs[r - 1];
-    ok = ok && !(out_rep[q] == rep && (out_job ? out_job[q] : 0u) == job);
-  }
-  if (!ok) {
-    atomicAdd(bad, 1ULL);
-    return;
-  }
-  HeadMeta<KT> m;
-  m.rep = rep;
-  m.off = (uint32_t)coff[r];
-  m.len = out_len[p];
-  m.job = job;
-  m.pad = 0;
-  meta[node] = m;
-}
-
-__global__ void k_take_len(const uint32_t* hs, const uint32_t* out_len, uint64_t nh, uint64_t* len) {
-  const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < nh) len[r] = out_len[hs[r]];
-}
-
-/* A listranked node at its place in output order: its k-mer (K on the
- * rep strand), its index among the listranked nodes and its distance. */
-template <typename KT>
-struct SortedRec {
-  KT k;
-  uint32_t p, dist;
-};
-
-/* every node to its chain's offset + its dist, as one record (its k-mer,
- * index and dist), so the output order's arrays and the FASTA writer read
- * in sequence; bad counts nodes whose head is missing, whose key differs
- * from the head's, or whose dist is past the chain's end (meta.len is 0
- * for a node that heads no chain) */
-template <typename KT>
-__global__ void k_scatter_ranked(const uint32_t* out_head, const uint32_t* out_dist, const KT* out_rep, const KT* out_k,
-                                 const uint32_t* out_job, uint64_t n, uint64_t n_chain, const HeadMeta<KT>* meta,
-                                 SortedRec<KT>* sr, unsigned long long* bad) {
-  const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const uint32_t h = out_head[p];
-  bool ok = h < n_chain;
-  if (ok) {
-    const HeadMeta<KT> m = meta[h];
-    const uint32_t d = out_dist[p];
-    const uint64_t pos = (uint64_t)m.off + d;
-    ok = d < m.len && pos < n && m.rep == out_rep[p] && m.job == (out_job ? out_job[p] : 0u);
-    if (ok) sr[pos] = SortedRec<KT>{out_k[p], (uint32_t)p, d};
-  }
-  if (!ok) atomicAdd(bad, 1ULL);
-}
-
-/* perm and the sorted distances from the placed records; positions no node
- * was placed at (the records are pre-filled with ones) count as bad */
-template <typename KT>
-__global__ __launch_bounds__(BLOCK) void k_sorted_split(const SortedRec<KT>* sr, uint64_t n, uint32_t* perm,
-                                                        uint32_t* dist_sorted, unsigned long long* bad) {
-  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
-  uint32_t holes = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += stride) {
-    const SortedRec<KT> r = sr[i];
-    perm[i] = r.p;
-    dist_sorted[i] = r.dist;
-    holes += r.p == ~0u;
-  }
-  if (holes) atomicAdd(bad, (unsigned long long)holes);
 }
 
 template <typename KT>
@@ -1208,29 +834,9 @@ __global__ void k_fasta_len(const uint32_t* dist_sorted, uint64_t n, int K, uint
   if (i < n) len[i] = dist_sorted[i] == 0 ? (uint64_t)(2 * K + 3) : 1ULL;
 }
 
-/* print_chain_as_fasta (debruijn_chain_operations.hpp:352-385): a node at
- * dist 0 starts a record "\n>" canonical(K) "\n" rep; every other node adds
- * the last base of K (its k-mer on the rep strand).  From the records in
- * output order (sr, after placement by chains) or through perm. */
-template <typename KT>
-__global__ void k_fasta_write_sorted(const SortedRec<KT>* sr, const KT* out_rep, const uint64_t* off, uint64_t n,
-                                     int K, char* buf) {
-  kops<KT> ops(K);
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const SortedRec<KT> r = sr[i];
-  char* o = buf + off[i];
-  if (r.dist == 0) {
-    o[0] = '\n';
-    o[1] = '>';
-    write_kmer<KT>(o + 2, ops.canon(r.k), K);
-    o[2 + K] = '\n';
-    write_kmer<KT>(o + 3 + K, out_rep[r.p], K);
-  } else {
-    const char A[4] = {'A', 'C', 'G', 'T'};
-    o[0] = A[(int)(r.k & 3)];
-  }
-}
+/* print_chain_as_fasta (debruijn_chain_operations.hpp:352-385) of sorted
+ * nodes: a node at dist 0 starts a record "\n>" canonical(K) "\n" rep;
+ * every other node adds the last base of K (its k-mer on the rep strand). */
 template <typename KT>
 __global__ void k_fasta_write(const uint32_t* perm, const KT* out_k, const KT* out_rep, const uint32_t* dist_sorted,
                               const uint64_t* off, uint64_t n, int K, char* buf) {
@@ -1418,17 +1024,16 @@ __global__ void k_get_nodes(const Slot<KT>* T, const uint64_t* present, uint64_t
 }
 
 template <typename KT>
-__global__ void k_get_chain_nodes(const uint32_t* perm, const KT* out_k, const KT* out_rep, const uint32_t* dist_sorted,
-                                  uint64_t n, bruno_chain_node* out) {
+__global__ void k_get_chain_nodes(OutView<KT> v, uint64_t c0, uint64_t n, bruno_chain_node* out) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  uint32_t m = perm[i];
+  const KT k = v.kmer(c0 + i), rep = v.rep_of(c0 + i);
   bruno_chain_node c;
-  c.k[0] = (uint64_t)out_k[m];
-  c.k[1] = (uint64_t)((u128)out_k[m] >> 64);
-  c.rep[0] = (uint64_t)out_rep[m];
-  c.rep[1] = (uint64_t)((u128)out_rep[m] >> 64);
-  c.dist = (int32_t)dist_sorted[i];
+  c.k[0] = (uint64_t)k;
+  c.k[1] = (uint64_t)((u128)k >> 64);
+  c.rep[0] = (uint64_t)rep;
+  c.rep[1] = (uint64_t)((u128)rep >> 64);
+  c.dist = (int32_t)v.dist_of(c0 + i);
   c.pad = 0;
   out[i] = c;
 }
@@ -1467,9 +1072,8 @@ __global__ void k_branch_nodes(const Slot<KT>* T, uint64_t tbase, uint64_t tcap,
  * the k-mer is the reverse strand of its canonical form. */
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_chain_edges(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, uint32_t rbits,
-                                                       int K, const uint32_t* perm, const KT* out_k,
-                                                       const uint32_t* starts, uint64_t n_unitigs,
-                                                       bruno_chain_edge* out, Counters* ctr) {
+                                                       int K, OutView<KT> v, uint64_t c0, const uint32_t* starts,
+                                                       uint64_t n_unitigs, bruno_chain_edge* out, Counters* ctr) {
   kops<KT> ops(K);
   const int lane = threadIdx.x & 63;
   const uint64_t wave = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
@@ -1479,7 +1083,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_edges(const Slot<KT>* T, uint64
     uint64_t sum = 0;
     uint32_t mn = 65535, mx = 0, missing = 0;
     for (uint32_t p = b + lane; p < e; p += 64) {
-      const NodeRec* r = node_rec<KT>(T, tbase, tcap, rbits, ops.canon(out_k[perm[p]]));
+      const NodeRec* r = node_rec<KT>(T, tbase, tcap, rbits, ops.canon(v.kmer(c0 + p)));
       const uint32_t c = r ? r->c[8] : 0;
       missing |= r == nullptr;
       sum += c;
@@ -1494,7 +1098,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_edges(const Slot<KT>* T, uint64
       missing |= __shfl_xor(missing, off);
     }
     if (lane == 0) {
-      const KT L = out_k[perm[b]], R = out_k[perm[e - 1]];
+      const KT L = v.kmer(c0 + b), R = v.kmer(c0 + e - 1);
       const KT cL = ops.canon(L), cR = ops.canon(R);
       const NodeRec* rl = node_rec<KT>(T, tbase, tcap, rbits, cL);
       const NodeRec* rr = node_rec<KT>(T, tbase, tcap, rbits, cR);
@@ -1690,11 +1294,18 @@ struct bruno_job {
   LRNode* lr = nullptr;
   uint32_t* list[2] = {nullptr, nullptr};
   uint8_t* alive = nullptr;
+  /* rulers of the list ranking (chains.h), marked by the chain extraction,
+   * and the contracted list's state */
+  uint64_t* ruler_bits = nullptr;
+  uint32_t *ruler_base = nullptr, *ruler_node = nullptr;
+  uint64_t n_rulers = 0;
+  uint64_t* lstate = nullptr;
   uint64_t vcap = 0;
   uint32_t iterations = 0;
   uint64_t n_cycle = 0, n_isolated = 0, conflicts = 0;
   bool lr_contracted = false; /* ranked by the contraction path (well-formed chains) */
   bool out_by_chains = false; /* unitig order placed from chain offsets, not sorted */
+  uint64_t n_units = 0, n_unit_nodes = 0; /* paths and their nodes (contraction) */
 
   /* output */
   uint64_t n_out = 0, n_unitigs = 0;
@@ -1703,6 +1314,12 @@ struct bruno_job {
   uint32_t* out_dist = nullptr;
   uint32_t* perm = nullptr;
   uint32_t* dist_sorted = nullptr;
+  /* placed by paths (out_by_chains): out_k is in output order; per node its
+   * path, per path its first place (coff[n_units] = n_out) and its
+   * representative, per job its first path */
+  uint32_t *uid = nullptr, *coff = nullptr;
+  void* urep = nullptr;
+  std::vector<uint64_t> unit_start;
   char* fasta = nullptr;
   uint64_t fasta_len = 0;
   void* bsorted = nullptr;
@@ -1802,6 +1419,24 @@ void fill64(bruno_job* j, void* p, uint64_t n_words, uint64_t v, hipStream_t st)
                      v);
 }
 void fill64(bruno_job* j, void* p, uint64_t n_words, uint64_t v) { fill64(j, p, n_words, v, j->stream); }
+
+/* the ranking's and the placed output's arrays are gone */
+void forget_ranking(bruno_job* j) {
+  j->ruler_bits = nullptr;
+  j->ruler_base = j->ruler_node = nullptr;
+  j->n_rulers = 0;
+  j->lstate = nullptr;
+  j->n_units = j->n_unit_nodes = 0;
+  j->uid = j->coff = nullptr;
+  j->urep = nullptr;
+  j->unit_start.clear();
+}
+
+template <typename KT>
+OutView<KT> out_view(const bruno_job* j) {
+  return OutView<KT>{(const KT*)j->out_k, j->uid,  j->coff,     (const KT*)j->urep,
+                     j->perm,             (const KT*)j->out_rep, j->dist_sorted};
+}
 
 size_t slot_bytes(const bruno_job* j) { return j->words == 1 ? sizeof(Slot<uint64_t>) : sizeof(Slot<u128>); }
 
@@ -2583,6 +2218,17 @@ bruno_status filter_t(bruno_job* j) {
   return BRUNO_OK;
 }
 
+/* One sampled ruler per this many chain nodes, at most the tuning knob's
+ * period.  A small graph's ranking lasts as long as its longest walk (period
+ * x ln(rulers) dependent reads), a large one's as its reads in all, to
+ * which denser rulers add.  List ranking + output, ms, by period 8 / 16 / 32
+ * / 64: 1 M nodes 0.45 / 0.50 / 0.61 / 0.94, 4.7 M 1.18 / 1.11 / 1.19 / 1.32,
+ * 10 M (k = 63) 1.96 / 1.82 / 1.91 / 2.15, 40 M 6.46 / 5.60 / 5.42 / 5.70. */
+uint64_t ruler_period(uint64_t n_chain) {
+  const uint64_t p = n_chain <= (1ULL << 21) ? 8 : n_chain <= (1ULL << 24) ? 16 : 32;
+  return std::min<uint64_t>(p, tuning().ruler_sample);
+}
+
 template <typename KT>
 bruno_status chains_t(bruno_job* j) {
   uint64_t nc = j->n_chain;
@@ -2591,15 +2237,26 @@ bruno_status chains_t(bruno_job* j) {
   TRY(dev_alloc(j, &j->vkmer, j->vcap * sizeof(KT)));
   TRY(dev_alloc(j, &j->bkmer, std::max<uint64_t>(1, j->n_branch) * sizeof(KT)));
   TRY(dev_alloc(j, (void**)&j->lr, std::max<uint64_t>(1, nc) * sizeof(LRNode)));
+  const uint64_t n_words = (nc + 63) / 64;
+  TRY(dev_alloc(j, (void**)&j->alive, std::max<uint64_t>(1, nc)));
+  TRY(dev_alloc(j, (void**)&j->ruler_bits, std::max<uint64_t>(1, n_words) * 8));
+  TRY(dev_alloc(j, (void**)&j->ruler_base, std::max<uint64_t>(1, n_words) * 4));
+  TRY(dev_alloc(j, (void**)&j->ruler_node, std::max<uint64_t>(1, nc) * 4));
   HIP_CHECK(hipMemsetAsync(&j->ctr->lr_ill, 0, sizeof(unsigned long long), j->stream));
+  HIP_CHECK(hipMemsetAsync(&j->ctr->lr_next, 0, sizeof(unsigned long long), j->stream));
   hipLaunchKernelGGL((k_chain_init<KT>), dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, (const Slot<KT>*)j->table,
                      probe_span(j), j->rbits, j->K, j->chain_slot, j->chain_job, j->d_seg, j->n_jobs, nc,
-                     (KT*)j->ckmer, j->cedge, j->lr, (KT*)j->vkmer, j->vcap, j->ctr);
+                     (KT*)j->ckmer, j->cedge, j->lr, (KT*)j->vkmer, j->vcap, ruler_period(nc) - 1, j->ruler_bits,
+                     j->alive, j->ctr);
+  if (nc)
+    hipLaunchKernelGGL(k_ruler_list, dim3(grid_for(n_words)), dim3(BLOCK), 0, j->stream, j->ruler_bits, n_words,
+                       j->ruler_base, j->ruler_node, j->ctr);
   hipLaunchKernelGGL((k_termini<KT>), dim3(grid_for(j->n_branch)), dim3(BLOCK), 0, j->stream,
                      (const Slot<KT>*)j->table, probe_span(j), j->rbits, j->K, j->branch_slot, j->branch_job,
                      j->d_seg, j->n_jobs, j->n_branch, j->lr, (KT*)j->bkmer);
   TRY(sync_counters(j));
   j->n_virt = j->hctr->n_virt;
+  j->n_rulers = j->hctr->lr_next;
   if (nc + j->n_virt >= (1ULL << 31)) return BRUNO_CAPACITY;
   return BRUNO_OK;
 }
@@ -2637,112 +2294,88 @@ bruno_status separate(bruno_job* j, const uint32_t* jcm) {
  * ran out) and the caller runs the round-by-round emulation instead. */
 bruno_status list_rank_fast(bruno_job* j, bool* used) {
   *used = false;
-  uint64_t nc = j->n_chain;
+  const uint64_t nc = j->n_chain, nr = j->n_rulers;
   if (nc == 0) return BRUNO_OK;
-  /* ruler flags as a bitmap (n_chain / 8 bytes: small enough to stay in
-   * the device caches for the walks' random tests) */
-  uint64_t* ruler = nullptr;
-  const uint64_t ruler_bytes = (nc + 63) / 64 * 8;
-  uint32_t* rlist = nullptr;
-  uint32_t* heads = nullptr;
-  WalkRec *rend = nullptr, *link = nullptr, *info = nullptr;
   /* k_chain_init counted the ill-formed ends */
-  const bool well_formed = j->hctr->lr_ill == 0;
-  if (!well_formed) return BRUNO_OK;
-  TRY(dev_alloc(j, (void**)&ruler, ruler_bytes));
-  j->hctr->lr_conflict = 0;
-  j->hctr->lr_next = 0;
-  j->hctr->lr_count = 0;
-  j->hctr->lr_cycle = 0;
-  HIP_CHECK(hipMemcpyAsync(&j->ctr->lr_count, &j->hctr->lr_count, 4 * sizeof(unsigned long long),
-                           hipMemcpyHostToDevice, j->stream));
-  TRY(dev_alloc(j, (void**)&rlist, nc * 4));
-  hipLaunchKernelGGL(k_lr_rulers, dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, j->lr, nc, ruler,
-                     (uint64_t)tuning().ruler_sample - 1, rlist, nc, j->ctr);
-  TRY(sync_counters(j));
-  uint64_t nr = j->hctr->lr_next;
-  TRY(dev_alloc(j, (void**)&rend, std::max<uint64_t>(1, nr) * 2 * sizeof(WalkRec)));
-  TRY(dev_alloc(j, (void**)&link, nc * 2 * sizeof(WalkRec)));
-  TRY(dev_alloc(j, (void**)&info, nc * 2 * sizeof(WalkRec)));
-  fill64(j, link, nc * 2, ~0ULL);
-  fill64(j, info, nc * 2, ~0ULL);
-  if (nr)
-    hipLaunchKernelGGL(k_lr_walk_nodes, dim3(grid_for(2 * nr, BLOCK, 1u << 20)), dim3(BLOCK), 0, j->stream, j->lr,
-                       ruler, rlist, nr, link, j->ctr);
-  TRY(dev_alloc(j, (void**)&heads, std::max<uint64_t>(1, 2 * nr) * 4));
-  j->hctr->lr_next = 0;
-  HIP_CHECK(hipMemcpyAsync(&j->ctr->lr_next, &j->hctr->lr_next, sizeof(unsigned long long), hipMemcpyHostToDevice,
-                           j->stream));
-  if (nr)
-    hipLaunchKernelGGL(k_lr_list_heads, dim3(grid_for(2 * nr, BLOCK, 1u << 20)), dim3(BLOCK), 0, j->stream, j->lr,
-                       rlist, nr, heads, j->ctr);
-  /* a walk that ran past its bound leaves the chain state untouched: clear
-   * the flag and let the round-by-round path run */
-  auto walk_failed = [&](bruno_status st, bool* fell_back) -> bruno_status {
-    *fell_back = false;
-    if (j->hctr->err == ERR_WALK) {
-      j->hctr->err = 0;
-      HIP_CHECK(hipMemsetAsync(&j->ctr->err, 0, 4, j->stream));
-      hipLaunchKernelGGL(k_lr_zero_mail, dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, j->lr, nc);
-      HIP_CHECK(hipStreamSynchronize(j->stream));
-      *fell_back = true;
-      return BRUNO_OK;
-    }
-    return st;
-  };
-  bool fell = false;
-  bruno_status s = sync_counters(j);
-  if (s != BRUNO_OK) {
-    s = walk_failed(s, &fell);
-    return s;
-  }
-  uint64_t nh = j->hctr->lr_next;
-  if (nh)
-    hipLaunchKernelGGL(k_lr_walk_rulers, dim3(grid_for(nh)), dim3(BLOCK), 0, j->stream, j->lr, link, heads, nh, nr,
-                       info, j->ctr);
-  s = sync_counters(j);
-  if (s != BRUNO_OK) {
-    s = walk_failed(s, &fell);
-    return s;
-  }
+  if (j->hctr->lr_ill != 0) return BRUNO_OK;
   const uint32_t nj = j->n_jobs;
-  uint8_t* cyc = nullptr;
-  uint32_t* jbuf = nullptr; /* jT[nj], jcyc[nj], jcm[nj] */
-  TRY(dev_alloc(j, (void**)&cyc, nc));
-  TRY(dev_alloc(j, (void**)&jbuf, 3 * nj * sizeof(uint32_t)));
-  HIP_CHECK(hipMemsetAsync(jbuf, 0, 2 * nj * sizeof(uint32_t), j->stream));
-  if (nr)
-    hipLaunchKernelGGL(k_lr_ruler_ends, dim3(grid_for(2 * nr, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, j->lr,
-                       rlist, nr, info, rend);
-  hipLaunchKernelGGL(k_lr_finish, dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, j->lr, nc, ruler, rend, info, cyc,
-                     j->chain_job, nj, jbuf, jbuf + nj, j->ctr);
-  std::vector<uint32_t> hj(3 * nj, 0);
-  HIP_CHECK(hipMemcpyAsync(hj.data(), jbuf, 2 * nj * sizeof(uint32_t), hipMemcpyDeviceToHost, j->stream));
-  TRY(sync_counters(j));
-  const uint64_t ncyc = j->hctr->lr_cycle;
-  /* per job: T = largest ceil(log2 L), at least 1 with a cycle; cycle nodes
-   * end at distance 2^T and are separated */
-  j->job_iters.assign(nj, 0);
-  uint32_t Tmax = 0;
-  for (uint32_t q = 0; q < nj; ++q) {
-    uint32_t T = hj[q];
-    if (hj[nj + q] && T < 1) T = 1;
-    if (T >= 30) return BRUNO_INTERNAL; /* the reference stops at 30 rounds; not reachable below 2^29 nodes */
-    j->job_iters[q] = T;
-    hj[2 * nj + q] = hj[nj + q] ? (1u << T) : 0u;
-    Tmax = std::max(Tmax, T);
+  const uint32_t* cjob = nj > 1 ? j->chain_job : nullptr;
+  const Rulers R{j->ruler_bits, j->ruler_base, j->ruler_node, nr};
+  /* totals, then per job T, isolated and cycle nodes, then the jump
+   * launches' flags */
+  const uint64_t n_tot = LRT_WORDS + 3 * (uint64_t)nj, n_flags = (LR_JUMP_LAUNCHES + 1) / 2;
+  unsigned long long* tot = nullptr;
+  TRY(dev_alloc(j, (void**)&j->lstate, std::max<uint64_t>(1, 2 * nr) * 8));
+  TRY(dev_alloc(j, (void**)&tot, (n_tot + n_flags) * 8));
+  unsigned long long *jT = tot + LRT_WORDS, *jiso = jT + nj, *jcyc = jiso + nj;
+  uint32_t* left = (uint32_t*)(tot + n_tot);
+  fill64(j, tot, n_tot + n_flags, 0);
+  if (nr) {
+    fill64(j, j->lstate, 2 * nr, LS_UNSET);
+    hipLaunchKernelGGL(k_lr_walk, dim3(grid_for(2 * nr)), dim3(BLOCK), 0, j->stream, j->lr, R, j->lstate, j->alive, cjob,
+                       tot, jiso, j->ctr);
+    /* entries covered grow at least by this factor a launch */
+    uint64_t covered = 1;
+    for (int q = 0; q < LR_JUMP_LAUNCHES && covered < 2 * nr; ++q, covered *= LR_JUMPS + 1)
+      hipLaunchKernelGGL(k_lr_jump, dim3(grid_for(2 * nr, BLOCK, 1u << 12)), dim3(BLOCK), 0, j->stream, j->lstate,
+                         2 * nr, q ? left + q - 1 : nullptr, left + q);
+    hipLaunchKernelGGL(k_lr_ends, dim3(grid_for(2 * nr, BLOCK, 2 * device_cus())), dim3(BLOCK), 0, j->stream, j->lr, R,
+                       j->lstate, cjob, tot, jT, j->ctr);
   }
-  uint32_t* jcm = jbuf + 2 * nj;
-  HIP_CHECK(hipMemcpyAsync(jcm, hj.data() + 2 * nj, nj * sizeof(uint32_t), hipMemcpyHostToDevice, j->stream));
-  if (ncyc)
-    hipLaunchKernelGGL(k_lr_cycles, dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, j->lr, nc, cyc, j->chain_job, nj,
-                       jcm);
-  j->iterations = Tmax;
-  j->conflicts = 0;
-  TRY(dev_alloc(j, (void**)&j->alive, nc));
-  TRY(separate(j, jcm));
-  *used = true;
-  return BRUNO_OK;
+  std::vector<unsigned long long> h(n_tot);
+  HIP_CHECK(hipMemcpyAsync(h.data(), tot, n_tot * 8, hipMemcpyDeviceToHost, j->stream));
+  bruno_status s = sync_counters(j);
+  if (j->hctr->err == ERR_WALK) {
+    /* a walk ran past its bound: the chain state is as it was, so clear the
+     * flag and let the round-by-round path run */
+    j->hctr->err = 0;
+    HIP_CHECK(hipMemsetAsync(&j->ctr->err, 0, 4, j->stream));
+    s = BRUNO_OK;
+  } else if (s == BRUNO_OK) {
+    j->n_units = h[LRT_HEADS] / 2 + h[LRT_SINGLES];
+    j->n_unit_nodes = h[LRT_SUM] / 2 + h[LRT_SINGLES];
+    j->n_isolated = h[LRT_ISOLATED];
+    const uint64_t on_paths = j->n_unit_nodes + j->n_isolated;
+    if (on_paths > nc) return BRUNO_INTERNAL;
+    j->n_cycle = nc - on_paths;
+    if (j->n_cycle) {
+      uint8_t* on_path = nullptr;
+      TRY(dev_alloc(j, (void**)&on_path, nc));
+      HIP_CHECK(hipMemsetAsync(on_path, 0, nc, j->stream));
+      hipLaunchKernelGGL(k_lr_mark_paths, dim3(grid_for(std::max<uint64_t>(1, 2 * nr))), dim3(BLOCK), 0, j->stream, j->lr,
+                         R, j->lstate, on_path);
+      hipLaunchKernelGGL(k_lr_drop_cycles, dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, on_path, nc, cjob, j->alive,
+                         jcyc);
+      HIP_CHECK(hipMemcpyAsync(h.data(), tot, n_tot * 8, hipMemcpyDeviceToHost, j->stream));
+      s = sync_counters(j);
+      void* a = on_path;
+      dev_free(j, a, nc);
+    }
+    /* per job: T = largest ceil(log2 L), at least 1 with a cycle (the
+     * reference stops at 30 rounds; not reachable below 2^29 nodes) */
+    j->job_iters.assign(nj, 0);
+    j->job_cycle.assign(nj, 0);
+    j->job_isolated.assign(nj, 0);
+    j->iterations = 0;
+    uint64_t cycles = 0;
+    for (uint32_t q = 0; q < nj; ++q) {
+      const uint64_t cyc = h[LRT_WORDS + 2 * (uint64_t)nj + q];
+      uint32_t T = (uint32_t)h[LRT_WORDS + q];
+      if (cyc && T < 1) T = 1;
+      if (T >= 30) return BRUNO_INTERNAL;
+      j->job_iters[q] = T;
+      j->iterations = std::max(j->iterations, T);
+      j->job_cycle[q] = cyc;
+      j->job_isolated[q] = nj > 1 ? h[LRT_WORDS + nj + q] : j->n_isolated;
+      cycles += cyc;
+    }
+    if (s == BRUNO_OK && cycles != j->n_cycle) s = BRUNO_INTERNAL;
+    j->conflicts = 0;
+    *used = s == BRUNO_OK;
+  }
+  void* a = tot;
+  dev_free(j, a, (n_tot + n_flags) * 8);
+  return s;
 }
 
 bruno_status list_rank_rounds(bruno_job* j, int variant) {
@@ -2751,7 +2384,7 @@ bruno_status list_rank_rounds(bruno_job* j, int variant) {
   const bool batch = nj > 1;
   TRY(dev_alloc(j, (void**)&j->list[0], std::max<uint64_t>(1, nc) * sizeof(uint32_t)));
   TRY(dev_alloc(j, (void**)&j->list[1], std::max<uint64_t>(1, nc) * sizeof(uint32_t)));
-  TRY(dev_alloc(j, (void**)&j->alive, std::max<uint64_t>(1, nc)));
+  if (nc) hipLaunchKernelGGL(k_lr_zero_mail, dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, j->lr, nc);
   /* batch: per-job round counters and active flags */
   unsigned long long* jctr = nullptr;
   uint8_t* active = nullptr;
@@ -2946,111 +2579,109 @@ bruno_status job_bounds(bruno_job* j, const uint32_t* job_of_item, const uint32_
 }
 
 /* chain_rep_less order without sorting every node: after the contraction
- * ranking each chain's nodes carry distances 0..m-1 from its rep end, so
- * only the chain heads are sorted (by job, then rep) and every node goes to
- * its chain's offset + its distance.  The result is the sorted order when
- * no node is rejected and no position stays empty: n nodes then fill n
- * places one each, the chains' keys strictly increase and each chain's
- * nodes sit in dist order.  Otherwise *placed = false and the caller
- * sorts. */
+ * ranking only the paths are sorted (by job, then representative), a prefix
+ * sum of their lengths gives every path's first place, and k_place writes
+ * the nodes to their places; k_path_fasta then writes the records. */
 template <typename KT>
-bruno_status place_by_chains(bruno_job* j, uint64_t n, const uint32_t* out_head, const uint32_t* out_len, bool* placed,
-                             SortedRec<KT>** sr_out) {
-  *placed = false;
-  *sr_out = nullptr;
-  const uint64_t nc = j->n_chain;
+bruno_status place_paths(bruno_job* j) {
   const uint32_t nj = j->n_jobs;
-  j->hctr->n_cand = 0;
-  HIP_CHECK(hipMemcpyAsync(&j->ctr->n_cand, &j->hctr->n_cand, 8, hipMemcpyHostToDevice, j->stream));
-  uint32_t* heads = nullptr;
-  TRY(dev_alloc(j, (void**)&heads, n * 4));
-  hipLaunchKernelGGL(k_list_heads_out, dim3(grid_for((n + HEAD_ITEMS - 1) / HEAD_ITEMS)), dim3(BLOCK), 0, j->stream,
-                     j->out_dist, n, heads, j->ctr);
-  TRY(sync_counters(j));
-  const uint64_t nh = j->hctr->n_cand;
-  void* a = nullptr;
-  if (nh == 0 || nh > n) {
-    a = heads;
-    dev_free(j, a, n * 4);
-    return BRUNO_OK;
-  }
-  const dim3 gh(grid_for(nh, BLOCK, 1u << 30)), gn(grid_for(n, BLOCK, 1u << 30));
-  /* heads in (job, rep) order */
-  KT* hkeys = nullptr;
-  uint32_t *hperm = nullptr, *hs = nullptr, *hjob = nullptr;
-  TRY(dev_alloc(j, (void**)&hkeys, nh * sizeof(KT)));
-  TRY(dev_alloc(j, (void**)&hperm, nh * 4));
-  TRY(dev_alloc(j, (void**)&hs, nh * 4));
-  hipLaunchKernelGGL((k_gather_kmer<KT>), gh, dim3(BLOCK), 0, j->stream, (const KT*)j->out_rep, heads, hkeys, nh);
-  TRY(sort_perm_kmer<KT>(j, hkeys, hperm, nh, j->K, false));
+  const uint64_t nu = j->n_units, n = j->n_unit_nodes, nr = j->n_rulers;
+  const uint32_t* cjob = nj > 1 ? j->chain_job : nullptr;
+  const Rulers R{j->ruler_bits, j->ruler_base, j->ruler_node, nr};
+  j->n_out = n;
+  j->fasta_len = n + nu * (2 * (uint64_t)j->K + 2);
+  j->fasta_off.assign(nj + 1, 0);
+  j->chain_start.assign(nj + 1, 0);
+  j->unit_start.assign(nj + 1, 0);
+  j->fasta_off[nj] = j->fasta_len;
+  j->chain_start[nj] = n;
+  j->unit_start[nj] = nu;
+  TRY(dev_alloc(j, &j->out_k, std::max<uint64_t>(1, n) * sizeof(KT)));
+  TRY(dev_alloc(j, (void**)&j->uid, std::max<uint64_t>(1, n) * 4));
+  TRY(dev_alloc(j, (void**)&j->coff, (nu + 1) * 4));
+  TRY(dev_alloc(j, &j->urep, std::max<uint64_t>(1, nu) * sizeof(KT)));
+  TRY(dev_alloc(j, (void**)&j->fasta, j->fasta_len + 1));
+  if (nu == 0) return BRUNO_OK;
+  KT* key = nullptr;
+  uint32_t *len = nullptr, *entry = nullptr, *job = nullptr, *perm = nullptr, *ulen = nullptr, *ujob = nullptr,
+           *unit_of = nullptr;
+  unsigned long long* tot = nullptr;
+  TRY(dev_alloc(j, (void**)&key, nu * sizeof(KT)));
+  TRY(dev_alloc(j, (void**)&len, nu * 4));
+  TRY(dev_alloc(j, (void**)&entry, nu * 4));
+  TRY(dev_alloc(j, (void**)&perm, nu * 4));
+  TRY(dev_alloc(j, (void**)&ulen, (nu + 1) * 4));
+  TRY(dev_alloc(j, (void**)&unit_of, 2 * nr * 4));
+  TRY(dev_alloc(j, (void**)&tot, LRT_WORDS * 8));
   if (nj > 1) {
-    TRY(dev_alloc(j, (void**)&hjob, nh * 4));
-    hipLaunchKernelGGL(k_gather_u32, gh, dim3(BLOCK), 0, j->stream, j->out_job, heads, hjob, nh);
-    TRY(sort_perm_u32(j, hjob, hperm, nh, job_bits(nj)));
+    TRY(dev_alloc(j, (void**)&job, nu * 4));
+    TRY(dev_alloc(j, (void**)&ujob, nu * 4));
   }
-  hipLaunchKernelGGL(k_gather_u32, gh, dim3(BLOCK), 0, j->stream, heads, hperm, hs, nh);
-  /* chain offsets in that order */
-  uint64_t *hl = nullptr, *coff = nullptr;
-  HeadMeta<KT>* meta = nullptr;
-  unsigned long long* bad = nullptr;
-  TRY(dev_alloc(j, (void**)&hl, nh * 8));
-  TRY(dev_alloc(j, (void**)&coff, nh * 8));
-  hipLaunchKernelGGL(k_take_len, gh, dim3(BLOCK), 0, j->stream, hs, out_len, nh, hl);
+  fill64(j, tot, LRT_WORDS, 0);
+  fill64(j, unit_of, nr, ~0ULL);
+  hipLaunchKernelGGL((k_chain_heads<KT>), dim3(grid_for(2 * nr, BLOCK, 1u << 12)), dim3(BLOCK), 0, j->stream, j->lr, R,
+                     j->lstate, j->K, cjob, nu, key, len, entry, job, tot, j->ctr);
+  TRY(sort_perm_kmer<KT>(j, key, perm, nu, j->K, false));
+  if (nj > 1) TRY(sort_perm_u32(j, job, perm, nu, job_bits(nj)));
+  hipLaunchKernelGGL((k_units<KT>), dim3(grid_for(nu + 1, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, perm, key, len,
+                     entry, job, nu, (KT*)j->urep, ulen, ujob, unit_of);
   size_t tmp = 0;
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, hl, coff, (int)nh, j->stream));
   void* t = nullptr;
-  TRY(dev_alloc(j, &t, tmp));
-  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(t, tmp, hl, coff, (int)nh, j->stream));
-  TRY(dev_alloc(j, (void**)&meta, nc * sizeof(HeadMeta<KT>)));
-  TRY(dev_alloc(j, (void**)&bad, 8));
-  /* len 0 marks a node that heads no chain */
-  SortedRec<KT>* sr = nullptr;
-  TRY(dev_alloc(j, (void**)&sr, n * sizeof(SortedRec<KT>)));
-  HIP_CHECK(hipMemsetAsync(meta, 0, nc * sizeof(HeadMeta<KT>), j->stream));
-  HIP_CHECK(hipMemsetAsync(sr, 0xFF, n * sizeof(SortedRec<KT>), j->stream));
-  HIP_CHECK(hipMemsetAsync(bad, 0, 8, j->stream));
-  hipLaunchKernelGGL((k_head_meta<KT>), gh, dim3(BLOCK), 0, j->stream, hs, coff, out_head, out_len,
-                     (const KT*)j->out_rep, j->out_job, nh, nc, meta, bad);
-  hipLaunchKernelGGL((k_scatter_ranked<KT>), gn, dim3(BLOCK), 0, j->stream, out_head, j->out_dist,
-                     (const KT*)j->out_rep, (const KT*)j->out_k, j->out_job, n, nc, meta, sr, bad);
-  hipLaunchKernelGGL((k_sorted_split<KT>), dim3(grid_for(n)), dim3(BLOCK), 0, j->stream, sr, n, j->perm,
-                     j->dist_sorted, bad);
-  unsigned long long hbad = 0;
-  HIP_CHECK(hipMemcpyAsync(&hbad, bad, 8, hipMemcpyDeviceToHost, j->stream));
-  HIP_CHECK(hipStreamSynchronize(j->stream));
-  *placed = hbad == 0;
-  if (*placed) {
-    *sr_out = sr;
-  } else {
-    a = sr;
-    dev_free(j, a, n * sizeof(SortedRec<KT>));
+  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, ulen, j->coff, (int)(nu + 1), j->stream));
+  TRY(dev_alloc(j, &t, std::max<size_t>(1, tmp)));
+  HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(t, tmp, ulen, j->coff, (int)(nu + 1), j->stream));
+  hipLaunchKernelGGL((k_place<KT>), dim3(grid_for(nr)), dim3(BLOCK), 0, j->stream, j->lr, R, j->lstate, unit_of,
+                     j->coff, j->K, (KT*)j->out_k, tot, j->ctr);
+  hipLaunchKernelGGL((k_path_fasta<KT>), dim3(grid_for((n + FASTA_ITEMS - 1) / FASTA_ITEMS)), dim3(BLOCK), 0, j->stream,
+                     (const KT*)j->out_k, j->coff, nu, n, j->K, j->uid, j->fasta);
+  uint64_t *us = nullptr, *cs = nullptr;
+  if (nj > 1) {
+    TRY(dev_alloc(j, (void**)&us, (nj + 1) * 8));
+    TRY(dev_alloc(j, (void**)&cs, (nj + 1) * 8));
+    hipLaunchKernelGGL(k_seg_bounds, dim3(grid_for(nu + 1, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, ujob, nu, nj,
+                       us);
+    hipLaunchKernelGGL(k_unit_starts, dim3(grid_for(nj + 1)), dim3(BLOCK), 0, j->stream, us, nj + 1, j->coff, cs);
+    HIP_CHECK(hipMemcpyAsync(j->unit_start.data(), us, (nj + 1) * 8, hipMemcpyDeviceToHost, j->stream));
+    HIP_CHECK(hipMemcpyAsync(j->chain_start.data(), cs, (nj + 1) * 8, hipMemcpyDeviceToHost, j->stream));
   }
-  a = heads;
-  dev_free(j, a, n * 4);
-  a = hkeys;
-  dev_free(j, a, nh * sizeof(KT));
-  a = hperm;
-  dev_free(j, a, nh * 4);
-  a = hs;
-  dev_free(j, a, nh * 4);
-  if (hjob) {
-    a = hjob;
-    dev_free(j, a, nh * 4);
+  unsigned long long h[LRT_WORDS];
+  HIP_CHECK(hipMemcpyAsync(h, tot, sizeof(h), hipMemcpyDeviceToHost, j->stream));
+  TRY(sync_counters(j));
+  /* every node of every path was placed, one place each */
+  if (h[LRT_UNITS] != nu || h[LRT_PLACED] != n || j->chain_start[nj] != n) return BRUNO_INTERNAL;
+  for (uint32_t q = 0; q <= nj; ++q)
+    j->fasta_off[q] = j->chain_start[q] + j->unit_start[q] * (2 * (uint64_t)j->K + 2);
+  void* a = key;
+  dev_free(j, a, nu * sizeof(KT));
+  a = len;
+  dev_free(j, a, nu * 4);
+  a = entry;
+  dev_free(j, a, nu * 4);
+  a = perm;
+  dev_free(j, a, nu * 4);
+  a = ulen;
+  dev_free(j, a, (nu + 1) * 4);
+  a = unit_of;
+  dev_free(j, a, 2 * nr * 4);
+  a = tot;
+  dev_free(j, a, LRT_WORDS * 8);
+  dev_free(j, t, std::max<size_t>(1, tmp));
+  if (nj > 1) {
+    a = job;
+    dev_free(j, a, nu * 4);
+    a = ujob;
+    dev_free(j, a, nu * 4);
+    a = us;
+    dev_free(j, a, (nj + 1) * 8);
+    a = cs;
+    dev_free(j, a, (nj + 1) * 8);
   }
-  a = hl;
-  dev_free(j, a, nh * 8);
-  a = coff;
-  dev_free(j, a, nh * 8);
-  dev_free(j, t, tmp);
-  a = meta;
-  dev_free(j, a, nc * sizeof(HeadMeta<KT>));
-  a = bad;
-  dev_free(j, a, 8);
   return BRUNO_OK;
 }
 
+/* The output of a round-by-round ranking: every node ranked, then sorted. */
 template <typename KT>
-bruno_status compact_t(bruno_job* j) {
+bruno_status sort_ranked(bruno_job* j) {
   uint64_t nc = j->n_chain;
   int K = j->K;
   TRY(dev_alloc(j, &j->out_k, std::max<uint64_t>(1, nc) * sizeof(KT)));
@@ -3063,25 +2694,17 @@ bruno_status compact_t(bruno_job* j) {
   j->hctr->n_out = 0;
   HIP_CHECK(hipMemcpyAsync(&j->ctr->n_out, &j->hctr->n_out, sizeof(unsigned long long), hipMemcpyHostToDevice,
                            j->stream));
-  uint32_t *out_head = nullptr, *out_len = nullptr;
-  if (j->lr_contracted) {
-    TRY(dev_alloc(j, (void**)&out_head, std::max<uint64_t>(1, nc) * 4));
-    TRY(dev_alloc(j, (void**)&out_len, std::max<uint64_t>(1, nc) * 4));
-  }
   hipLaunchKernelGGL((k_ranked<KT>), dim3(grid_for((nc + RANKED_ITEMS - 1) / RANKED_ITEMS)), dim3(BLOCK), 0,
                      j->stream, j->lr, (const KT*)j->ckmer, nc, (const KT*)j->vkmer, j->alive, K, j->chain_job,
-                     (KT*)j->out_k, (KT*)j->out_rep, j->out_dist, j->out_job, out_head, out_len, j->ctr);
+                     (KT*)j->out_k, (KT*)j->out_rep, j->out_dist, j->out_job, j->ctr);
   TRY(sync_counters(j));
   uint64_t n = j->hctr->n_out;
   j->n_out = n;
   /* chain_rep_less: by rep, then |dist| -> LSD: dist first, then rep words;
    * a batch adds a last pass on the job, so each job's nodes are contiguous */
   j->fasta_off.assign(nj + 1, 0);
-  bool placed = false;
-  SortedRec<KT>* sr = nullptr; /* the nodes in output order, when placed by chains */
-  if (n > 0 && out_head) TRY(place_by_chains<KT>(j, n, out_head, out_len, &placed, &sr));
-  j->out_by_chains = placed;
-  if (n > 0 && !placed) {
+  j->out_by_chains = false;
+  if (n > 0) {
     uint32_t* pin = nullptr;
     TRY(dev_alloc(j, (void**)&pin, n * 4));
     hipLaunchKernelGGL(k_iota, dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, pin, n);
@@ -3103,19 +2726,12 @@ bruno_status compact_t(bruno_job* j) {
     if (nj > 1) TRY(sort_perm_u32(j, j->out_job, j->perm, n, job_bits(nj)));
   }
   void* a = nullptr;
-  if (out_head) {
-    a = out_head;
-    dev_free(j, a, std::max<uint64_t>(1, nc) * 4);
-    a = out_len;
-    dev_free(j, a, std::max<uint64_t>(1, nc) * 4);
-  }
   if (n > 0) {
     void* t = nullptr;
     size_t tmp = 0;
     TRY(job_bounds(j, j->out_job, j->perm, n, j->chain_start));
-    if (!sr)
-      hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, j->out_dist,
-                         j->perm, j->dist_sorted, n);
+    hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, j->out_dist,
+                       j->perm, j->dist_sorted, n);
     /* .chain.fasta */
     uint64_t *len = nullptr, *off = nullptr;
     TRY(dev_alloc(j, (void**)&len, n * 8));
@@ -3132,12 +2748,8 @@ bruno_status compact_t(bruno_job* j) {
     HIP_CHECK(hipStreamSynchronize(j->stream));
     dev_free(j, t, tmp);
     TRY(dev_alloc(j, (void**)&j->fasta, total + 1));
-    if (sr)
-      hipLaunchKernelGGL((k_fasta_write_sorted<KT>), dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
-                         sr, (const KT*)j->out_rep, off, n, K, j->fasta);
-    else
-      hipLaunchKernelGGL((k_fasta_write<KT>), dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, j->perm,
-                         (const KT*)j->out_k, (const KT*)j->out_rep, j->dist_sorted, off, n, K, j->fasta);
+    hipLaunchKernelGGL((k_fasta_write<KT>), dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, j->perm,
+                       (const KT*)j->out_k, (const KT*)j->out_rep, j->dist_sorted, off, n, K, j->fasta);
     j->fasta_len = total;
     /* byte range of each job's records */
     j->fasta_off[nj] = total;
@@ -3158,13 +2770,21 @@ bruno_status compact_t(bruno_job* j) {
     dev_free(j, a, n * 8);
     a = off;
     dev_free(j, a, (n + 1) * 8);
-    a = sr;
-    dev_free(j, a, n * sizeof(SortedRec<KT>));
   } else {
     j->fasta_len = 0;
     j->chain_start.assign(nj + 1, 0);
     TRY(dev_alloc(j, (void**)&j->fasta, 16));
   }
+  return BRUNO_OK;
+}
+
+template <typename KT>
+bruno_status compact_t(bruno_job* j) {
+  const int K = j->K;
+  const uint32_t nj = j->n_jobs;
+  j->out_by_chains = j->lr_contracted && j->n_units > 0;
+  if (j->lr_contracted) TRY(place_paths<KT>(j));
+  else TRY(sort_ranked<KT>(j));
   /* .branch.fasta: sorted branch k-mers */
   uint64_t nb = j->n_branch;
   j->branch_start.assign(nj + 1, 0);
@@ -3329,6 +2949,7 @@ bruno_status bruno_job_reset(bruno_job* j) {
   j->list[0] = j->list[1] = nullptr;
   j->alive = nullptr;
   j->out_dist = j->perm = j->dist_sorted = nullptr;
+  forget_ranking(j);
   j->chain_job = j->branch_job = j->out_job = nullptr;
   j->fasta = j->bfasta = nullptr;
   j->n_present = j->n_branch = j->n_chain = j->n_virt = 0;
@@ -3582,6 +3203,55 @@ bruno_status bruno_compact(bruno_job* j) {
   return BRUNO_OK;
 }
 
+/* Unitig starts of job idx, whose m output nodes begin at c0: starts[u] +
+ * *off is unitig u's first node, starts[nu] + *off the end.  After a placing
+ * by paths the paths' first places; after a sort the dist-0 positions,
+ * selected into *own (m + 1 entries the caller frees) and checked against
+ * the unitig count before anything reads them. */
+static bruno_status unitig_starts(bruno_job* j, uint32_t idx, uint64_t c0, uint64_t m, uint64_t nu, uint32_t** own,
+                                  const uint32_t** starts, uint64_t* off) {
+  *own = nullptr;
+  if (j->uid) {
+    *starts = j->coff + j->unit_start[idx];
+    *off = 0;
+    return nu == j->unit_start[idx + 1] - j->unit_start[idx] ? BRUNO_OK : BRUNO_INTERNAL;
+  }
+  uint8_t* flags = nullptr;
+  uint32_t* n_sel = nullptr;
+  void* t = nullptr;
+  size_t tmp = 0;
+  uint32_t got = 0;
+  const uint32_t mm = (uint32_t)m;
+  hipcub::CountingInputIterator<uint32_t> pos(0);
+  TRY(dev_alloc(j, (void**)own, (m + 1) * 4));
+  bruno_status st = dev_alloc(j, (void**)&flags, m);
+  if (st == BRUNO_OK) st = dev_alloc(j, (void**)&n_sel, 4);
+  if (st == BRUNO_OK) {
+    hipLaunchKernelGGL(k_head_flags, dim3(grid_for(m, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
+                       j->dist_sorted + c0, m, flags);
+    if (hipcub::DeviceSelect::Flagged(nullptr, tmp, pos, flags, *own, n_sel, (int)m, j->stream) != hipSuccess)
+      st = BRUNO_INTERNAL;
+  }
+  if (st == BRUNO_OK) st = dev_alloc(j, &t, std::max<size_t>(tmp, 1));
+  if (st == BRUNO_OK &&
+      (hipcub::DeviceSelect::Flagged(t, tmp, pos, flags, *own, n_sel, (int)m, j->stream) != hipSuccess ||
+       hipMemcpyAsync(&got, n_sel, 4, hipMemcpyDeviceToHost, j->stream) != hipSuccess ||
+       hipStreamSynchronize(j->stream) != hipSuccess || got != nu ||
+       hipMemcpyAsync(*own + nu, &mm, 4, hipMemcpyHostToDevice, j->stream) != hipSuccess ||
+       hipStreamSynchronize(j->stream) != hipSuccess)) {
+    (void)hipGetLastError();
+    st = BRUNO_INTERNAL;
+  }
+  void* a = flags;
+  dev_free(j, a, m);
+  a = n_sel;
+  dev_free(j, a, 4);
+  dev_free(j, t, std::max<size_t>(tmp, 1));
+  *starts = *own;
+  *off = c0;
+  return st;
+}
+
 /* ================================================================== */
 /* graph cleaning (host side)                                           */
 /* ================================================================== */
@@ -3603,6 +3273,7 @@ static void free_after_lists(bruno_job* j) {
   j->list[0] = j->list[1] = nullptr;
   j->alive = nullptr;
   j->out_dist = j->perm = j->dist_sorted = nullptr;
+  forget_ranking(j);
   j->out_job = nullptr;
   j->fasta = j->bfasta = nullptr;
   j->cbits = j->sbits = nullptr;
@@ -3693,35 +3364,20 @@ static bruno_status pick_t(bruno_job* j, uint64_t min_freq, EdgeQuery<KT>** dq, 
   const uint64_t n = j->n_out, nu = j->n_unitigs;
   if (nu == 0) return BRUNO_OK;
   const uint64_t tcap = probe_span(j); /* plain jobs: one probe window per k-mer over the table */
-  uint8_t* flags = nullptr;
   uint32_t* starts = nullptr;
+  const uint32_t* st0 = nullptr;
+  uint64_t off = 0;
   ChainSummary<KT>*S = nullptr, *N = nullptr;
   unsigned long long* cnt = nullptr;
-  void* t = nullptr;
-  size_t tmp = 0;
-  hipcub::CountingInputIterator<uint32_t> pos(0);
-  TRY(dev_alloc(j, (void**)&flags, n));
-  TRY(dev_alloc(j, (void**)&starts, (n + 1) * 4)); /* room for every node: checked against nu below */
+  TRY(unitig_starts(j, 0, 0, n, nu, &starts, &st0, &off));
   TRY(dev_alloc(j, (void**)&cnt, 4 * sizeof(unsigned long long)));
   TRY(dev_alloc(j, (void**)&S, nu * sizeof(ChainSummary<KT>)));
   TRY(dev_alloc(j, (void**)&N, nu * sizeof(ChainSummary<KT>)));
   TRY(dev_alloc(j, (void**)dq, nu * sizeof(EdgeQuery<KT>)));
   *dq_bytes = nu * sizeof(EdgeQuery<KT>);
   HIP_CHECK(hipMemsetAsync(cnt, 0, 4 * sizeof(unsigned long long), j->stream));
-  hipLaunchKernelGGL(k_head_flags, dim3(grid_for(n, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, j->dist_sorted, n,
-                     flags);
-  HIP_CHECK(hipcub::DeviceSelect::Flagged(nullptr, tmp, pos, flags, starts, (uint32_t*)(cnt + 3), (int)n, j->stream));
-  TRY(dev_alloc(j, &t, std::max<size_t>(tmp, 1)));
-  HIP_CHECK(hipcub::DeviceSelect::Flagged(t, tmp, pos, flags, starts, (uint32_t*)(cnt + 3), (int)n, j->stream));
-  uint32_t heads = 0;
-  HIP_CHECK(hipMemcpyAsync(&heads, cnt + 3, 4, hipMemcpyDeviceToHost, j->stream));
-  HIP_CHECK(hipStreamSynchronize(j->stream));
-  if (heads != nu) return BRUNO_INTERNAL; /* one dist-0 node per unitig */
-  const uint32_t n32 = (uint32_t)n;
-  HIP_CHECK(hipMemcpyAsync(starts + nu, &n32, 4, hipMemcpyHostToDevice, j->stream));
   hipLaunchKernelGGL((k_chain_summaries<KT>), dim3(grid_for(nu)), dim3(BLOCK), 0, j->stream,
-                     (const Slot<KT>*)j->table, tcap, j->rbits, j->K, j->perm, (const KT*)j->out_k, j->dist_sorted,
-                     starts, nu, S, j->ctr);
+                     (const Slot<KT>*)j->table, tcap, j->rbits, j->K, out_view<KT>(j), st0, nu, S, j->ctr);
   hipLaunchKernelGGL((k_pick_chains<KT>), dim3(grid_for(nu)), dim3(BLOCK), 0, j->stream, S, nu, j->K, min_freq, *dq,
                      cnt, nu, N, cnt + 1, j->ctr);
   unsigned long long h[4];
@@ -3768,9 +3424,7 @@ static bruno_status pick_t(bruno_job* j, uint64_t min_freq, EdgeQuery<KT>** dq, 
     dev_free(j, a, nn * 4);
   }
   if (j->hctr->err) return BRUNO_INTERNAL;
-  void* a = flags;
-  dev_free(j, a, n);
-  a = starts;
+  void* a = starts;
   dev_free(j, a, (n + 1) * 4);
   a = cnt;
   dev_free(j, a, 4 * sizeof(unsigned long long));
@@ -3778,7 +3432,6 @@ static bruno_status pick_t(bruno_job* j, uint64_t min_freq, EdgeQuery<KT>** dq, 
   dev_free(j, a, nu * sizeof(ChainSummary<KT>));
   a = N;
   dev_free(j, a, nu * sizeof(ChainSummary<KT>));
-  dev_free(j, t, std::max<size_t>(tmp, 1));
   return BRUNO_OK;
 }
 
@@ -4161,11 +3814,10 @@ bruno_status bruno_batch_get_chain_nodes(bruno_job* j, uint32_t idx, bruno_chain
     TRY(dev_alloc(j, (void**)&d, m * sizeof(bruno_chain_node)));
     if (j->words == 1)
       hipLaunchKernelGGL((k_get_chain_nodes<uint64_t>), dim3(grid_for(m, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
-                         j->perm + c0, (const uint64_t*)j->out_k, (const uint64_t*)j->out_rep, j->dist_sorted + c0, m,
-                         d);
+                         out_view<uint64_t>(j), c0, m, d);
     else
       hipLaunchKernelGGL((k_get_chain_nodes<u128>), dim3(grid_for(m, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
-                         j->perm + c0, (const u128*)j->out_k, (const u128*)j->out_rep, j->dist_sorted + c0, m, d);
+                         out_view<u128>(j), c0, m, d);
     HIP_CHECK(hipMemcpyAsync(buf, d, m * sizeof(bruno_chain_node), hipMemcpyDeviceToHost, j->stream));
     HIP_CHECK(hipStreamSynchronize(j->stream));
     void* a = d;
@@ -4251,67 +3903,24 @@ extern "C++" {
 template <typename KT>
 static bruno_status chain_edges_t(bruno_job* j, uint32_t idx, uint64_t c0, uint64_t m, uint64_t nu,
                                   bruno_chain_edge* buf) {
-  /* unitig starts: positions of the dist-0 nodes among the job's sorted
-   * chain nodes, in order, then m (room for m + 1: the selection is checked
-   * against the unitig count before anything reads it) */
-  uint8_t* flags = nullptr;
-  uint32_t *starts = nullptr, *n_sel = nullptr;
+  uint32_t* starts = nullptr; /* room for every node: unitig_starts checks the count */
   bruno_chain_edge* d = nullptr;
-  void* t = nullptr;
-  size_t tmp = 0;
-  bruno_status st = BRUNO_OK;
-  uint32_t got = 0;
-  hipcub::CountingInputIterator<uint32_t> pos(0);
-  TRY(dev_alloc(j, (void**)&flags, m));
-  if ((st = dev_alloc(j, (void**)&starts, (m + 1) * 4)) != BRUNO_OK) goto done;
-  if ((st = dev_alloc(j, (void**)&n_sel, 4)) != BRUNO_OK) goto done;
-  if ((st = dev_alloc(j, (void**)&d, nu * sizeof(bruno_chain_edge))) != BRUNO_OK) goto done;
-  hipLaunchKernelGGL(k_head_flags, dim3(grid_for(m, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
-                     j->dist_sorted + c0, m, flags);
-  if (hipcub::DeviceSelect::Flagged(nullptr, tmp, pos, flags, starts, n_sel, (int)m, j->stream) != hipSuccess) {
-    st = BRUNO_INTERNAL;
-    goto done;
-  }
-  if ((st = dev_alloc(j, &t, std::max<size_t>(tmp, 1))) != BRUNO_OK) goto done;
-  if (hipcub::DeviceSelect::Flagged(t, tmp, pos, flags, starts, n_sel, (int)m, j->stream) != hipSuccess ||
-      copy_out(j, &got, n_sel, 4) != hipSuccess) {
-    st = BRUNO_INTERNAL;
-    goto done;
-  }
-  if (got != nu) {
-    st = BRUNO_INTERNAL;
-    goto done;
-  }
-  {
-    const uint32_t mm = (uint32_t)m;
-    if (hipMemcpyAsync(starts + nu, &mm, 4, hipMemcpyHostToDevice, j->stream) != hipSuccess) {
-      st = BRUNO_INTERNAL;
-      goto done;
-    }
+  const uint32_t* st0 = nullptr;
+  uint64_t off = 0;
+  bruno_status st = unitig_starts(j, idx, c0, m, nu, &starts, &st0, &off);
+  if (st == BRUNO_OK) st = dev_alloc(j, (void**)&d, nu * sizeof(bruno_chain_edge));
+  if (st == BRUNO_OK) {
     uint64_t tbase, tcap;
     job_segment(j, idx, tbase, tcap);
     hipLaunchKernelGGL((k_chain_edges<KT>), dim3(grid_for(nu * 64, BLOCK, 1u << 16)), dim3(BLOCK), 0, j->stream,
-                       (const Slot<KT>*)j->table, tbase, tcap, j->rbits, j->K, j->perm + c0, (const KT*)j->out_k,
-                       starts, nu, d, j->ctr);
+                       (const Slot<KT>*)j->table, tbase, tcap, j->rbits, j->K, out_view<KT>(j), off, st0, nu, d, j->ctr);
     st = sync_counters(j);
     if (st == BRUNO_OK && copy_out(j, buf, d, nu * sizeof(bruno_chain_edge)) != hipSuccess) st = BRUNO_INTERNAL;
   }
-done:
-  void* a = flags;
-  dev_free(j, a, m);
-  if (starts) {
-    a = starts;
-    dev_free(j, a, (m + 1) * 4);
-  }
-  if (n_sel) {
-    a = n_sel;
-    dev_free(j, a, 4);
-  }
-  if (d) {
-    a = d;
-    dev_free(j, a, nu * sizeof(bruno_chain_edge));
-  }
-  if (t) dev_free(j, t, std::max<size_t>(tmp, 1));
+  void* a = starts;
+  dev_free(j, a, (m + 1) * 4);
+  a = d;
+  dev_free(j, a, nu * sizeof(bruno_chain_edge));
   return st;
 }
 

@@ -50,16 +50,15 @@ __device__ __forceinline__ int edge_index(bool canonical, bool out, int c) {
 /* One thread per unitig u: starts[u] and starts[u + 1] - 1 are the sorted
  * positions of its first and last node. */
 template <typename KT>
-__global__ void k_chain_summaries(const Slot<KT>* T, uint64_t tcap, uint32_t rbits, int K, const uint32_t* perm,
-                                  const KT* out_k, const uint32_t* dist_sorted, const uint32_t* starts, uint64_t nu,
-                                  ChainSummary<KT>* out, Counters* ctr) {
+__global__ void k_chain_summaries(const Slot<KT>* T, uint64_t tcap, uint32_t rbits, int K, OutView<KT> v,
+                                  const uint32_t* starts, uint64_t nu, ChainSummary<KT>* out, Counters* ctr) {
   kops<KT> ops(K);
   for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t h = starts[u], t = starts[u + 1] - 1;
     ChainSummary<KT> s;
-    s.t5 = out_k[perm[h]];
-    s.t3 = out_k[perm[t]];
-    s.len = dist_sorted[t];
+    s.t5 = v.kmer(h);
+    s.t3 = v.kmer(t);
+    s.len = v.dist_of(t);
     s.b5 = 0;
     s.b3 = 0;
     const KT c5 = ops.canon(s.t5), c3 = ops.canon(s.t3);

@@ -371,9 +371,10 @@ typedef struct {
   uint32_t parse_block;    /* workgroup size of the parse + count kernel: 128, 256 or 512    */
   uint32_t parse_grid;     /* most waves of the parse + count launch (one read per wave)     */
   uint32_t scan_grid;      /* most workgroups of the filter's table scan                     */
-  uint32_t ruler_sample;   /* list ranking: one sampled ruler per this many chain nodes on
-                              average (power of two, 8..4096): the walk length between
-                              rulers and the size of the contracted list                    */
+  uint32_t ruler_sample;   /* list ranking: one sampled ruler per at most this many chain
+                              nodes on average (power of two, 8..4096; small graphs take
+                              fewer): the walk length between rulers and the size of the
+                              contracted list                                               */
   uint32_t count_regions;  /* 1 or 2: plain jobs (k <= 63) with tables of >= 2^22 slots lay
                               the table out in LDS-sized regions and count by writing
                               instance records grouped by region, then building each region
