@@ -900,7 +900,7 @@ __global__ __launch_bounds__(BLOCK) void k_move_slots(const Slot<KT>* O, uint64_
     for (int q = 0; q < Slot<KT>::NSUB; ++q) {
       const uint64_t v = p->sub[q];
       if (v != EMPTY64)
-        add_k2<KT>(T, s, (uint8_t)((v >> 48) - 1), sp, spcap, &ctr->err, v & 0xFFFFFFFFFFFFULL);
+        add_k2<KT>(T, s, v >> 48, sp, spcap, &ctr->err, v & 0xFFFFFFFFFFFFULL);
     }
   }
 }
@@ -917,7 +917,7 @@ __global__ __launch_bounds__(BLOCK) void k_move_spill(const Spill* O, uint64_t o
     for (int q = 0; q < SPILL_SUB; ++q) {
       const uint64_t v = O[i].sub[q];
       if (v != EMPTY64)
-        add_k2<KT>(T, s, (uint8_t)((v >> 48) - 1), sp, spcap, &ctr->err, v & 0xFFFFFFFFFFFFULL);
+        add_k2<KT>(T, s, v >> 48, sp, spcap, &ctr->err, v & 0xFFFFFFFFFFFFULL);
     }
   }
 }
@@ -971,7 +971,7 @@ __global__ __launch_bounds__(BLOCK) void k_get_k2(const Slot<KT>* T, uint64_t s0
         }
         kmers[(pos + j) * W] = (uint64_t)k;
         if (W == 2) kmers[(pos + j) * W + 1] = (uint64_t)((u128)k >> 64);
-        biedges[pos + j] = L.e[j];
+        biedges[pos + j] = biedge_byte(L.e[j]);
         counts[pos + j] = L.c[j];
       }
     }

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
             SlotOps<KT>::find_or_insert((Slot<KT>*)a.table + tbase, tcap, a.rbits, km, &a.ctr->err, &claimed);
         if (slot != ~0ULL) {
           my_new += claimed;
-          my_k2 += add_k2<KT>((Slot<KT>*)a.table, tbase + slot, e, a.spill, a.spcap, &a.ctr->err);
+          my_k2 += add_k2<KT>((Slot<KT>*)a.table, tbase + slot, biedge_index(e) + 1, a.spill, a.spcap, &a.ctr->err);
         }
       }
       ++my_inst;
@@ -399,12 +399,8 @@ __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
 /* ------------------------------------------------------------------ */
 /* per-slot k2 gathering                                                */
 /* ------------------------------------------------------------------ */
-/* All 25 biedge bytes possible for ACGT-only reads (nibbles 0,1,2,4,8). */
-__device__ __constant__ uint8_t BIEDGE25[25] = {
-    0x00, 0x01, 0x02, 0x04, 0x08, 0x10, 0x11, 0x12, 0x14, 0x18, 0x20, 0x21, 0x22,
-    0x24, 0x28, 0x40, 0x41, 0x42, 0x44, 0x48, 0x80, 0x81, 0x82, 0x84, 0x88};
-
-/* k2 entries of one slot.  N is a compile-time bound so that every array
+/* k2 entries of one slot: e the biedge's sides (biedge_sides), c its count.
+ * N is a compile-time bound so that every array
  * index below is a constant after unrolling and the lists stay in registers
  * (N = NSUB for slots without spilled entries, 25 for the rest). */
 template <int N>
@@ -418,17 +414,28 @@ typedef K2L<25> K2List;
 template <typename KT, int N>
 __device__ __forceinline__ uint64_t sub_entries(const Slot<KT>* p, K2L<N>& L) {
   static_assert(N >= Slot<KT>::NSUB, "list too small");
+  /* the whole slot at once, then no branch per entry: with one the
+   * compiler waits for each entry's load by itself (five dependent misses
+   * for a 64-byte slot) */
+  constexpr int W = sizeof(Slot<KT>) / 8, S0 = W - Slot<KT>::NSUB;
+  uint64_t w[W];
+#pragma unroll
+  for (int j = 0; j < W / 2; ++j) {
+    const ulonglong2 x = ((const ulonglong2*)p)[j];
+    w[2 * j] = x.x;
+    w[2 * j + 1] = x.y;
+  }
   L.n = 0;
   uint64_t kf = 0;
 #pragma unroll
   for (int j = 0; j < Slot<KT>::NSUB; ++j) {
-    uint64_t v = p->sub[j];
-    bool ok = v != EMPTY64;
+    const uint64_t v = w[S0 + j];
+    const uint64_t ok = v != EMPTY64 ? ~0ULL : 0ULL;
     /* sub-entries fill in order, so the valid ones are a prefix */
-    L.e[j] = ok ? (uint8_t)((v >> 48) - 1) : 0;
-    L.c[j] = ok ? (uint32_t)(v & 0xFFFFFFFFFFFFULL) : 0;
-    L.n += ok;
-    kf += ok ? (v & 0xFFFFFFFFFFFFULL) : 0;
+    L.e[j] = (uint8_t)(biedge_sides((uint32_t)(v >> 48) - 1) & ok);
+    L.c[j] = (uint32_t)(v & ok);
+    L.n += (int)(ok & 1);
+    kf += v & 0xFFFFFFFFFFFFULL & ok;
   }
   return kf;
 }
@@ -439,7 +446,7 @@ __device__ __forceinline__ void gather_k2(const Slot<KT>* p, uint64_t s, const S
   if (SlotOps<KT>::flags(p) & F_SPILL) {
     spill_each(sp, spcap, s, [&](uint64_t code, uint64_t cnt) {
       if (L.n < 25) {
-        L.e[L.n] = (uint8_t)(code - 1);
+        L.e[L.n] = biedge_sides((uint32_t)code - 1);
         L.c[L.n] = (uint32_t)cnt;
         ++L.n;
       }
@@ -447,7 +454,8 @@ __device__ __forceinline__ void gather_k2(const Slot<KT>* p, uint64_t s, const S
   }
 }
 
-__device__ __forceinline__ int nib_idx(int n) { return n == 1 ? 0 : n == 2 ? 1 : n == 4 ? 2 : n == 8 ? 3 : 8; }
+/* base of a side number (-1: no edge) */
+__device__ __forceinline__ int side_base(int n) { return n - 1; }
 __device__ __forceinline__ uint16_t sat_add16(uint32_t a, uint32_t b) {
   uint32_t c = a + b;
   return (uint16_t)(c > 65535u ? 65535u : c);
@@ -455,7 +463,7 @@ __device__ __forceinline__ uint16_t sat_add16(uint32_t a, uint32_t b) {
 /* compact_multi_biedge::update(edges, cnt) (debruijn_graph_node.hpp:200-211),
  * written with constant indices only */
 __device__ __forceinline__ void node_update(uint16_t (&c)[9], uint8_t e, uint32_t cnt) {
-  int o = nib_idx(e & 0xF), i = nib_idx(e >> 4);
+  int o = side_base(e & 0xF), i = side_base(e >> 4);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     if (q == o) c[q] = sat_add16(c[q], cnt);
@@ -504,14 +512,14 @@ __device__ bool p2_counts(const kops<KT>& ops, KT k, const K2L<N>& L, const Thre
     kf += cu;
     int ch = L.e[j] >> 4;
     if (ch) {
-      int ci = nib_idx(ch);
+      int ci = side_base(ch);
       /* is_k1_rc_palindrome(l, k, high): last base == comp(l) && high */
       bool split = ((ops.K & 1) && lastb == 3 - ci && high) && !kpal;
       add_sel4(k1in, ci, split ? ((cu + 1) >> 1) : cu);
     }
     ch = L.e[j] & 0xF;
     if (ch) {
-      int ci = nib_idx(ch);
+      int ci = side_base(ch);
       bool split = ((ops.K & 1) && firstb == 3 - ci && low) && !kpal;
       add_sel4(k1out, ci, split ? ((cu + 1) >> 1) : cu);
     }
@@ -533,9 +541,9 @@ __device__ bool p2_counts(const kops<KT>& ops, KT k, const K2L<N>& L, const Thre
     if (cnt < t.t2lo || cnt >= t.t2hi) flag |= 4;
     if (kf < t.t0lo || kf >= t.t0hi) flag |= 8;
     int in = L.e[j] >> 4, out = L.e[j] & 0xF;
-    uint64_t k1 = get_sel4(k1in, nib_idx(in), t.t1hi);
+    uint64_t k1 = get_sel4(k1in, side_base(in), t.t1hi);
     if (k1 < t.t1lo || k1 >= t.t1hi) flag |= 2;
-    k1 = get_sel4(k1out, nib_idx(out), t.t1hi);
+    k1 = get_sel4(k1out, side_base(out), t.t1hi);
     if (k1 < t.t1lo || k1 >= t.t1hi) flag |= 1;
     if (flag >= 3) continue;
     uint8_t e = L.e[j];
@@ -573,8 +581,8 @@ __device__ __forceinline__ bool p2_counts_slot(const kops<KT>& ops, const KmerFa
                  hi2 = th(t.t2hi);
   const bool odd = ops.K & 1;
   /* the edge whose k+1-mer is an rc palindrome counts half (is_k1_rc_palindrome) */
-  const uint32_t split_in = (odd && f.high && !f.kpal) ? (1u << (3 - f.last)) : 0u;
-  const uint32_t split_out = (odd && f.low && !f.kpal) ? (1u << (3 - f.first)) : 0u;
+  const uint32_t split_in = (odd && f.high && !f.kpal) ? 4 - f.last : 15u;
+  const uint32_t split_out = (odd && f.low && !f.kpal) ? 4 - f.first : 15u;
   uint32_t kf = 0, kin[4] = {0, 0, 0, 0}, kout[4] = {0, 0, 0, 0};
 #pragma unroll
   for (int j = 0; j < N; ++j) {
@@ -584,8 +592,8 @@ __device__ __forceinline__ bool p2_counts_slot(const kops<KT>& ops, const KmerFa
     kf += min(cu, M);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      kin[q] += ni == (1u << q) ? vi : 0u;
-      kout[q] += no == (1u << q) ? vo : 0u;
+      kin[q] += ni == q + 1u ? vi : 0u;
+      kout[q] += no == q + 1u ? vo : 0u;
     }
   }
   kf = min(kf, M);
@@ -600,16 +608,16 @@ __device__ __forceinline__ bool p2_counts_slot(const kops<KT>& ops, const KmerFa
     uint32_t k1i = 65536u, k1o = 65536u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      k1i = ni == (1u << q) ? min(kin[q], M) : k1i;
-      k1o = no == (1u << q) ? min(kout[q], M) : k1o;
+      k1i = ni == q + 1u ? min(kin[q], M) : k1i;
+      k1o = no == q + 1u ? min(kout[q], M) : k1o;
     }
     const bool f2 = k1i < lo1 || k1i >= hi1, f1 = k1o < lo1 || k1o >= hi1;
     const bool keep = j < L.n && !(cu < lo2 || cu >= hi2) && !kf_bad && !(f1 && f2);
     const uint32_t ki = keep && !f2 ? ni : 0u, ko = keep && !f1 ? no : 0u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      acc[q] += ko == (1u << q) ? cu : 0u;
-      acc[4 + q] += ki == (1u << q) ? cu : 0u;
+      acc[q] += ko == q + 1u ? cu : 0u;
+      acc[4 + q] += ki == q + 1u ? cu : 0u;
     }
     acc[8] += keep ? cu : 0u;
     have |= keep;
@@ -668,9 +676,9 @@ __device__ bool edge_counts(const kops<KT>& ops, KT k, const K2L<N>& L, const Th
     if (j >= L.n) break;
     const uint64_t cu = L.c[j];
     int ch = L.e[j] >> 4;
-    if (ch) add_sel4(sin, nib_idx(ch), cu);
+    if (ch) add_sel4(sin, side_base(ch), cu);
     ch = L.e[j] & 0xF;
-    if (ch) add_sel4(sout, nib_idx(ch), cu);
+    if (ch) add_sel4(sout, side_base(ch), cu);
   }
   uint64_t win_in[4], win_out[4];
 #pragma unroll
@@ -694,7 +702,7 @@ __device__ bool edge_counts(const kops<KT>& ops, KT k, const K2L<N>& L, const Th
   for (int j = 0; j < N; ++j) {
     if (j >= L.n) break;
     const int in = L.e[j] >> 4, out = L.e[j] & 0xF;
-    const uint64_t wi = get_sel4(win_in, nib_idx(in), 0), wo = get_sel4(win_out, nib_idx(out), 0);
+    const uint64_t wi = get_sel4(win_in, side_base(in), 0), wo = get_sel4(win_out, side_base(out), 0);
     const bool in_ok = in && wi >= t.t1lo && wi < t.t1hi;
     const bool out_ok = out && wo >= t.t1lo && wo < t.t1hi;
     if (!in_ok && !out_ok) continue;

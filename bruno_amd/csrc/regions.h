@@ -49,13 +49,6 @@ constexpr uint64_t REGION_BUILD_CU_SLOTS = 512; /* build workgroups resident on 
 constexpr int REC_BS = 512, REC_PF = 8, REC_STAGE = 192, REC_FLUSH = 32;
 constexpr int REGION_ITEMS = 8;              /* records per thread loaded at once by the build */
 
-/* biedge byte (nibbles 0, 1, 2, 4, 8 per side) -> index into BIEDGE25 */
-__device__ __forceinline__ uint32_t biedge_index(uint8_t e) {
-  const uint32_t l = e >> 4, r = e & 15;
-  const uint32_t il = l ? 1 + __builtin_ctz(l) : 0, ir = r ? 1 + __builtin_ctz(r) : 0;
-  return il * 5 + ir;
-}
-
 /* Records of a bucket fill chunks of `chunk` slots taken from the front of
  * the bucket's area with one atomic each (a workgroup keeps one open chunk
  * per bucket and pads it with skipped records at the end); records that
@@ -324,6 +317,9 @@ constexpr uint64_t LIST_HOLE = ~0ULL;
 __device__ __forceinline__ uint64_t lds_load(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ void lds_store(uint64_t* p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 /* A region in LDS, one row per slot word (row 0 the key / meta word, then
  * the two-word key's words, then the sub-entries): a wave's lanes touch
@@ -373,82 +369,139 @@ struct LdsRegion {
   }
 };
 
-/* Find or claim k-mer v in the LDS region L of span slots from home slot
- * s; returns the slot, or ~0u when the region is full.  *claimed as in
- * SlotOps::find_or_insert. */
-template <uint32_t SLOTS>
-__device__ __forceinline__ uint32_t lds_claim(LdsRegion<uint64_t, SLOTS>& L, uint32_t span, uint32_t s, uint64_t v,
-                                              int* claimed) {
-  for (uint32_t probe = 0; probe < span; ++probe) {
-    uint64_t k0 = lds_load(L.flag(s));
-    if (k0 == EMPTY64) {
-      const uint64_t old = atomicCAS((unsigned long long*)L.flag(s), EMPTY64, (unsigned long long)v);
-      if (old == EMPTY64) {
-        *claimed = 1;
-        return s;
-      }
-      k0 = old;
-    }
-    if ((k0 & KEY_BITS) == v) return s;
-    s = (s + 1 == span) ? 0 : s + 1;
-  }
-  return ~0u;
-}
-/* Two-word keys: meta is claimed by CAS (EMPTY -> LOCK), the words are
- * stored and meta published with a release store, all in one block ahead
- * of any wait, so a lane of the claiming wave never waits for its own
- * wave; readers wait (bounded) while meta is LOCK. */
-template <uint32_t SLOTS>
-__device__ __forceinline__ uint32_t lds_claim(LdsRegion<u128, SLOTS>& L, uint32_t span, uint32_t s, u128 v,
-                                              int* claimed) {
-  const uint64_t lo = (uint64_t)v, hi = (uint64_t)(v >> 64);
-  for (uint32_t probe = 0; probe < span; ++probe) {
-    uint64_t m = __hip_atomic_load(L.flag(s), __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (m == EMPTY64) {
-      const uint64_t old = atomicCAS((unsigned long long*)L.flag(s), EMPTY64, (unsigned long long)LOCK64);
-      if (old == EMPTY64) {
-        L.w[1][s] = lo;
-        L.w[2][s] = hi;
-        __hip_atomic_store(L.flag(s), (uint64_t)0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        *claimed = 1;
-        return s;
-      }
-      m = old;
-    }
-    for (uint32_t spin = 0; m == LOCK64 && spin < MAX_SPIN; ++spin)
-      m = __hip_atomic_load(L.flag(s), __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (m == LOCK64) return ~0u;
-    if (L.w[1][s] == lo && L.w[2][s] == hi) return s;
-    s = (s + 1 == span) ? 0 : s + 1;
-  }
-  return ~0u;
+/* An EMPTY word by its high half: no key, meta or sub-entry word of a
+ * region being counted has an all-ones high half (F_PRESENT is never set
+ * there, a biedge code is at most 25), so one 32-bit compare decides. */
+__device__ __forceinline__ bool lds_empty(uint64_t v) { return (uint32_t)(v >> 32) == ~0u; }
+
+/* v, with what the compiler knows of it forgotten: the word a loop ended
+ * with is tested again after the loop (two instructions), where the
+ * compiler would carry each test's result through the loop as a lane mask
+ * (three scalar instructions a pass, more than the pass itself). */
+__device__ __forceinline__ uint64_t opaque(uint64_t v) {
+  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
+  asm("" : "+v"(lo), "+v"(hi));
+  return ((uint64_t)hi << 32) | lo;
 }
 
-/* add_k2 on LDS slot s; gs is the slot's table index (side-table key).
- * Returns 1 for a new k2 entry in the slot, 0 for a count added, and
- * LDS_SPILL when the entry belongs in the side table (the slot is marked
- * as having spilled entries; the caller queues the entry). */
+/* Find or claim the k-mer of a record in the LDS region L of span slots
+ * from home slot s; returns the slot, or ~0u when the region is full.
+ * fresh: this call inserted the key.  During the adds a slot's first word
+ * holds the record's 59 hash bits (with the region they determine a one-word
+ * k-mer), so a record needs no unhashing; lds_finish puts the k-mers in.
+ * (One exit and no state but the word read: a wave runs the loop to its
+ * longest probe sequence, so what counts is the instructions per probe,
+ * vector and scalar.) */
+template <uint32_t SLOTS>
+__device__ __forceinline__ uint32_t lds_claim(LdsRegion<uint64_t, SLOTS>& L, uint32_t span, const uint32_t home,
+                                              const uint64_t& rec, bool& fresh) {
+  const uint64_t v = rec >> REC_BUCKET_BITS;
+  uint32_t s = home, at;
+  uint64_t k0;
+  bool miss;
+  do {
+    at = s;
+    k0 = lds_load(L.flag(s));
+    if (lds_empty(k0)) k0 = atomicCAS((unsigned long long*)L.flag(s), EMPTY64, (unsigned long long)v);
+    miss = !lds_empty(k0) && (k0 & ~F_SPILL) != v;
+    s = (s + 1 == span) ? 0 : s + 1;
+  } while (miss && s != home);
+  k0 = opaque(k0);
+  fresh = lds_empty(k0);
+  return fresh || (k0 & ~F_SPILL) == v ? at : ~0u;
+}
+/* Two-word k-mers: the hash word is claimed, then the high word stored
+ * (all ones until then, which no k-mer's high word is); a slot whose hash
+ * word agrees is read on, waiting (bounded) for its high word.  The claiming
+ * lanes of a wave store before any lane of it waits.  A probe that misses
+ * costs one LDS read; with the k-mer's own words as the key it was three. */
+template <uint32_t SLOTS>
+__device__ __forceinline__ uint32_t lds_claim(LdsRegion<u128, SLOTS>& L, uint32_t span, const uint32_t home,
+                                              const ulonglong2& rec, bool& fresh) {
+  const uint64_t v = rec.x >> REC_BUCKET_BITS, hi = rec.y;
+  uint32_t s = home, at;
+  uint64_t k0;
+  bool miss, same;
+  do {
+    at = s;
+    k0 = lds_load(L.flag(s));
+    if (lds_empty(k0)) {
+      k0 = atomicCAS((unsigned long long*)L.flag(s), EMPTY64, (unsigned long long)v);
+      if (lds_empty(k0)) lds_store(&L.w[2][s], hi);
+    }
+    same = (k0 & ~F_SPILL) == v;
+    if (same) {
+      uint64_t h2 = lds_load(&L.w[2][s]);
+      for (uint32_t spin = 0; h2 == EMPTY64 && spin < MAX_SPIN; ++spin) h2 = lds_load(&L.w[2][s]);
+      same = h2 == hi;
+    }
+    miss = !(lds_empty(k0) || same);
+    s = (s + 1 == span) ? 0 : s + 1;
+  } while (miss && s != home);
+  k0 = opaque(k0);
+  fresh = lds_empty(k0);
+  return fresh || same ? at : ~0u;
+}
+
+/* Between the adds' slots and the table's: the hash word of slot i made
+ * from its k-mer (after a load) and back (before a write-back; h_top: the
+ * hash's top bits, the region's bucket). */
+template <uint32_t SLOTS>
+__device__ __forceinline__ void lds_begin(LdsRegion<uint64_t, SLOTS>& L, uint32_t i) {
+  const uint64_t w = L.w[0][i];
+  if (!lds_empty(w)) L.w[0][i] = (w & F_SPILL) | (kmer_hash(w & KEY_BITS) << REC_BUCKET_BITS >> REC_BUCKET_BITS);
+}
+template <uint32_t SLOTS>
+__device__ __forceinline__ void lds_begin(LdsRegion<u128, SLOTS>& L, uint32_t i) {
+  const uint64_t w = L.w[0][i];
+  if (w != EMPTY64)
+    L.w[0][i] = (w & F_SPILL) |
+                (kmer_hash(((u128)L.w[2][i] << 64) | L.w[1][i]) << REC_BUCKET_BITS >> REC_BUCKET_BITS);
+}
+template <uint32_t SLOTS>
+__device__ __forceinline__ void lds_finish(LdsRegion<uint64_t, SLOTS>& L, uint32_t i, uint64_t h_top) {
+  const uint64_t w = L.w[0][i];
+  if (!lds_empty(w)) L.w[0][i] = (w & F_SPILL) | kmer_unhash(h_top | (w & ~F_SPILL));
+}
+template <uint32_t SLOTS>
+__device__ __forceinline__ void lds_finish(LdsRegion<u128, SLOTS>& L, uint32_t i, uint64_t h_top) {
+  const uint64_t w = L.w[0][i];
+  if (!lds_empty(w)) {
+    L.w[1][i] = (uint64_t)kmer_unhash(h_top | (w & ~F_SPILL), L.w[2][i]);
+    L.w[0][i] = w & F_SPILL;
+  }
+}
+
+/* add_k2 on LDS slot s (code = biedge index + 1).  Returns 1 for a new k2
+ * entry in the slot, 0 for a count added, and LDS_SPILL when the entry
+ * belongs in the side table (the slot is marked as having spilled entries;
+ * the caller queues the entry).  A loop over the sub-entry rows: almost
+ * every record ends at the first or second. */
 constexpr int LDS_SPILL = 2;
 template <typename KT, uint32_t SLOTS>
-__device__ __forceinline__ int lds_add_k2(LdsRegion<KT, SLOTS>& L, uint32_t s, uint8_t e) {
-  const uint64_t code = (uint64_t)e + 1;
-#pragma unroll
-  for (int j = 0; j < Slot<KT>::NSUB; ++j) {
-    uint64_t* q = L.sub(j, s);
-    uint64_t v = lds_load(q);
-    if (v == EMPTY64) {
-      const uint64_t old = atomicCAS((unsigned long long*)q, EMPTY64, (unsigned long long)((code << 48) | 1));
-      if (old == EMPTY64) return 1;
-      v = old;
-    }
-    if ((v >> 48) == code) {
-      atomicAdd((unsigned long long*)q, 1ULL);
-      return 0;
-    }
+__device__ __forceinline__ int lds_add_k2(LdsRegion<KT, SLOTS>& L, uint32_t s, uint32_t code) {
+  constexpr int N = Slot<KT>::NSUB;
+  uint64_t* q = L.sub(0, s);
+  uint64_t* const end = q + (size_t)N * SLOTS;
+  const uint64_t first = ((uint64_t)code << 48) | 1;
+  uint64_t* at;
+  uint64_t v;
+  bool more;
+  do {
+    at = q;
+    v = lds_load(q);
+    if (lds_empty(v)) v = atomicCAS((unsigned long long*)q, EMPTY64, (unsigned long long)first);
+    more = !lds_empty(v) && (uint32_t)(v >> 48) != code;
+    q += SLOTS;
+  } while (more && q != end);
+  v = opaque(v);
+  if ((uint32_t)(v >> 48) == code) atomicAdd((unsigned long long*)at, 1ULL);
+  else if (!lds_empty(v)) {
+    uint64_t* fw = L.flag(s);
+    if (!(lds_load(fw) & F_SPILL)) atomicOr((unsigned long long*)fw, (unsigned long long)F_SPILL);
+    return LDS_SPILL;
   }
-  uint64_t* fw = L.flag(s);
-  if (!(lds_load(fw) & F_SPILL)) atomicOr((unsigned long long*)fw, (unsigned long long)F_SPILL);
-  return LDS_SPILL;
+  return lds_empty(v) ? 1 : 0;
 }
 
 /* an empty use of a register: the compiler waits for its load here */
@@ -458,63 +511,46 @@ __device__ __forceinline__ void consume(const ulonglong2& v) {
   asm volatile("" ::"v"(v.y));
 }
 
-/* the k-mer of a record of region q */
-__device__ __forceinline__ uint64_t rec_hash(const RegionArgs& g, uint64_t q, uint64_t key) {
-  /* the bucket bits (the region's top 5 bits), then the record's */
-  return ((q >> (g.rbits - REC_BUCKET_BITS)) << (64 - REC_BUCKET_BITS)) | (key >> REC_BUCKET_BITS);
-}
-__device__ __forceinline__ uint64_t rec_kmer(uint64_t h, uint64_t) { return kmer_unhash(h); }
-__device__ __forceinline__ u128 rec_kmer(uint64_t h, const ulonglong2& r) { return kmer_unhash(h, r.y); }
-
-/* The biedge byte of biedge index i = il * 5 + ir (nibble 0 for side index
- * 0, else 1 << (index - 1)), computed: a table lookup would be a global
- * load per record on the build's critical path. */
-__device__ __forceinline__ uint32_t biedge_of_index(uint32_t i) {
-  const uint32_t il = (i * 52u) >> 8, ir = i - 5u * il; /* i / 5 for i < 25 */
-  return (((1u << il) >> 1) << 4) | ((1u << ir) >> 1);
-}
-
-/* Add one record of region q (table slots from base) to the LDS region.
- * Returns the side-table entry to queue (slot << 5 | biedge index), or
- * NO_SPILL. */
-constexpr uint64_t NO_SPILL = ~0ULL;
+/* Add one record to its region in LDS.  Returns the LDS slot of a
+ * side-table entry to queue (of the record's biedge index), or NO_SPILL. */
+constexpr uint32_t NO_SPILL = ~0u;
 template <typename KT, uint32_t SLOTS, typename R>
-__device__ __forceinline__ uint64_t region_add(const RegionArgs& g, LdsRegion<KT, SLOTS>& L, uint32_t span,
-                                               uint64_t q, uint64_t base, const R& rec, unsigned long long& my_new,
-                                               unsigned long long& my_k2) {
+__device__ __forceinline__ uint32_t region_add(const RegionArgs& g, LdsRegion<KT, SLOTS>& L, uint32_t span,
+                                               const R& rec, uint32_t& my_new, uint32_t& my_k2) {
   const uint64_t key = rec_key(rec);
-  const uint32_t code = (uint32_t)(key & 31);
-  const uint64_t h = rec_hash(g, q, key);
-  const KT km = rec_kmer(h, rec);
-  int claimed = 0;
-  const uint32_t s = lds_claim(L, span, (uint32_t)__umul64hi(h << g.rbits, g.span), km, &claimed);
+  bool fresh;
+  /* the record's hash bits below the region's, as region_home takes them */
+  const uint32_t home = region_home(key, g.rbits - REC_BUCKET_BITS, span);
+  const uint32_t s = lds_claim(L, span, home, rec, fresh);
   if (s == ~0u) {
     atomicOr(&g.ctr->err, ERR_TABLE_FULL);
     return NO_SPILL;
   }
-  my_new += claimed;
-  const int r = lds_add_k2<KT, SLOTS>(L, s, (uint8_t)biedge_of_index(code));
-  if (r == LDS_SPILL) return ((base + s) << 5) | code;
-  my_k2 += r;
-  return NO_SPILL;
+  my_new += fresh ? 1 : 0;
+  const int r = lds_add_k2<KT, SLOTS>(L, s, (uint32_t)(key & 31) + 1);
+  my_k2 += r & 1;
+  return r == LDS_SPILL ? s : NO_SPILL;
 }
 
-/* Queue side-table entries from converged code: one ballot per record
- * slot of the tile; qn (this wave's queue fill) stays wave-uniform.  A full
- * queue adds the entry inline. */
-__device__ __forceinline__ void spill_queue(const RegionArgs& g, uint64_t* q, uint32_t& qn, uint64_t e,
-                                            unsigned long long& my_k2) {
-  const uint64_t m = __ballot(e != NO_SPILL);
+/* a side-table entry added at once: the wave's queue is full (kept out of
+ * line: inlined at every record slot it was most of the build's code) */
+__device__ __noinline__ int spill_add_now(Spill* sp, uint64_t spcap, uint64_t e, uint32_t* err) {
+  return spill_add(sp, spcap, e >> 5, (e & 31) + 1, err);
+}
+
+/* Queue side-table entries (table slot << 5 | biedge index) from converged
+ * code: one ballot per record slot of the tile; qn (this wave's queue fill)
+ * stays wave-uniform.  A full queue adds the entry at once.  s: LDS slot or
+ * NO_SPILL; base: the region's first table slot. */
+__device__ __forceinline__ void spill_queue(const RegionArgs& g, uint64_t* q, uint32_t& qn, uint32_t s, uint64_t base,
+                                            uint32_t code, uint32_t& my_k2) {
+  const uint64_t m = __ballot(s != NO_SPILL);
   if (!m) return;
-  const uint32_t lane = __lane_id();
-  const uint32_t at = qn + (uint32_t)__popcll(m & ((1ULL << lane) - 1));
-  if (e != NO_SPILL) {
-    if (at < g.spq_cap) {
-      q[at] = e;
-    } else {
-      const uint64_t bq = biedge_of_index((uint32_t)(e & 31)) + 1;
-      my_k2 += spill_add(g.spill, g.spcap, e >> 5, bq, &g.ctr->err);
-    }
+  const uint32_t at = qn + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+  if (s != NO_SPILL) {
+    const uint64_t e = ((base + s) << 5) | code;
+    if (at < g.spq_cap) q[at] = e;
+    else my_k2 += spill_add_now(g.spill, g.spcap, e, &g.ctr->err);
   }
   qn += (uint32_t)__popcll(m);
 }
@@ -605,7 +641,7 @@ __device__ __forceinline__ bool fuse_nodes(const RegionArgs& g, LdsRegion<KT, SL
     for (int j = 0; j < N; ++j) {
       const uint64_t v = *L.sub(j, qs);
       const bool ok = v != EMPTY64;
-      Lk.e[j] = ok ? (uint8_t)((v >> 48) - 1) : 0;
+      Lk.e[j] = ok ? biedge_sides((uint32_t)(v >> 48) - 1) : 0;
       Lk.c[j] = ok ? (uint32_t)(v & 0xFFFFFFFFFFFFULL) : 0;
       Lk.n += ok;
     }
@@ -651,7 +687,7 @@ __global__ __launch_bounds__(BLOCK) void k_spill_flush(const uint64_t* spq, cons
   unsigned long long mine = 0;
   for (uint32_t i = threadIdx.x; i < n; i += BLOCK) {
     const uint64_t e = q[i];
-    mine += spill_add(spill, spcap, e >> 5, biedge_of_index((uint32_t)(e & 31)) + 1, &ctr->err);
+    mine += spill_add(spill, spcap, e >> 5, (e & 31) + 1, &ctr->err);
   }
   block_add(mine, &ctr->n_k2);
 }
@@ -664,7 +700,16 @@ __global__ __launch_bounds__(BLOCK) void k_spill_flush(const uint64_t* spq, cons
  * stores, a slot per lane).  The next region's first records are loaded
  * before this region's records are added, so their latency hides behind
  * the LDS work; barriers order LDS only, so one region's write-back
- * overlaps the next region's set-up. */
+ * overlaps the next region's set-up.
+ *
+ * Bound by the instructions per record (vector and scalar; LDS is busy a
+ * third of the time), so the adds carry no lane masks through their loops,
+ * compare one 32-bit half for EMPTY, take the home slot from one 32-bit
+ * product and leave the k-mer to the write-back (a record needs no
+ * unhashing; one slot in two holds a k-mer).  184 M records into 113 M slots:
+ * 1.86 -> 1.56 ms; 301 M 16-byte records (k = 63): 5.5 -> 4.55 ms.  Twice the
+ * waves (1,024 threads a workgroup, half the registers) were slower, 2.34 and
+ * 6.2 ms. */
 template <typename KT, uint32_t SLOTS, int BS, bool FUSE>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_region_build(RegionArgs g) {
   typedef typename RecOf<KT>::T R;
@@ -678,7 +723,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const uint64_t qa = g.q0 + (uint64_t)blockIdx.x * nlaunch / gridDim.x,
                  qb = g.q0 + ((uint64_t)blockIdx.x + 1) * nlaunch / gridDim.x;
   const R* recs = (const R*)g.recs;
-  unsigned long long my_new = 0, my_k2 = 0;
+  uint32_t my_new = 0, my_k2 = 0; /* a lane's records of one launch: far below 2^32 */
   constexpr uint64_t TILE = (uint64_t)REGION_ITEMS * BS;
   /* region_start[q] for the workgroup's regions, 64 at a time: lane l of
    * every wave holds entry rs_base + l and the next 64 are loaded ahead,
@@ -729,6 +774,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
     Slot<KT>* T = (Slot<KT>*)g.table + base;
     if (g.valid) {
       L.template load<BS>(span, T);
+      lds_barrier();
+      for (uint32_t i = threadIdx.x; i < span; i += BS) lds_begin(L, i);
     } else {
       L.template clear<BS>(span);
     }
@@ -739,9 +786,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
      * wait for nothing) */
 #pragma unroll
     for (int k = 0; k < REGION_ITEMS; ++k) {
-      uint64_t e = NO_SPILL;
-      if (lo + (uint64_t)k * BS + threadIdx.x < hi) e = region_add<KT, SLOTS, R>(g, L, span, q, base, rr[k], my_new, my_k2);
-      spill_queue(g, spq, qn, e, my_k2);
+      uint32_t e = NO_SPILL;
+      if (lo + (uint64_t)k * BS + threadIdx.x < hi) e = region_add<KT, SLOTS, R>(g, L, span, rr[k], my_new, my_k2);
+      spill_queue(g, spq, qn, e, base, (uint32_t)rec_key(rr[k]) & 31, my_k2);
     }
     for (uint64_t i0 = lo + TILE; i0 < hi; i0 += TILE) {
       R rt[REGION_ITEMS];
@@ -752,10 +799,10 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
       }
 #pragma unroll
       for (int k = 0; k < REGION_ITEMS; ++k) {
-        uint64_t e = NO_SPILL;
+        uint32_t e = NO_SPILL;
         if (i0 + (uint64_t)k * BS + threadIdx.x < hi)
-          e = region_add<KT, SLOTS, R>(g, L, span, q, base, rt[k], my_new, my_k2);
-        spill_queue(g, spq, qn, e, my_k2);
+          e = region_add<KT, SLOTS, R>(g, L, span, rt[k], my_new, my_k2);
+        spill_queue(g, spq, qn, e, base, (uint32_t)rec_key(rt[k]) & 31, my_k2);
       }
     }
     /* the next region's records (loaded since this region began) are
@@ -765,6 +812,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
     for (int k = 0; k < REGION_ITEMS; ++k) consume(rn[k]);
     lds_barrier();
+    /* a slot's words are finished by the thread that reads them below (the
+     * fused filter: by a lane of the same wave) */
+    const uint64_t h_top = (q >> (g.rbits - REC_BUCKET_BITS)) << (64 - REC_BUCKET_BITS);
+    if (FUSE || !g.cbits)
+      for (uint32_t i = threadIdx.x; i < span; i += BS) lds_finish(L, i, h_top);
     bool left = false; /* a candidate of this wave's slots found its list full */
     if constexpr (FUSE) {
       /* each wave queues the candidates of its slots (lane l holds the
@@ -803,7 +855,10 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
       for (uint32_t i0 = 0; i0 < span; i0 += BS) {
         const uint32_t i = i0 + threadIdx.x;
         bool c = false, sp = false;
-        if (i < span) c = lds_candidate(g, L, i, sp);
+        if (i < span) {
+          c = lds_candidate(g, L, i, sp);
+          if (!FUSE) lds_finish(L, i, h_top);
+        }
         if (FUSE && !left) c = false;
         const uint64_t bc = __ballot(c), bsp = __ballot(sp);
         const uint32_t w0 = i0 + (threadIdx.x & ~63u);
@@ -813,7 +868,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
         }
       }
     }
-    if (FUSE) lds_barrier(); /* the node records are in LDS */
+    lds_barrier(); /* the k-mers and node records are in LDS */
     L.template store<BS>(span, T);
     lds_barrier();
   }

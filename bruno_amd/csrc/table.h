@@ -19,8 +19,9 @@
  *   words, so a slot is claimed by CAS on meta (EMPTY -> LOCK), the k-mer is
  *   written, then meta is published as its flag word (bit 63 spilled, bit 62
  *   present).
- * Sub-entry: (code << 48) | count with code = biedge + 1 (1..256); EMPTY =
- *   all ones.
+ * Sub-entry: (code << 48) | count with code = biedge index + 1 (1..25, the
+ *   index of an instance record, so the region build stores it as it comes);
+ *   EMPTY = all ones.
  */
 #ifndef BRUNO_TABLE_H_
 #define BRUNO_TABLE_H_
@@ -102,17 +103,39 @@ __device__ __forceinline__ void or64(uint64_t* p, uint64_t v) {
 
 __device__ __forceinline__ uint64_t home_slot(uint64_t h, uint64_t cap) { return __umul64hi(h, cap); }
 
+/* A biedge's two sides as numbers (0 no edge, else 1 + base; in << 4 | out),
+ * from its index il * 5 + ir, and the biedge byte (nibbles 0, 1, 2, 4, 8 per
+ * side) they stand for; the index of a byte. */
+__device__ __forceinline__ uint8_t biedge_sides(uint32_t i) {
+  const uint32_t il = (13u * i) >> 6; /* i / 5 for i < 25 */
+  return (uint8_t)(i + 11u * il);     /* il << 4 | (i - 5 il) */
+}
+__device__ __forceinline__ uint8_t biedge_byte(uint8_t sides) {
+  return (uint8_t)((((1u << (sides >> 4)) >> 1) << 4) | ((1u << (sides & 15)) >> 1));
+}
+__device__ __forceinline__ uint32_t biedge_index(uint8_t e) {
+  const uint32_t l = e >> 4, r = e & 15;
+  const uint32_t il = l ? 1 + __builtin_ctz(l) : 0, ir = r ? 1 + __builtin_ctz(r) : 0;
+  return il * 5 + ir;
+}
+
 /* Probe window of a k-mer hash.  rbits == 0: the whole table of span slots
  * (home = fastrange(h, span), wrapping at span).  rbits > 0: the table is
  * 2^rbits regions of span slots each; the top rbits hash bits pick the
  * region, the rest the home slot inside it, and probes wrap inside the
- * region, so every slot a k-mer can occupy lies in one region. */
+ * region, so every slot a k-mer can occupy lies in one region.  The home
+ * slot there takes the 32 hash bits below the region's: a region has far
+ * fewer slots, and the region build computes it for every instance, where
+ * a 64 x 64-bit high product is four quarter-rate multiplies. */
+__device__ __forceinline__ uint32_t region_home(uint64_t h, uint32_t rbits, uint32_t span) {
+  return __umulhi((uint32_t)((h << rbits) >> 32), span);
+}
 struct Probe {
   uint64_t lo, hi, s;
   __device__ __forceinline__ Probe(uint64_t h, uint64_t span, uint32_t rbits) {
     lo = rbits ? (h >> (64 - rbits)) * span : 0;
     hi = lo + span;
-    s = lo + __umul64hi(h << rbits, span);
+    s = rbits ? lo + region_home(h, rbits, (uint32_t)span) : __umul64hi(h, span);
   }
   __device__ __forceinline__ void next() { s = (s + 1 == hi) ? lo : s + 1; }
 };
@@ -281,7 +304,8 @@ __device__ __forceinline__ Spill* spill_record(Spill* sp, uint64_t spcap, uint64
 }
 
 /* Count n instances (one unless a table is being moved) of entry code
- * (biedge + 1) of slot s in the side table.  Returns 1 if the entry is new. */
+ * (biedge index + 1) of slot s in the side table.  Returns 1 if the entry is
+ * new. */
 __device__ __forceinline__ int spill_add(Spill* sp, uint64_t spcap, uint64_t s, uint64_t code, uint32_t* err,
                                          uint64_t n = 1) {
   for (int part = 0; part < SPILL_PARTS; ++part) {
@@ -319,13 +343,12 @@ __device__ __forceinline__ void spill_each(const Spill* sp, uint64_t spcap, uint
   }
 }
 
-/* Add n instances (one unless a table is being moved) of biedge e to slot
- * s.  Returns 1 if a new k2 entry was created. */
+/* Add n instances (one unless a table is being moved) of entry code (biedge
+ * index + 1) to slot s.  Returns 1 if a new k2 entry was created. */
 template <typename KT>
-__device__ int add_k2(Slot<KT>* T, uint64_t s, uint8_t e, Spill* sp, uint64_t spcap, uint32_t* err,
+__device__ int add_k2(Slot<KT>* T, uint64_t s, uint64_t code, Spill* sp, uint64_t spcap, uint32_t* err,
                       uint64_t n = 1) {
   Slot<KT>* p = T + s;
-  const uint64_t code = (uint64_t)e + 1;
 #pragma unroll
   for (int j = 0; j < Slot<KT>::NSUB; ++j) {
     uint64_t v = ld_relaxed(&p->sub[j]);
