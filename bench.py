@@ -353,7 +353,7 @@ def main():
                                            "n_unitigs", "n_cycle_nodes", "iterations", "capacity", "device_bytes",
                                            "peak_device_bytes")},
         "roofline": {
-            "kernel": ("count phase: k_parse_records + k_split1 + k_split2 + k_region_build%s + k_spill_flush "
+            "kernel": ("count phase: k_parse_records + k_split + k_region_build%s + k_spill_flush "
                        "(device events around the phase)" % (" (with the filter fused into its write-back)"
                                                               if fused else "")) if stats["count_by_regions"] else
                       "k_parse (parse + atomic k2 count)",
@@ -560,7 +560,7 @@ def run_batched(args, free):
         "per_job_results_equal": bool(same and inst1 == inst),
         "peak_device_gb": peak / 1e9,
         "roofline": {
-            "kernel": "count phase, all groups (a batch: k_parse, the atomic count; a large job alone: the region count)",
+            "kernel": "count phase, all groups (the region count; groups of small tables: k_parse, the atomic count)",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,

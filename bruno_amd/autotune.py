@@ -3,9 +3,9 @@
 The knobs change speed only, never results:
   load factor   hash slots per distinct k-mer (count probes vs. table size,
                 which the filter scan and the table reset stream);
-  region_slots  region size of a region-layout table (k <= 31 plain jobs);
-  count_groups  sub-bucket groups of the region count's split / build
-                pipeline (0: automatic);
+  region_slots  region size of a region-layout table;
+  count_groups  bucket groups of the region count's split / build pipeline
+                (0 and 1: one after the other);
   parse_block   workgroup size of the atomic parse + count kernel;
   parse_grid    waves of the atomic parse + count launch;
   scan_grid     workgroups of the filter's table scan (atomic-count tables);

@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <queue>
 #include <type_traits>
 #include <vector>
 
@@ -148,26 +149,32 @@ __global__ __launch_bounds__(BLOCK) void k_filter_scan(const Slot<KT>* T, uint64
 
 /* The filter pre-pass from the bits a region build left (regions.h):
  * candidate and spilled slots of a region-layout table in slot order,
- * FILTER_BITS_WPT words per thread per reservation. */
+ * FILTER_BITS_WPT words per thread per reservation.  Word w belongs to
+ * region w / stride (stride: the words of the largest region of any job). */
 constexpr int FILTER_BITS_WPT = 8;
 __global__ __launch_bounds__(BLOCK) void k_filter_bits(const uint64_t* cbits, const uint64_t* sbits, uint64_t n_regions,
-                                                       uint64_t stride, uint64_t span, uint64_t* cand,
-                                                       uint64_t cand_cap, uint64_t* spilled, uint64_t spilled_cap,
-                                                       Counters* ctr) {
+                                                       uint64_t stride, const JobLayout* lay, uint32_t n_jobs,
+                                                       uint64_t* cand, uint64_t cand_cap, uint64_t* spilled,
+                                                       uint64_t spilled_cap, Counters* ctr) {
   __shared__ ReserveSmem sm;
   __shared__ ReserveSmem sm2;
-  const uint64_t n_words = n_regions * stride, used = (span + 63) / 64;
+  const uint64_t n_words = n_regions * stride;
   const uint64_t tile = (uint64_t)BLOCK * FILTER_BITS_WPT;
   for (uint64_t base = (uint64_t)blockIdx.x * tile; base < n_words; base += (uint64_t)gridDim.x * tile) {
-    uint64_t cw[FILTER_BITS_WPT], sw[FILTER_BITS_WPT];
+    uint64_t cw[FILTER_BITS_WPT], sw[FILTER_BITS_WPT], s0[FILTER_BITS_WPT];
     uint32_t nc = 0, ns = 0;
 #pragma unroll
     for (int q = 0; q < FILTER_BITS_WPT; ++q) {
       const uint64_t w = base + (uint64_t)q * BLOCK + threadIdx.x;
-      cw[q] = sw[q] = 0;
-      if (w < n_words && w % stride < used) {
-        cw[q] = cbits[w];
-        sw[q] = sbits[w];
+      cw[q] = sw[q] = s0[q] = 0;
+      if (w < n_words) {
+        const uint32_t r = (uint32_t)(w / stride), at = (uint32_t)(w - (uint64_t)r * stride) * 64;
+        const JobLayout& l = lay[n_jobs > 1 ? count_job_of(n_jobs, r, [&](uint32_t j) { return lay[j].region0; }) : 0];
+        if (at < l.span) {
+          cw[q] = cbits[w];
+          sw[q] = sbits[w];
+          s0[q] = l.slot0 + (uint64_t)(r - l.region0) * l.span + at;
+        }
       }
       nc += __popcll(cw[q]);
       ns += __popcll(sw[q]);
@@ -176,14 +183,12 @@ __global__ __launch_bounds__(BLOCK) void k_filter_bits(const uint64_t* cbits, co
     unsigned long long ps = block_reserve(ns, &ctr->n_spill, sm2);
 #pragma unroll
     for (int q = 0; q < FILTER_BITS_WPT; ++q) {
-      const uint64_t w = base + (uint64_t)q * BLOCK + threadIdx.x;
-      const uint64_t s0 = (w / stride) * span + (w % stride) * 64;
       for (uint64_t m = cw[q]; m; m &= m - 1) {
-        if (pc < cand_cap) cand[pc] = s0 + __builtin_ctzll(m);
+        if (pc < cand_cap) cand[pc] = s0[q] + __builtin_ctzll(m);
         ++pc;
       }
       for (uint64_t m = sw[q]; m; m &= m - 1) {
-        if (ps < spilled_cap) spilled[ps] = s0 + __builtin_ctzll(m);
+        if (ps < spilled_cap) spilled[ps] = s0[q] + __builtin_ctzll(m);
         ++ps;
       }
     }
@@ -449,7 +454,7 @@ __device__ void resolve_pair(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, u
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_t cap, uint32_t rbits, int K,
                                                       const uint64_t* chain_slot,
-                                                      const uint32_t* chain_job, const uint64_t* seg, uint32_t n_jobs,
+                                                      const uint32_t* chain_job, const JobLayout* lay, uint32_t n_jobs,
                                                       uint64_t n_chain, KT* ckmer, const uint8_t* cedge, LRNode* lr,
                                                       KT* vkmer, uint64_t vcap, uint64_t ruler_mask,
                                                       uint64_t* ruler_bits, uint8_t* alive, Counters* ctr) {
@@ -458,10 +463,12 @@ __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_
   unsigned long long ill = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n_chain; i += stride) {
     uint64_t tbase = 0, tcap = cap;
+    uint32_t rb = rbits;
     if (n_jobs > 1) {
-      const uint32_t job = chain_job[i];
-      tbase = seg[job];
-      tcap = seg[job + 1] - tbase;
+      const JobLayout l = lay[chain_job[i]];
+      tbase = l.slot0;
+      tcap = l.span;
+      rb = l.rbits;
     }
     /* a chain node has at most one in and one out edge: from the filter's
      * k-mer and edge byte when it left them, else from the node's slot */
@@ -489,7 +496,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_
     /* in neighbour c.k[0..K-2]: when canonical its OUT end faces k; out
      * neighbour k[1..].c: when canonical its IN end faces k */
     bool in_branch = false, out_branch = false;
-    resolve_pair<KT>(T, tbase, tcap, rbits, ops, k, (uint32_t)i, ci >= 0, ops.in_nbr(k, ci < 0 ? 0 : ci), co >= 0,
+    resolve_pair<KT>(T, tbase, tcap, rb, ops, k, (uint32_t)i, ci >= 0, ops.in_nbr(k, ci < 0 ? 0 : ci), co >= 0,
                      ops.out_nbr(k, co < 0 ? 0 : co), n_chain, vkmer, vcap, ctr, st.p[0], st.p[1], in_branch, out_branch,
                      ill);
     if (ci >= 0) st.d[0] = in_branch ? 0 : 1;
@@ -510,17 +517,19 @@ __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_termini(const Slot<KT>* T, uint64_t cap, uint32_t rbits, int K,
                                                    const uint64_t* branch_slot,
-                                                   const uint32_t* branch_job, const uint64_t* seg, uint32_t n_jobs,
+                                                   const uint32_t* branch_job, const JobLayout* lay, uint32_t n_jobs,
                                                    uint64_t n_branch, LRNode* lr, KT* bkmer) {
   kops<KT> ops(K);
   const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n_branch; i += stride) {
     const Slot<KT>* p = T + branch_slot[i];
     uint64_t tbase = 0, tcap = cap;
+    uint32_t rb = rbits;
     if (n_jobs > 1) {
-      const uint32_t job = branch_job[i];
-      tbase = seg[job];
-      tcap = seg[job + 1] - tbase;
+      const JobLayout l = lay[branch_job[i]];
+      tbase = l.slot0;
+      tcap = l.span;
+      rb = l.rbits;
     }
     KT k = SlotOps<KT>::kmer(p);
     bkmer[i] = k;
@@ -535,7 +544,7 @@ __global__ __launch_bounds__(BLOCK) void k_termini(const Slot<KT>* T, uint64_t c
         KT rn = ops.rc(n);
         bool flipped = !(n < rn);
         KT cn = flipped ? rn : n;
-        uint64_t s = SlotOps<KT>::find(T + tbase, tcap, rbits, cn, true);
+        uint64_t s = SlotOps<KT>::find(T + tbase, tcap, rb, cn, true);
         if (s == ~0ULL) continue;
         const NodeRec* q = (const NodeRec*)&T[tbase + s].sub[0];
         if (q->cls != CLS_CHAIN) continue;
@@ -797,8 +806,21 @@ __global__ void k_gather_kmer(const KT* src, const uint32_t* perm, KT* dst, uint
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[perm[i]];
 }
-__global__ void k_add_u64(unsigned long long* dst, const unsigned long long* src, uint32_t n) {
-  if (threadIdx.x < n) dst[threadIdx.x] += src[threadIdx.x];
+/* a region count's instances and dropped reads (stat, per job) into the
+ * table's counters and a batch's per-job ones (n_jobs instances, then
+ * n_jobs dropped reads); nothing when the count gave up */
+__global__ void k_add_job_stats(const unsigned long long* stat, uint32_t ja, uint32_t jb, const uint32_t* overflow,
+                                unsigned long long* jstat, uint32_t n_jobs, Counters* ctr) {
+  if (*overflow) return;
+  for (uint32_t q = ja + blockIdx.x * blockDim.x + threadIdx.x; q < jb; q += gridDim.x * blockDim.x) {
+    const unsigned long long n = stat[2 * (uint64_t)q], d = stat[2 * (uint64_t)q + 1];
+    if (n) atomicAdd(&ctr->n_instances, n);
+    if (d) atomicAdd(&ctr->n_dropped, d);
+    if (jstat) {
+      jstat[q] += n;
+      jstat[n_jobs + q] += d;
+    }
+  }
 }
 __global__ void k_gather_u32(const uint32_t* src, const uint32_t* perm, uint32_t* dst, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1211,9 +1233,9 @@ inline hipStream_t shared_count_stream() {
   }
   return s[dev];
 }
-/* sub-bucket groups of a pipelined region count: at most this many chosen
- * automatically, at most MAX_COUNT_GROUPS by the tuning knob */
-constexpr uint64_t COUNT_GROUPS = 16, MAX_COUNT_GROUPS = 64;
+/* groups of buckets of a pipelined region count: at most this many
+ * (the count_groups knob) */
+constexpr uint64_t MAX_COUNT_GROUPS = 64;
 
 enum Stage { ST_CREATED = 0, ST_COUNTED = 1, ST_FILTERED = 2, ST_CHAINS = 3, ST_RANKED = 4, ST_COMPACTED = 5 };
 
@@ -1230,14 +1252,18 @@ struct bruno_job {
 
   uint64_t cap = 0, spcap = 0;
   void* table = nullptr;
-  /* Region layout (plain jobs with k <= 31 and a large table): 2^rbits
-   * regions of rspan slots, each small enough for one workgroup's LDS, so
-   * a count can build every region on chip from instance records grouped
-   * by region.  rbits == 0: one probe window over the whole table (or a
-   * batch job's segment). */
+  /* Region layout (large tables): every job of the table has 2^rbits
+   * regions of span slots, each small enough for one workgroup's LDS, so a
+   * count can build every region on chip from instance records grouped by
+   * region.  Else one probe window over the whole table (or a batch job's
+   * segment).  lay: per job (d_lay on the device); rbits, rspan: a plain
+   * job's. */
+  bool regions = false;
+  std::vector<JobLayout> lay;
+  JobLayout* d_lay = nullptr;
   uint32_t rbits = 0;
   uint64_t rspan = 0;
-  bool region_ok = false;     /* plain job: the region layout may be chosen */
+  uint64_t n_regions = 0, n_buckets = 0, bit_stride = 0;
   bool table_valid = false;   /* every slot holds a key or EMPTY (else it is stale) */
   bool by_regions = false;    /* the last count built the table region by region */
   /* the only count since the reset built every region and left the filter
@@ -1444,7 +1470,7 @@ size_t slot_bytes(const bruno_job* j) { return j->words == 1 ? sizeof(Slot<uint6
  * region-layout table is only marked stale: the next count writes every
  * slot (or ensure_table_valid fills it). */
 void clear_table(bruno_job* j, hipStream_t st) {
-  if (j->rbits) {
+  if (j->regions) {
     j->table_valid = false;
   } else {
     fill64(j, j->table, j->cap * slot_bytes(j) / 8, EMPTY64, st);
@@ -1468,33 +1494,76 @@ double ev_ms(bruno_job* j, int a, int b) {
 }
 
 
-/* Tables of at least this many slots get the region layout (count_regions
- * 1 or 2).  Measured on jobs of 2^22 to 2^26 slots counted alone, the
- * region count and the filter after it save 1.1 to 6.7 ms per job over
- * the atomic count (below 2^22 the layout is not offered). */
+/* Tables of at least this many slots (all jobs of a batch together) get the
+ * region layout (count_regions 1 or 2).  Measured on jobs of 2^22 to 2^26
+ * slots counted alone, the region count and the filter after it save 1.1 to
+ * 6.7 ms per job over the atomic count (below 2^22 the layout is not
+ * offered); a batch of 16 jobs with 2^28 slots together, 243 M instances,
+ * counts in 5.9 ms instead of 18.6. */
 constexpr uint64_t REGION_MIN_CAP = 1ULL << 22;
 constexpr uint64_t REGION_MIN_CAP_ANY = 1ULL << 22;
 
-/* One table for all jobs: job i gets caps[i] slots from seg[i].  A plain
- * k <= 31 job with a large table gets 2^rbits regions of at most
- * region_slots slots (the capacity rounds up to a whole number of
- * regions); its slots are written by the first count, not filled here. */
+/* Region layout of a table of cap slots: at least 2^REC_BUCKET_BITS regions
+ * of at most `most` slots.  A batch job's capacity is its caller's number,
+ * filled as far as the caller likes, so its regions get room for the spread
+ * of their k-mers (six standard deviations of a region's mean at load 1); a
+ * plain job's table only rounds up to whole regions. */
+void region_layout(uint64_t cap, uint64_t most, bool spread, uint32_t* rbits, uint64_t* span) {
+  uint32_t b = REC_BUCKET_BITS;
+  for (;; ++b) {
+    uint64_t s = (cap + (1ULL << b) - 1) >> b;
+    if (spread) s += (uint64_t)(6.0 * std::sqrt((double)s)) + 16;
+    if (s <= most) {
+      *rbits = b;
+      *span = s;
+      return;
+    }
+  }
+}
+
+/* One table for all jobs: job i gets caps[i] slots (with the region layout,
+ * a whole number of regions) from seg[i].  A region table's slots are
+ * written by the first count, not filled here. */
 bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
   const uint32_t nj = j->n_jobs;
-  j->seg.assign(nj + 1, 0);
-  for (uint32_t i = 0; i < nj; ++i) j->seg[i + 1] = j->seg[i] + caps[i];
-  j->rbits = 0;
-  j->rspan = 0;
   const uint32_t cr = tuning().count_regions;
-  if (nj == 1 && j->region_ok && cr && j->seg[1] >= (cr >= 2 ? REGION_MIN_CAP_ANY : REGION_MIN_CAP)) {
-    uint32_t b = REC_BUCKET_BITS;
-    /* the knob counts 32-byte slots: a 64-byte-slot region holds half */
-    const uint64_t most = j->words == 1 ? tuning().region_slots : tuning().region_slots / 2;
-    while ((j->seg[1] + (1ULL << b) - 1) >> b > most) ++b;
-    j->rbits = b;
-    j->rspan = (j->seg[1] + (1ULL << b) - 1) >> b;
-    j->seg[1] = j->rspan << b;
+  uint64_t total = 0, n_reg = 0, n_buck = 0, max_span = 0;
+  for (uint32_t i = 0; i < nj; ++i) total += caps[i];
+  j->regions = cr && total >= (cr >= 2 ? REGION_MIN_CAP_ANY : REGION_MIN_CAP);
+  /* the knob counts 32-byte slots: a 64-byte-slot region holds half */
+  const uint64_t most = j->words == 1 ? tuning().region_slots : tuning().region_slots / 2;
+  j->lay.assign(nj, JobLayout{});
+  if (j->regions) {
+    for (uint32_t i = 0; i < nj; ++i) {
+      JobLayout& l = j->lay[i];
+      region_layout(caps[i], most, nj > 1, &l.rbits, &l.span);
+      /* buckets: one per CU, 512 when one split pass would have more than
+       * SPLIT_BITS region bits left */
+      l.beta = std::min<uint32_t>(l.rbits, l.rbits > 8 + SPLIT_BITS ? MAX_BUCKET_BITS : 8);
+      l.region0 = (uint32_t)n_reg;
+      l.bucket0 = (uint32_t)n_buck;
+      n_reg += 1ULL << l.rbits;
+      n_buck += 1ULL << l.beta;
+      max_span = std::max(max_span, l.span);
+    }
+    /* regions and buckets are numbered in 32 bits */
+    if (n_reg >= (1ULL << 31) || n_buck >= (1ULL << 31)) j->regions = false;
   }
+  j->seg.assign(nj + 1, 0);
+  for (uint32_t i = 0; i < nj; ++i) {
+    JobLayout& l = j->lay[i];
+    if (!j->regions) {
+      l = JobLayout{};
+      l.span = caps[i];
+    }
+    l.slot0 = j->seg[i];
+    j->seg[i + 1] = j->seg[i] + (l.span << l.rbits);
+  }
+  j->n_regions = n_reg;
+  j->n_buckets = n_buck;
+  j->bit_stride = (max_span + 63) / 64;
+  j->rbits = nj == 1 ? j->lay[0].rbits : 0;
+  j->rspan = nj == 1 && j->regions ? j->lay[0].span : 0;
   const uint64_t cap = j->seg[nj];
   j->cap = cap;
   TRY(dev_alloc(j, &j->table, cap * slot_bytes(j)));
@@ -1503,10 +1572,12 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
   j->spcap = std::max<uint64_t>(1024, cap / 32);
   TRY(dev_alloc(j, (void**)&j->spill, j->spcap * sizeof(Spill)));
   TRY(dev_alloc(j, (void**)&j->d_seg, (nj + 1) * sizeof(uint64_t)));
+  TRY(dev_alloc(j, (void**)&j->d_lay, nj * sizeof(JobLayout)));
   TRY(dev_alloc(j, (void**)&j->d_jstat, 2 * nj * sizeof(unsigned long long)));
   HIP_CHECK(hipMemcpyAsync(j->d_seg, j->seg.data(), (nj + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, j->stream));
+  HIP_CHECK(hipMemcpyAsync(j->d_lay, j->lay.data(), nj * sizeof(JobLayout), hipMemcpyHostToDevice, j->stream));
   j->table_valid = false;
-  if (!j->rbits) {
+  if (!j->regions) {
     fill64(j, j->table, cap * slot_bytes(j) / 8, EMPTY64);
     j->table_valid = true;
   }
@@ -1516,7 +1587,7 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
 }
 
 /* probe span of a plain job: one region, or the whole table */
-uint64_t probe_span(const bruno_job* j) { return j->rbits ? j->rspan : j->cap; }
+uint64_t probe_span(const bruno_job* j) { return j->regions && j->n_jobs == 1 ? j->rspan : j->cap; }
 
 /* The filter pre-pass keeps a k-mer when its count can reach the lower
  * bound.  An edge count of the k2 filter is at most the k-mer count, and so
@@ -1537,12 +1608,13 @@ void ensure_table_valid(bruno_job* j) {
 }
 
 bool persistent(const bruno_job* j, const void* p) {
-  return p == j->table || p == j->spill || p == j->d_seg || p == j->d_jstat || (p && p == j->sketch);
+  return p == j->table || p == j->spill || p == j->d_seg || p == j->d_lay || p == j->d_jstat || (p && p == j->sketch);
 }
 uint64_t persistent_bytes(const bruno_job* j) {
   const uint64_t sk = j->sketch ? SKETCH_M * 4 : 0;
   if (!j->table) return sk;
   return j->cap * slot_bytes(j) + j->spcap * sizeof(Spill) + (j->n_jobs + 1) * sizeof(uint64_t) +
+         j->n_jobs * sizeof(JobLayout) +
          2 * j->n_jobs * sizeof(unsigned long long) + sk;
 }
 
@@ -1623,12 +1695,17 @@ bruno_status grow_table(bruno_job* j, uint64_t want) {
   void* osp = j->spill;
   void* oseg = j->d_seg;
   void* ojs = j->d_jstat;
+  void* olay = j->d_lay;
+  const bool oregions = j->regions;
+  const std::vector<JobLayout> olay_h = j->lay;
+  const uint64_t onreg = j->n_regions, onbuck = j->n_buckets, ostride = j->bit_stride;
   const uint64_t ocap = j->cap, ospcap = j->spcap;
   const uint32_t orbits = j->rbits;
   const uint64_t orspan = j->rspan;
   const std::vector<uint64_t> oseg_h = j->seg;
   j->table = j->spill = nullptr;
   j->d_seg = nullptr;
+  j->d_lay = nullptr;
   j->d_jstat = nullptr;
   bruno_status st = alloc_table(j, &want);
   uint64_t* remap = nullptr;
@@ -1640,6 +1717,13 @@ bruno_status grow_table(bruno_job* j, uint64_t want) {
     p = j->spill; dev_free(j, p, j->spcap * sizeof(Spill));
     p = j->d_seg; dev_free(j, p, (j->n_jobs + 1) * 8);
     p = j->d_jstat; dev_free(j, p, 2 * j->n_jobs * 8);
+    p = j->d_lay; dev_free(j, p, j->n_jobs * sizeof(JobLayout));
+    j->d_lay = (JobLayout*)olay;
+    j->regions = oregions;
+    j->lay = olay_h;
+    j->n_regions = onreg;
+    j->n_buckets = onbuck;
+    j->bit_stride = ostride;
     j->table = otab;
     j->spill = (Spill*)osp;
     j->d_seg = (uint64_t*)oseg;
@@ -1673,6 +1757,7 @@ bruno_status grow_table(bruno_job* j, uint64_t want) {
   dev_free(j, osp, ospcap * sizeof(Spill));
   dev_free(j, oseg, (j->n_jobs + 1) * 8);
   dev_free(j, ojs, 2 * j->n_jobs * 8);
+  dev_free(j, olay, j->n_jobs * sizeof(JobLayout));
   j->bits_fresh = false;
   j->by_regions = false;
   return s2;
@@ -1703,220 +1788,176 @@ bruno_status autosize(bruno_job* j, const char* d_bases, const uint64_t* d_offse
   return BRUNO_OK;
 }
 
-/* Count one batch of reads into a region-layout table (regions.h): bucketed
- * instance records, two multisplit passes that group each bucket's records
- * by region (partition.h), one on-chip build per region.  *done = false
- * (and nothing counted) when the record buffers do not fit, a bucket
- * overflowed its share, or the table has more regions than two passes
- * split; the caller then counts with atomics. */
-/* record staging per bucket in the parser's LDS: 48 KB of records */
-/* the record parser's shape: 16-byte records (k > 31) stage half as many
- * per bucket in the same LDS, so the workgroup appends four times as often
- * (a quarter of the records per append, under the halved threshold) */
-template <typename KT> struct RecShape {
-  static constexpr bool wide = sizeof(typename RecOf<KT>::T) == 16;
-  static constexpr int BS = REC_BS, PF = wide ? REC_PF / 4 : REC_PF;
-  static constexpr int STAGE = wide ? REC_STAGE / 2 : REC_STAGE, FLUSH = wide ? REC_FLUSH / 2 : REC_FLUSH;
-};
+/* Records of a region count's pass over several jobs of a batch: at most
+ * this many bytes of them (a job with more is a pass of its own), so the record
+ * buffers of a batch stay small beside its table. */
+constexpr uint64_t REC_PASS_BYTES = 1ULL << 32;
 
+/* Jobs [ja, jb) counted by regions: the reads of these jobs into bucketed
+ * instance records, one multisplit pass that groups each bucket's records by
+ * region (partition.h), one on-chip build per region.  *done = false (and
+ * nothing counted) when the record buffers do not fit or a bucket got a
+ * large share of the records; the caller then counts with atomics. */
 template <typename KT>
-bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, bool* done) {
+bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t* d_first, const uint64_t* h_first,
+                                uint32_t ja, uint32_t jb, const std::vector<unsigned long long>& inst, int valid,
+                                uint64_t* cbits, uint64_t* sbits, bool* done) {
   typedef typename RecOf<KT>::T R;
-  constexpr int STAGE = RecShape<KT>::STAGE;
   constexpr uint64_t RB = sizeof(R);
   *done = false;
-  const uint64_t n_reads = a.n_reads;
-  const int rb = (int)j->rbits - REC_BUCKET_BITS; /* region bits inside a bucket */
-  const int b1 = std::min(std::max(rb - 8, 0), SPLIT1_MAX_BITS), b2 = rb - b1;
-  if (rb < 0 || b2 > SPLIT2_MAX_BITS) return BRUNO_OK;
-  const uint64_t n_sb = (uint64_t)REC_BUCKETS << b1, nreg = 1ULL << j->rbits;
-  /* scratch: front / back per bucket, instances and dropped reads, the
-   * instance bound, the first pass's overflow flag, its cursors and exact
-   * counts (when the first try overflows) */
-  const uint64_t NS = 2 * REC_BUCKETS + 4 + 2 * n_sb;
-  unsigned long long* scratch = nullptr;
-  TRY(dev_alloc(j, (void**)&scratch, NS * 8));
-  unsigned long long *front = scratch, *back = scratch + REC_BUCKETS, *stat = scratch + 2 * REC_BUCKETS,
-                     *bound = stat + 2, *overflow = bound + 1, *cursor = overflow + 1, *counts = cursor + n_sb;
-  void* sp = scratch;
-  HIP_CHECK(hipMemsetAsync(scratch, 0, NS * 8, j->stream));
-  hipLaunchKernelGGL(k_count_instances, dim3(grid_for(n_reads)), dim3(BLOCK), 0, j->stream, a, bound);
-  unsigned long long n_bound = 0;
-  HIP_CHECK(hipMemcpyAsync(&n_bound, bound, 8, hipMemcpyDeviceToHost, j->stream));
-  HIP_CHECK(hipStreamSynchronize(j->stream));
-  typedef RecShape<KT> RS;
-  auto parse_kernel = k_parse_records<KT, RS::BS, RS::PF, RS::STAGE, RS::FLUSH>;
-  /* persistent: exactly the workgroups that fit on the device at once */
-  static int per_cu = 0;
-  if (per_cu == 0) {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, parse_kernel, RS::BS, 0) != hipSuccess || per_cu <= 0) {
-      (void)hipGetLastError();
-      per_cu = 1;
-    }
+  const uint32_t nj = j->n_jobs;
+  const uint64_t cus = device_cus();
+  const uint32_t b_lo = j->lay[ja].bucket0, b_hi = jb < nj ? j->lay[jb].bucket0 : (uint32_t)j->n_buckets;
+  const uint32_t q_lo = j->lay[ja].region0, q_hi = jb < nj ? j->lay[jb].region0 : (uint32_t)j->n_regions;
+  const uint64_t n_sb = b_hi - b_lo;
+  uint64_t n_inst = 0;
+  uint32_t beta_min = MAX_BUCKET_BITS, beta_max = 0;
+  int b2_max = 0;
+  for (uint32_t q = ja; q < jb; ++q) {
+    n_inst += inst[q];
+    beta_min = std::min(beta_min, j->lay[q].beta);
+    beta_max = std::max(beta_max, j->lay[q].beta);
+    b2_max = std::max(b2_max, (int)(j->lay[q].rbits - j->lay[q].beta));
   }
-  const uint64_t groups =
-      std::max<uint64_t>(1, std::min<uint64_t>((n_reads + RS::BS - 1) / RS::BS, (uint64_t)device_cus() * per_cu));
-  /* chunks of up to 2048 records, smaller for small inputs so padding
-   * stays under ~1/8 of the records; a flush appends at most REC_STAGE
-   * records, so a chunk holds at least that many */
-  uint32_t chunk = 2048;
-  while (chunk / 2 >= (uint32_t)STAGE && (uint64_t)chunk * groups * REC_BUCKETS * 8 > n_bound) chunk >>= 1;
-  const uint64_t bcap = n_bound / REC_BUCKETS + n_bound / (4 * REC_BUCKETS) + 65536 + groups * chunk;
-  /* each sub-bucket's room in the first pass's output: its share of the
-   * bucket plus 3% and a constant (a sub-bucket's count strays from its
-   * share by about its square root) */
-  auto room = [&](uint64_t n_b) { return (n_b >> b1) + (n_b >> b1) / 32 + 256; };
-  const uint64_t out_cap = n_sb * room(bcap);
-  R* recs = nullptr;
-  /* the parser's buffer also takes the second pass's output (<= the first's) */
-  const uint64_t recs_n = std::max<uint64_t>(REC_BUCKETS * bcap, out_cap);
-  if (dev_alloc(j, (void**)&recs, recs_n * RB) != BRUNO_OK) {
-    dev_free(j, sp, NS * 8);
-    return BRUNO_OK;
-  }
-  void* rp = recs;
-  RecArgs ra{recs, bcap, front, back, stat, chunk};
-  hipLaunchKernelGGL(parse_kernel, dim3((unsigned)groups), dim3(RS::BS), 0,
-                     j->stream, a, ra);
-  std::vector<unsigned long long> hcur(2 * REC_BUCKETS);
-  HIP_CHECK(hipMemcpyAsync(hcur.data(), front, 2 * REC_BUCKETS * 8, hipMemcpyDeviceToHost, j->stream));
-  HIP_CHECK(hipStreamSynchronize(j->stream));
-  bool over = false;
-  for (int b = 0; b < REC_BUCKETS; ++b) over |= hcur[b] + hcur[REC_BUCKETS + b] > bcap;
-  /* sub-bucket rooms from the bucket sizes (records plus chunk padding) */
-  std::vector<uint64_t> base(n_sb + 1, 0);
-  for (uint64_t q = 0; q < n_sb; ++q) base[q + 1] = base[q] + room(hcur[q >> b1] + hcur[REC_BUCKETS + (q >> b1)]);
-  R* recs2 = nullptr;
-  uint64_t *d_base = nullptr, *d_out = nullptr, *rstart = nullptr;
-  const uint64_t C = base[n_sb];
-  auto give_up = [&]() {
-    void* p = rstart;
-    dev_free(j, p, (nreg + 1) * 8);
-    p = d_out;
-    dev_free(j, p, (n_sb + 1) * 8);
-    p = d_base;
-    dev_free(j, p, (n_sb + 1) * 8);
-    p = recs2;
-    dev_free(j, p, std::max<uint64_t>(1, C) * RB);
-    dev_free(j, rp, recs_n * RB);
-    dev_free(j, sp, NS * 8);
+  if (b2_max > SPLIT_MAX_BITS) return BRUNO_OK;
+  /* parser workgroups: one per CU and at least one per job with reads, each
+   * next one to the job whose workgroups have the most instances (a wave's
+   * reads or more per workgroup) */
+  std::vector<uint32_t> wgs(jb - ja, 0);
+  std::priority_queue<std::pair<double, uint32_t>> most;
+  uint64_t given = 0;
+  auto give = [&](uint32_t q) {
+    const uint64_t nr = h_first[q + 1] - h_first[q], w = ++wgs[q - ja];
+    ++given;
+    if (w * 64 < nr) most.push({(double)inst[q] / (double)w, q});
   };
-  if (over || dev_alloc(j, (void**)&recs2, std::max<uint64_t>(1, C) * RB) != BRUNO_OK ||
-      dev_alloc(j, (void**)&d_base, (n_sb + 1) * 8) != BRUNO_OK ||
-      dev_alloc(j, (void**)&d_out, (n_sb + 1) * 8) != BRUNO_OK ||
-      dev_alloc(j, (void**)&rstart, (nreg + 1) * 8) != BRUNO_OK) {
-    give_up();
-    return BRUNO_OK;
+  for (uint32_t q = ja; q < jb; ++q)
+    if (h_first[q + 1] > h_first[q]) give(q);
+  while (given < cus && !most.empty()) {
+    const uint32_t q = most.top().second;
+    most.pop();
+    give(q);
   }
-  /* pass 1: the chunked front of every bucket and the records appended
-   * from its back, by the top b1 region bits */
-  Split1Args s1{};
-  s1.in = recs;
-  s1.b1 = b1;
-  s1.cursor = cursor;
-  s1.limit = d_base + 1;
-  s1.out = recs2;
-  s1.overflow = overflow;
-  /* segments (tiles numbered through them) grouped by the XCD that splits
-   * their bucket, bucket % SPLIT_XCDS */
-  uint64_t tiles = 0;
-  for (int x = 0; x < SPLIT_XCDS; ++x) {
-    s1.xcd_tiles[x] = tiles;
-    for (int b = x; b < REC_BUCKETS; b += SPLIT_XCDS) {
-      const uint64_t ranges[2][2] = {{(uint64_t)b * bcap, (uint64_t)b * bcap + hcur[b]},
-                                     {(uint64_t)(b + 1) * bcap - hcur[REC_BUCKETS + b], (uint64_t)(b + 1) * bcap}};
-      for (auto& r : ranges) {
-        if (r[1] <= r[0]) continue;
-        s1.seg[s1.n_seg++] = SplitSeg{r[0], r[1], tiles, (uint32_t)b, 0};
-        tiles += (r[1] - r[0] + SplitShape<R>::TILE - 1) / SplitShape<R>::TILE;
-      }
-    }
+  std::vector<ParseShare> share;
+  uint64_t open = 0; /* (workgroup, bucket) pairs: chunks that may stay partly filled */
+  for (uint32_t q = ja; q < jb; ++q) {
+    const uint32_t w = wgs[q - ja];
+    open += (uint64_t)w << j->lay[q].beta;
+    for (uint32_t i = 0; i < w; ++i) share.push_back(ParseShare{q, i, w, 0});
   }
-  s1.xcd_tiles[SPLIT_XCDS] = tiles;
-  s1.n_tiles = tiles;
-  const unsigned split_grid = device_cus() * 4;
-  /* k_split1: a multiple of SPLIT_XCDS workgroups */
-  const dim3 g1((unsigned)(SPLIT_XCDS * std::max<uint64_t>(1, std::min<uint64_t>(tiles, split_grid) / SPLIT_XCDS)));
-  std::vector<unsigned long long> cur(n_sb + 1);
-  for (int attempt = 0; attempt < 2; ++attempt) {
-    HIP_CHECK(hipMemcpyAsync(d_base, base.data(), (n_sb + 1) * 8, hipMemcpyHostToDevice, j->stream));
-    HIP_CHECK(hipMemcpyAsync(cursor, base.data(), n_sb * 8, hipMemcpyHostToDevice, j->stream));
-    if (tiles) hipLaunchKernelGGL(k_split1<R>, g1, dim3(SPLIT_BS), 0, j->stream, s1);
-    HIP_CHECK(hipMemcpyAsync(cur.data(), cursor, n_sb * 8, hipMemcpyDeviceToHost, j->stream));
-    HIP_CHECK(hipMemcpyAsync(&cur[n_sb], overflow, 8, hipMemcpyDeviceToHost, j->stream));
-    HIP_CHECK(hipStreamSynchronize(j->stream));
-    if (!cur[n_sb]) break;
-    if (attempt == 1) {
-      give_up();
-      return BRUNO_INTERNAL; /* exact room cannot overflow */
-    }
-    /* a sub-bucket ran out of room: exact counts, then the pass again */
-    HIP_CHECK(hipMemsetAsync(counts, 0, n_sb * 8, j->stream));
-    HIP_CHECK(hipMemsetAsync(overflow, 0, 8, j->stream));
-    hipLaunchKernelGGL(k_split_count<R>, g1, dim3(SPLIT_BS), 0, j->stream, s1, counts);
-    std::vector<unsigned long long> hc(n_sb);
-    HIP_CHECK(hipMemcpyAsync(hc.data(), counts, n_sb * 8, hipMemcpyDeviceToHost, j->stream));
-    HIP_CHECK(hipStreamSynchronize(j->stream));
-    for (uint64_t q = 0; q < n_sb; ++q) base[q + 1] = base[q] + hc[q];
-    if (base[n_sb] > C) {
-      give_up();
-      return BRUNO_INTERNAL;
-    }
-  }
-  /* pass 2: each sub-bucket by the remaining b2 region bits, into the
-   * parser's buffer without gaps, with every region's first record */
-  std::vector<uint64_t> out(n_sb + 1, 0);
-  for (uint64_t q = 0; q < n_sb; ++q) out[q + 1] = out[q] + (cur[q] - base[q]);
-  HIP_CHECK(hipMemcpyAsync(d_out, out.data(), (n_sb + 1) * 8, hipMemcpyHostToDevice, j->stream));
-  HIP_CHECK(hipMemcpyAsync(d_base, base.data(), n_sb * 8, hipMemcpyHostToDevice, j->stream));
-  HIP_CHECK(hipMemcpyAsync(rstart + nreg, &out[n_sb], 8, hipMemcpyHostToDevice, j->stream));
-  hipLaunchKernelGGL(k_region_bounds, dim3(grid_for(n_sb + 1, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream, d_out, n_sb,
-                     b2, rstart);
-  Split2Args s2{recs2, d_base, d_out, 0, n_sb, 64 - b1 - b2, b2, recs, rstart};
-  const int valid = j->table_valid ? 1 : 0;
-  /* a first count builds every region: it also leaves the filter scan's
-   * bits (stale once another count follows) */
-  const uint64_t stride = (j->rspan + 63) / 64, nbits = nreg * stride;
-  uint64_t *cbits = nullptr, *sbits = nullptr;
-  if (!valid && dev_alloc(j, (void**)&cbits, nbits * 8) == BRUNO_OK &&
-      dev_alloc(j, (void**)&sbits, nbits * 8) != BRUNO_OK) {
-    void* cp = cbits;
-    dev_free(j, cp, nbits * 8);
-    cbits = nullptr;
-  }
-  if (!sbits) cbits = nullptr;
-  const dim3 g4((unsigned)std::min<uint64_t>(nreg, 4 * REGION_BUILD_CU_SLOTS)),
-      g2((unsigned)std::min<uint64_t>(nreg, 2 * REGION_BUILD_CU_SLOTS));
-  const bool small = RB == 8 ? j->rspan <= REGION_SMALL_SLOTS : j->rspan <= REGION_WIDE_SMALL_SLOTS;
-  const uint64_t n_waves = small ? (uint64_t)g4.x * 4 : (uint64_t)g2.x * 8;
+  /* chunks of up to 1024 records, smaller for small inputs so padding stays
+   * under ~1/8 of the records; an append holds at most a bucket's stage */
+  const uint64_t stage = (REC_STAGE_BYTES / RB) >> beta_min;
+  uint32_t clog = 10;
+  while (clog > 6 && (1ULL << (clog - 1)) >= stage && (open << clog) * 4 > n_inst) --clog;
+  /* every record's chunk, the partly filled ones, and the numbers struck out
+   * (up to CHUNK_LOW of a batch, a batch at the end) */
+  const uint64_t n_full = (n_inst >> clog) + open;
+  const uint64_t n_chunks = n_full + n_full * CHUNK_LOW / (CHUNK_BATCH - CHUNK_LOW) + (2 * CHUNK_BATCH) * share.size() + 64;
+  if (n_chunks >= (1ULL << 31)) return BRUNO_OK;
+  /* one bucket with more than a 26th of the records (beyond a constant) */
+  const uint64_t limit = ((n_inst / 32 + n_inst / 128 + 65536) >> clog) + 2 * share.size() + 1;
+  const uint64_t nreg = q_hi - q_lo;
+  const uint64_t n_pieces = (n_chunks << (clog - PIECE_LOG)) + nreg;
+  if (n_pieces >= (1ULL << 32)) return BRUNO_OK;
+  uint64_t span_max = 0;
+  for (uint32_t q = ja; q < jb; ++q) span_max = std::max(span_max, j->lay[q].span);
+  const bool small_build = span_max <= (RB == 8 ? REGION_SMALL_SLOTS : REGION_WIDE_SMALL_SLOTS);
+  const uint64_t g_small = 4 * REGION_BUILD_CU_SLOTS, g_large = 2 * REGION_BUILD_CU_SLOTS;
+  const uint64_t build_grid = std::min<uint64_t>(nreg, small_build ? g_small : g_large);
+  const uint64_t n_waves = build_grid * (small_build ? 4 : 8);
   /* side-table queues: a wave's share of the instances / 128 (a k-mer
    * spills only past its slot's sub-entries), at least 1024 entries; a
    * full queue adds inline */
-  uint32_t spq_cap = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(1024, n_bound / 128 / n_waves));
+  uint32_t spq_cap = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(1024, n_inst / 128 / n_waves));
+  /* device buffers, all given back at the end */
+  struct Buf {
+    void* p;
+    uint64_t bytes;
+  };
+  std::vector<Buf> bufs;
+  bool room = true;
+  auto get = [&](uint64_t bytes) -> void* {
+    void* p = nullptr;
+    if (!room || dev_alloc(j, &p, std::max<uint64_t>(16, bytes)) != BRUNO_OK) {
+      room = false;
+      return nullptr;
+    }
+    bufs.push_back(Buf{p, std::max<uint64_t>(16, bytes)});
+    return p;
+  };
+  auto give_back = [&]() {
+    for (Buf& b : bufs) dev_free(j, b.p, b.bytes);
+    bufs.clear();
+  };
+  R* recs = (R*)get((n_chunks << clog) * RB);
+  R* out = (R*)get((n_pieces << PIECE_LOG) * RB);
+  uint16_t* digit_of = (uint16_t*)get(n_pieces * 2);
+  uint32_t* pieces = (uint32_t*)get(n_pieces * 4);
+  uint32_t* owner = (uint32_t*)get(n_chunks * 4);
+  uint32_t* list = (uint32_t*)get(n_chunks * 4);
+  uint32_t* rstart = (uint32_t*)get(nreg * 4);
+  uint32_t* rcount = (uint32_t*)get(nreg * 4);
+  uint32_t* first = (uint32_t*)get((n_sb + 1) * 4);
+  ParseShare* d_share = (ParseShare*)get(share.size() * sizeof(ParseShare));
+  /* zeroed: chunks taken in all and overflow flag, statistics, per bucket
+   * chunks taken and listed */
+  const uint64_t n_zero = 1 + 2 * (uint64_t)nj + (n_sb + 1) / 2 + n_sb * (LISTED_STRIDE / 2);
+  uint64_t* zero = (uint64_t*)get(n_zero * 8);
+  uint32_t* spq_n = (uint32_t*)get(n_waves * 4);
+  if (!room) {
+    give_back();
+    return BRUNO_OK;
+  }
   uint64_t* spq = nullptr;
-  uint32_t* spq_n = nullptr;
-  TRY(dev_alloc(j, (void**)&spq_n, n_waves * 4));
-  if (dev_alloc(j, (void**)&spq, n_waves * spq_cap * 8) != BRUNO_OK) spq_cap = 0;
+  if (dev_alloc(j, (void**)&spq, n_waves * spq_cap * 8) == BRUNO_OK) bufs.push_back(Buf{spq, n_waves * spq_cap * 8});
+  else spq_cap = 0;
+  uint32_t* next = (uint32_t*)zero;
+  uint32_t* overflow = next + 1;
+  unsigned long long* stat = (unsigned long long*)(zero + 1);
+  uint32_t* taken = (uint32_t*)(zero + 1 + 2 * (uint64_t)nj);
+  uint32_t* listed = (uint32_t*)(zero + 1 + 2 * (uint64_t)nj + (n_sb + 1) / 2);
+  fill64(j, zero, n_zero, 0);
+  /* the kernels number buckets and regions through all jobs */
+  ChunkPool pool{recs, clog, (uint32_t)n_chunks, next, taken - b_lo, owner, overflow};
+  if (!share.empty()) {
+    HIP_CHECK(hipMemcpyAsync(d_share, share.data(), share.size() * sizeof(ParseShare), hipMemcpyHostToDevice, j->stream));
+    RecArgs ra{pool, j->d_lay, d_first, d_share, stat};
+    constexpr int PF = RB == 8 ? 8 : 4;
+    const dim3 g((unsigned)share.size());
+    if (beta_max <= 8)
+      hipLaunchKernelGGL((k_parse_records<KT, 256, PF>), g, dim3(REC_BS), 0, j->stream, a, ra);
+    else
+      hipLaunchKernelGGL((k_parse_records<KT, 512, PF / 2>), g, dim3(REC_BS), 0, j->stream, a, ra);
+  }
+  hipLaunchKernelGGL(k_chunk_first, dim3(1), dim3(1024), 0, j->stream, pool, b_lo, b_hi,
+                     (uint32_t)std::min<uint64_t>(limit, ~0u), first - b_lo);
+  hipLaunchKernelGGL(k_chunk_list, dim3(grid_for(n_chunks, BLOCK, 4 * cus)), dim3(BLOCK), 0, j->stream, pool, b_lo,
+                     first - b_lo, listed, list);
+  SplitArgs sa{pool, first - b_lo, list, j->d_lay, nj, b_lo, b_hi, q_lo, out, digit_of, pieces, rstart - q_lo,
+               rcount - q_lo};
+  auto split = [&]() {
+    const dim3 g((unsigned)std::min<uint64_t>(sa.b1 - sa.b0, cus));
+    if (b2_max <= SPLIT_BITS) hipLaunchKernelGGL((k_split<R, SPLIT_BITS>), g, dim3(SPLIT_BS), 0, j->stream, sa);
+    else hipLaunchKernelGGL((k_split<R, SPLIT_MAX_BITS>), g, dim3(SPLIT_BS), 0, j->stream, sa);
+  };
   /* the filter fused into the build (a first count, by request): node
    * lists with room for the nodes the table can hold (at most half its
    * slots, and at most the instances / the count threshold) plus every
    * wave's open chunks; a node that finds no room stays a candidate for
    * the filter pass */
-  bool fuse = j->fuse_filter && cbits && j->n_jobs == 1;
+  bool fuse = j->fuse_filter && cbits && nj == 1;
   NodeLists nl{};
   uint64_t* holes = nullptr;
   uint64_t lcap = 0;
   if (fuse) {
     const uint64_t lo = j->thresholding ? std::max<uint64_t>(1, scan_lo(j)) : 1;
-    lcap = std::min<uint64_t>(j->cap / 2, n_bound / lo) + 2 * FUSE_CHUNK * n_waves + 1024;
+    lcap = std::min<uint64_t>(j->cap / 2, n_inst / lo) + 2 * FUSE_CHUNK * n_waves + 1024;
     lcap = std::min<uint64_t>(lcap, 0x7FFFFFFFULL);
     if (tuning().fuse_list_cap) lcap = std::min<uint64_t>(lcap, tuning().fuse_list_cap);
     uint64_t *cs = nullptr, *bs = nullptr;
     if (dev_alloc(j, (void**)&cs, lcap * 8) == BRUNO_OK && dev_alloc(j, (void**)&bs, lcap * 8) == BRUNO_OK &&
         dev_alloc(j, (void**)&holes, 2 * n_waves * 8) == BRUNO_OK) {
-      j->chain_slot = cs;
-      j->branch_slot = bs;
-      j->list_cap = lcap;
       nl = NodeLists{cs, bs, nullptr, nullptr, lcap, j->d_seg, 1};
       HIP_CHECK(hipMemsetAsync(&j->ctr->n_present, 0, 3 * sizeof(unsigned long long), j->stream));
     } else {
@@ -1930,38 +1971,31 @@ bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, bool* done) {
       fuse = false;
     }
   }
-  RegionArgs g{j->table, j->rspan, j->rbits, nreg, 0, nreg, recs, rstart, valid, j->spill, j->spcap, spq, spq_n,
-               spq_cap, j->ctr, cbits, sbits, stride, j->thresholding, scan_lo(j), fuse ? 1 : 0, j->K, j->th, nl,
-               holes};
-  auto build = [&](auto fuse_tag, hipStream_t st, dim3 b4, dim3 b2_) {
+  RegionArgs g{j->table, j->d_lay, nj, q_lo, q_hi, out, pieces, rstart - q_lo, rcount - q_lo, overflow, valid, j->spill, j->spcap,
+               spq, spq_n, spq_cap, j->ctr, cbits, sbits, j->bit_stride, j->thresholding, scan_lo(j), fuse ? 1 : 0, j->K,
+               j->th, nl, holes};
+  auto build = [&](auto fuse_tag, hipStream_t st) {
     constexpr bool F = decltype(fuse_tag)::value;
+    const dim3 b((unsigned)std::min<uint64_t>(g.q1 - g.q0, build_grid));
     if (RB == 8) {
-      if (j->rspan <= REGION_SMALL_SLOTS)
-        hipLaunchKernelGGL((k_region_build<uint64_t, REGION_SMALL_SLOTS, 256, F>), b4, dim3(256), 0, st, g);
-      else
-        hipLaunchKernelGGL((k_region_build<uint64_t, REGION_MAX_SLOTS, 512, F>), b2_, dim3(512), 0, st, g);
+      if (small_build) hipLaunchKernelGGL((k_region_build<uint64_t, REGION_SMALL_SLOTS, 256, F>), b, dim3(256), 0, st, g);
+      else hipLaunchKernelGGL((k_region_build<uint64_t, REGION_MAX_SLOTS, 512, F>), b, dim3(512), 0, st, g);
     } else {
-      if (j->rspan <= REGION_WIDE_SMALL_SLOTS)
-        hipLaunchKernelGGL((k_region_build<u128, REGION_WIDE_SMALL_SLOTS, 256, F>), b4, dim3(256), 0, st, g);
-      else
-        hipLaunchKernelGGL((k_region_build<u128, REGION_WIDE_SLOTS, 512, F>), b2_, dim3(512), 0, st, g);
+      if (small_build) hipLaunchKernelGGL((k_region_build<u128, REGION_WIDE_SMALL_SLOTS, 256, F>), b, dim3(256), 0, st, g);
+      else hipLaunchKernelGGL((k_region_build<u128, REGION_WIDE_SLOTS, 512, F>), b, dim3(512), 0, st, g);
     }
+    /* this launch's waves' side-table queues */
+    if (spq_cap)
+      hipLaunchKernelGGL(k_spill_flush, dim3(b.x * (small_build ? 4 : 8)), dim3(BLOCK), 0, st, spq, spq_n, spq_cap, overflow,
+                         j->spill, j->spcap, j->ctr);
   };
-  /* Pass 2 and the builds, pipelined by groups of sub-buckets: the build
-   * of a group (bound by instruction issue and LDS) runs on a second stream
-   * beside the next group's multisplit (bound by HBM).  A pipelined pass 2
-   * runs one workgroup per CU, which leaves every CU's LDS room for a
-   * region build beside it.  By default only large counts are pipelined,
-   * from 8 sub-buckets per CU, in groups of at least half a sub-bucket per
-   * CU: on fewer sub-buckets the split's narrower launches and the builds'
-   * shared CUs cost more than the overlap gives (measured: 512 sub-buckets
-   * in two groups, 4.5 -> 5.6 ms).  One group when the filter is fused (its
-   * list chunks and holes belong to one launch). */
-  const uint64_t cus = device_cus();
-  uint64_t want = tuning().count_groups;
-  if (want == 0) want = n_sb >= 8 * cus ? std::min<uint64_t>(COUNT_GROUPS, 2 * n_sb / cus) : 1;
-  want = std::min<uint64_t>(std::min<uint64_t>(want, MAX_COUNT_GROUPS), n_sb);
-  hipStream_t bst = (fuse || want < 2) ? nullptr : shared_count_stream();
+  /* Split and builds one after the other, or (count_groups) in groups of a
+   * plain job's buckets, a group's builds on a second stream beside the
+   * next group's split.  One split workgroup fills a CU's LDS, so the two
+   * share the device by CUs, not within them: one group is the default. */
+  uint64_t ng = std::min<uint64_t>(std::min<uint64_t>(tuning().count_groups, MAX_COUNT_GROUPS), n_sb);
+  if (ng < 2 || fuse || nj > 1) ng = 1;
+  hipStream_t bst = ng > 1 ? shared_count_stream() : nullptr;
   if (bst) {
     for (hipEvent_t& e : j->cev)
       if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
@@ -1970,66 +2004,150 @@ bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, bool* done) {
         bst = nullptr;
       }
   }
-  const uint64_t ng = bst ? want : 1;
-  if (!bst) bst = j->stream;
+  if (!bst) {
+    ng = 1;
+    bst = j->stream;
+  }
+  const uint32_t b2 = j->lay[ja].rbits - j->lay[ja].beta;
   for (uint64_t gi = 0; gi < ng; ++gi) {
-    const uint64_t sb0 = n_sb * gi / ng, sb1 = n_sb * (gi + 1) / ng;
-    if (sb1 == sb0) continue;
-    s2.sb0 = sb0;
-    s2.n_sb = sb1 - sb0;
-    hipLaunchKernelGGL(k_split2<R>, dim3((unsigned)std::min<uint64_t>(sb1 - sb0, ng > 1 ? device_cus() : split_grid)),
-                       dim3(SPLIT_BS), 0, j->stream, s2);
+    if (ng > 1) {
+      sa.b0 = (uint32_t)(n_sb * gi / ng);
+      sa.b1 = (uint32_t)(n_sb * (gi + 1) / ng);
+      if (sa.b0 == sa.b1) continue;
+      g.q0 = sa.b0 << b2;
+      g.q1 = sa.b1 << b2;
+    }
+    split();
     if (bst != j->stream) {
       HIP_CHECK(hipEventRecord(j->cev[0], j->stream));
       HIP_CHECK(hipStreamWaitEvent(bst, j->cev[0], 0));
     }
-    g.q0 = sb0 << b2;
-    g.q1 = sb1 << b2;
-    const uint64_t nq = g.q1 - g.q0;
-    const dim3 b4((unsigned)std::min<uint64_t>(nq, 4 * REGION_BUILD_CU_SLOTS)),
-        b2d((unsigned)std::min<uint64_t>(nq, 2 * REGION_BUILD_CU_SLOTS));
-    if (fuse) build(std::true_type{}, bst, b4, b2d);
-    else build(std::false_type{}, bst, b4, b2d);
-    /* this launch's waves' side-table queues */
-    if (spq_cap)
-      hipLaunchKernelGGL(k_spill_flush, dim3(small ? b4.x * 4 : b2d.x * 8), dim3(BLOCK), 0, bst, spq, spq_n, spq_cap,
-                         j->spill, j->spcap, j->ctr);
+    if (fuse) build(std::true_type{}, bst);
+    else build(std::false_type{}, bst);
   }
   if (bst != j->stream) {
     HIP_CHECK(hipEventRecord(j->cev[1], bst));
     HIP_CHECK(hipStreamWaitEvent(j->stream, j->cev[1], 0));
   }
-  /* instances and dropped reads into the job's counters */
-  hipLaunchKernelGGL(k_add_u64, dim3(1), dim3(64), 0, j->stream, (unsigned long long*)&j->ctr->n_instances, stat, 1);
-  hipLaunchKernelGGL(k_add_u64, dim3(1), dim3(64), 0, j->stream, (unsigned long long*)&j->ctr->n_dropped, stat + 1,
-                     1);
+  hipLaunchKernelGGL(k_add_job_stats, dim3(grid_for(jb - ja)), dim3(BLOCK), 0, j->stream, stat, ja, jb, overflow,
+                     nj > 1 ? j->d_jstat : nullptr, nj, j->ctr);
+  uint32_t h[2];
+  HIP_CHECK(hipMemcpyAsync(h, next, 8, hipMemcpyDeviceToHost, j->stream));
   HIP_CHECK(hipStreamSynchronize(j->stream));
-  void* qp = spq;
-  dev_free(j, qp, n_waves * spq_cap * 8);
-  qp = spq_n;
-  dev_free(j, qp, n_waves * 4);
-  give_up(); /* every buffer of the count back to the pool */
-  j->table_valid = true;
-  j->cbits = cbits;
-  j->sbits = sbits;
-  j->bits_fresh = cbits != nullptr;
-  j->fused = fuse;
-  j->holes = holes;
-  j->n_hole_waves = fuse ? n_waves : 0;
-  *done = true;
+  give_back();
+  *done = h[1] == 0;
+  if (fuse && *done) {
+    j->chain_slot = nl.chain_slot;
+    j->branch_slot = nl.branch_slot;
+    j->list_cap = lcap;
+    j->fused = true;
+    j->holes = holes;
+    j->n_hole_waves = n_waves;
+  } else if (fuse) {
+    void* p = nl.chain_slot;
+    dev_free(j, p, lcap * 8);
+    p = nl.branch_slot;
+    dev_free(j, p, lcap * 8);
+    p = holes;
+    dev_free(j, p, 2 * n_waves * 8);
+  }
   return BRUNO_OK;
 }
 
+/* reads [first[ja], first[jb]) counted with atomics in HBM */
+template <typename KT>
+void count_atomic(bruno_job* j, ParseArgs a, uint64_t r0, uint64_t r1) {
+  const bruno_tuning t = tuning();
+  a.read0 = r0;
+  a.n_reads = r1;
+  const unsigned wpb = t.parse_block / 64;
+  const uint64_t waves = std::min<uint64_t>(r1 - r0, t.parse_grid);
+  const unsigned g = (unsigned)std::max<uint64_t>(1, (waves + wpb - 1) / wpb);
+  switch (t.parse_block) {
+    case 128: hipLaunchKernelGGL((k_parse<KT, 2, 128>), dim3(g), dim3(128), 0, j->stream, a); break;
+    case 512: hipLaunchKernelGGL((k_parse<KT, 2, 512>), dim3(g), dim3(512), 0, j->stream, a); break;
+    default: hipLaunchKernelGGL((k_parse<KT, 2, 256>), dim3(g), dim3(256), 0, j->stream, a); break;
+  }
+}
+
+/* Count one call's reads into a region-layout table, job by job or several
+ * jobs of a batch at a time; jobs whose pass could not be counted by regions
+ * are counted with atomics. */
+template <typename KT>
+bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, const uint64_t* d_first, const uint64_t* h_first) {
+  const uint32_t nj = j->n_jobs;
+  const int valid = j->table_valid ? 1 : 0;
+  /* instances per job (an upper bound: reads to be dropped included) */
+  std::vector<ParseShare> share;
+  const uint64_t n_reads = h_first[nj];
+  for (uint32_t q = 0; q < nj; ++q) {
+    const uint64_t nr = h_first[q + 1] - h_first[q];
+    if (!nr) continue;
+    const uint64_t w = std::min<uint64_t>(std::max<uint64_t>(1, 2 * device_cus() * nr / n_reads), (nr + BLOCK - 1) / BLOCK);
+    for (uint32_t i = 0; i < w; ++i) share.push_back(ParseShare{q, i, (uint32_t)w, 0});
+  }
+  std::vector<unsigned long long> inst(nj, 0);
+  {
+    ParseShare* d_share = nullptr;
+    unsigned long long* d_inst = nullptr;
+    const uint64_t sb = std::max<uint64_t>(1, share.size()) * sizeof(ParseShare);
+    TRY(dev_alloc(j, (void**)&d_share, sb));
+    TRY(dev_alloc(j, (void**)&d_inst, nj * 8));
+    HIP_CHECK(hipMemcpyAsync(d_share, share.data(), share.size() * sizeof(ParseShare), hipMemcpyHostToDevice, j->stream));
+    fill64(j, d_inst, nj, 0);
+    if (!share.empty())
+      hipLaunchKernelGGL(k_count_instances, dim3((unsigned)share.size()), dim3(BLOCK), 0, j->stream, a, d_first, d_share,
+                         d_inst);
+    HIP_CHECK(hipMemcpyAsync(inst.data(), d_inst, nj * 8, hipMemcpyDeviceToHost, j->stream));
+    HIP_CHECK(hipStreamSynchronize(j->stream));
+    void* p = d_share;
+    dev_free(j, p, sb);
+    p = d_inst;
+    dev_free(j, p, nj * 8);
+  }
+  /* a first count builds every region: it also leaves the filter scan's
+   * bits (stale once another count follows) */
+  const uint64_t nbits = j->n_regions * j->bit_stride;
+  uint64_t *cbits = nullptr, *sbits = nullptr;
+  if (!valid && dev_alloc(j, (void**)&cbits, nbits * 8) == BRUNO_OK &&
+      dev_alloc(j, (void**)&sbits, nbits * 8) != BRUNO_OK) {
+    void* p = cbits;
+    dev_free(j, p, nbits * 8);
+    cbits = nullptr;
+  }
+  if (!sbits) cbits = nullptr;
+  bool all = true;
+  for (uint32_t ja = 0, jb; ja < nj; ja = jb) {
+    uint64_t n = inst[ja];
+    for (jb = ja + 1; jb < nj && n + inst[jb] <= REC_PASS_BYTES / sizeof(typename RecOf<KT>::T); ++jb) n += inst[jb];
+    bool done = false;
+    TRY(count_regions_pass<KT>(j, a, d_first, h_first, ja, jb, inst, valid, cbits, sbits, &done));
+    if (done) continue;
+    all = false;
+    if (!valid)
+      fill64(j, (char*)j->table + j->seg[ja] * slot_bytes(j), (j->seg[jb] - j->seg[ja]) * slot_bytes(j) / 8, EMPTY64);
+    if (h_first[jb] > h_first[ja]) count_atomic<KT>(j, a, h_first[ja], h_first[jb]);
+  }
+  j->table_valid = true;
+  j->by_regions = all;
+  j->cbits = cbits;
+  j->sbits = sbits;
+  j->bits_fresh = cbits && all;
+  return BRUNO_OK;
+}
+
+/* d_first / h_first: every job's first read of this call, n_jobs + 1 entries
+ * (device and host; d_first may be null for a plain job) */
 template <typename KT>
 bruno_status parse_count_t(bruno_job* j, const char* d_bases, const uint64_t* d_offsets, uint64_t n_reads,
-                           const uint64_t* d_first, const uint64_t* d_starts = nullptr,
+                           const uint64_t* d_first, const uint64_t* h_first, const uint64_t* d_starts = nullptr,
                            const uint64_t* d_ends = nullptr) {
   ParseArgs a{};
   a.starts = d_starts;
   a.ends = d_ends;
   a.n_jobs = j->n_jobs;
   a.job_first = d_first;
-  a.seg = j->d_seg;
+  a.lay = j->d_lay;
   a.job_inst = j->d_jstat;
   a.job_drop = j->d_jstat + j->n_jobs;
   a.bases = (const uint8_t*)d_bases;
@@ -2042,26 +2160,11 @@ bruno_status parse_count_t(bruno_job* j, const char* d_bases, const uint64_t* d_
   a.spill = j->spill;
   a.spcap = j->spcap;
   a.ctr = j->ctr;
-  const bruno_tuning t = tuning();
   j->by_regions = false;
   j->bits_fresh = false;
-  if (j->rbits && t.count_regions) {
-    bool done = false;
-    TRY(count_by_regions<KT>(j, a, &done));
-    if (done) {
-      j->by_regions = true;
-      return BRUNO_OK;
-    }
-  }
+  if (j->regions && tuning().count_regions) return count_by_regions<KT>(j, a, d_first, h_first);
   ensure_table_valid(j);
-  const unsigned wpb = t.parse_block / 64;
-  const uint64_t waves = std::min<uint64_t>(n_reads, t.parse_grid);
-  const unsigned g = (unsigned)std::max<uint64_t>(1, (waves + wpb - 1) / wpb);
-  switch (t.parse_block) {
-    case 128: hipLaunchKernelGGL((k_parse<KT, 2, 128>), dim3(g), dim3(128), 0, j->stream, a); break;
-    case 512: hipLaunchKernelGGL((k_parse<KT, 2, 512>), dim3(g), dim3(512), 0, j->stream, a); break;
-    default: hipLaunchKernelGGL((k_parse<KT, 2, 256>), dim3(g), dim3(256), 0, j->stream, a); break;
-  }
+  count_atomic<KT>(j, a, 0, n_reads);
   return BRUNO_OK;
 }
 
@@ -2146,10 +2249,10 @@ bruno_status filter_t(bruno_job* j) {
   TRY(dev_alloc(j, (void**)&spilled, n_spill_cap * sizeof(uint64_t)));
   if (j->bits_fresh) {
     /* the last count built every region and left the scan's choice */
-    const uint64_t nreg = 1ULL << j->rbits, stride = (j->rspan + 63) / 64;
+    const uint64_t nreg = j->n_regions, stride = j->bit_stride;
     hipLaunchKernelGGL(k_filter_bits, dim3(grid_for((nreg * stride + FILTER_BITS_WPT - 1) / FILTER_BITS_WPT)),
-                       dim3(BLOCK), 0, j->stream, j->cbits, j->sbits, nreg, stride, j->rspan, cand, n_distinct,
-                       spilled, n_spill_cap, j->ctr);
+                       dim3(BLOCK), 0, j->stream, j->cbits, j->sbits, nreg, stride, j->d_lay, j->n_jobs, cand,
+                       n_distinct, spilled, n_spill_cap, j->ctr);
   } else {
     hipLaunchKernelGGL((k_filter_scan<KT>),
                        dim3(grid_for((j->cap + FILTER_SPT - 1) / FILTER_SPT, BLOCK, tuning().scan_grid)),
@@ -2245,7 +2348,7 @@ bruno_status chains_t(bruno_job* j) {
   HIP_CHECK(hipMemsetAsync(&j->ctr->lr_ill, 0, sizeof(unsigned long long), j->stream));
   HIP_CHECK(hipMemsetAsync(&j->ctr->lr_next, 0, sizeof(unsigned long long), j->stream));
   hipLaunchKernelGGL((k_chain_init<KT>), dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream, (const Slot<KT>*)j->table,
-                     probe_span(j), j->rbits, j->K, j->chain_slot, j->chain_job, j->d_seg, j->n_jobs, nc,
+                     probe_span(j), j->rbits, j->K, j->chain_slot, j->chain_job, j->d_lay, j->n_jobs, nc,
                      (KT*)j->ckmer, j->cedge, j->lr, (KT*)j->vkmer, j->vcap, ruler_period(nc) - 1, j->ruler_bits,
                      j->alive, j->ctr);
   if (nc)
@@ -2253,7 +2356,7 @@ bruno_status chains_t(bruno_job* j) {
                        j->ruler_base, j->ruler_node, j->ctr);
   hipLaunchKernelGGL((k_termini<KT>), dim3(grid_for(j->n_branch)), dim3(BLOCK), 0, j->stream,
                      (const Slot<KT>*)j->table, probe_span(j), j->rbits, j->K, j->branch_slot, j->branch_job,
-                     j->d_seg, j->n_jobs, j->n_branch, j->lr, (KT*)j->bkmer);
+                     j->d_lay, j->n_jobs, j->n_branch, j->lr, (KT*)j->bkmer);
   TRY(sync_counters(j));
   j->n_virt = j->hctr->n_virt;
   j->n_rulers = j->hctr->lr_next;
@@ -2834,8 +2937,7 @@ const char* bruno_status_string(bruno_status s) {
   return "unknown";
 }
 
-static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, const uint64_t* caps, bruno_job** out,
-                                  bool plain = false) {
+static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, const uint64_t* caps, bruno_job** out) {
   if (!d || !out) return BRUNO_BAD_INPUT;
   *out = nullptr;
   if (d->k < 3 || d->k > 63 || n_jobs == 0 || d->thresholding < 0 || d->thresholding > 2) return BRUNO_BAD_INPUT;
@@ -2854,7 +2956,6 @@ static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, cons
   j->load_factor = (d->load_factor > 0 && d->load_factor < 1) ? d->load_factor : 0.5;
   j->stream = (hipStream_t)d->stream;
   j->n_jobs = n_jobs;
-  j->region_ok = plain;
   j->job_reads.assign(n_jobs, 0);
   if (pool_alloc((void**)&j->ctr, sizeof(Counters)) != hipSuccess ||
       hipHostMalloc((void**)&j->hctr, sizeof(Counters), hipHostMallocDefault) != hipSuccess) {
@@ -2891,7 +2992,7 @@ static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, cons
 bruno_status bruno_job_create(const bruno_job_desc* d, bruno_job** out) {
   if (!d) return BRUNO_BAD_INPUT;
   const uint64_t cap = d->capacity;
-  return create_common(d, 1, cap ? &cap : nullptr, out, true);
+  return create_common(d, 1, cap ? &cap : nullptr, out);
 }
 
 bruno_status bruno_batch_create(const bruno_job_desc* d, uint32_t n_jobs, const uint64_t* capacities,
@@ -2899,8 +3000,7 @@ bruno_status bruno_batch_create(const bruno_job_desc* d, uint32_t n_jobs, const 
   if (!capacities || n_jobs == 0 || n_jobs > BRUNO_MAX_BATCH_JOBS) return BRUNO_BAD_INPUT;
   for (uint32_t i = 0; i < n_jobs; ++i)
     if (capacities[i] == 0) return BRUNO_BAD_INPUT;
-  /* one job: a plain job (the region layout when its table is large) */
-  return create_common(d, n_jobs, capacities, out, n_jobs == 1);
+  return create_common(d, n_jobs, capacities, out);
 }
 
 /* Slots from which a one-job table counts by regions (0: never, the
@@ -2992,14 +3092,22 @@ bruno_status bruno_job_reset(bruno_job* j) {
 }
 
 static bruno_status parse_count_common(bruno_job* j, const char* d_bases, const uint64_t* d_offsets, uint64_t n_reads,
-                                       const uint64_t* d_first, const uint64_t* d_starts = nullptr,
+                                       const uint64_t* h_first, const uint64_t* d_starts = nullptr,
                                        const uint64_t* d_ends = nullptr) {
   if (j->fused) return BRUNO_STATE; /* the filter already ran on the table */
   ev_record(j, 0);
-  if (j->words == 1) TRY(parse_count_t<uint64_t>(j, d_bases, d_offsets, n_reads, d_first, d_starts, d_ends));
-  else TRY(parse_count_t<u128>(j, d_bases, d_offsets, n_reads, d_first, d_starts, d_ends));
+  const uint64_t all[2] = {0, n_reads}, nf = (j->n_jobs + 1) * 8;
+  uint64_t* d_first = nullptr;
+  if (!h_first) h_first = all;
+  TRY(dev_alloc(j, (void**)&d_first, nf));
+  HIP_CHECK(hipMemcpyAsync(d_first, h_first, nf, hipMemcpyHostToDevice, j->stream));
+  if (j->words == 1) TRY(parse_count_t<uint64_t>(j, d_bases, d_offsets, n_reads, d_first, h_first, d_starts, d_ends));
+  else TRY(parse_count_t<u128>(j, d_bases, d_offsets, n_reads, d_first, h_first, d_starts, d_ends));
   ev_record(j, 1);
-  TRY(sync_counters(j));
+  const bruno_status st = sync_counters(j);
+  void* p = d_first;
+  dev_free(j, p, nf);
+  TRY(st);
   j->ms.parse_count_ms += ev_ms(j, 0, 1);
   j->n_reads += n_reads;
   /* No limit on a job's instances: sub-entries count to 2^48, and every
@@ -3044,17 +3152,7 @@ bruno_status bruno_batch_parse_count(bruno_job* j, const char* d_bases, const ui
     return BRUNO_OK;
   }
   if (!d_bases || !d_offsets || j->cap == 0) return BRUNO_BAD_INPUT;
-  uint64_t* d_first = nullptr;
-  if (nj > 1) {
-    TRY(dev_alloc(j, (void**)&d_first, (nj + 1) * 8));
-    HIP_CHECK(hipMemcpyAsync(d_first, job_first_read, (nj + 1) * 8, hipMemcpyHostToDevice, j->stream));
-  }
-  bruno_status s = parse_count_common(j, d_bases, d_offsets, n_reads, d_first);
-  if (d_first) {
-    (void)hipStreamSynchronize(j->stream);
-    void* a = d_first;
-    dev_free(j, a, (nj + 1) * 8);
-  }
+  bruno_status s = parse_count_common(j, d_bases, d_offsets, n_reads, job_first_read);
   if (s == BRUNO_OK)
     for (uint32_t i = 0; i < nj; ++i) j->job_reads[i] += job_first_read[i + 1] - job_first_read[i];
   return s;
@@ -3857,14 +3955,10 @@ bruno_status bruno_batch_get_branch_fasta(bruno_job* j, uint32_t idx, char* buf,
 }
 
 /* table segment of job idx: first slot and probe span */
-static void job_segment(const bruno_job* j, uint32_t idx, uint64_t& tbase, uint64_t& tcap) {
-  if (j->n_jobs == 1) {
-    tbase = 0;
-    tcap = probe_span(j);
-  } else {
-    tbase = j->seg[idx];
-    tcap = j->seg[idx + 1] - j->seg[idx];
-  }
+static void job_segment(const bruno_job* j, uint32_t idx, uint64_t& tbase, uint64_t& tcap, uint32_t& rbits) {
+  tbase = j->lay[idx].slot0;
+  tcap = j->lay[idx].span;
+  rbits = j->lay[idx].rbits;
 }
 
 extern "C++" {
@@ -3873,9 +3967,10 @@ static bruno_status branch_nodes_t(bruno_job* j, uint32_t idx, uint64_t b0, uint
   bruno_node* d = nullptr;
   TRY(dev_alloc(j, (void**)&d, nb * sizeof(bruno_node)));
   uint64_t tbase, tcap;
-  job_segment(j, idx, tbase, tcap);
+  uint32_t rbits;
+  job_segment(j, idx, tbase, tcap, rbits);
   hipLaunchKernelGGL((k_branch_nodes<KT>), dim3(grid_for(nb, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
-                     (const Slot<KT>*)j->table, tbase, tcap, j->rbits, (const KT*)j->bsorted + b0, nb, d, j->ctr);
+                     (const Slot<KT>*)j->table, tbase, tcap, rbits, (const KT*)j->bsorted + b0, nb, d, j->ctr);
   bruno_status st = sync_counters(j);
   if (st == BRUNO_OK && copy_out(j, buf, d, nb * sizeof(bruno_node)) != hipSuccess) st = BRUNO_INTERNAL;
   void* a = d;
@@ -3911,9 +4006,10 @@ static bruno_status chain_edges_t(bruno_job* j, uint32_t idx, uint64_t c0, uint6
   if (st == BRUNO_OK) st = dev_alloc(j, (void**)&d, nu * sizeof(bruno_chain_edge));
   if (st == BRUNO_OK) {
     uint64_t tbase, tcap;
-    job_segment(j, idx, tbase, tcap);
+    uint32_t rbits;
+    job_segment(j, idx, tbase, tcap, rbits);
     hipLaunchKernelGGL((k_chain_edges<KT>), dim3(grid_for(nu * 64, BLOCK, 1u << 16)), dim3(BLOCK), 0, j->stream,
-                       (const Slot<KT>*)j->table, tbase, tcap, j->rbits, j->K, out_view<KT>(j), off, st0, nu, d, j->ctr);
+                       (const Slot<KT>*)j->table, tbase, tcap, rbits, j->K, out_view<KT>(j), off, st0, nu, d, j->ctr);
     st = sync_counters(j);
     if (st == BRUNO_OK && copy_out(j, buf, d, nu * sizeof(bruno_chain_edge)) != hipSuccess) st = BRUNO_INTERNAL;
   }

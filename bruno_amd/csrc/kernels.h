@@ -208,10 +208,11 @@ struct ParseArgs {
   Spill* spill;
   uint64_t spcap;
   /* batches: job j owns reads [job_first[j], job_first[j+1]) of this call
-   * and table slots [seg[j], seg[j+1]); n_jobs == 1 uses the whole table */
+   * and the table slots of lay[j]; n_jobs == 1 uses the whole table */
   uint32_t n_jobs;
   const uint64_t* job_first;
-  const uint64_t* seg;
+  const JobLayout* lay;
+  uint64_t read0;       /* count mode: reads [read0, n_reads) */
   unsigned long long* job_inst; /* per-job k-mer instances (n_jobs > 1) */
   unsigned long long* job_drop; /* per-job dropped reads (n_jobs > 1) */
   /* sketch mode: SKETCH_M HyperLogLog registers per job */
@@ -318,16 +319,18 @@ __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
    * the job changes, so the per-job counters see few atomics) */
   uint32_t cj = 0;
   uint64_t j_lo = 0, j_hi = 0, tbase = 0, tcap = a.cap;
+  uint32_t rbits = a.rbits;
   unsigned long long j_inst = 0;
-  for (uint64_t r = wave; r < a.n_reads; r += nwaves) {
+  for (uint64_t r = a.read0 + wave; r < a.n_reads; r += nwaves) {
     if ((MODE == 2 || MODE == 3) && a.n_jobs > 1 && !(r >= j_lo && r < j_hi)) {
       if (lane == 0 && j_inst) atomicAdd(&a.job_inst[cj], j_inst);
       j_inst = 0;
       cj = job_of(a.job_first, a.n_jobs, r);
       j_lo = a.job_first[cj];
       j_hi = a.job_first[cj + 1];
-      tbase = a.seg[cj];
-      tcap = a.seg[cj + 1] - tbase;
+      tbase = a.lay[cj].slot0;
+      tcap = a.lay[cj].span;
+      rbits = a.lay[cj].rbits;
     }
     const uint64_t off = a.starts ? a.starts[r] : a.offsets[r];
     const uint64_t L = (a.starts ? a.ends[r] : a.offsets[r + 1]) - off;
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
       } else {
         int claimed = 0;
         uint64_t slot =
-            SlotOps<KT>::find_or_insert((Slot<KT>*)a.table + tbase, tcap, a.rbits, km, &a.ctr->err, &claimed);
+            SlotOps<KT>::find_or_insert((Slot<KT>*)a.table + tbase, tcap, rbits, km, &a.ctr->err, &claimed);
         if (slot != ~0ULL) {
           my_new += claimed;
           my_k2 += add_k2<KT>((Slot<KT>*)a.table, tbase + slot, biedge_index(e) + 1, a.spill, a.spcap, &a.ctr->err);

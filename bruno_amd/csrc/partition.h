@@ -1,35 +1,34 @@
 /*
- * partition.h -- grouping the count's instance records by table region.
+ * partition.h -- grouping a count's instance records by table region.
  *
- * The record parser (k_parse_records, regions.h) leaves one 8-byte record
- * per k-mer instance, rec = (hash << 5) | biedge index, in 32 buckets picked
- * by the hash's top 5 bits.  The next rb hash bits (the record's top rb
- * bits) name the region inside the bucket.  Two multisplit passes, both
- * hand-written and each one read and one write of the records, group them
- * by region so that a region build reads each region's records as one
- * contiguous run:
+ * The record parser (k_parse_records, regions.h) leaves one record per k-mer
+ * instance, rec = (hash << 5) | biedge index, in buckets picked by the
+ * hash's top `beta` bits (up to 512 buckets per job).  A bucket is a list of
+ * chunks taken from one pool, so no bucket has a capacity of its own.  The
+ * next hash bits (b2 of them) name the region inside the bucket, and one
+ * multisplit pass, k_split, groups every bucket's records by region, in
+ * pieces of 64 records that a region's build reads with one wave each.
  *
- *   k_split1   all buckets at once, by the top b1 region bits (up to 128
- *              sub-buckets per bucket).  Each sub-bucket gets room for its
- *              share of the bucket plus a margin (hash bits are uniform, so a
- *              sub-bucket holds 1/2^b1 of its bucket up to sampling noise);
- *              a workgroup sorts a tile of records by digit in LDS and
- *              reserves each digit's run with one atomic per tile.  A
- *              sub-bucket that would overflow its room (a k-mer in a large
- *              share of all instances) is reported, and the pass runs again
- *              with room from exact counts (k_split_count).  The chunk
- *              padding the parser left behind (code 31) is dropped.
- *   k_split2   one workgroup per sub-bucket (persistent), by the remaining
- *              b2 <= 9 region bits: a count pass over the sub-bucket, then
- *              the same LDS tile sort with workgroup-local cursors, into a
- *              compact output.  It also writes the first record of every
- *              region.
+ * One workgroup owns a bucket: it sorts tile after tile by digit in LDS and
+ * appends each digit's run to the digit's open piece, taking new pieces from
+ * the bucket's own room (its chunks, and one piece per region) with a counter
+ * of its own: no global atomic, and no pass over the records to count them
+ * first (a region's count cannot be estimated: a k-mer repeated thousands of
+ * times puts all its instances in one region).  The pieces' regions, a 64th
+ * of the records, are grouped at the end instead.  A tile fills 128 KB of
+ * LDS, one 1,024-thread workgroup per CU, so that a run of a tile is still
+ * 64 bytes when a bucket has 2,048 regions; 256 buckets are one per CU.
  *
- * Both passes load the next tile while sorting and writing the current one.
+ * The records are read and written once, 2.7 TB/s at 1.6 G records of 8
+ * bytes (9.4 ms; LDS work and the barriers between a tile's steps take the
+ * rest).  Contiguous regions behind a count pass took 12.9 ms.  Before that, 32
+ * coarser buckets and two passes (on small tables, 32 workgroups in the
+ * second) took 0.73 ms for 21 M records (now 0.13), 1.84 for 184 M (1.09),
+ * 5.5 for 301 M of 16 bytes (3.6).
  *
- * Neither pass keeps the order of records inside a digit, which nothing
- * downstream depends on (a region's slots come out the same up to the
- * order of keys inside a probe run).
+ * The order of records inside a region is not kept, which nothing
+ * downstream depends on (a region's slots come out the same up to the order
+ * of keys inside a probe run).
  */
 #ifndef BRUNO_PARTITION_H_
 #define BRUNO_PARTITION_H_
@@ -38,16 +37,18 @@
 
 namespace br {
 
-constexpr int SPLIT_BS = 512;
-constexpr int SPLIT_ITEMS = 8;
-constexpr int SPLIT_TILE = SPLIT_BS * SPLIT_ITEMS;  /* records per tile */
-constexpr int SPLIT1_MAX_BITS = 7;
-constexpr int SPLIT2_MAX_BITS = 9;
-constexpr uint32_t REC_CODE_FILL = 31;              /* chunk padding, never a biedge index (0..24) */
+/* A record drops the hash's top REC_BUCKET_BITS bits, so every job has at
+ * least that many bucket bits. */
+constexpr int REC_BUCKET_BITS = 5;
+constexpr int MAX_BUCKET_BITS = 9;
+constexpr int SPLIT_BS = 1024;
+constexpr int SPLIT_BITS = 11, SPLIT_MAX_BITS = 12; /* region bits a bucket is split by: usual, largest tables */
+constexpr uint32_t REC_CODE_FILL = 31; /* chunk padding, never a biedge index (0..24) */
+constexpr uint32_t NO_CHUNK = ~0u;
 
 /* A record: one word (k <= 31) or the key word and the k-mer's high word
- * (k <= 63).  The key word, (hash << 5) | biedge index, is what the passes
- * split on. */
+ * (k <= 63).  The key word, (hash << 5) | biedge index, is what the split
+ * goes by. */
 template <typename KT> struct RecOf;
 template <> struct RecOf<uint64_t> { typedef uint64_t T; };
 template <> struct RecOf<u128> { typedef ulonglong2 T; };
@@ -57,285 +58,282 @@ template <typename R> __device__ __forceinline__ R rec_zero();
 template <> __device__ __forceinline__ uint64_t rec_zero<uint64_t>() { return 0; }
 template <> __device__ __forceinline__ ulonglong2 rec_zero<ulonglong2>() { return make_ulonglong2(0, 0); }
 
-/* One segment of a bucket's record area: [begin, end) holds records of
- * bucket `bucket`; its tiles are numbered from first_tile. */
-struct SplitSeg {
-  uint64_t begin, end, first_tile;
-  uint32_t bucket, pad;
-};
-constexpr int SPLIT_MAX_SEGS = 64;
-
-/* Workgroups go to the device's XCDs (each with its own L2) in turn:
- * workgroup w runs on XCD w % SPLIT_XCDS. */
-constexpr int SPLIT_XCDS = 8;
-
-struct Split1Args {
-  const void* in;                 /* records (RecOf<KT>::T) */
-  SplitSeg seg[SPLIT_MAX_SEGS];   /* grouped by bucket % SPLIT_XCDS */
-  int n_seg;
-  uint64_t n_tiles;
-  uint64_t xcd_tiles[SPLIT_XCDS + 1]; /* tiles of XCD x's buckets: [xcd_tiles[x], xcd_tiles[x + 1]) */
-  int b1;                         /* digit bits (0: one sub-bucket per bucket) */
-  unsigned long long* cursor;     /* [32 << b1]: next free position of each sub-bucket */
-  const uint64_t* limit;          /* [32 << b1]: end of each sub-bucket's room */
-  void* out;
-  unsigned long long* overflow;   /* set when a sub-bucket ran out of room */
-};
-
-/* Exclusive prefix of cnt[0..n) into start[0..n) (n <= 512), computed by
- * the first wave; returns nothing, the caller synchronises. */
-__device__ __forceinline__ void wave_exclusive_scan(const uint32_t* cnt, uint32_t* start, int n) {
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    const int per = (n + 63) / 64;
-    uint32_t mine = 0;
-    for (int i = 0; i < per; ++i) {
-      const int q = lane * per + i;
-      mine += q < n ? cnt[q] : 0;
-    }
-    uint32_t incl = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t v = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += v;
-    }
-    uint32_t run = incl - mine;
-    for (int i = 0; i < per; ++i) {
-      const int q = lane * per + i;
-      if (q < n) {
-        start[q] = run;
-        run += cnt[q];
-      }
-    }
+/* the job holding bucket / region x: the largest j with first(j) <= x */
+template <typename F>
+__device__ __forceinline__ uint32_t count_job_of(uint32_t n_jobs, uint32_t x, F first) {
+  uint32_t lo = 0, hi = n_jobs;
+  while (hi - lo > 1) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (first(mid) <= x) lo = mid;
+    else hi = mid;
   }
+  return lo;
 }
 
-/* The LDS tile sort both passes share: the tile's records (ITEMS per
- * thread, `ok` false for holes and padding) are ranked by digit with LDS
- * atomics and scattered into buf in digit order; reserve(d, count) (one
- * thread per digit) fixes where digit d's records of this tile go, and
- * store(d, j, rec) writes the j-th of them, so each digit's run is written
- * to consecutive places. */
-template <typename R, int ITEMS, typename DigitF, typename ReserveF, typename StoreF>
-__device__ __forceinline__ void tile_split(const R (&r)[ITEMS], const bool (&ok)[ITEMS], int nbins, R* buf,
-                                           uint32_t* cnt, uint32_t* start, DigitF digit, ReserveF reserve,
-                                           StoreF store) {
-  for (int i = threadIdx.x; i < nbins; i += SPLIT_BS) cnt[i] = 0;
-  __syncthreads();
-  uint32_t rank[ITEMS], d[ITEMS];
-#pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    d[k] = ok[k] ? digit(rec_key(r[k])) : 0;
-    rank[k] = ok[k] ? atomicAdd(&cnt[d[k]], 1u) : 0;
-  }
-  __syncthreads();
-  wave_exclusive_scan(cnt, start, nbins);
-  __syncthreads();
-  /* per digit: its count in this tile -> its output position */
-  for (int i = threadIdx.x; i < nbins; i += SPLIT_BS) reserve(i, cnt[i]);
-#pragma unroll
-  for (int k = 0; k < ITEMS; ++k)
-    if (ok[k]) buf[start[d[k]] + rank[k]] = r[k];
-  __syncthreads();
-  /* records in digit order; each digit's run goes to consecutive places */
-  const uint32_t total = start[nbins - 1] + cnt[nbins - 1];
-  for (uint32_t i = threadIdx.x; i < total; i += SPLIT_BS) {
-    const R x = buf[i];
-    const uint32_t dx = digit(rec_key(x));
-    store(dx, i - start[dx], x);
-  }
-  __syncthreads();
-}
-
-/* Both passes sort 8-byte records in tiles of 8,192 (16 per thread), so a
- * sub-bucket's or region's run of a tile is twice as long as with 4,096;
- * 16-byte records keep 4,096 (the tile fills the same 64 KB of LDS). */
-template <typename R> struct SplitShape {
-  static constexpr int ITEMS = sizeof(R) == 8 ? 2 * SPLIT_ITEMS : SPLIT_ITEMS;
-  static constexpr int TILE = SPLIT_BS * ITEMS;
+/* The chunk pool: chunk c holds records [c << clog, (c + 1) << clog) of one
+ * bucket.  Chunk numbers are taken CHUNK_BATCH at a time. */
+constexpr uint32_t CHUNK_BATCH = 128, CHUNK_LOW = 16;
+struct ChunkPool {
+  void* recs;                 /* RecOf<KT>::T */
+  uint32_t clog;              /* log2 records per chunk */
+  uint32_t n_max;             /* chunks the pool has room for */
+  uint32_t* next;             /* chunks taken */
+  uint32_t* taken;            /* per bucket: chunks taken */
+  uint32_t* owner;            /* per chunk: its bucket (NO_CHUNK: not used) */
+  uint32_t* overflow;         /* set when records found no room (the count then starts over with atomics) */
 };
 
-/* the records of tile t of the split segments (ok: a real record) */
-template <typename R, int ITEMS>
-__device__ __forceinline__ void seg_tile_load(const Split1Args& a, uint64_t t, R (&r)[ITEMS], bool (&ok)[ITEMS],
-                                              uint32_t& bucket) {
-  int g = 0;
-  while (g + 1 < a.n_seg && a.seg[g + 1].first_tile <= t) ++g;
-  const SplitSeg& sg = a.seg[g];
-  const uint64_t lo = sg.begin + (t - sg.first_tile) * (uint64_t)(SPLIT_BS * ITEMS);
-  const R* in = (const R*)a.in;
-  bucket = sg.bucket;
-#pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const uint64_t i = lo + (uint64_t)k * SPLIT_BS + threadIdx.x;
-    r[k] = i < sg.end ? in[i] : rec_zero<R>();
-    ok[k] = i < sg.end && (uint32_t)(rec_key(r[k]) & 31) != REC_CODE_FILL;
-  }
-}
-
-/* The buckets of one XCD are split by that XCD's workgroups only, so the
- * runs that neighbouring tiles append next to each other (sharing cache
- * lines at their ends) meet in one L2 instead of being written back in
- * parts by two.  The grid is a multiple of SPLIT_XCDS. */
-template <typename R>
-__global__ __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(4))) void k_split1(Split1Args a) {
-  constexpr int ITEMS = SplitShape<R>::ITEMS;
-  __shared__ R buf[SplitShape<R>::TILE];
-  __shared__ uint32_t cnt[1 << SPLIT1_MAX_BITS], start[1 << SPLIT1_MAX_BITS];
-  __shared__ unsigned long long pos[1 << SPLIT1_MAX_BITS], lim[1 << SPLIT1_MAX_BITS];
-  R* out = (R*)a.out;
-  const int b1 = a.b1;
-  const int nb = 1 << b1;
-  const uint32_t x = blockIdx.x % SPLIT_XCDS, per = gridDim.x / SPLIT_XCDS;
-  const uint64_t t0 = a.xcd_tiles[x] + blockIdx.x / SPLIT_XCDS, t1 = a.xcd_tiles[x + 1];
-  R rn[ITEMS];
-  bool okn[ITEMS];
-  uint32_t bn = 0;
-  if (t0 < t1) seg_tile_load(a, t0, rn, okn, bn);
-  for (uint64_t t = t0; t < t1; t += per) {
-    R r[ITEMS];
-    bool ok[ITEMS];
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      r[k] = rn[k];
-      ok[k] = okn[k];
-    }
-    const uint32_t bucket = bn;
-    /* the next tile's loads go out before this tile is sorted and written */
-    if (t + per < t1) seg_tile_load(a, t + per, rn, okn, bn);
-    unsigned long long* cur = a.cursor + ((uint64_t)bucket << b1);
-    const uint64_t* limit = a.limit + ((uint64_t)bucket << b1);
-    tile_split<R, ITEMS>(
-        r, ok, nb, buf, cnt, start, [&](uint64_t x) -> uint32_t { return b1 ? (uint32_t)(x >> (64 - b1)) : 0u; },
-        [&](int i, uint32_t c) {
-          pos[i] = c ? atomicAdd(&cur[i], (unsigned long long)c) : 0ULL;
-          lim[i] = limit[i];
-        },
-        [&](uint32_t dx, uint32_t j, const R& x) {
-          /* a sub-bucket past its room: reported, and the pass runs again
-           * with exact room */
-          const uint64_t at = pos[dx] + j;
-          if (at < lim[dx]) out[at] = x;
-          else atomicOr(a.overflow, 1ULL);
-        });
-  }
-}
-
-/* Exact records per (bucket, top b1 region bits): the room k_split1 takes
- * when the estimate ran short. */
-template <typename R>
-__global__ __launch_bounds__(SPLIT_BS) void k_split_count(Split1Args a, unsigned long long* counts) {
-  __shared__ uint32_t cnt[1 << SPLIT1_MAX_BITS];
-  const int b1 = a.b1;
-  const int nb = 1 << b1;
-  constexpr int ITEMS = SplitShape<R>::ITEMS;
-  for (uint64_t t = blockIdx.x; t < a.n_tiles; t += gridDim.x) {
-    R r[ITEMS];
-    bool ok[ITEMS];
-    uint32_t bucket = 0;
-    seg_tile_load(a, t, r, ok, bucket);
-    for (int i = threadIdx.x; i < nb; i += SPLIT_BS) cnt[i] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k)
-      if (ok[k]) atomicAdd(&cnt[b1 ? (uint32_t)(rec_key(r[k]) >> (64 - b1)) : 0u], 1u);
-    __syncthreads();
-    for (int i = threadIdx.x; i < nb; i += SPLIT_BS)
-      if (cnt[i]) atomicAdd(&counts[((uint64_t)bucket << b1) + i], (unsigned long long)cnt[i]);
+/* first[b] = chunks of the buckets from b_lo to b (first[b_hi] = all); a
+ * bucket with more than `limit` chunks sets the overflow flag: one k-mer in a large
+ * share of all instances would leave one workgroup the work of the whole
+ * device.  One workgroup. */
+__global__ __launch_bounds__(1024) void k_chunk_first(ChunkPool p, uint32_t b_lo, uint32_t b_hi, uint32_t limit,
+                                                      uint32_t* first) {
+  typedef hipcub::BlockScan<uint32_t, 1024> Scan;
+  __shared__ typename Scan::TempStorage tmp;
+  uint32_t before = 0;
+  for (uint32_t b0 = b_lo; b0 < b_hi; b0 += 1024) {
+    const uint32_t b = b0 + threadIdx.x;
+    const uint32_t v = b < b_hi ? p.taken[b] : 0;
+    if (v > limit) *p.overflow = 1;
+    uint32_t at, total;
+    Scan(tmp).ExclusiveSum(v, at, total);
+    if (b < b_hi) first[b] = before + at;
+    before += total;
     __syncthreads();
   }
+  if (threadIdx.x == 0) first[b_hi] = before;
 }
 
-/* region_start of every sub-bucket's first region (its output start), so a
- * region build of the sub-buckets before sb finds its last region's end
- * before the pass over sb has run */
-__global__ void k_region_bounds(const uint64_t* out_start, uint64_t n_sb, int b2, uint64_t* region_start) {
-  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s <= n_sb) region_start[s << b2] = out_start[s];
+/* The chunks in bucket order (in any order within a bucket).  listed counts
+ * a bucket's chunks so far, one counter per cache line: with 32 in a line
+ * the atomics on it took 0.5 ms for 1.6 M chunks. */
+constexpr uint32_t LISTED_STRIDE = 32;
+__global__ __launch_bounds__(BLOCK) void k_chunk_list(ChunkPool p, uint32_t b_lo, const uint32_t* first,
+                                                      uint32_t* listed, uint32_t* list) {
+  const uint32_t n = min(*p.next, p.n_max);
+  for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < n; c += gridDim.x * BLOCK) {
+    const uint32_t b = p.owner[c];
+    if (b != NO_CHUNK) list[first[b] + atomicAdd(&listed[(uint64_t)(b - b_lo) * LISTED_STRIDE], 1u)] = c;
+  }
 }
 
-struct Split2Args {
-  const void* in;                 /* records (RecOf<KT>::T) */
-  const uint64_t* in_start;       /* [n_sb]: sub-bucket s holds in[in_start[s], + its count) */
-  const uint64_t* out_start;      /* [n_sb + 1]: and goes to out[out_start[s], out_start[s + 1]) */
-  uint64_t sb0;                   /* this launch: sub-buckets [sb0, sb0 + n_sb) */
-  uint64_t n_sb;
-  int shift;                      /* digit = (rec >> shift) & (2^b2 - 1) */
-  int b2;
-  void* out;                      /* grouped by region */
-  uint64_t* region_start;         /* [n_sb << b2 (+1)]: first record of every region */
+/* The split's output: pieces of 64 records (one per lane of a build's wave).
+ * A region's records are the pieces list[region_start ...], all full but
+ * the last. */
+constexpr int PIECE_LOG = 6;
+constexpr uint32_t PIECE = 1u << PIECE_LOG;
+
+/* tile of the split: 128 KB of records, less with twice the digits (both
+ * beside the digits' state in the CU's 160 KB) */
+template <typename R, int BITS> struct SplitShape {
+  static constexpr int FULL = (int)((128 << 10) / sizeof(R) / SPLIT_BS);
+  static constexpr int ITEMS = BITS > SPLIT_BITS ? FULL * 13 / 16 : FULL;
+  static constexpr int TILE = ITEMS * SPLIT_BS;
 };
 
-template <typename R>
-__global__ __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(4))) void k_split2(Split2Args a) {
-  constexpr int ITEMS = SplitShape<R>::ITEMS, TILE = SplitShape<R>::TILE;
+struct SplitArgs {
+  ChunkPool pool;
+  const uint32_t* first;      /* by bucket, see k_chunk_first */
+  const uint32_t* list;       /* chunks in bucket order */
+  const JobLayout* jobs;
+  uint32_t n_jobs;
+  uint32_t b0, b1;            /* this launch: buckets [b0, b1) */
+  uint32_t q_lo;              /* the pass's first region */
+  void* out;                  /* pieces; bucket b's from piece_base(b) */
+  uint16_t* digit_of;         /* per piece: its region's place in the bucket */
+  uint32_t* pieces;           /* per region its pieces, from region_start on */
+  uint32_t* region_start;
+  uint32_t* region_count;     /* records */
+};
+
+template <typename R, int BITS>
+__global__ __launch_bounds__(SPLIT_BS) void k_split(SplitArgs a) {
+  constexpr int ITEMS = SplitShape<R, BITS>::ITEMS, TILE = SplitShape<R, BITS>::TILE;
+  constexpr int MAXD = 1 << BITS, DPT = MAXD / SPLIT_BS; /* digits per thread of the scan */
   __shared__ R buf[TILE];
-  const R* in = (const R*)a.in;
-  R* out = (R*)a.out;
-  __shared__ uint32_t cnt[1 << SPLIT2_MAX_BITS], start[1 << SPLIT2_MAX_BITS];
-  __shared__ unsigned long long pos[1 << SPLIT2_MAX_BITS], next[1 << SPLIT2_MAX_BITS];
-  const int b2 = a.b2, shift = a.shift;
-  const uint32_t nb = 1u << b2, m = nb - 1;
-  auto digit = [&](uint64_t x) -> uint32_t { return b2 ? (uint32_t)(x >> shift) & m : 0u; };
-  for (uint64_t s = a.sb0 + blockIdx.x; s < a.sb0 + a.n_sb; s += gridDim.x) {
-    const uint64_t o0 = a.out_start[s], n = a.out_start[s + 1] - o0;
-    const uint64_t lo = a.in_start[s], hi = lo + n;
-    /* count pass: every digit's records in the sub-bucket (a region's
-     * count cannot be estimated: a k-mer repeated thousands of times puts
-     * all its instances in one region) */
-    for (uint32_t i = threadIdx.x; i < nb; i += SPLIT_BS) cnt[i] = 0;
-    __syncthreads();
-    for (uint64_t i0 = lo; i0 < hi; i0 += 2 * SPLIT_TILE) {
-      uint64_t r[2 * SPLIT_ITEMS];
-#pragma unroll
-      for (int k = 0; k < 2 * SPLIT_ITEMS; ++k) {
-        const uint64_t i = i0 + (uint64_t)k * SPLIT_BS + threadIdx.x;
-        r[k] = i < hi ? rec_key(in[i]) : 0;
-      }
-#pragma unroll
-      for (int k = 0; k < 2 * SPLIT_ITEMS; ++k)
-        if (i0 + (uint64_t)k * SPLIT_BS + threadIdx.x < hi) atomicAdd(&cnt[digit(r[k])], 1u);
-    }
-    __syncthreads();
-    wave_exclusive_scan(cnt, start, (int)nb);
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < nb; i += SPLIT_BS) {
-      next[i] = o0 + start[i];
-      a.region_start[(s << b2) + i] = o0 + start[i];
-    }
-    __syncthreads();
-    /* scatter pass: tile by tile, each digit's run after the previous
-     * tile's; the next tile loads while one is sorted and written */
-    R rn[ITEMS];
-    bool okn[ITEMS];
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const uint64_t i = lo + (uint64_t)k * SPLIT_BS + threadIdx.x;
-      okn[k] = i < hi;
-      rn[k] = okn[k] ? in[i] : rec_zero<R>();
-    }
-    for (uint64_t i0 = lo; i0 < hi; i0 += TILE) {
-      R r[ITEMS];
-      bool ok[ITEMS];
+  __shared__ uint32_t cnt[MAXD + 1]; /* a tile's counts, then first place | first new piece << 16 */
+  __shared__ uint32_t nxt[MAXD];     /* next place of each digit in the bucket's pieces (a multiple of PIECE: none open) */
+  __shared__ uint32_t tot[MAXD];     /* records so far */
+  __shared__ uint32_t part[SPLIT_BS / 64];
+  if (*a.pool.overflow) return;
+  const R* in = (const R*)a.pool.recs;
+  const uint32_t clog = a.pool.clog, cmask = (1u << clog) - 1;
+  for (uint32_t b = a.b0 + blockIdx.x; b < a.b1; b += gridDim.x) {
+    const uint32_t ji = count_job_of(a.n_jobs, b, [&](uint32_t q) { return a.jobs[q].bucket0; });
+    const uint32_t beta = a.jobs[ji].beta, b2 = a.jobs[ji].rbits - beta;
+    /* the digit: the b2 hash bits below the bucket's */
+    const uint32_t nd = 1u << b2, dmask = nd - 1;
+    const int sh = 64 + REC_BUCKET_BITS - (int)beta - (int)b2;
+    auto digit = [&](uint64_t x) -> uint32_t { return b2 ? (uint32_t)(x >> sh) & dmask : 0u; };
+    const uint32_t l0 = a.first[b];
+    const uint64_t n = (uint64_t)(a.first[b + 1] - l0) << clog;
+    const uint32_t* list = a.list + l0;
+    /* the bucket's pieces: room for its chunks and one more per region */
+    const uint32_t g0 = a.jobs[ji].region0 + ((b - a.jobs[ji].bucket0) << b2);
+    const uint32_t p0 = (l0 << (clog - PIECE_LOG)) + (g0 - a.q_lo);
+    R* out = (R*)a.out + ((uint64_t)p0 << PIECE_LOG);
+    uint16_t* digit_of = a.digit_of + p0;
+    /* Record slot k of a tile is the tile's record k * SPLIT_BS + thread; m
+     * (wave-uniform) is what is left of the bucket, so a slot is filled when
+     * thread < m - k * SPLIT_BS.  A chunk holds 64 to SPLIT_BS records, so a
+     * wave's record slot has one chunk and a thread one place in it; the
+     * chunk numbers are read a tile ahead of the records. */
+    const uint32_t in_chunk = threadIdx.x & cmask;
+    auto left = [&](uint64_t i0) -> int { return i0 < n ? (int)(n - i0 < (uint64_t)TILE ? n - i0 : TILE) : 0; };
+    auto load_list = [&](uint64_t i0, uint32_t (&ln)[ITEMS]) {
+      const int m = left(i0);
+      const uint32_t* l = list + (i0 >> clog);
+      const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x) >> clog;
 #pragma unroll
       for (int k = 0; k < ITEMS; ++k) {
-        r[k] = rn[k];
-        ok[k] = okn[k];
+        ln[k] = 0;
+        if ((int)threadIdx.x < m - k * SPLIT_BS) ln[k] = l[w + ((uint32_t)(k * SPLIT_BS) >> clog)];
       }
+    };
+    auto load = [&](uint64_t i0, const uint32_t (&ln)[ITEMS], R (&r)[ITEMS]) {
+      const int m = left(i0);
 #pragma unroll
       for (int k = 0; k < ITEMS; ++k) {
-        const uint64_t i = i0 + TILE + (uint64_t)k * SPLIT_BS + threadIdx.x;
-        okn[k] = i < hi;
-        rn[k] = okn[k] ? in[i] : rec_zero<R>();
+        r[k] = rec_zero<R>();
+        if ((int)threadIdx.x < m - k * SPLIT_BS)
+          r[k] = in[((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)ln[k]) << clog) + in_chunk];
       }
-      tile_split<R, ITEMS>(
-          r, ok, (int)nb, buf, cnt, start, digit,
-          [&](int i, uint32_t c) {
-            pos[i] = next[i];
-            next[i] += c;
-          },
-          [&](uint32_t dx, uint32_t j, const R& x) { out[pos[dx] + j] = x; });
+    };
+    /* exclusive prefix of v over the digits, thread t holding digits
+     * t * DPT ...; v is replaced by it, the sum returned.  One barrier (LDS
+     * only: records in flight are not waited for). */
+    auto scan = [&](uint32_t (&v)[DPT]) -> uint32_t {
+      uint32_t mine = 0;
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) {
+        const uint32_t c = v[q];
+        v[q] = mine;
+        mine += c;
+      }
+      uint32_t incl = mine;
+      const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+      }
+      if (lane == 63) part[w] = incl;
+      lds_barrier();
+      /* the waves' sums: lane l takes wave l's */
+      constexpr int NW = SPLIT_BS / 64;
+      uint32_t x = part[lane & (NW - 1)];
+#pragma unroll
+      for (int off = 1; off < NW; off <<= 1) {
+        const uint32_t o = __shfl_up(x, off, 64);
+        if (lane >= off) x += o;
+      }
+      const uint32_t sum = (uint32_t)__builtin_amdgcn_readlane((int)x, NW - 1);
+      const int wu = __builtin_amdgcn_readfirstlane(w);
+      const uint32_t before = incl - mine + (wu ? (uint32_t)__builtin_amdgcn_readlane((int)x, wu - 1) : 0u);
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) v[q] += before;
+      return sum;
+    };
+    for (uint32_t d = threadIdx.x; d < MAXD; d += SPLIT_BS) cnt[d] = nxt[d] = tot[d] = 0;
+    lds_barrier();
+    uint32_t n_pieces = 0;
+    uint32_t ln[ITEMS];
+    R r[ITEMS];
+    load_list(0, ln);
+    load(0, ln, r);
+    load_list(TILE, ln);
+    for (uint64_t i0 = 0; i0 < n; i0 += TILE) {
+      uint32_t okm = 0;
+      const int m = left(i0);
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k)
+        if ((int)threadIdx.x < m - k * SPLIT_BS && (rec_key(r[k]) & 31) != REC_CODE_FILL) okm |= 1u << k;
+      /* digit << 16 | rank among the tile's records of the digit (a tile has
+       * at most 2^14 records, a digit 12 bits) */
+      uint32_t dr[ITEMS];
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k) {
+        const uint32_t d = digit(rec_key(r[k]));
+        dr[k] = d << 16 | (okm >> k & 1u ? atomicAdd(&cnt[d], 1u) : 0u);
+      }
+      lds_barrier();
+      /* A digit's run fills its open piece (`room` places), then new pieces
+       * in a row.  Counts and new pieces are scanned as one word (sums of at
+       * most 2^14 and 2^14 / PIECE + 2^12). */
+      uint32_t c[DPT], v[DPT];
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) {
+        const uint32_t d = threadIdx.x * DPT + q, room = -nxt[d] & (PIECE - 1);
+        c[q] = cnt[d];
+        v[q] = c[q] | (c[q] > room ? (c[q] - room + PIECE - 1) >> PIECE_LOG : 0) << 16;
+      }
+      const uint32_t sum = scan(v), total = sum & 0xFFFF;
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) cnt[threadIdx.x * DPT + q] = v[q];
+      lds_barrier();
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k)
+        if (okm >> k & 1u) buf[(cnt[dr[k] >> 16] & 0xFFFFu) + (dr[k] & 0xFFFFu)] = r[k];
+      lds_barrier();
+      /* the next tile's records, ahead of this one's stores (loads and
+       * stores complete in order) */
+      if (i0 + TILE < n) {
+        load(i0 + TILE, ln, r);
+        load_list(i0 + 2 * (uint64_t)TILE, ln);
+      }
+#pragma unroll 1
+      for (uint32_t i = threadIdx.x; i < total; i += SPLIT_BS) {
+        const R x = buf[i];
+        const uint32_t d = digit(rec_key(x)), w = cnt[d], p = nxt[d];
+        const uint32_t rank = i - (w & 0xFFFFu), room = -p & (PIECE - 1);
+        out[rank < room ? p + rank : ((n_pieces + (w >> 16)) << PIECE_LOG) + (rank - room)] = x;
+      }
+      lds_barrier();
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) {
+        const uint32_t d = threadIdx.x * DPT + q, p = nxt[d], room = -p & (PIECE - 1);
+        const uint32_t np = n_pieces + (v[q] >> 16);
+        if (c[q] > room) {
+          const uint32_t more = c[q] - room;
+#pragma unroll 1
+          for (uint32_t i = 0; i << PIECE_LOG < more; ++i) digit_of[np + i] = (uint16_t)d;
+          nxt[d] = (np << PIECE_LOG) + more;
+        } else {
+          nxt[d] = p + c[q];
+        }
+        tot[d] += c[q];
+        cnt[d] = 0;
+      }
+      n_pieces += sum >> 16;
+      lds_barrier();
     }
+    /* the regions' pieces in order: the full ones as they come, an open one
+     * last */
+    {
+      uint32_t v[DPT];
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) v[q] = (tot[threadIdx.x * DPT + q] + PIECE - 1) >> PIECE_LOG;
+      scan(v);
+#pragma unroll
+      for (int q = 0; q < DPT; ++q) {
+        const uint32_t d = threadIdx.x * DPT + q;
+        cnt[d] = v[q];
+        if (d < nd) {
+          a.region_start[g0 + d] = p0 + v[q];
+          a.region_count[g0 + d] = tot[d];
+        }
+      }
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < n_pieces; i += SPLIT_BS) {
+        const uint32_t d = digit_of[i], p = nxt[d];
+        if (p >> PIECE_LOG != i || !(p & (PIECE - 1))) a.pieces[p0 + atomicAdd(&cnt[d], 1u)] = p0 + i;
+      }
+      __syncthreads();
+      for (uint32_t d = threadIdx.x; d < nd; d += SPLIT_BS)
+        if (nxt[d] & (PIECE - 1)) a.pieces[p0 + cnt[d]] = p0 + (nxt[d] >> PIECE_LOG);
+    }
+    __syncthreads();
   }
 }
 

@@ -1,25 +1,28 @@
 /*
- * regions.h -- counting by table region (plain jobs, k <= 63).
+ * regions.h -- counting by table region (k <= 63).
  *
- * The table is 2^rbits regions of rspan slots (one region fills a build
- * workgroup's LDS); a k-mer's probe window never leaves the region its
- * hash's top rbits bits pick (see Probe in table.h).  Counting then needs no
- * HBM atomics on the table:
+ * A job's table is 2^rbits regions of span slots (one region fills a build
+ * workgroup's LDS at most); a k-mer's probe window never leaves the region
+ * its hash's top rbits bits pick (see Probe in table.h).  Counting then needs
+ * no HBM atomics on the table:
  *
  *   1. k_parse_records: one read per lane, k-mer and reverse complement
  *      rolled along the read; each instance becomes a record (8 bytes,
  *      (hash bits 0..58) << 5 | biedge index; k > 31 adds the k-mer's high
- *      word) in one of 32 buckets picked by hash bits 59..63, so a record's
- *      top bits are its region inside the bucket.  A workgroup stages
- *      records per bucket in LDS and appends runs of >= FLUSH with one
- *      atomic per chunk.
- *   2. two multisplit passes (partition.h) group each bucket's records by
- *      region and note where every region's records start.
+ *      word) in one of its job's 2^beta buckets picked by the top hash bits.
+ *      A workgroup stages records per bucket in LDS and appends whole cache
+ *      lines to chunks of a common pool.
+ *   2. k_split (partition.h) groups each bucket's records by region, in
+ *      pieces of 64, and lists every region's pieces.
  *   3. k_region_build: a workgroup takes regions one by one; per region it
  *      loads the slots into LDS (or starts from EMPTY when the table holds
  *      nothing yet), adds the region's records with LDS atomics, and writes
  *      the region back with coalesced stores.  Entries beyond a slot's NSUB
  *      sub-entries go to the HBM side table exactly as in the atomic count.
+ *
+ * A batch's jobs go through the same launches: every parser workgroup reads
+ * one job's reads, buckets and regions are numbered through all jobs, and a
+ * region's job gives its layout.
  *
  * The table contents equal those of the atomic count up to the order of
  * keys inside a probe run, which no result depends on.
@@ -32,8 +35,6 @@
 
 namespace br {
 
-constexpr int REC_BUCKET_BITS = 5;
-constexpr int REC_BUCKETS = 1 << REC_BUCKET_BITS;
 /* Region sizes: 2560 slots (80 KB of LDS, two 512-thread builds per CU) or
  * 1280 (40 KB, four 256-thread builds per CU); the region_slots knob picks
  * one when a table is allocated. */
@@ -43,36 +44,41 @@ constexpr uint32_t REGION_SMALL_SLOTS = 1280;
 constexpr uint32_t REGION_WIDE_SLOTS = 1280;
 constexpr uint32_t REGION_WIDE_SMALL_SLOTS = 640;
 constexpr uint64_t REGION_BUILD_CU_SLOTS = 512; /* build workgroups resident on the device (x2 for small) */
-/* record parser (k <= 31): workgroup size, positions between appends,
- * staged records per bucket, append threshold (16-byte records, k > 31:
- * a quarter of the positions, half the stage and half the threshold) */
-constexpr int REC_BS = 512, REC_PF = 8, REC_STAGE = 192, REC_FLUSH = 32;
+/* record parser: workgroup size, staged records of all its buckets (128 KB),
+ * records parked while their bucket's stage is full */
+constexpr int REC_BS = 1024, REC_PARK = 512;
+constexpr uint32_t REC_STAGE_BYTES = 128 << 10;
 constexpr int REGION_ITEMS = 8;              /* records per thread loaded at once by the build */
 
-/* Records of a bucket fill chunks of `chunk` slots taken from the front of
- * the bucket's area with one atomic each (a workgroup keeps one open chunk
- * per bucket and pads it with skipped records at the end); records that
- * find their workgroup's stage full (reads longer than the stage) are
- * appended one by one from the back. */
-struct RecArgs {
-  void* recs;                /* REC_BUCKETS x bcap records (RecOf<KT>::T) */
-  uint64_t bcap;
-  unsigned long long* front; /* per bucket: records in chunks taken (> bcap - back: overflow) */
-  unsigned long long* back;  /* per bucket: records appended from the back */
-  unsigned long long* stat;  /* [0] instances, [1] dropped reads */
-  uint32_t chunk;            /* power of two, >= REC_STAGE */
+/* A parser workgroup's share: reads of job `job`, part i of n of them. */
+struct ParseShare {
+  uint32_t job, i, n, pad;
 };
 
-/* Upper bound of the instances of a batch of reads (reads with non-ACGT
- * bases included). */
-__global__ __launch_bounds__(BLOCK) void k_count_instances(ParseArgs a, unsigned long long* out) {
+struct RecArgs {
+  ChunkPool pool;
+  const JobLayout* jobs;
+  const uint64_t* first;     /* job q holds reads [first[q], first[q + 1]) */
+  const ParseShare* share;   /* per workgroup */
+  unsigned long long* stat;  /* per job: instances, dropped reads */
+};
+
+/* Instances of each job's reads (reads with non-ACGT bases included, so an
+ * upper bound).  A few workgroups per job: their totals are one atomic each
+ * (with a workgroup per 256 reads the atomics took 0.63 ms for 13 M reads,
+ * whose offsets are read in 0.03 ms). */
+__global__ __launch_bounds__(BLOCK) void k_count_instances(ParseArgs a, const uint64_t* first, const ParseShare* share,
+                                                           unsigned long long* out) {
+  const ParseShare sh = share[blockIdx.x];
+  const uint64_t r0 = first[sh.job], nr = first[sh.job + 1] - r0;
+  const uint64_t lo = r0 + nr * sh.i / sh.n, hi = r0 + nr * (sh.i + 1) / sh.n;
   unsigned long long n = 0;
-  for (uint64_t r = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; r < a.n_reads; r += (uint64_t)gridDim.x * BLOCK) {
+  for (uint64_t r = lo + threadIdx.x; r < hi; r += BLOCK) {
     const uint64_t off = a.starts ? a.starts[r] : a.offsets[r];
     const uint64_t L = (a.starts ? a.ends[r] : a.offsets[r + 1]) - off;
     if (L >= (uint64_t)a.K + 2) n += L - a.K + 1;
   }
-  block_add(n, out);
+  block_add(n, out + sh.job);
 }
 
 /* A k-mer instance's record: the key word (hash << 5) | biedge index, and
@@ -84,12 +90,7 @@ template <> __device__ __forceinline__ ulonglong2 make_rec<u128>(uint64_t key, u
   return make_ulonglong2(key, (uint64_t)(km >> 64));
 }
 
-template <typename R>
-__device__ __forceinline__ void rec_put(const RecArgs& ra, uint32_t b, uint64_t at, const R& rec) {
-  if (at < ra.bcap) ((R*)ra.recs)[(uint64_t)b * ra.bcap + at] = rec;
-}
-
-/* chunk padding: a record the first multisplit pass drops (code 31) */
+/* chunk padding: a record the split drops (code 31) */
 template <typename R> __device__ __forceinline__ R rec_filler();
 template <> __device__ __forceinline__ uint64_t rec_filler<uint64_t>() { return REC_CODE_FILL; }
 template <> __device__ __forceinline__ ulonglong2 rec_filler<ulonglong2>() { return make_ulonglong2(REC_CODE_FILL, 0); }
@@ -101,73 +102,171 @@ template <> __device__ __forceinline__ ulonglong2 rec_filler<ulonglong2>() { ret
  * step through their reads in aligned 16-byte blocks, all lanes of the
  * workgroup at the same block index (bases before a read's start or past
  * its end are masked off), loading the next block while the current one
- * is parsed; every PF positions the workgroup appends its staged records
- * (about BS x PF / 32 per bucket), so the loop runs to the longest read of
- * the workgroup's BS reads.  A read with a non-ACGT base is dropped whole
+ * is parsed.  A read with a non-ACGT base is dropped whole
  * (NFilterSequencesIterator, compact_dbg_freq_construct_clean.cpp:210-213),
- * found by a first pass over its blocks. */
-template <typename KT, int BS, int PF, int STAGE, int FLUSH>
-__global__ __launch_bounds__(BS) void k_parse_records(ParseArgs a, RecArgs ra) {
+ * found by a first pass over its blocks.
+ *
+ * Staging: the LDS stage is divided among the job's buckets; every PF
+ * positions the workgroup appends each bucket's whole 128-byte lines to the
+ * bucket's open chunk (the rest moves to the front of its stage), so chunks
+ * are written in full lines whatever their number.  A record that finds its
+ * stage full is parked and staged again when the park is half full; one that
+ * finds the park full too gives the count up (the caller counts with
+ * atomics), which takes one bucket getting a fifteenth of all records.
+ *
+ * One 1,024-thread workgroup per CU with 256 buckets (512 for the largest
+ * tables).  Bound by instruction issue; the appends to 256 buckets cost
+ * 5-15% over 32 (1.6 G instances 7.4 -> 7.8 ms, 184 M 0.84 -> 0.96, 301 M of
+ * k = 63 2.48 -> 2.59; 21 M, where a workgroup has two rounds of 600 reads,
+ * 0.15 -> 0.21), and the split after it needs one pass instead of two: the
+ * count phase as a whole 35.9 -> 30.1, 4.5 -> 3.8, 13.2 -> 10.7 and 1.39 ->
+ * 0.81 ms.  A batch of 16 jobs of 0.05 to 2 Mbp (243 M instances), which HBM
+ * atomics counted in 18.6 ms, takes 5.9. */
+template <typename KT, int MAXB, int PF>
+__global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs ra) {
   typedef typename RecOf<KT>::T R;
-  __shared__ R stg[REC_BUCKETS][STAGE];
-  __shared__ uint32_t cnt[REC_BUCKETS];
-  __shared__ unsigned long long ch_base[REC_BUCKETS]; /* open chunk (~0: none) */
-  __shared__ uint32_t ch_fill[REC_BUCKETS];
-  __shared__ uint32_t fl_n1[REC_BUCKETS], fl_n2[REC_BUCKETS];
-  __shared__ unsigned long long fl_d1[REC_BUCKETS], fl_d2[REC_BUCKETS];
-  __shared__ uint32_t blocks_max;
-  constexpr int WPB = BS / 64;
+  constexpr uint32_t LINE = 128 / sizeof(R);
+  constexpr uint32_t STAGE = REC_STAGE_BYTES / sizeof(R);
+  __shared__ R stg[STAGE];
+  __shared__ uint32_t cnt[MAXB];
+  __shared__ uint32_t ch_id[MAXB], ch_fill[MAXB];     /* open chunk (NO_CHUNK: none) */
+  __shared__ uint32_t fl_n1[MAXB], fl_n[MAXB], fl_c1[MAXB], fl_f1[MAXB]; /* an append: see flush */
+  __shared__ R park[REC_PARK];
+  __shared__ uint16_t park_b[REC_PARK];
+  __shared__ uint32_t n_park, blocks_max;
+  __shared__ uint32_t pl_base, pl_used, pl_size; /* chunk numbers in hand */
   static_assert(16 % PF == 0, "flush points split a block evenly");
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint32_t tid = threadIdx.x;
+  const ParseShare sh = ra.share[blockIdx.x];
+  const JobLayout* jb = ra.jobs + sh.job;
+  const uint32_t beta = jb->beta, nb_ = 1u << beta, S = STAGE >> beta, bucket0 = jb->bucket0;
+  const uint32_t clog = ra.pool.clog, C = 1u << clog;
   const int K = a.K;
-  const uint32_t C = ra.chunk;
   kops<KT> ops(K);
   unsigned long long my_inst = 0, my_drop = 0;
-  if (threadIdx.x < REC_BUCKETS) {
-    cnt[threadIdx.x] = 0;
-    ch_base[threadIdx.x] = ~0ULL;
-    ch_fill[threadIdx.x] = 0;
+  for (uint32_t b = tid; b < nb_; b += REC_BS) {
+    cnt[b] = 0;
+    ch_id[b] = NO_CHUNK;
+    ch_fill[b] = 0;
   }
+  if (tid == 0) n_park = pl_base = pl_used = pl_size = 0;
   __syncthreads();
-  /* append every bucket holding >= at staged records to its open chunk
-   * (the rest to a new chunk), then empty them */
-  auto flush = [&](uint32_t at) {
-    if (threadIdx.x < REC_BUCKETS) {
-      const uint32_t t = threadIdx.x;
-      const uint32_t c = cnt[t];
-      uint32_t n = c < (uint32_t)STAGE ? c : (uint32_t)STAGE;
-      if (n < at) n = 0;
-      const unsigned long long base = ch_base[t];
-      const uint32_t fill = ch_fill[t];
-      const uint32_t room = base == ~0ULL ? 0u : C - fill;
-      const uint32_t m1 = n < room ? n : room, m2 = n - m1;
-      fl_n1[t] = m1;
-      fl_d1[t] = base + fill;
-      fl_n2[t] = m2;
-      if (m2) {
-        const unsigned long long nb = atomicAdd(&ra.front[t], (unsigned long long)C);
-        fl_d2[t] = nb;
-        ch_base[t] = nb;
-        ch_fill[t] = m2;
+  R* const recs = (R*)ra.pool.recs;
+  auto put = [&](uint32_t b, const R& rec) {
+    const uint32_t pos = atomicAdd(&cnt[b], 1u);
+    if (pos < S) {
+      stg[b * S + pos] = rec;
+    } else {
+      const uint32_t p = atomicAdd(&n_park, 1u);
+      if (p < REC_PARK) {
+        park[p] = rec;
+        park_b[p] = (uint16_t)b;
       } else {
-        ch_fill[t] = fill + m1;
+        *ra.pool.overflow = 1;
       }
-      if (n) cnt[t] = 0;
+    }
+  };
+  auto unused = [&](uint32_t c) {
+    if (c < ra.pool.n_max) ra.pool.owner[c] = NO_CHUNK;
+  };
+  /* append every bucket's whole lines (last: everything) to its open chunk,
+   * the rest to a new one: fl_n records, of which fl_n1 go to chunk fl_c1
+   * from place fl_f1 and the others to the front of chunk ch_id */
+  auto flush = [&](bool last) {
+    if (tid < nb_) {
+      const uint32_t c = cnt[tid], n = c < S ? c : S;
+      const uint32_t m = last ? n : n & ~(LINE - 1);
+      const uint32_t id = ch_id[tid], fill = ch_fill[tid];
+      const uint32_t room = id == NO_CHUNK ? 0u : C - fill;
+      const uint32_t m1 = m < room ? m : room, m2 = m - m1;
+      fl_n[tid] = m;
+      fl_n1[tid] = m1;
+      fl_c1[tid] = id;
+      fl_f1[tid] = fill;
+      cnt[tid] = n - m;
+      ch_fill[tid] = m2 ? m2 : fill + m1;
+      /* One chunk number per bucket that needs one, from those in hand
+       * (an atomic in HBM here would hold up the whole workgroup at the
+       * next barrier: 2 of 9 ms); a wave that finds too few takes its own,
+       * and strikes out what was left. */
+      const uint64_t need = __ballot(m2 != 0);
+      if (need) {
+        const uint32_t lane = tid & 63, want = (uint32_t)__popcll(need);
+        uint32_t nid = 0;
+        if (lane == 0) {
+          const uint32_t u = atomicAdd(&pl_used, want);
+          nid = pl_base + u;
+          if (u + want > pl_size) {
+            for (uint32_t q = u; q < pl_size; ++q) unused(pl_base + q);
+            nid = atomicAdd(ra.pool.next, want);
+          }
+        }
+        nid = (uint32_t)__builtin_amdgcn_readfirstlane((int)nid) + (uint32_t)__popcll(need & ((1ULL << lane) - 1));
+        if (m2) {
+          atomicAdd(&ra.pool.taken[bucket0 + tid], 1u);
+          if (nid < ra.pool.n_max) ra.pool.owner[nid] = bucket0 + tid;
+          else *ra.pool.overflow = 1;
+          ch_id[tid] = nid < ra.pool.n_max ? nid : ra.pool.n_max - 1;
+        }
+      }
     }
     lds_barrier();
-    for (int b = w; b < REC_BUCKETS; b += WPB) {
-      const uint32_t m1 = fl_n1[b], m2 = fl_n2[b];
-      const unsigned long long d1 = fl_d1[b], d2 = fl_d2[b];
-      for (uint32_t i = lane; i < m1 + m2; i += 64) rec_put(ra, b, i < m1 ? d1 + i : d2 + (i - m1), stg[b][i]);
+    /* numbers for the next appends, while the other waves copy */
+    if (tid == REC_BS - 1 && !last && pl_used + CHUNK_LOW > pl_size) {
+      for (uint32_t q = pl_used; q < pl_size; ++q) unused(pl_base + q);
+      pl_base = atomicAdd(ra.pool.next, CHUNK_BATCH);
+      pl_size = CHUNK_BATCH;
+      pl_used = 0;
+    }
+    /* LINE lanes per bucket */
+    const uint32_t gl = tid & (LINE - 1);
+    for (uint32_t b = tid / LINE; b < nb_; b += REC_BS / LINE) {
+      const uint32_t m = fl_n[b];
+      if (m == 0) continue;
+      const uint32_t m1 = fl_n1[b];
+      R* d1 = recs + ((uint64_t)fl_c1[b] << clog) + fl_f1[b];
+      R* d2 = recs + ((uint64_t)ch_id[b] << clog);
+      for (uint32_t i = gl; i < m; i += LINE) {
+        R* d = i < m1 ? d1 + i : d2 + (i - m1);
+        *d = stg[b * S + i];
+      }
+      /* fewer than LINE records are left; the lanes read before they write */
+      if (gl < cnt[b]) stg[b * S + gl] = stg[b * S + m + gl];
     }
     lds_barrier();
   };
-  const int sh = 2 * (K - 1);
+  /* stage the parked records again until none is left (every bucket has
+   * room for S - LINE of its own each time) */
+  auto unpark = [&]() {
+    for (;;) {
+      const uint32_t n = n_park < REC_PARK ? n_park : REC_PARK;
+      if (n == 0) break;
+      R rec = rec_zero<R>();
+      uint32_t b = 0;
+      if (tid < n) {
+        rec = park[tid];
+        b = park_b[tid];
+      }
+      lds_barrier();
+      if (tid == 0) n_park = 0;
+      lds_barrier();
+      if (tid < n) put(b, rec);
+      lds_barrier();
+      flush(false);
+    }
+  };
+  const int sh2 = 2 * (K - 1);
   const KT kmask = ops.mask;
-  for (uint64_t r0 = (uint64_t)blockIdx.x * BS; r0 < a.n_reads; r0 += (uint64_t)gridDim.x * BS) {
-    const uint64_t r = r0 + threadIdx.x;
+  /* the share's reads, in as many rounds of up to REC_BS lanes as it takes,
+   * evenly filled */
+  const uint64_t r_job = ra.first[sh.job], n_job = ra.first[sh.job + 1] - r_job;
+  const uint64_t lo_r = r_job + n_job * sh.i / sh.n, hi_r = r_job + n_job * (sh.i + 1) / sh.n;
+  const uint64_t rounds = (hi_r - lo_r + REC_BS - 1) / REC_BS;
+  for (uint64_t round = 0; round < rounds; ++round) {
+    const uint64_t ra0 = lo_r + (hi_r - lo_r) * round / rounds, ra1 = lo_r + (hi_r - lo_r) * (round + 1) / rounds;
+    const uint64_t r = ra0 + tid;
     uint64_t lo = 0, L = 0;
-    if (r < a.n_reads) {
+    if (r < ra1) {
       lo = a.starts ? a.starts[r] : a.offsets[r];
       L = (a.starts ? a.ends[r] : a.offsets[r + 1]) - lo;
     }
@@ -194,7 +293,7 @@ __global__ __launch_bounds__(BS) void k_parse_records(ParseArgs a, RecArgs ra) {
     const uint64_t nb = Lp ? (uint64_t)(mis + (int64_t)Lp + 16) / 16 : 0; /* through position Lp */
     /* every thread has read the last round's maximum before it is reset */
     __syncthreads();
-    if (threadIdx.x == 0) blocks_max = 0;
+    if (tid == 0) blocks_max = 0;
     __syncthreads();
     if (nb) atomicMax(&blocks_max, (uint32_t)nb);
     __syncthreads();
@@ -206,6 +305,10 @@ __global__ __launch_bounds__(BS) void k_parse_records(ParseArgs a, RecArgs ra) {
      * the first instance). */
     KT fw = 0, rv = 0;
     uint32_t gone = 0;
+    /* a round of few reads fills its stages more slowly: an append at every
+     * PF-th position, or once a block when a bucket's share of the block's
+     * records leaves a quarter of its stage to chance and what stays behind */
+    const bool often = (ra1 - ra0) * 16 > (uint64_t)(STAGE - STAGE / 4 - nb_ * (LINE / 2));
     uint4 cur = nb ? blk[0] : make_uint4(0, 0, 0, 0);
     for (uint32_t t = 0; t < nbw; ++t) {
       const uint4 nxt = (t + 1 < nb && t + 1 < nblk) ? blk[t + 1] : make_uint4(0, 0, 0, 0);
@@ -228,55 +331,53 @@ __global__ __launch_bounds__(BS) void k_parse_records(ParseArgs a, RecArgs ra) {
             const uint32_t il2 = flip && has_out ? 4u - c : il;
             const uint32_t ir2 = flip && has_in ? 4u - gone : ir;
             const uint64_t h = kmer_hash(km);
-            const uint32_t b = (uint32_t)(h >> (64 - REC_BUCKET_BITS));
             const uint64_t key = (h << REC_BUCKET_BITS) | (il2 * 5u + ir2);
-            const R rec = make_rec<KT>(key, km);
-            const uint32_t pos = atomicAdd(&cnt[b], 1u);
-            if (pos < (uint32_t)STAGE) {
-              stg[b][pos] = rec;
-            } else {
-              /* stage full: one record from the back */
-              const unsigned long long k = atomicAdd(&ra.back[b], 1ULL);
-              if (k < ra.bcap) rec_put(ra, b, ra.bcap - 1 - k, rec);
-            }
+            put((uint32_t)(h >> (64 - beta)), make_rec<KT>(key, km));
             ++my_inst;
           }
           if (in_read) {
-            gone = (uint32_t)(fw >> sh) & 3u;
+            gone = (uint32_t)(fw >> sh2) & 3u;
             fw = ((fw << 2) | (KT)c) & kmask;
-            rv = (rv >> 2) | ((KT)(3u - c) << sh);
+            rv = (rv >> 2) | ((KT)(3u - c) << sh2);
           }
         }
-        if (q % PF == PF - 1) {
+        if (q % PF == PF - 1 && (often || q == 15)) {
           lds_barrier();
-          flush(FLUSH);
+          flush(false);
+          if (n_park > REC_PARK / 2) unpark();
         }
       }
       cur = nxt;
     }
   }
-  flush(1);
+  unpark();
+  flush(true);
+  if (tid == 0)
+    for (uint32_t q = pl_used; q < pl_size; ++q) unused(pl_base + q);
   /* pad the open chunks */
-  for (int b = w; b < REC_BUCKETS; b += WPB) {
-    const unsigned long long base = ch_base[b];
-    if (base == ~0ULL) continue;
-    for (uint32_t i = ch_fill[b] + lane; i < C; i += 64) rec_put(ra, b, base + i, rec_filler<R>());
+  for (uint32_t b = tid / 64; b < nb_; b += REC_BS / 64) {
+    if (ch_id[b] == NO_CHUNK) continue;
+    R* d = recs + ((uint64_t)ch_id[b] << clog);
+    for (uint32_t i = ch_fill[b] + (tid & 63); i < C; i += 64) d[i] = rec_filler<R>();
   }
   const unsigned long long si = wave_sum(my_inst), sd = wave_sum(my_drop);
-  if (lane == 0) {
-    if (si) atomicAdd(&ra.stat[0], si);
-    if (sd) atomicAdd(&ra.stat[1], sd);
+  if ((tid & 63) == 0) {
+    if (si) atomicAdd(&ra.stat[2 * sh.job], si);
+    if (sd) atomicAdd(&ra.stat[2 * sh.job + 1], sd);
   }
 }
 
 struct RegionArgs {
   void* table;               /* Slot<KT> */
-  uint64_t span;             /* slots per region */
-  uint32_t rbits;            /* region bits (the bucket's 5 and rb below them) */
-  uint64_t n_regions;        /* 2^rbits */
-  uint64_t q0, q1;           /* this launch: regions [q0, q1) */
-  const void* recs;          /* records (RecOf<KT>::T) grouped by region */
-  const uint64_t* region_start; /* [n_regions + 1]: region q holds recs[region_start[q], region_start[q + 1]) */
+  const JobLayout* jobs;      /* their table layouts; regions are numbered through all of them */
+  uint32_t n_jobs;
+  uint32_t q0, q1;           /* this launch: regions [q0, q1) */
+  const void* recs;          /* pieces of PIECE records (RecOf<KT>::T) */
+  const uint32_t* pieces;    /* region q holds region_count[q] records, in the pieces
+                                pieces[region_start[q] ...] */
+  const uint32_t* region_start;
+  const uint32_t* region_count;
+  const uint32_t* overflow;  /* set: the records are not complete, nothing is built */
   int valid;                 /* the table holds earlier counts (else start from EMPTY) */
   Spill* spill;
   uint64_t spcap;
@@ -289,7 +390,7 @@ struct RegionArgs {
   uint32_t* spq_n;
   uint32_t spq_cap;
   Counters* ctr;
-  /* filter pre-pass (optional): per region `stride` words of candidate
+  /* filter pre-pass (optional): from word q * stride, region q's candidate
    * bits (occupied, no spilled entries, k-mer count >= t1lo when
    * thresholding) and of spilled-slot bits, bit i of word w = slot 64 w + i */
   uint64_t* cbits;
@@ -516,11 +617,11 @@ __device__ __forceinline__ void consume(const ulonglong2& v) {
 constexpr uint32_t NO_SPILL = ~0u;
 template <typename KT, uint32_t SLOTS, typename R>
 __device__ __forceinline__ uint32_t region_add(const RegionArgs& g, LdsRegion<KT, SLOTS>& L, uint32_t span,
-                                               const R& rec, uint32_t& my_new, uint32_t& my_k2) {
+                                               uint32_t rbits, const R& rec, uint32_t& my_new, uint32_t& my_k2) {
   const uint64_t key = rec_key(rec);
   bool fresh;
   /* the record's hash bits below the region's, as region_home takes them */
-  const uint32_t home = region_home(key, g.rbits - REC_BUCKET_BITS, span);
+  const uint32_t home = region_home(key, rbits - REC_BUCKET_BITS, span);
   const uint32_t s = lds_claim(L, span, home, rec, fresh);
   if (s == ~0u) {
     atomicOr(&g.ctr->err, ERR_TABLE_FULL);
@@ -681,7 +782,9 @@ __device__ __forceinline__ bool fuse_nodes(const RegionArgs& g, LdsRegion<KT, SL
 
 /* Side-table entries the region builds queued, one workgroup per queue. */
 __global__ __launch_bounds__(BLOCK) void k_spill_flush(const uint64_t* spq, const uint32_t* spq_n, uint32_t spq_cap,
-                                                        Spill* spill, uint64_t spcap, Counters* ctr) {
+                                                        const uint32_t* overflow, Spill* spill, uint64_t spcap,
+                                                        Counters* ctr) {
+  if (*overflow) return; /* nothing was built */
   const uint32_t n = min(spq_n[blockIdx.x], spq_cap);
   const uint64_t* q = spq + (uint64_t)blockIdx.x * spq_cap;
   unsigned long long mine = 0;
@@ -692,7 +795,9 @@ __global__ __launch_bounds__(BLOCK) void k_spill_flush(const uint64_t* spq, cons
   block_add(mine, &ctr->n_k2);
 }
 
-/* Build regions [q0, q1), workgroup i taking an even share [qa, qb) of them.
+/* Build regions [q0, q1), workgroup i taking every gridDim-th of them (the
+ * jobs of a batch differ in records per region, so neighbours in one
+ * workgroup would leave some with the work of several).
  * Per region: set up the slots in LDS (EMPTY, or the table's slots when an
  * earlier count wrote them; a region without records is then left as it
  * is), add the region's records (REGION_ITEMS per thread at a time), write
@@ -700,7 +805,11 @@ __global__ __launch_bounds__(BLOCK) void k_spill_flush(const uint64_t* spq, cons
  * stores, a slot per lane).  The next region's first records are loaded
  * before this region's records are added, so their latency hides behind
  * the LDS work; barriers order LDS only, so one region's write-back
- * overlaps the next region's set-up.
+ * overlaps the next region's set-up.  Nothing between two write-backs may
+ * wait for a load issued after the first one (loads and stores complete in
+ * order): piece numbers are read two regions ahead and region bounds three,
+ * and a job's layout only when a workgroup comes to it (184 M records: 1.70
+ * -> 1.52 ms; 301 M of 16 bytes: 5.13 -> 4.40).
  *
  * Bound by the instructions per record (vector and scalar; LDS is busy a
  * third of the time), so the adds carry no lane masks through their loops,
@@ -717,28 +826,34 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
    * slots, so half as many (and the registers stay without spills) */
   constexpr int REGION_ITEMS = sizeof(R) == 8 ? br::REGION_ITEMS : br::REGION_ITEMS / 2;
   __shared__ LdsRegion<KT, SLOTS> L;
-  const uint32_t span = (uint32_t)g.span;
-  const uint64_t nreg = g.n_regions;
-  const uint64_t nlaunch = g.q1 - g.q0;
-  const uint64_t qa = g.q0 + (uint64_t)blockIdx.x * nlaunch / gridDim.x,
-                 qb = g.q0 + ((uint64_t)blockIdx.x + 1) * nlaunch / gridDim.x;
+  if (*g.overflow) return;
+  const uint32_t qa = g.q0 + blockIdx.x, step = gridDim.x;
   const R* recs = (const R*)g.recs;
   uint32_t my_new = 0, my_k2 = 0; /* a lane's records of one launch: far below 2^32 */
-  constexpr uint64_t TILE = (uint64_t)REGION_ITEMS * BS;
-  /* region_start[q] for the workgroup's regions, 64 at a time: lane l of
-   * every wave holds entry rs_base + l and the next 64 are loaded ahead,
-   * so a region's bounds are two lane reads, not a dependent load */
+  constexpr uint32_t TILE = REGION_ITEMS * BS;
+  /* first piece and record count of the workgroup's regions, 64 at a
+   * time: lane l of every wave holds its region number rs_n + l and the
+   * next 64 are loaded ahead, so a region's bounds are lane reads, not
+   * dependent loads */
   const int lane = threadIdx.x & 63;
-  uint64_t rs_base = qa;
-  auto rs_load = [&](uint64_t b) -> uint64_t { return b + lane <= nreg ? g.region_start[b + lane] : 0; };
-  uint64_t rs = rs_load(qa), rs_nx = rs_load(qa + 64);
-  auto rstart = [&](uint64_t q) -> uint64_t { /* q never decreases */
-    while (q >= rs_base + 64) {
+  uint32_t rs_n = 0;
+  auto rs_load = [&](uint32_t n, uint32_t& st, uint32_t& c) {
+    const uint64_t q = qa + (uint64_t)(n + lane) * step;
+    st = q < g.q1 ? g.region_start[q] : 0;
+    c = q < g.q1 ? g.region_count[q] : 0;
+  };
+  uint32_t rs, rs_nx, rc, rc_nx;
+  rs_load(0, rs, rc);
+  rs_load(64, rs_nx, rc_nx);
+  auto bounds = [&](uint32_t n, uint32_t& start, uint32_t& count) { /* n never decreases */
+    while (n >= rs_n + 64) {
       rs = rs_nx;
-      rs_base += 64;
-      rs_nx = rs_load(rs_base + 64);
+      rc = rc_nx;
+      rs_n += 64;
+      rs_load(rs_n + 64, rs_nx, rc_nx);
     }
-    return readlane64(rs, (int)(q - rs_base));
+    start = (uint32_t)__builtin_amdgcn_readlane((int)rs, (int)(n - rs_n));
+    count = (uint32_t)__builtin_amdgcn_readlane((int)rc, (int)(n - rs_n));
   };
   /* this wave's side-table queue */
   const uint64_t wave_id = (uint64_t)blockIdx.x * (BS / 64) + (threadIdx.x >> 6);
@@ -746,31 +861,88 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
   uint32_t qn = 0;
   /* this wave's open chunks of the chain and branch lists (fused filter) */
   ListChunk ch[2] = {{0, FUSE_CHUNK}, {0, FUSE_CHUNK}};
-  /* first tile of the next region with records, loaded ahead */
-  R rn[REGION_ITEMS];
-  uint64_t nq = qa, nlo = 0, nhi = 0;
-  auto ahead = [&](uint64_t from) {
-    nq = from;
-    for (; nq < qb; ++nq) {
-      nlo = rstart(nq);
-      nhi = rstart(nq + 1);
-      if (!(g.valid && nlo == nhi)) break; /* no records: the region stays as it is */
-    }
-    if (nq < qb) {
+  /* A region's piece numbers, 64 of this wave's at a time: record slot k
+   * of tile t is the region's piece (t * REGION_ITEMS + k) * NW + wave, so
+   * lane l loads the number of piece l * NW + wave, for 64 / REGION_ITEMS
+   * tiles. */
+  constexpr uint32_t NW = BS / 64, TILES = 64 / REGION_ITEMS;
+  auto numbers = [&](uint32_t start, uint32_t count, uint32_t t) -> uint32_t {
+    const uint32_t i = (t * REGION_ITEMS + lane) * NW + (threadIdx.x >> 6);
+    /* (no branch: a value of two paths would be copied, and waited for) */
+    return g.pieces[i << PIECE_LOG < count ? start + i : 0];
+  };
+  auto load = [&](uint32_t count, uint32_t nums, uint32_t t, R (&r)[REGION_ITEMS]) {
 #pragma unroll
-      for (int k = 0; k < REGION_ITEMS; ++k) {
-        const uint64_t i = nlo + (uint64_t)k * BS + threadIdx.x;
-        rn[k] = i < nhi ? recs[i] : rec_zero<R>();
-      }
+    for (int k = 0; k < REGION_ITEMS; ++k) {
+      const uint32_t p = (uint32_t)__builtin_amdgcn_readlane((int)nums, (int)((t % TILES) * REGION_ITEMS + k));
+      r[k] = rec_zero<R>();
+      if (t * TILE + k * BS + threadIdx.x < count) r[k] = recs[((uint64_t)p << PIECE_LOG) + lane];
     }
   };
-  ahead(qa);
-  while (nq < qb) {
-    const uint64_t q = nq, lo = nlo, hi = nhi;
+  /* Read ahead of the region being built: the next one's first tile, the
+   * piece numbers of the one after, and where the pieces of the third are (a
+   * region without records in a written table stays as it is and is passed
+   * over; past the last one the counts are 0). */
+  struct Ahead {
+    uint32_t q, start, count;
+  };
+  Ahead nx, af, th; /* next, after it, third */
+  uint32_t th_n = 0; /* number of the third of the workgroup's regions */
+  R rn[REGION_ITEMS];
+  uint32_t af_nums;
+  auto find = [&]() {
+    for (;; ++th_n) {
+      th.q = qa + th_n * step;
+      th.start = th.count = 0;
+      if (th.q >= g.q1) return;
+      bounds(th_n, th.start, th.count);
+      if (!(g.valid && th.count == 0)) break;
+    }
+    ++th_n;
+  };
+  auto ahead = [&]() {
+    nx = af;
+    load(nx.count, af_nums, 0, rn);
+    af = th;
+    af_nums = numbers(af.start, af.count, 0);
+  };
+  /* the current region's job (read when a workgroup comes to it: a load at
+   * each region would wait for the write-back before it) */
+  uint32_t ji = count_job_of(g.n_jobs, qa, [&](uint32_t j) { return g.jobs[j].region0; });
+  uint32_t ji_end, span, rbits, region0;
+  uint64_t slot0;
+  auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+  auto job = [&]() {
+    ji_end = ji + 1 < g.n_jobs ? uniform(g.jobs[ji + 1].region0) : ~0u;
+    span = uniform((uint32_t)g.jobs[ji].span);
+    rbits = uniform(g.jobs[ji].rbits);
+    region0 = uniform(g.jobs[ji].region0);
+    slot0 = readlane64(g.jobs[ji].slot0, 0);
+  };
+  job();
+  find();
+  af = th;
+  af_nums = numbers(af.start, af.count, 0);
+  find();
+  uint32_t nums = af_nums;
+  ahead();
+  find();
+  /* nothing read ahead is under way where the loop is entered or repeated:
+   * a wait inside it then covers its own loads only */
+#pragma unroll
+  for (int k = 0; k < REGION_ITEMS; ++k) consume(rn[k]);
+  consume((uint64_t)af_nums);
+  while (nx.q < g.q1) {
+    const uint32_t q = nx.q, count = nx.count, start = nx.start;
+    while (q >= ji_end) {
+      ++ji;
+      job();
+    }
+    const uint32_t rq = q - region0;
     R rr[REGION_ITEMS];
 #pragma unroll
     for (int k = 0; k < REGION_ITEMS; ++k) rr[k] = rn[k];
-    const uint64_t base = q * g.span;
+    const uint64_t base = slot0 + (uint64_t)rq * span;
     Slot<KT>* T = (Slot<KT>*)g.table + base;
     if (g.valid) {
       L.template load<BS>(span, T);
@@ -779,7 +951,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
     } else {
       L.template clear<BS>(span);
     }
-    ahead(q + 1);
+    uint32_t nums_nx = af_nums;
+    ahead();
     lds_barrier();
     /* the first tile, loaded ahead; a region longer than one tile loads
      * the rest here (in registers of their own, so the first tile's adds
@@ -787,34 +960,35 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
     for (int k = 0; k < REGION_ITEMS; ++k) {
       uint32_t e = NO_SPILL;
-      if (lo + (uint64_t)k * BS + threadIdx.x < hi) e = region_add<KT, SLOTS, R>(g, L, span, rr[k], my_new, my_k2);
+      if (k * BS + threadIdx.x < count) e = region_add<KT, SLOTS, R>(g, L, span, rbits, rr[k], my_new, my_k2);
       spill_queue(g, spq, qn, e, base, (uint32_t)rec_key(rr[k]) & 31, my_k2);
     }
-    for (uint64_t i0 = lo + TILE; i0 < hi; i0 += TILE) {
+    for (uint32_t t = 1; t * TILE < count; ++t) {
+      if (t % TILES == 0) nums = numbers(start, count, t);
       R rt[REGION_ITEMS];
+      load(count, nums, t, rt);
 #pragma unroll
-      for (int k = 0; k < REGION_ITEMS; ++k) {
-        const uint64_t i = i0 + (uint64_t)k * BS + threadIdx.x;
-        rt[k] = i < hi ? recs[i] : rec_zero<R>();
-      }
+      for (int k = 0; k < REGION_ITEMS; ++k) consume(rt[k]);
 #pragma unroll
       for (int k = 0; k < REGION_ITEMS; ++k) {
         uint32_t e = NO_SPILL;
-        if (i0 + (uint64_t)k * BS + threadIdx.x < hi)
-          e = region_add<KT, SLOTS, R>(g, L, span, rt[k], my_new, my_k2);
+        if (t * TILE + k * BS + threadIdx.x < count)
+          e = region_add<KT, SLOTS, R>(g, L, span, rbits, rt[k], my_new, my_k2);
         spill_queue(g, spq, qn, e, base, (uint32_t)rec_key(rt[k]) & 31, my_k2);
       }
     }
-    /* the next region's records (loaded since this region began) are
-     * waited for here, before the write-back's stores: stores and loads
+    /* what was read ahead since this region began is waited for here, before the write-back's stores: stores and loads
      * share one in-order counter, so waiting for them after the stores
      * would wait for the stores too */
 #pragma unroll
     for (int k = 0; k < REGION_ITEMS; ++k) consume(rn[k]);
+    consume((uint64_t)af_nums);
+    find();
+    nums = nums_nx;
     lds_barrier();
     /* a slot's words are finished by the thread that reads them below (the
      * fused filter: by a lane of the same wave) */
-    const uint64_t h_top = (q >> (g.rbits - REC_BUCKET_BITS)) << (64 - REC_BUCKET_BITS);
+    const uint64_t h_top = (uint64_t)(rq >> (rbits - REC_BUCKET_BITS)) << (64 - REC_BUCKET_BITS);
     if (FUSE || !g.cbits)
       for (uint32_t i = threadIdx.x; i < span; i += BS) lds_finish(L, i, h_top);
     bool left = false; /* a candidate of this wave's slots found its list full */
@@ -863,8 +1037,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const uint64_t bc = __ballot(c), bsp = __ballot(sp);
         const uint32_t w0 = i0 + (threadIdx.x & ~63u);
         if ((threadIdx.x & 63) == 0 && w0 < span) {
-          g.cbits[q * g.stride + w0 / 64] = bc;
-          g.sbits[q * g.stride + w0 / 64] = bsp;
+          g.cbits[(uint64_t)q * g.stride + w0 / 64] = bc;
+          g.sbits[(uint64_t)q * g.stride + w0 / 64] = bsp;
         }
       }
     }

@@ -10,9 +10,8 @@
  * one batch (bruno_batch_create ... bruno_run_pipeline).  Requests that
  * arrive while batches are on the device wait for the next free worker and
  * the memory the running batches give back, so several batches overlap on
- * the device.  A request with a large table (2^26 slots or more) runs on
- * its own, counted by regions, which beats its share of a batch's atomic
- * count.  A request whose table proves too small is retried on its own
+ * the device.  A request with a large table (2^26 slots or more) fills the
+ * device by itself and runs on its own, so that no small one waits for it.  A request whose table proves too small is retried on its own
  * with more slots.  All device memory comes from the library's pool,
  * so a running server makes no hipMalloc / hipFree calls.
  *
@@ -401,8 +400,7 @@ bruno_status bruno_server_submit(bruno_server* S, const bruno_request* q, uint64
   r->capacity = q->job.capacity;
   if (r->capacity == 0) r->capacity = std::max<uint64_t>(4096, 2 * r->n_bases);
   r->footprint = footprint(r->job, r->capacity, r->n_reads, r->n_bases);
-  /* a large table runs as a batch of its own, counted by regions: from
-   * about 2^26 slots that beats the job's share of a batch (atomic count) */
+  /* a large table, counted by regions, runs as a batch of its own */
   const uint64_t region = br_region_count_min_slots();
   r->alone = region && r->capacity >= std::max<uint64_t>(region, SOLO_MIN_SLOTS);
   std::lock_guard<std::mutex> lk(S->mu);

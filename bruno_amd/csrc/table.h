@@ -130,6 +130,13 @@ __device__ __forceinline__ uint32_t biedge_index(uint8_t e) {
 __device__ __forceinline__ uint32_t region_home(uint64_t h, uint32_t rbits, uint32_t span) {
   return __umulhi((uint32_t)((h << rbits) >> 32), span);
 }
+/* A job's table: slots from slot0, 2^rbits regions of span slots (rbits 0:
+ * one probe window of span slots).  For a region count also its bucket bits,
+ * and its first region and bucket among those of all jobs of the table. */
+struct JobLayout {
+  uint64_t slot0, span;
+  uint32_t rbits, beta, region0, bucket0;
+};
 struct Probe {
   uint64_t lo, hi, s;
   __device__ __forceinline__ Probe(uint64_t h, uint64_t span, uint32_t rbits) {

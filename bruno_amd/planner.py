@@ -39,11 +39,8 @@ def footprint(s, k, load_factor=0.5, cap=None):
     return int(table + present + reads + chains)
 
 
-# A job with a table of at least this many slots runs alone.  Alone, a job
-# of 2^22 slots or more counts by regions (the batched count is the atomic
-# one); measured on config-4 jobs, from about 5e7 k-mer instances (tables of
-# about 2^26 slots) its region count and later phases alone cost less than
-# its share of a batch.
+# A job with a table of at least this many slots (about 5e7 k-mer instances)
+# runs alone: it fills the device by itself, so a batch gains nothing on it.
 SOLO_SLOTS = 1 << 26
 
 
@@ -51,9 +48,8 @@ def plan_groups(cfgs, k, budget_bytes, load_factor=0.5, solo_slots=SOLO_SLOTS):
     """Jobs packed in arrival order into launch groups whose estimated
     footprint stays within the budget (a job larger than the budget runs
     alone).  A job whose table reaches solo_slots (0: none) runs alone too,
-    in its place: counted by regions it goes faster than in a batch, and a
-    batch gains nothing on a job that fills the device by itself.  The
-    other jobs keep filling the open group past it, which then runs when
+    in its place: a batch gains nothing on a job that fills the device by
+    itself.  The other jobs keep filling the open group past it, which then runs when
     it is full (or at the end)."""
     groups, cur, used = [], [], 0
     for i, s in enumerate(cfgs):

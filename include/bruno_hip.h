@@ -168,7 +168,7 @@ bruno_status bruno_job_set_recycle(bruno_job* job, int on);
  * further batch (bruno_parse_count* returns BRUNO_STATE until
  * bruno_job_reset) and the k2 / count getters return BRUNO_STATE, since
  * node records replace the k2 entries.  Off by default; a count that falls
- * back to atomics (small tables, batches) is not fused.  No counterpart in
+ * back to atomics (small tables) is not fused, nor is a batch's.  No counterpart in
  * the reference, whose filter is a pass of its own over the count map. */
 bruno_status bruno_job_set_fused_filter(bruno_job* job, int on);
 
@@ -375,21 +375,20 @@ typedef struct {
                               nodes on average (power of two, 8..4096; small graphs take
                               fewer): the walk length between rulers and the size of the
                               contracted list                                               */
-  uint32_t count_regions;  /* 1 or 2: plain jobs (k <= 63) with tables of >= 2^22 slots lay
-                              the table out in LDS-sized regions and count by writing
-                              instance records grouped by region, then building each region
-                              on chip; 0: one probe window and atomic counting in HBM.  Read
+  uint32_t count_regions;  /* 1 or 2: tables (k <= 63) of >= 2^22 slots, all jobs of a batch
+                              together, are laid out in LDS-sized regions and count by
+                              writing instance records grouped by region, then building each
+                              region on chip; 0: one probe window and atomic counting in HBM.  Read
                               when a table is allocated and at each count.                   */
   uint32_t region_slots;   /* most slots of a region when a region table is allocated:
                               2560 (80 KB of LDS per build workgroup) or 1280 (40 KB)       */
   uint32_t fuse_list_cap;  /* a count with the filter fused gives each node list room for at
                               most this many nodes (0: every node the table can hold); the
                               nodes beyond it are left to bruno_filter                      */
-  uint32_t count_groups;   /* a region count's second split pass and region builds run in
-                              this many groups of sub-buckets, a group's builds beside the
-                              next group's split (1: one after the other; at most 64);
-                              0: 16 groups from 8 sub-buckets per CU (the largest tables),
-                              else 1                                                         */
+  uint32_t count_groups;   /* a plain job's region count: the split and the region builds
+                              run in this many groups of buckets, a group's builds beside
+                              the next group's split (at most 64); 0 and 1: one after the
+                              other                                                          */
 } bruno_tuning;
 bruno_status bruno_set_tuning(const bruno_tuning* t);
 bruno_status bruno_get_tuning(bruno_tuning* t);
