@@ -1495,13 +1495,28 @@ double ev_ms(bruno_job* j, int a, int b) {
 
 
 /* Tables of at least this many slots (all jobs of a batch together) get the
- * region layout (count_regions 1 or 2).  Measured on jobs of 2^22 to 2^26
- * slots counted alone, the region count and the filter after it save 1.1 to
- * 6.7 ms per job over the atomic count (below 2^22 the layout is not
- * offered); a batch of 16 jobs with 2^28 slots together, 243 M instances,
- * counts in 5.9 ms instead of 18.6. */
-constexpr uint64_t REGION_MIN_CAP = 1ULL << 22;
-constexpr uint64_t REGION_MIN_CAP_ANY = 1ULL << 22;
+ * region layout (count_regions 1 or 2).  A table so small that the count's
+ * dozen launches (180 us, against 40 for the atomic kernel's one) outweigh
+ * the atomics of any call it has room for keeps one probe window. */
+constexpr uint64_t REGION_MIN_CAP = 1ULL << 19;
+/* Below this a plain job's regions get room for the spread of the hash
+ * (region_layout), so that a tight table takes what one probe window takes. */
+constexpr uint64_t REGION_TIGHT_CAP = 1ULL << 22;
+
+/* Fewest instances of a call counted by regions (count_regions 1), in a
+ * table that holds counts already or, below REGION_TIGHT_CAP, in an empty
+ * one; larger empty tables have to be written in any case, and their filter
+ * then reads the build's bits instead of the table.  The region count costs
+ * 0.2 ms and up to 0.1 ms per M instances, and in a written table every slot
+ * read and written; the atomics of reads not seen before 0.25 to 0.45 ms per
+ * M instances.  Measured, us, atomic / regions: k = 31, empty, 2^20 slots,
+ * 0.3 M instances 140 / 302, 1.05 M 372 / 336, 3.1 M 993 / 410; written,
+ * 2^20, 0.63 M 235 / 329; 2^22, 0.42 M 170 / 325, 1.3 M 415 / 450, 2.5 M 783 /
+ * 490; 2^24, 0.5 M 211 / 420, 1.7 M 564 / 483, 5.0 M 1524 / 633; k = 63, 2^22,
+ * 0.42 M 244 / 349, 1.3 M 579 / 441; 2^24, 0.5 M 311 / 604, 1.7 M 795 / 658. */
+uint64_t region_min_instances(uint64_t cap, bool valid) {
+  return valid || cap < REGION_TIGHT_CAP ? (1ULL << 19) + cap / 16 : 0;
+}
 
 /* Region layout of a table of cap slots: at least 2^REC_BUCKET_BITS regions
  * of at most `most` slots.  A batch job's capacity is its caller's number,
@@ -1529,14 +1544,14 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
   const uint32_t cr = tuning().count_regions;
   uint64_t total = 0, n_reg = 0, n_buck = 0, max_span = 0;
   for (uint32_t i = 0; i < nj; ++i) total += caps[i];
-  j->regions = cr && total >= (cr >= 2 ? REGION_MIN_CAP_ANY : REGION_MIN_CAP);
+  j->regions = cr && total >= REGION_MIN_CAP;
   /* the knob counts 32-byte slots: a 64-byte-slot region holds half */
   const uint64_t most = j->words == 1 ? tuning().region_slots : tuning().region_slots / 2;
   j->lay.assign(nj, JobLayout{});
   if (j->regions) {
     for (uint32_t i = 0; i < nj; ++i) {
       JobLayout& l = j->lay[i];
-      region_layout(caps[i], most, nj > 1, &l.rbits, &l.span);
+      region_layout(caps[i], most, nj > 1 || caps[i] < REGION_TIGHT_CAP, &l.rbits, &l.span);
       /* buckets: one per CU, 512 when one split pass would have more than
        * SPLIT_BITS region bits left */
       l.beta = std::min<uint32_t>(l.rbits, l.rbits > 8 + SPLIT_BITS ? MAX_BUCKET_BITS : 8);
@@ -1850,10 +1865,9 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   const uint64_t stage = (REC_STAGE_BYTES / RB) >> beta_min;
   uint32_t clog = 10;
   while (clog > 6 && (1ULL << (clog - 1)) >= stage && (open << clog) * 4 > n_inst) --clog;
-  /* every record's chunk, the partly filled ones, and the numbers struck out
-   * (up to CHUNK_LOW of a batch, a batch at the end) */
-  const uint64_t n_full = (n_inst >> clog) + open;
-  const uint64_t n_chunks = n_full + n_full * CHUNK_LOW / (CHUNK_BATCH - CHUNK_LOW) + (2 * CHUNK_BATCH) * share.size() + 64;
+  /* every record's chunk, the partly filled ones, and at most two per
+   * (workgroup, bucket) taken ahead and not used */
+  const uint64_t n_chunks = (n_inst >> clog) + 3 * open + 1;
   if (n_chunks >= (1ULL << 31)) return BRUNO_OK;
   /* one bucket with more than a 26th of the records (beyond a constant) */
   const uint64_t limit = ((n_inst / 32 + n_inst / 128 + 65536) >> clog) + 2 * share.size() + 1;
@@ -2072,11 +2086,26 @@ void count_atomic(bruno_job* j, ParseArgs a, uint64_t r0, uint64_t r1) {
 
 /* Count one call's reads into a region-layout table, job by job or several
  * jobs of a batch at a time; jobs whose pass could not be counted by regions
- * are counted with atomics. */
+ * are counted with atomics, and so is a call of few instances. */
 template <typename KT>
 bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, const uint64_t* d_first, const uint64_t* h_first) {
   const uint32_t nj = j->n_jobs;
   const int valid = j->table_valid ? 1 : 0;
+  auto atomic = [&](uint32_t ja, uint32_t jb) {
+    if (!valid)
+      fill64(j, (char*)j->table + j->seg[ja] * slot_bytes(j), (j->seg[jb] - j->seg[ja]) * slot_bytes(j) / 8, EMPTY64);
+    if (h_first[jb] > h_first[ja]) count_atomic<KT>(j, a, h_first[ja], h_first[jb]);
+  };
+  auto all_atomic = [&]() {
+    atomic(0, nj);
+    j->table_valid = true;
+    j->by_regions = false;
+    return BRUNO_OK;
+  };
+  const uint64_t least = tuning().count_regions == 1 ? region_min_instances(j->cap, valid) : 0;
+  /* too few reads for it (up to 256 instances each; the instances are not
+   * counted for that: with it a small call would take twice as long) */
+  if (j->cap < REGION_TIGHT_CAP && h_first[nj] * 256 < least) return all_atomic();
   /* instances per job (an upper bound: reads to be dropped included) */
   std::vector<ParseShare> share;
   const uint64_t n_reads = h_first[nj];
@@ -2105,6 +2134,9 @@ bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, const uint64_t* 
     p = d_inst;
     dev_free(j, p, nj * 8);
   }
+  unsigned long long n_inst = 0;
+  for (unsigned long long v : inst) n_inst += v;
+  if (n_inst < least) return all_atomic();
   /* a first count builds every region: it also leaves the filter scan's
    * bits (stale once another count follows) */
   const uint64_t nbits = j->n_regions * j->bit_stride;
@@ -2124,9 +2156,7 @@ bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, const uint64_t* 
     TRY(count_regions_pass<KT>(j, a, d_first, h_first, ja, jb, inst, valid, cbits, sbits, &done));
     if (done) continue;
     all = false;
-    if (!valid)
-      fill64(j, (char*)j->table + j->seg[ja] * slot_bytes(j), (j->seg[jb] - j->seg[ja]) * slot_bytes(j) / 8, EMPTY64);
-    if (h_first[jb] > h_first[ja]) count_atomic<KT>(j, a, h_first[ja], h_first[jb]);
+    atomic(ja, jb);
   }
   j->table_valid = true;
   j->by_regions = all;
@@ -3007,7 +3037,7 @@ bruno_status bruno_batch_create(const bruno_job_desc* d, uint32_t n_jobs, const 
  * region count switched off); for the request server, not exported. */
 __attribute__((visibility("hidden"))) uint64_t br_region_count_min_slots() {
   const uint32_t cr = tuning().count_regions;
-  return cr == 0 ? 0 : cr >= 2 ? REGION_MIN_CAP_ANY : REGION_MIN_CAP;
+  return cr == 0 ? 0 : REGION_MIN_CAP;
 }
 
 bruno_status bruno_job_destroy(bruno_job* j) {

@@ -71,8 +71,8 @@ __device__ __forceinline__ uint32_t count_job_of(uint32_t n_jobs, uint32_t x, F 
 }
 
 /* The chunk pool: chunk c holds records [c << clog, (c + 1) << clog) of one
- * bucket.  Chunk numbers are taken CHUNK_BATCH at a time. */
-constexpr uint32_t CHUNK_BATCH = 128, CHUNK_LOW = 16;
+ * bucket.  A parser workgroup takes numbers ahead, as many as it has
+ * buckets at a time. */
 struct ChunkPool {
   void* recs;                 /* RecOf<KT>::T */
   uint32_t clog;              /* log2 records per chunk */

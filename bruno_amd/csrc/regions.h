@@ -134,7 +134,9 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   __shared__ R park[REC_PARK];
   __shared__ uint16_t park_b[REC_PARK];
   __shared__ uint32_t n_park, blocks_max;
-  __shared__ uint32_t pl_base, pl_used, pl_size; /* chunk numbers in hand */
+  /* chunk numbers in hand, at least one per bucket before an append: pl_n0
+   * from pl_b0, then up to pl_n from pl_b1; pl_used are given out */
+  __shared__ uint32_t pl_b0, pl_n0, pl_b1, pl_n, pl_used;
   static_assert(16 % PF == 0, "flush points split a block evenly");
   const uint32_t tid = threadIdx.x;
   const ParseShare sh = ra.share[blockIdx.x];
@@ -149,7 +151,11 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
     ch_id[b] = NO_CHUNK;
     ch_fill[b] = 0;
   }
-  if (tid == 0) n_park = pl_base = pl_used = pl_size = 0;
+  if (tid == 0) {
+    n_park = pl_b0 = pl_n0 = pl_used = 0;
+    pl_b1 = atomicAdd(ra.pool.next, nb_);
+    pl_n = nb_;
+  }
   __syncthreads();
   R* const recs = (R*)ra.pool.recs;
   auto put = [&](uint32_t b, const R& rec) {
@@ -165,9 +171,6 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
         *ra.pool.overflow = 1;
       }
     }
-  };
-  auto unused = [&](uint32_t c) {
-    if (c < ra.pool.n_max) ra.pool.owner[c] = NO_CHUNK;
   };
   /* append every bucket's whole lines (last: everything) to its open chunk,
    * the rest to a new one: fl_n records, of which fl_n1 go to chunk fl_c1
@@ -185,24 +188,17 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       fl_f1[tid] = fill;
       cnt[tid] = n - m;
       ch_fill[tid] = m2 ? m2 : fill + m1;
-      /* One chunk number per bucket that needs one, from those in hand
-       * (an atomic in HBM here would hold up the whole workgroup at the
-       * next barrier: 2 of 9 ms); a wave that finds too few takes its own,
-       * and strikes out what was left. */
+      /* One chunk number per bucket that needs one, from those in hand (an
+       * atomic in HBM here would hold up the whole workgroup at the next
+       * barrier: 2 of 9 ms). */
       const uint64_t need = __ballot(m2 != 0);
       if (need) {
-        const uint32_t lane = tid & 63, want = (uint32_t)__popcll(need);
-        uint32_t nid = 0;
-        if (lane == 0) {
-          const uint32_t u = atomicAdd(&pl_used, want);
-          nid = pl_base + u;
-          if (u + want > pl_size) {
-            for (uint32_t q = u; q < pl_size; ++q) unused(pl_base + q);
-            nid = atomicAdd(ra.pool.next, want);
-          }
-        }
-        nid = (uint32_t)__builtin_amdgcn_readfirstlane((int)nid) + (uint32_t)__popcll(need & ((1ULL << lane) - 1));
+        const uint32_t lane = tid & 63;
+        uint32_t u = 0;
+        if (lane == 0) u = atomicAdd(&pl_used, (uint32_t)__popcll(need));
+        u = (uint32_t)__builtin_amdgcn_readfirstlane((int)u) + (uint32_t)__popcll(need & ((1ULL << lane) - 1));
         if (m2) {
+          const uint32_t nid = u < pl_n0 ? pl_b0 + u : pl_b1 + (u - pl_n0);
           atomicAdd(&ra.pool.taken[bucket0 + tid], 1u);
           if (nid < ra.pool.n_max) ra.pool.owner[nid] = bucket0 + tid;
           else *ra.pool.overflow = 1;
@@ -211,11 +207,14 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       }
     }
     lds_barrier();
-    /* numbers for the next appends, while the other waves copy */
-    if (tid == REC_BS - 1 && !last && pl_used + CHUNK_LOW > pl_size) {
-      for (uint32_t q = pl_used; q < pl_size; ++q) unused(pl_base + q);
-      pl_base = atomicAdd(ra.pool.next, CHUNK_BATCH);
-      pl_size = CHUNK_BATCH;
+    /* numbers for the next append, while the other waves copy: those left
+     * (fewer than nb_, so all of the later range), then nb_ more */
+    if (tid == REC_BS - 1 && pl_n - pl_used < nb_) {
+      const uint32_t left = pl_n - pl_used;
+      pl_b0 = pl_b1 + (pl_used - pl_n0);
+      pl_n0 = left;
+      pl_b1 = atomicAdd(ra.pool.next, nb_);
+      pl_n = left + nb_;
       pl_used = 0;
     }
     /* LINE lanes per bucket */
@@ -352,8 +351,10 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   }
   unpark();
   flush(true);
-  if (tid == 0)
-    for (uint32_t q = pl_used; q < pl_size; ++q) unused(pl_base + q);
+  for (uint32_t u = pl_used + tid; u < pl_n; u += REC_BS) {
+    const uint32_t nid = u < pl_n0 ? pl_b0 + u : pl_b1 + (u - pl_n0);
+    if (nid < ra.pool.n_max) ra.pool.owner[nid] = NO_CHUNK;
+  }
   /* pad the open chunks */
   for (uint32_t b = tid / 64; b < nb_; b += REC_BS / 64) {
     if (ch_id[b] == NO_CHUNK) continue;

@@ -375,10 +375,11 @@ typedef struct {
                               nodes on average (power of two, 8..4096; small graphs take
                               fewer): the walk length between rulers and the size of the
                               contracted list                                               */
-  uint32_t count_regions;  /* 1 or 2: tables (k <= 63) of >= 2^22 slots, all jobs of a batch
+  uint32_t count_regions;  /* 1 or 2: tables (k <= 63) of >= 2^19 slots, all jobs of a batch
                               together, are laid out in LDS-sized regions and count by
                               writing instance records grouped by region, then building each
-                              region on chip; 0: one probe window and atomic counting in HBM.  Read
+                              region on chip (1: the calls with enough instances for that to
+                              be faster, 2: every call); 0: one probe window and atomic counting in HBM.  Read
                               when a table is allocated and at each count.                   */
   uint32_t region_slots;   /* most slots of a region when a region table is allocated:
                               2560 (80 KB of LDS per build workgroup) or 1280 (40 KB)       */

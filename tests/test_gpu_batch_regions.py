@@ -94,3 +94,23 @@ def test_widest_splits(k, cap):
     job.parse_count(b, off)
     assert {q: c[-1] for q, c in node_table(job.counts()).items()} == {q: 2 * c[-1] for q, c in want.items()}
     job.close()
+
+
+@pytest.mark.parametrize("k", [31, 24, 63])
+@pytest.mark.parametrize("sizes", [(100, 20000, 100), (20000, 100, 20000)])
+def test_calls_of_few_and_many_instances(k, sizes):
+    """count_regions 1 in a table of about 2^19 slots filled to the last one:
+    calls below and above the line between atomics and regions, in either
+    order, give what the oracle gives."""
+    set_tuning(count_regions=1)
+    rng = np.random.default_rng(k)
+    g = "".join(rng.choice(list("ACGT"), 530_000))
+    parts = [[g[i:i + 180] for i in rng.integers(0, len(g) - 180, n)] for n in sizes]
+    b, off = pack([r for p in parts for r in p])
+    want = oracle_node_table(run_oracle(k, None, b, off).unfiltered())
+    job = bruno_amd.GraphJob(k, None, capacity=max(len(want), 1 << 19))
+    for p in parts:
+        job.parse_count(*pack(p))
+        assert job.stats()["count_by_regions"] == (len(p) > 100)
+    assert node_table(job.counts()) == want
+    job.close()

@@ -5,9 +5,19 @@ import numpy as np
 import pytest
 
 import bruno_amd
+from bruno_amd.autotune import get_tuning, set_tuning
 from tests.gpu_common import node_table, oracle_node_table, run_oracle
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def every_call_by_regions():
+    old = get_tuning()
+    set_tuning(count_regions=2)
+    yield
+    set_tuning(**old)
+
 
 M = (1 << 64) - 1
 MUL, ADD = 0xD6E8FEB86659FD93, 0x9E3779B97F4A7C15
