@@ -1658,6 +1658,13 @@ uint64_t capacity_from_estimate(double est, uint64_t n_instances, double load_fa
   return (uint64_t)(d / load_factor) + 4096;
 }
 
+/* Reads from which the sketch takes one per lane: fewer do not fill the
+ * device that way, and a wave per read is over sooner (an estimate, launch
+ * and copies with it, of 2^15 reads of 150 bases: 95 us, a lane per read 111;
+ * of 250 bases 102, 126; of 2^16: a lane per read 122 and 139, the waves
+ * about as long; of 300,000 the kernel alone 137, 67). */
+constexpr uint64_t SKETCH_LANE_READS = 1ULL << 16;
+
 /* sketch of the canonical k-mers of reads (device pointers) */
 template <typename KT>
 bruno_status sketch_t(int K, const char* d_bases, const uint64_t* d_offsets, uint64_t n_reads, uint32_t* regs,
@@ -1672,6 +1679,11 @@ bruno_status sketch_t(int K, const char* d_bases, const uint64_t* d_offsets, uin
   a.n_jobs = 1;
   a.sketch = regs;
   a.ctr = ctr;
+  if (n_reads >= SKETCH_LANE_READS) {
+    const uint64_t g = std::min<uint64_t>((n_reads + SKETCH_BS - 1) / SKETCH_BS, 8 * device_cus());
+    hipLaunchKernelGGL(k_sketch<KT>, dim3((unsigned)g), dim3(SKETCH_BS), 0, st, a);
+    return BRUNO_OK;
+  }
   const uint64_t waves = std::min<uint64_t>(n_reads, tuning().parse_grid);
   const unsigned g = (unsigned)std::max<uint64_t>(1, (waves + 3) / 4);
   hipLaunchKernelGGL((k_parse<KT, 3, 256>), dim3(g), dim3(256), 0, st, a);

@@ -215,7 +215,7 @@ struct ParseArgs {
   uint64_t read0;       /* count mode: reads [read0, n_reads) */
   unsigned long long* job_inst; /* per-job k-mer instances (n_jobs > 1) */
   unsigned long long* job_drop; /* per-job dropped reads (n_jobs > 1) */
-  /* sketch mode: SKETCH_M HyperLogLog registers per job */
+  /* sketch: SKETCH_M HyperLogLog registers */
   uint32_t* sketch;
   /* record mode */
   const uint64_t* rec_base; /* per-read first record index */
@@ -296,6 +296,61 @@ __device__ __forceinline__ void for_each_instance(const uint8_t* s, uint64_t L, 
   }, f);
 }
 
+/* The codes of four bases (a word of their bytes), one per byte: A, C, G, T
+ * of either case 0 to 3, anything else some code. */
+__device__ __forceinline__ uint32_t codes4(uint32_t w) { return ((w >> 1) ^ (w >> 2)) & 0x03030303u; }
+/* nonzero in every byte of w that is not a base: its code does not give its
+ * letter back */
+__device__ __forceinline__ uint32_t not_bases4(uint32_t w) {
+  return __builtin_amdgcn_perm(0u, 0x74676361u /* "acgt" */, codes4(w)) ^ (w | 0x20202020u);
+}
+/* ones in the bytes [0, n) of a word, n clamped to 0 .. 4 */
+__device__ __forceinline__ uint32_t first_bytes(int n) {
+  return n <= 0 ? 0u : n >= 4 ? ~0u : (1u << (8 * n)) - 1;
+}
+/* A read of L bases as one lane walks it, in aligned 16-byte blocks: bases
+ * [16 t - mis, 16 t - mis + 16) of it in block t.  (An aligned block that
+ * holds a byte of the read never crosses a page the read does not touch.) */
+struct LaneRead {
+  const uint4* blk;
+  int mis;
+  uint32_t n_blk; /* blocks that hold a base */
+  __device__ __forceinline__ LaneRead(const uint8_t* s, uint64_t L) {
+    blk = (const uint4*)((uintptr_t)s & ~(uintptr_t)15);
+    mis = (int)((uintptr_t)s & 15);
+    n_blk = L ? (uint32_t)((mis + L + 15) / 16) : 0;
+  }
+  /* Blocks t .. t + 3 (zero past the last): read together, as the waves of
+   * a CU walk more lines at once than its L1 holds, and a line read block by
+   * block would be fetched up to eight times (sketch of 184 M instances 535 ->
+   * 333 us, record parser 957 -> 906). */
+  __device__ __forceinline__ void four(uint32_t t, uint4 (&v)[4]) const {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = t + q < n_blk ? blk[t + q] : make_uint4(0, 0, 0, 0);
+  }
+  /* a byte of the read is no base */
+  __device__ __forceinline__ bool bad(uint64_t L) const {
+    uint32_t any = 0;
+    for (uint32_t t = 0; t < n_blk; t += 4) {
+      uint4 v[4];
+      four(t, v);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const uint32_t w[4] = {not_bases4(v[b].x), not_bases4(v[b].y), not_bases4(v[b].z), not_bases4(v[b].w)};
+        const int64_t j0 = (int64_t)(16ULL * (t + b)) - mis, left = (int64_t)L - j0;
+        if (j0 >= 0 && left >= 16) {
+          any |= w[0] | w[1] | w[2] | w[3];
+        } else {
+          const int lo = j0 < 0 ? (int)-j0 : 0, hi = left < 0 ? 0 : left < 16 ? (int)left : 16;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) any |= w[q] & first_bytes(hi - 4 * q) & ~first_bytes(lo - 4 * q);
+        }
+      }
+    }
+    return any != 0;
+  }
+};
+
 /* lane l's value of a 64-bit register (l wave-uniform) */
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
@@ -303,8 +358,92 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
   return ((uint64_t)hi << 32) | lo;
 }
 
+/* A sampled k-mer's HyperLogLog register and its value there. */
+template <typename KT, typename F>
+__device__ __forceinline__ void sketch_kmer(KT km, F&& f) {
+  const uint64_t h = sketch_hash(km);
+  if ((h >> (64 - SKETCH_SAMPLE_BITS)) != 0) return;
+  const uint32_t idx = (uint32_t)(h >> (64 - SKETCH_SAMPLE_BITS - SKETCH_INDEX_BITS)) & (SKETCH_M - 1);
+  const uint64_t rest = (h << (SKETCH_SAMPLE_BITS + SKETCH_INDEX_BITS)) |
+                        (1ULL << (SKETCH_SAMPLE_BITS + SKETCH_INDEX_BITS - 1));
+  f(idx, (uint32_t)__clzll(rest) + 1);
+}
+
+/* Distinct-k-mer sketch, one read per lane: k-mer and reverse complement
+ * rolled along it as the record parser does, where a wave per read (k_parse)
+ * extracts each instance's from packed words and waits for a register of
+ * the sketch in L2 at most steps; here the registers are the workgroup's
+ * own, in LDS, and merged at the end.  A read longer than SKETCH_LONG, which
+ * the 63 others would wait for, is parsed by the whole wave.  Bound by
+ * instruction issue, two thirds of it the hash's three 64-bit multiplies:
+ * 184 M instances 820 -> 333 us (535 when a lane read one block at a time), 21 M
+ * 137 -> 67. */
+constexpr int SKETCH_BS = 256;
+constexpr uint64_t SKETCH_LONG = 2048;
+template <typename KT>
+__global__ __launch_bounds__(SKETCH_BS) void k_sketch(ParseArgs a) {
+  __shared__ uint32_t reg[SKETCH_M];
+  for (int i = threadIdx.x; i < SKETCH_M; i += SKETCH_BS) reg[i] = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const uint64_t wave = ((uint64_t)blockIdx.x * SKETCH_BS + threadIdx.x) >> 6;
+  const uint64_t nwaves = ((uint64_t)gridDim.x * SKETCH_BS) >> 6;
+  const int K = a.K, sh2 = 2 * (K - 1);
+  const kops<KT> ops(K);
+  const KT kmask = ops.mask;
+  auto put = [&](KT km) { sketch_kmer<KT>(km, [&](uint32_t idx, uint32_t rank) { atomicMax(&reg[idx], rank); }); };
+  for (uint64_t r0 = wave * 64; r0 < a.n_reads; r0 += nwaves * 64) {
+    const uint64_t r = r0 + lane;
+    uint64_t off = 0, L = 0;
+    if (r < a.n_reads) {
+      off = a.starts ? a.starts[r] : a.offsets[r];
+      L = (a.starts ? a.ends[r] : a.offsets[r + 1]) - off;
+    }
+    const uint64_t m_long = __ballot(L > SKETCH_LONG);
+    const int n = L <= SKETCH_LONG && L >= (uint64_t)K + 2 ? (int)L : 0;
+    const LaneRead rd(a.bases + off, n);
+    /* a read with a non-ACGT base is dropped whole */
+    const int Lp = rd.bad(n) ? 0 : n;
+    const uint32_t nb = Lp ? rd.n_blk : 0;
+    KT fw = 0, rv = 0;
+    uint4 v[4];
+    for (uint32_t t = 0; t < nb; ++t) {
+      if (t % 4 == 0) rd.four(t, v);
+      const uint4 cur = v[0];
+      v[0] = v[1];
+      v[1] = v[2];
+      v[2] = v[3];
+      const uint32_t cw[4] = {codes4(cur.x), codes4(cur.y), codes4(cur.z), codes4(cur.w)};
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int j = (int)(16 * t) + q - rd.mis;
+        if (j >= 0 && j < Lp) {
+          const uint32_t c = (cw[q >> 2] >> (8 * (q & 3))) & 3u;
+          fw = ((fw << 2) | (KT)c) & kmask;
+          rv = (rv >> 2) | ((KT)(3u - c) << sh2);
+          if (j >= K - 1) put(fw < rv ? fw : rv);
+        }
+      }
+    }
+    for (uint64_t m = m_long; m; m &= m - 1) {
+      const int l = __ffsll((unsigned long long)m) - 1;
+      const uint8_t* s = a.bases + readlane64(off, l);
+      const uint64_t len = readlane64(L, l);
+      int bad = 0;
+      for (uint64_t i = lane; i < len; i += 64) bad |= (base_code(s[i]) < 0);
+      if (__any(bad) || len < (uint64_t)K + 2) continue;
+      for_each_instance<KT>(s, len, K, lane, ops, [&](uint64_t, KT km, uint8_t) { put(km); });
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < SKETCH_M; i += SKETCH_BS) {
+    const uint32_t v = reg[i];
+    if (v && v > __hip_atomic_load(a.sketch + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a.sketch + i, v);
+  }
+}
+
 /* MODE 0: count records per read; MODE 1: write records; MODE 2: count into
- * the table; MODE 3: distinct-k-mer sketch only.  BS is the workgroup size
+ * the table; MODE 3: distinct-k-mer sketch of a few reads (see k_sketch).  BS is the workgroup size
  * (the work is per wave, so any multiple of 64 works; it is a tuning knob). */
 template <typename KT, int MODE, int BS = BLOCK>
 __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
@@ -322,7 +461,7 @@ __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
   uint32_t rbits = a.rbits;
   unsigned long long j_inst = 0;
   for (uint64_t r = a.read0 + wave; r < a.n_reads; r += nwaves) {
-    if ((MODE == 2 || MODE == 3) && a.n_jobs > 1 && !(r >= j_lo && r < j_hi)) {
+    if (MODE == 2 && a.n_jobs > 1 && !(r >= j_lo && r < j_hi)) {
       if (lane == 0 && j_inst) atomicAdd(&a.job_inst[cj], j_inst);
       j_inst = 0;
       cj = job_of(a.job_first, a.n_jobs, r);
@@ -359,15 +498,10 @@ __global__ __launch_bounds__(BS) void k_parse(ParseArgs a) {
     if (MODE == 2 && a.n_jobs > 1) j_inst += nk;
     for_each_instance<KT>(s, L, K, lane, ops, [&](uint64_t i, KT km, uint8_t e) {
       if (MODE == 3) {
-        const uint64_t h = sketch_hash(km);
-        if ((h >> (64 - SKETCH_SAMPLE_BITS)) == 0) {
-          const uint32_t idx = (uint32_t)(h >> (64 - SKETCH_SAMPLE_BITS - SKETCH_INDEX_BITS)) & (SKETCH_M - 1);
-          const uint64_t rest = (h << (SKETCH_SAMPLE_BITS + SKETCH_INDEX_BITS)) |
-                                (1ULL << (SKETCH_SAMPLE_BITS + SKETCH_INDEX_BITS - 1));
-          const uint32_t rank = (uint32_t)__clzll(rest) + 1;
-          uint32_t* reg = a.sketch + (uint64_t)cj * SKETCH_M + idx;
+        sketch_kmer<KT>(km, [&](uint32_t idx, uint32_t rank) {
+          uint32_t* reg = a.sketch + idx;
           if (rank > __hip_atomic_load(reg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(reg, rank);
-        }
+        });
       } else if (MODE == 1) {
         a.out_kmers[(rbase + i) * kt_traits<KT>::words] = (uint64_t)km;
         if (kt_traits<KT>::words == 2)

@@ -101,8 +101,7 @@ template <> __device__ __forceinline__ ulonglong2 rec_filler<ulonglong2>() { ret
  * record, not a window extraction and a reverse complement.  The lanes
  * step through their reads in aligned 16-byte blocks, all lanes of the
  * workgroup at the same block index (bases before a read's start or past
- * its end are masked off), loading the next block while the current one
- * is parsed.  A read with a non-ACGT base is dropped whole
+ * its end are masked off).  A read with a non-ACGT base is dropped whole
  * (NFilterSequencesIterator, compact_dbg_freq_construct_clean.cpp:210-213),
  * found by a first pass over its blocks.
  *
@@ -115,10 +114,11 @@ template <> __device__ __forceinline__ ulonglong2 rec_filler<ulonglong2>() { ret
  * atomics), which takes one bucket getting a fifteenth of all records.
  *
  * One 1,024-thread workgroup per CU with 256 buckets (512 for the largest
- * tables).  Bound by instruction issue; the appends to 256 buckets cost
- * 5-15% over 32 (1.6 G instances 7.4 -> 7.8 ms, 184 M 0.84 -> 0.96, 301 M of
- * k = 63 2.48 -> 2.59; 21 M, where a workgroup has two rounds of 600 reads,
- * 0.15 -> 0.21), and the split after it needs one pass instead of two: the
+ * tables).  Bound by instruction issue.  The appends to 256 buckets cost
+ * 5-15% over 32 and the split after it needs one pass instead of two; the
+ * bases tested and coded four at a time and read four blocks at a time give
+ * it back (1.6 G instances 7.4 ms with 32 buckets, 7.8 with 256, now 7.2; 184
+ * M 0.84, 0.96, 0.91; 301 M of k = 63 2.48, 2.59, 2.42).  With the split the
  * count phase as a whole 35.9 -> 30.1, 4.5 -> 3.8, 13.2 -> 10.7 and 1.39 ->
  * 0.81 ms.  A batch of 16 jobs of 0.05 to 2 Mbp (243 M instances), which HBM
  * atomics counted in 18.6 ms, takes 5.9. */
@@ -269,22 +269,9 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       lo = a.starts ? a.starts[r] : a.offsets[r];
       L = (a.starts ? a.ends[r] : a.offsets[r + 1]) - lo;
     }
-    const uint8_t* s = a.bases + lo;
-    const uint4* blk = (const uint4*)((uintptr_t)s & ~(uintptr_t)15);
-    const int64_t mis = (int64_t)((uintptr_t)s & 15);
-    /* the blocks holding the read; an aligned block that holds a byte of
-     * the read never crosses a page the read does not touch */
-    const uint64_t nblk = L ? (uint64_t)(mis + (int64_t)L + 15) / 16 : 0;
-    bool bad = false;
-    for (uint64_t t = 0; t < nblk; ++t) {
-      const uint4 v = blk[t];
-      const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int64_t j = (int64_t)(16 * t) + q - mis;
-        if (j >= 0 && j < (int64_t)L) bad |= base_code((uint8_t)(wv[q >> 2] >> (8 * (q & 3)))) < 0;
-      }
-    }
+    const LaneRead rd(a.bases + lo, L);
+    const int64_t mis = rd.mis;
+    const bool bad = rd.bad(L);
     if (bad) ++my_drop;
     /* reads shorter than the parser window k + 2 give nothing
      * (debruijn_biedge_loader.hpp:464-465) */
@@ -308,16 +295,19 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
      * PF-th position, or once a block when a bucket's share of the block's
      * records leaves a quarter of its stage to chance and what stays behind */
     const bool often = (ra1 - ra0) * 16 > (uint64_t)(STAGE - STAGE / 4 - nb_ * (LINE / 2));
-    uint4 cur = nb ? blk[0] : make_uint4(0, 0, 0, 0);
+    uint4 v[4] = {};
     for (uint32_t t = 0; t < nbw; ++t) {
-      const uint4 nxt = (t + 1 < nb && t + 1 < nblk) ? blk[t + 1] : make_uint4(0, 0, 0, 0);
-      const uint32_t wv[4] = {cur.x, cur.y, cur.z, cur.w};
+      if (t % 4 == 0) rd.four(t, v);
+      const uint4 cur = v[0];
+      v[0] = v[1];
+      v[1] = v[2];
+      v[2] = v[3];
+      const uint32_t cw[4] = {codes4(cur.x), codes4(cur.y), codes4(cur.z), codes4(cur.w)};
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         const int64_t j = (int64_t)(16 * t) + q - mis;
         if (j >= 0 && j <= (int64_t)Lp) {
-          const uint32_t x = ((wv[q >> 2] >> (8 * (q & 3))) & 0xFFu) | 0x20u;
-          const uint32_t c = ((x >> 1) ^ (x >> 2)) & 3u; /* A/C/G/T, either case */
+          const uint32_t c = (cw[q >> 2] >> (8 * (q & 3))) & 3u;
           const bool in_read = j < (int64_t)Lp;
           if (j >= K) {
             const bool flip = !(fw < rv);
@@ -346,7 +336,6 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
           if (n_park > REC_PARK / 2) unpark();
         }
       }
-      cur = nxt;
     }
   }
   unpark();
