@@ -1085,62 +1085,102 @@ __global__ void k_branch_nodes(const Slot<KT>* T, uint64_t tbase, uint64_t tcap,
   out[i] = nd;
 }
 
+/* Self counts of a unitig's chain nodes: sum, largest, and 65535 less the
+ * smallest (so zero is where all three begin). */
+struct ChainSum {
+  unsigned long long sum;
+  uint32_t mx, mn;
+};
+
 /* .chain.edges (compute_freq_map, compact_dbg_stats.hpp:783-816, and
- * print_chain_frequencies, :879-1065), one wave per unitig: the unitig's
- * sorted chain nodes [starts[u], starts[u+1]) run from its rep L (dist 0)
- * to its last k-mer R on the rep strand.  The lanes look up the self counts
- * of the nodes in the table and reduce their sum, min and max; lane 0 reads
- * L's in-edge and R's out-edge counts, complemented in reverse order when
- * the k-mer is the reverse strand of its canonical form. */
+ * print_chain_frequencies, :879-1065), first the self counts: a wave looks up
+ * 64 consecutive nodes of the unitigs' sorted chain nodes (unitig u's are
+ * [starts[u], starts[u + 1])), whichever unitigs they belong to, sums them
+ * by unitig in the wave and adds one ChainSum per unitig it met.  Bound by
+ * the lookups' latency: with one wave per unitig the longest one's nodes
+ * were a chain of them (1 M nodes, 1.93 ms, now 0.11). */
+template <typename KT>
+__global__ __launch_bounds__(BLOCK) void k_chain_sums(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, uint32_t rbits,
+                                                      int K, OutView<KT> v, uint64_t c0, const uint32_t* starts,
+                                                      uint64_t n_unitigs, ChainSum* out, Counters* ctr) {
+  kops<KT> ops(K);
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t wave = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
+  const uint64_t n_waves = ((uint64_t)gridDim.x * BLOCK) >> 6;
+  const uint32_t first = starts[0], end = starts[n_unitigs];
+  for (uint64_t p0 = first + wave * 64; p0 < end; p0 += n_waves * 64) {
+    const uint64_t u0 = wave_find(starts, (uint32_t)n_unitigs, (uint32_t)p0); /* node p0's unitig */
+    /* this lane's unitig: the starts after u0's at or before its node */
+    const uint64_t p = p0 + lane;
+    const uint32_t s = u0 + 1 + lane < n_unitigs ? starts[u0 + 1 + lane] : ~0u;
+    uint32_t k = 0;
+#pragma unroll
+    for (uint32_t step = 32; step; step >>= 1)
+      if ((uint32_t)__shfl(s, (int)(k + step - 1)) <= p) k += step;
+    const bool in = p < end;
+    uint32_t sum = 0, mx = 0, mn = 0;
+    bool missing = false;
+    if (in) {
+      const NodeRec* r = node_rec<KT>(T, tbase, tcap, rbits, ops.canon(v.kmer(c0 + p)));
+      missing = r == nullptr;
+      sum = r ? r->c[8] : 0;
+      mx = sum;
+      mn = 65535 - sum;
+    }
+    /* over the lanes of the same unitig up to this one */
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t ks = __shfl_up(k, off), a = __shfl_up(sum, off), x = __shfl_up(mx, off), y = __shfl_up(mn, off);
+      if ((int)lane >= off && ks == k) {
+        sum += a;
+        mx = x > mx ? x : mx;
+        mn = y > mn ? y : mn;
+      }
+    }
+    const uint32_t kn = __shfl_down(k, 1);
+    if (in && (lane == 63 || kn != k || p + 1 == end)) {
+      ChainSum* o = out + u0 + k;
+      atomicAdd(&o->sum, (unsigned long long)sum);
+      atomicMax(&o->mx, mx);
+      atomicMax(&o->mn, mn);
+    }
+    if (missing) atomicOr(&ctr->err, ERR_NO_NODE);
+  }
+}
+
+/* ... then a unitig's record per thread: its nodes run from its rep L (dist
+ * 0) to its last k-mer R on the rep strand; L's in-edge and R's out-edge
+ * counts are complemented in reverse order when the k-mer is the reverse
+ * strand of its canonical form. */
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_chain_edges(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, uint32_t rbits,
                                                        int K, OutView<KT> v, uint64_t c0, const uint32_t* starts,
-                                                       uint64_t n_unitigs, bruno_chain_edge* out, Counters* ctr) {
+                                                       uint64_t n_unitigs, const ChainSum* sums, bruno_chain_edge* out,
+                                                       Counters* ctr) {
   kops<KT> ops(K);
-  const int lane = threadIdx.x & 63;
-  const uint64_t wave = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
-  const uint64_t n_waves = ((uint64_t)gridDim.x * BLOCK) >> 6;
-  for (uint64_t u = wave; u < n_unitigs; u += n_waves) {
-    const uint32_t b = starts[u], e = starts[u + 1];
-    uint64_t sum = 0;
-    uint32_t mn = 65535, mx = 0, missing = 0;
-    for (uint32_t p = b + lane; p < e; p += 64) {
-      const NodeRec* r = node_rec<KT>(T, tbase, tcap, rbits, ops.canon(v.kmer(c0 + p)));
-      const uint32_t c = r ? r->c[8] : 0;
-      missing |= r == nullptr;
-      sum += c;
-      mn = c < mn ? c : mn;
-      mx = c > mx ? c : mx;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      sum += __shfl_xor(sum, off);
-      const uint32_t a = __shfl_xor(mn, off), z = __shfl_xor(mx, off);
-      mn = a < mn ? a : mn;
-      mx = z > mx ? z : mx;
-      missing |= __shfl_xor(missing, off);
-    }
-    if (lane == 0) {
-      const KT L = v.kmer(c0 + b), R = v.kmer(c0 + e - 1);
-      const KT cL = ops.canon(L), cR = ops.canon(R);
-      const NodeRec* rl = node_rec<KT>(T, tbase, tcap, rbits, cL);
-      const NodeRec* rr = node_rec<KT>(T, tbase, tcap, rbits, cR);
-      bruno_chain_edge o;
-      o.left[0] = (uint64_t)L;
-      o.left[1] = (uint64_t)((u128)L >> 64);
-      o.right[0] = (uint64_t)R;
-      o.right[1] = (uint64_t)((u128)R >> 64);
-      o.sum = sum;
-      o.n_nodes = e - b;
-      for (int c = 0; c < 4; ++c) {
-        o.in[c] = rl ? (cL == L ? rl->c[4 + c] : rl->c[3 - c]) : 0;
-        o.out[c] = rr ? (cR == R ? rr->c[c] : rr->c[7 - c]) : 0;
-      }
-      o.min = (uint16_t)mn;
-      o.max = (uint16_t)mx;
-      if (missing || !rl || !rr) atomicOr(&ctr->err, ERR_NO_NODE);
-      out[u] = o;
-    }
+  const uint64_t u = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+  if (u >= n_unitigs) return;
+  const uint32_t b = starts[u], e = starts[u + 1];
+  const KT L = v.kmer(c0 + b), R = v.kmer(c0 + e - 1);
+  const KT cL = ops.canon(L), cR = ops.canon(R);
+  const NodeRec* rl = node_rec<KT>(T, tbase, tcap, rbits, cL);
+  const NodeRec* rr = node_rec<KT>(T, tbase, tcap, rbits, cR);
+  const ChainSum cs = sums[u];
+  bruno_chain_edge o;
+  o.left[0] = (uint64_t)L;
+  o.left[1] = (uint64_t)((u128)L >> 64);
+  o.right[0] = (uint64_t)R;
+  o.right[1] = (uint64_t)((u128)R >> 64);
+  o.sum = cs.sum;
+  o.n_nodes = e - b;
+  for (int c = 0; c < 4; ++c) {
+    o.in[c] = rl ? (cL == L ? rl->c[4 + c] : rl->c[3 - c]) : 0;
+    o.out[c] = rr ? (cR == R ? rr->c[c] : rr->c[7 - c]) : 0;
   }
+  o.min = (uint16_t)(65535 - cs.mn);
+  o.max = (uint16_t)cs.mx;
+  if (!rl || !rr) atomicOr(&ctr->err, ERR_NO_NODE);
+  out[u] = o;
 }
 
 /* 1 where a sorted chain node starts a unitig (dist 0) */
@@ -4045,13 +4085,18 @@ static bruno_status chain_edges_t(bruno_job* j, uint32_t idx, uint64_t c0, uint6
   const uint32_t* st0 = nullptr;
   uint64_t off = 0;
   bruno_status st = unitig_starts(j, idx, c0, m, nu, &starts, &st0, &off);
+  ChainSum* sums = nullptr;
   if (st == BRUNO_OK) st = dev_alloc(j, (void**)&d, nu * sizeof(bruno_chain_edge));
+  if (st == BRUNO_OK) st = dev_alloc(j, (void**)&sums, nu * sizeof(ChainSum));
   if (st == BRUNO_OK) {
     uint64_t tbase, tcap;
     uint32_t rbits;
     job_segment(j, idx, tbase, tcap, rbits);
-    hipLaunchKernelGGL((k_chain_edges<KT>), dim3(grid_for(nu * 64, BLOCK, 1u << 16)), dim3(BLOCK), 0, j->stream,
-                       (const Slot<KT>*)j->table, tbase, tcap, rbits, j->K, out_view<KT>(j), off, st0, nu, d, j->ctr);
+    fill64(j, sums, nu * sizeof(ChainSum) / 8, 0);
+    hipLaunchKernelGGL((k_chain_sums<KT>), dim3(grid_for(m, BLOCK, 1u << 16)), dim3(BLOCK), 0, j->stream,
+                       (const Slot<KT>*)j->table, tbase, tcap, rbits, j->K, out_view<KT>(j), off, st0, nu, sums, j->ctr);
+    hipLaunchKernelGGL((k_chain_edges<KT>), dim3(grid_for(nu, BLOCK, 1u << 30)), dim3(BLOCK), 0, j->stream,
+                       (const Slot<KT>*)j->table, tbase, tcap, rbits, j->K, out_view<KT>(j), off, st0, nu, sums, d, j->ctr);
     st = sync_counters(j);
     if (st == BRUNO_OK && copy_out(j, buf, d, nu * sizeof(bruno_chain_edge)) != hipSuccess) st = BRUNO_INTERNAL;
   }
@@ -4059,6 +4104,8 @@ static bruno_status chain_edges_t(bruno_job* j, uint32_t idx, uint64_t c0, uint6
   dev_free(j, a, (m + 1) * 4);
   a = d;
   dev_free(j, a, nu * sizeof(bruno_chain_edge));
+  a = sums;
+  dev_free(j, a, nu * sizeof(ChainSum));
   return st;
 }
 
