@@ -202,6 +202,21 @@ def status_string(code):
         return "status %d" % code
 
 
+_new_bytes = ctypes.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype = ctypes.py_object
+_new_bytes.argtypes = (ctypes.c_char_p, ctypes.c_ssize_t)
+
+
+def text(n, fill):
+    """n bytes, written in place by fill(buffer): a ctypes buffer would be
+    zeroed first and copied afterwards (13 MB: 5.6 ms against 0.7)."""
+    if n == 0:
+        return b""
+    out = _new_bytes(None, n)
+    fill(ctypes.c_char_p(out))
+    return out
+
+
 def check(code, what):
     if code != OK:
         raise BrunoError(code, what)

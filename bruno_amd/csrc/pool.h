@@ -22,17 +22,80 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 #include <vector>
 
 namespace br {
 
+/* Pinned chunks for one device-to-host copy at a time, with an event each. */
+struct PinnedRing {
+  static constexpr int CHUNKS = 16;
+  static constexpr uint64_t CHUNK = 512 << 10;
+  char* mem = nullptr;
+  hipEvent_t ev[CHUNKS] = {};
+
+  bool make() {
+    if (hipHostMalloc((void**)&mem, CHUNKS * CHUNK, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      mem = nullptr;
+      return false;
+    }
+    for (hipEvent_t& e : ev)
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        e = nullptr;
+        return false;
+      }
+    return true;
+  }
+  void drop() {
+    for (hipEvent_t& e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (mem) (void)hipHostFree(mem);
+  }
+};
+
 class DevicePool {
  public:
+  /* A ring for the caller alone until it is given back (null: no pinned
+   * memory to be had).  Up to KEEP_RINGS that nobody holds are kept, until
+   * trim. */
+  static constexpr size_t KEEP_RINGS = 4;
+  PinnedRing* take_ring() {
+    {
+      std::lock_guard<std::mutex> g(mu_);
+      if (!rings_.empty()) {
+        PinnedRing* r = rings_.back();
+        rings_.pop_back();
+        return r;
+      }
+    }
+    PinnedRing* r = new (std::nothrow) PinnedRing;
+    if (r && !r->make()) {
+      r->drop();
+      delete r;
+      r = nullptr;
+    }
+    return r;
+  }
+  void give_ring(PinnedRing* r) {
+    {
+      std::lock_guard<std::mutex> g(mu_);
+      if (rings_.size() < KEEP_RINGS) {
+        rings_.push_back(r);
+        return;
+      }
+    }
+    r->drop();
+    delete r;
+  }
+
   static constexpr uint64_t ALIGN = 256;
   static constexpr uint64_t GROW_MIN = 1ULL << 30;  /* chunk for small requests */
   static constexpr uint64_t CHUNK_ROUND = 2ULL << 20;
 
+  DevicePool() { rings_.reserve(KEEP_RINGS); }
   static DevicePool& current() {
     static DevicePool pools[64];
     int dev = 0;
@@ -105,6 +168,11 @@ class DevicePool {
   void trim() {
     std::lock_guard<std::mutex> g(mu_);
     trim_locked();
+    for (PinnedRing* r : rings_) {
+      r->drop();
+      delete r;
+    }
+    rings_.clear();
   }
 
   void stats(uint64_t* reserved, uint64_t* in_use, uint64_t* largest_free) {
@@ -175,6 +243,7 @@ class DevicePool {
   std::map<int, Chunk> chunks_;
   std::map<char*, Blk> free_;
   std::unordered_map<char*, Blk> used_;
+  std::vector<PinnedRing*> rings_;
   int next_chunk_ = 0;
   uint64_t reserved_ = 0, in_use_ = 0;
 };

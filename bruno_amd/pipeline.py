@@ -38,9 +38,7 @@ class _Views:
         n = ctypes.c_uint64(0)
         self._call(name, None, ctypes.byref(n))
         if text:
-            buf = ctypes.create_string_buffer(max(1, n.value))
-            self._call(name, buf, ctypes.byref(n))
-            return buf.raw[:n.value]
+            return _lib.text(n.value, lambda buf: self._call(name, buf, ctypes.byref(n)))
         out = np.zeros(n.value, dtype)
         if n.value:
             self._call(name, _ptr(out), ctypes.byref(n))

@@ -14,7 +14,7 @@ import ctypes
 import numpy as np
 
 from . import _lib
-from ._lib import check, lib
+from ._lib import check, lib, text
 from .pipeline import DEFAULT_THRESH
 
 
@@ -88,9 +88,7 @@ class Server:
     def _text(self, fn, ticket):
         n = ctypes.c_uint64()
         check(fn(self.h, int(ticket), None, ctypes.byref(n)), fn.__name__)
-        buf = ctypes.create_string_buffer(max(1, n.value))
-        check(fn(self.h, int(ticket), buf, ctypes.byref(n)), fn.__name__)
-        return buf.raw[:n.value]
+        return text(n.value, lambda buf: check(fn(self.h, int(ticket), buf, ctypes.byref(n)), fn.__name__))
 
     def unitigs(self, ticket):
         return self._text(lib().bruno_server_get_unitigs, ticket)
