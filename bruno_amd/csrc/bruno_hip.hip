@@ -2053,9 +2053,10 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
       else hipLaunchKernelGGL((k_region_build<u128, REGION_WIDE_SLOTS, 512, F>), b, dim3(512), 0, st, g);
     }
     /* this launch's waves' side-table queues */
+    const uint32_t nq = b.x * (small_build ? 4 : 8);
     if (spq_cap)
-      hipLaunchKernelGGL(k_spill_flush, dim3(b.x * (small_build ? 4 : 8)), dim3(BLOCK), 0, st, spq, spq_n, spq_cap, overflow,
-                         j->spill, j->spcap, j->ctr);
+      hipLaunchKernelGGL(k_spill_flush, dim3((unsigned)std::min<uint64_t>((nq + BLOCK / 64 - 1) / (BLOCK / 64), 4 * cus)),
+                         dim3(BLOCK), 0, st, spq, spq_n, nq, spq_cap, overflow, j->spill, j->spcap, j->ctr);
   };
   /* Split and builds one after the other, or (count_groups) in groups of a
    * plain job's buckets, a group's builds on a second stream beside the
