@@ -31,6 +31,29 @@ struct ChainSummary {
   uint16_t f5, f6;
 };
 
+/* Chain summaries by (5' branch, 3' branch, length, 5' end, 3' end). */
+template <typename KT>
+struct SummaryKey {
+  KT b5, b3;
+  uint32_t len;
+  KT t5, t3;
+  __device__ __forceinline__ bool operator<(const SummaryKey& o) const {
+    if (b5 != o.b5) return b5 < o.b5;
+    if (b3 != o.b3) return b3 < o.b3;
+    if (len != o.len) return len < o.len;
+    if (t5 != o.t5) return t5 < o.t5;
+    return t3 < o.t3;
+  }
+};
+template <typename KT>
+struct SummaryKeys {
+  typedef SummaryKey<KT> Item;
+  const ChainSummary<KT>* S;
+  __device__ __forceinline__ Item operator()(uint32_t i) const {
+    return Item{S[i].b5, S[i].b3, S[i].len, S[i].t5, S[i].t3};
+  }
+};
+
 /* An edge to erase: oriented k-mer, side (1 = out, 0 = in) and base. */
 template <typename KT>
 struct EdgeQuery {
