@@ -3537,12 +3537,14 @@ static bruno_status drop_separated_t(bruno_job* j) {
                      j->rbits, j->K, j->chain_slot, j->alive, nc, mark);
   hipLaunchKernelGGL((k_drop_separated_edges<KT>), dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream,
                      (Slot<KT>*)j->table, tcap, j->rbits, j->K, j->chain_slot, mark, nc);
+  hipLaunchKernelGGL((k_drop_beside_separated<KT>), dim3(grid_for(nc)), dim3(BLOCK), 0, j->stream,
+                     (Slot<KT>*)j->table, tcap, j->rbits, j->K, j->chain_slot, mark, nc);
   void* a = mark;
   dev_free(j, a, nc);
   return BRUNO_OK;
 }
 
-/* erase_if(IsIsolated) over both node lists */
+/* erase_if(IsIsolated) over both node lists; once, see k_drop_at_erased */
 template <typename KT>
 static bruno_status drop_edgeless_t(bruno_job* j) {
   if (j->n_chain)
@@ -3649,7 +3651,8 @@ static bruno_status pick_t(bruno_job* j, uint64_t min_freq, EdgeQuery<KT>** dq, 
   return BRUNO_OK;
 }
 
-/* the queried edges below min_freq, erased on both nodes */
+/* the queried edges below min_freq, erased on both nodes, and the nodes that
+ * have no other */
 template <typename KT>
 static bruno_status erase_t(bruno_job* j, const EdgeQuery<KT>* q, uint64_t n, uint64_t min_freq, uint64_t* erased) {
   *erased = 0;
@@ -3664,6 +3667,8 @@ static bruno_status erase_t(bruno_job* j, const EdgeQuery<KT>* q, uint64_t n, ui
                      j->rbits, j->K, q, n, min_freq, hit);
   hipLaunchKernelGGL((k_erase_edges<KT>), dim3(grid_for(n)), dim3(BLOCK), 0, j->stream, (Slot<KT>*)j->table, tcap,
                      j->rbits, j->K, q, n, hit, cnt);
+  hipLaunchKernelGGL((k_drop_at_erased<KT>), dim3(grid_for(n)), dim3(BLOCK), 0, j->stream, (Slot<KT>*)j->table, tcap,
+                     j->rbits, j->K, q, n, hit);
   unsigned long long h = 0;
   HIP_CHECK(hipMemcpyAsync(&h, cnt, sizeof(h), hipMemcpyDeviceToHost, j->stream));
   HIP_CHECK(hipStreamSynchronize(j->stream));
@@ -3686,9 +3691,7 @@ static bruno_status clean_t(bruno_job* j, int variant, uint64_t k1_lo, bruno_cle
     uint64_t ndq = 0, nbq = 0, e1 = 0, e2 = 0, dqb = 0, bqb = 0;
     bruno_status s = pick_t<KT>(j, min_freq, &dq, &ndq, &bq, &nbq, &dqb, &bqb);
     if (s == BRUNO_OK) s = erase_t<KT>(j, dq, ndq, min_freq, &e1);
-    if (s == BRUNO_OK) s = drop_edgeless_t<KT>(j);
     if (s == BRUNO_OK) s = erase_t<KT>(j, bq, nbq, min_freq, &e2);
-    if (s == BRUNO_OK) s = drop_edgeless_t<KT>(j);
     void* a = dq;
     dev_free(j, a, dqb);
     a = bq;
@@ -3702,7 +3705,6 @@ static bruno_status clean_t(bruno_job* j, int variant, uint64_t k1_lo, bruno_cle
     if (e1 + e2 == 0) break;
     TRY(recompact_t<KT>(j, variant));
     TRY(drop_separated_t<KT>(j));
-    TRY(drop_edgeless_t<KT>(j));
     ++st->rounds;
   }
   /* the outputs of the cleaned graph (its branch points and unitigs) */

@@ -293,6 +293,51 @@ __global__ void k_drop_separated_edges(Slot<KT>* T, uint64_t tcap, uint32_t rbit
   }
 }
 
+/* erase_if(IsIsolated) after edges were erased, at the nodes that lost one
+ * only: with every edgeless node gone before, no other can have become
+ * edgeless (a pass over 2.4 M nodes of the lists took 66 us, nine times in a
+ * cleaning of three rounds). */
+template <typename KT>
+__device__ __forceinline__ void drop_if_edgeless(Slot<KT>* T, uint64_t tcap, uint32_t rbits, const kops<KT>& ops, KT u) {
+  const uint64_t s = SlotOps<KT>::find(T, tcap, rbits, ops.canon(u), true);
+  if (s == ~0ULL) return;
+  Slot<KT>* p = T + s;
+  const NodeRec* r = (const NodeRec*)&p->sub[0];
+  bool any = false;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) any |= r->c[q] > 0;
+  uint64_t* fw = SlotOps<KT>::flag_word(p);
+  if (!any) *fw = *fw & ~F_PRESENT; /* the same word whoever writes it */
+}
+/* ... of the edges k_erase_edges erased */
+template <typename KT>
+__global__ void k_drop_at_erased(Slot<KT>* T, uint64_t tcap, uint32_t rbits, int K, const EdgeQuery<KT>* Q, uint64_t n,
+                                 const uint8_t* hit) {
+  kops<KT> ops(K);
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    if (!hit[i]) continue;
+    const EdgeQuery<KT> e = Q[i];
+    drop_if_edgeless<KT>(T, tcap, rbits, ops, e.x);
+    drop_if_edgeless<KT>(T, tcap, rbits, ops, e.out ? ops.out_nbr(e.x, (int)e.c) : ops.in_nbr(e.x, (int)e.c));
+  }
+}
+/* ... of the edges k_drop_separated_edges took */
+template <typename KT>
+__global__ void k_drop_beside_separated(Slot<KT>* T, uint64_t tcap, uint32_t rbits, int K, const uint64_t* chain_slot,
+                                        const uint8_t* mark, uint64_t nc) {
+  kops<KT> ops(K);
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += (uint64_t)gridDim.x * blockDim.x) {
+    if (!mark[i]) continue;
+    const Slot<KT>* p = T + chain_slot[i];
+    const KT x = SlotOps<KT>::kmer(p);
+    const NodeRec* r = (const NodeRec*)&p->sub[0];
+    for (int c = 0; c < 4; ++c) {
+      if (r->c[c] > 0) drop_if_edgeless<KT>(T, tcap, rbits, ops, ops.out_nbr(x, c));
+      if (r->c[4 + c] > 0) drop_if_edgeless<KT>(T, tcap, rbits, ops, ops.in_nbr(x, c));
+    }
+  }
+}
+
 /* The node lists again after edges changed: every node still in the graph
  * is classified from its counters (IsBranchPoint / IsChainNode) and
  * appended to the chain or the branch list (one thread per old list entry,
