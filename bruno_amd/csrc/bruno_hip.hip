@@ -3765,54 +3765,74 @@ bruno_status bruno_get_phase_ms(bruno_job* j, bruno_phase_ms* o) {
 }
 
 /* ---- per-job views ------------------------------------------------- */
-/* One device-to-host copy through a pinned ring: chunk c goes through slot c
- * mod CHUNKS, and whoever has copied it on to the caller's memory sends the
- * slot's next chunk off.  run() is called by one thread or by several. */
+/* One device-to-host copy through a pinned ring, piece by piece: the piece
+ * in slot c mod CHUNKS is copied on to the caller's memory, a share by each
+ * thread, while the next one comes in. */
 struct RingCopy {
   PinnedRing* r;
   hipStream_t st;
-  int dev;
   char* dst;
   const char* src; /* aligned; the caller's first byte is `skip` further on */
   uint64_t skip, total, n;
-  std::atomic<uint64_t> next{0};
-  std::atomic<uint64_t> sent[PinnedRing::CHUNKS]; /* chunks sent through the slot */
-  std::atomic<int> err{0};
+  unsigned threads = 1;
+  std::atomic<uint64_t> ready{0}; /* pieces that are in, or given up */
+  std::atomic<uint64_t> copied{0}; /* shares of pieces copied on */
+  std::atomic<bool> bad{false};
 
-  void send(uint64_t c) {
+  bool send(uint64_t c) {
     const int s = (int)(c % PinnedRing::CHUNKS);
     const uint64_t o = c * PinnedRing::CHUNK;
-    if (!err.load() &&
-        (hipMemcpyAsync(r->mem + s * PinnedRing::CHUNK, src + o, std::min(PinnedRing::CHUNK, total - o),
-                        hipMemcpyDeviceToHost, st) != hipSuccess ||
-         hipEventRecord(r->ev[s], st) != hipSuccess))
-      err = 1;
-    sent[s].fetch_add(1, std::memory_order_release);
+    return hipMemcpyAsync(r->mem + s * PinnedRing::CHUNK, src + o, std::min(PinnedRing::CHUNK, total - o),
+                          hipMemcpyDeviceToHost, st) == hipSuccess &&
+           hipEventRecord(r->ev[s], st) == hipSuccess;
   }
-  void run() {
-    for (uint64_t c; (c = next.fetch_add(1)) < n;) {
-      const int s = (int)(c % PinnedRing::CHUNKS);
-      while (sent[s].load(std::memory_order_acquire) <= c / PinnedRing::CHUNKS) std::this_thread::yield();
-      if (!err.load() && hipEventSynchronize(r->ev[s]) != hipSuccess) err = 1;
-      if (!err.load()) {
-        const uint64_t a = std::max(c * PinnedRing::CHUNK, skip), b = std::min((c + 1) * PinnedRing::CHUNK, total);
-        memcpy(dst + (a - skip), r->mem + s * PinnedRing::CHUNK + (a - c * PinnedRing::CHUNK), b - a);
-      }
-      if (c + PinnedRing::CHUNKS < n) send(c + PinnedRing::CHUNKS);
+  /* share t of piece c, whole 4 KB of the ring's memory */
+  void share(uint64_t c, unsigned t) {
+    const uint64_t o = c * PinnedRing::CHUNK, end = std::min(o + PinnedRing::CHUNK, total);
+    const uint64_t part = ((end - o) / threads + 4096) & ~(uint64_t)4095;
+    const uint64_t a = std::max(std::min(o + t * part, end), skip), b = t + 1 == threads ? end : std::min(o + (t + 1) * part, end);
+    if (a < b) memcpy(dst + (a - skip), r->mem + (c % PinnedRing::CHUNKS) * PinnedRing::CHUNK + (a - o), b - a);
+    copied.fetch_add(1, std::memory_order_release);
+  }
+  void help(unsigned t) {
+    for (uint64_t c = 0; c < n; ++c) {
+      while (ready.load(std::memory_order_acquire) <= c) std::this_thread::yield();
+      if (bad.load()) return;
+      share(c, t);
     }
+  }
+  hipError_t run() {
+    bool ok = send(0);
+    for (uint64_t c = 0; c < n && ok; ++c) {
+      if (c + 1 < n) ok = send(c + 1); /* its slot's last piece has been copied on */
+      ok = ok && hipEventSynchronize(r->ev[c % PinnedRing::CHUNKS]) == hipSuccess;
+      if (!ok) break;
+      ready.store(c + 1, std::memory_order_release);
+      share(c, 0);
+      while (copied.load(std::memory_order_acquire) < (c + 1) * threads) std::this_thread::yield();
+    }
+    if (!ok) {
+      bad = true;
+      ready.store(n, std::memory_order_release);
+    }
+    const hipError_t e = hipStreamSynchronize(st);
+    return ok ? e : hipErrorUnknown;
   }
 };
 
-/* Bytes from which three more threads help copy to the caller's memory: the
- * first touch of its pages costs more than the copy (36 MB to new pages 7.9
- * ms with one thread, 3.7 with four; 4 MB either way 0.18). */
-constexpr uint64_t COPY_THREADS_MIN = 8 << 20;
+/* Bytes from which three more threads help copy to the caller's memory,
+ * whose first touch costs more than the copy (36 MB to new pages 7.9 ms with
+ * one thread, 3.7 with four). */
+constexpr uint64_t COPY_THREADS_MIN = 2 << 20;
 
 /* device -> host on the job's stream (never the null stream, which would
  * wait for every other job's work), through pinned memory and from an
  * aligned address: HIP copies text from an odd address, as a job's unitigs
- * are, with a byte-wise kernel when it is small (1.0 MB 430 us, here 70), and
- * waits long for its own staging otherwise (16 MB 1.0 ms, 0.65). */
+ * are, byte by byte or after pinning the caller's pages (in two processes, one
+ * after the other: 1.0 MB 430 and 500 us, here 62 and 148; 5.3 MB 320 and 870,
+ * 213 and 436; 47 MB 6.7 ms in the second, 1.05 and 1.8).  In large pieces: in
+ * the first process on a device a copy and its event take 25 us, later 115, so
+ * 512 KB ones took 10.6 ms for the 47 MB. */
 static hipError_t copy_out(bruno_job* j, void* dst, const void* src, uint64_t bytes) {
   if (!bytes) return hipStreamSynchronize(j->stream);
   DevicePool& pool = DevicePool::current();
@@ -3830,24 +3850,29 @@ static hipError_t copy_out(bruno_job* j, void* dst, const void* src, uint64_t by
     c.src = (const char*)src - c.skip;
     c.total = bytes + c.skip;
     c.n = (c.total + PinnedRing::CHUNK - 1) / PinnedRing::CHUNK;
-    for (auto& x : c.sent) x = 0;
-    (void)hipGetDevice(&c.dev);
-    for (uint64_t q = 0; q < std::min<uint64_t>(c.n, PinnedRing::CHUNKS); ++q) c.send(q);
-    std::thread help[3];
+    std::thread helper[3];
+    unsigned t = 0;
     if (bytes >= COPY_THREADS_MIN) {
+      c.threads = 4;
       try {
-        for (std::thread& t : help) t = std::thread([&c] {
-          if (hipSetDevice(c.dev) == hipSuccess) c.run();
-          else (void)hipGetLastError();
-        });
-      } catch (...) { /* fewer threads */
+        for (; t < 3; ++t) helper[t] = std::thread([&c, t] { c.help(t + 1); });
+      } catch (...) { /* one thread then */
       }
     }
-    c.run();
-    for (std::thread& t : help)
-      if (t.joinable()) t.join();
-    e = hipStreamSynchronize(j->stream);
-    if (e == hipSuccess && c.err) e = hipErrorUnknown;
+    /* threads that could not be had */
+    if (t + 1 < c.threads) {
+      c.bad = true;
+      c.ready.store(c.n, std::memory_order_release);
+      for (std::thread& h : helper)
+        if (h.joinable()) h.join();
+      c.bad = false;
+      c.ready = 0;
+      c.copied = 0;
+      c.threads = 1;
+    }
+    e = c.run();
+    for (std::thread& h : helper)
+      if (h.joinable()) h.join();
     pool.give_ring(r);
   }
   if (e != hipSuccess) (void)hipGetLastError();

@@ -28,10 +28,11 @@
 
 namespace br {
 
-/* Pinned chunks for one device-to-host copy at a time, with an event each. */
+/* Two pinned pieces for one device-to-host copy at a time, with an event
+ * each. */
 struct PinnedRing {
-  static constexpr int CHUNKS = 16;
-  static constexpr uint64_t CHUNK = 512 << 10;
+  static constexpr int CHUNKS = 2;
+  static constexpr uint64_t CHUNK = 8 << 20;
   char* mem = nullptr;
   hipEvent_t ev[CHUNKS] = {};
 
