@@ -1596,8 +1596,10 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
       JobLayout& l = j->lay[i];
       region_layout(caps[i], most, nj > 1 || caps[i] < REGION_TIGHT_CAP, &l.rbits, &l.span);
       /* buckets: one per CU, 512 when one split pass would have more than
-       * SPLIT_BITS region bits left */
-      l.beta = std::min<uint32_t>(l.rbits, l.rbits > 8 + SPLIT_BITS ? MAX_BUCKET_BITS : 8);
+       * SPLIT_MAX_BITS region bits left (2^20 regions, 4.0 G instances:
+       * parser 17.2 and split 32.1 ms with 256 buckets and 12 bits, 26.3 and
+       * 27.5 with 512 and 11) */
+      l.beta = std::min<uint32_t>(l.rbits, l.rbits > 8 + SPLIT_MAX_BITS ? MAX_BUCKET_BITS : 8);
       l.region0 = (uint32_t)n_reg;
       l.bucket0 = (uint32_t)n_buck;
       n_reg += 1ULL << l.rbits;

@@ -42,7 +42,7 @@ namespace br {
 constexpr int REC_BUCKET_BITS = 5;
 constexpr int MAX_BUCKET_BITS = 9;
 constexpr int SPLIT_BS = 1024;
-constexpr int SPLIT_BITS = 11, SPLIT_MAX_BITS = 12; /* region bits a bucket is split by: usual, largest tables */
+constexpr int SPLIT_BITS = 11, SPLIT_MAX_BITS = 12; /* region bits a bucket is split by: usual, more than 2^19 regions */
 constexpr uint32_t REC_CODE_FILL = 31; /* chunk padding, never a biedge index (0..24) */
 constexpr uint32_t NO_CHUNK = ~0u;
 

@@ -83,7 +83,7 @@ def test_one_kmer_in_most_records(first):
 
 @pytest.mark.parametrize("k,cap", [(31, 700_000_000), (31, 1_400_000_000), (63, 350_000_000)])
 def test_widest_splits(k, cap):
-    """2^20 regions (512 buckets, 11 region bits) and 2^21 (12 bits)."""
+    """2^20 regions (256 buckets, 12 region bits) and 2^21 (512 buckets)."""
     set_tuning(region_slots=1280)
     b, off = pack(random_reads(5, 20000, 2000, (80, 200), 0.01)[1])
     job = bruno_amd.GraphJob(k, None, capacity=cap)
