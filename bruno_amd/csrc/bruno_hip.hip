@@ -1312,6 +1312,10 @@ struct bruno_job {
   /* the only count since the reset built every region and left the filter
    * scan's candidate / spilled-slot bits */
   bool bits_fresh = false;
+  /* a plain job whose table was asked for with REGION_TIGHT_CAP slots or
+   * more: a smaller one takes further batches after any count, which a fused
+   * count would end */
+  bool fusable = false;
   uint64_t* cbits = nullptr;
   uint64_t* sbits = nullptr;
   /* fuse_filter: a count that builds every region also filters (asked by
@@ -1588,6 +1592,7 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
   uint64_t total = 0, n_reg = 0, n_buck = 0, max_span = 0;
   for (uint32_t i = 0; i < nj; ++i) total += caps[i];
   j->regions = cr && total >= REGION_MIN_CAP;
+  j->fusable = nj == 1 && caps[0] >= REGION_TIGHT_CAP;
   /* the knob counts 32-byte slots: a 64-byte-slot region holds half */
   const uint64_t most = j->words == 1 ? tuning().region_slots : tuning().region_slots / 2;
   j->lay.assign(nj, JobLayout{});
@@ -1768,7 +1773,7 @@ bruno_status grow_table(bruno_job* j, uint64_t want) {
   void* oseg = j->d_seg;
   void* ojs = j->d_jstat;
   void* olay = j->d_lay;
-  const bool oregions = j->regions;
+  const bool oregions = j->regions, ofusable = j->fusable;
   const std::vector<JobLayout> olay_h = j->lay;
   const uint64_t onreg = j->n_regions, onbuck = j->n_buckets, ostride = j->bit_stride;
   const uint64_t ocap = j->cap, ospcap = j->spcap;
@@ -1792,6 +1797,7 @@ bruno_status grow_table(bruno_job* j, uint64_t want) {
     p = j->d_lay; dev_free(j, p, j->n_jobs * sizeof(JobLayout));
     j->d_lay = (JobLayout*)olay;
     j->regions = oregions;
+    j->fusable = ofusable;
     j->lay = olay_h;
     j->n_regions = onreg;
     j->n_buckets = onbuck;
@@ -2017,7 +2023,7 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
    * slots, and at most the instances / the count threshold) plus every
    * wave's open chunks; a node that finds no room stays a candidate for
    * the filter pass */
-  bool fuse = j->fuse_filter && cbits && nj == 1;
+  bool fuse = j->fuse_filter && cbits && j->fusable;
   NodeLists nl{};
   uint64_t* holes = nullptr;
   uint64_t lcap = 0;

@@ -111,6 +111,7 @@ __global__ __launch_bounds__(1024) void k_chunk_first(ChunkPool p, uint32_t b_lo
 constexpr uint32_t LISTED_STRIDE = 32;
 __global__ __launch_bounds__(BLOCK) void k_chunk_list(ChunkPool p, uint32_t b_lo, const uint32_t* first,
                                                       uint32_t* listed, uint32_t* list) {
+  if (*p.overflow) return; /* chunks may be missing, or a bucket too large */
   const uint32_t n = min(*p.next, p.n_max);
   for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < n; c += gridDim.x * BLOCK) {
     const uint32_t b = p.owner[c];

@@ -168,7 +168,8 @@ bruno_status bruno_job_set_recycle(bruno_job* job, int on);
  * further batch (bruno_parse_count* returns BRUNO_STATE until
  * bruno_job_reset) and the k2 / count getters return BRUNO_STATE, since
  * node records replace the k2 entries.  Off by default; a count that falls
- * back to atomics (small tables) is not fused, nor is a batch's.  No counterpart in
+ * back to atomics is not fused, nor is one of a batch or of a table asked for
+ * with fewer than 2^22 slots.  No counterpart in
  * the reference, whose filter is a pass of its own over the count map. */
 bruno_status bruno_job_set_fused_filter(bruno_job* job, int on);
 

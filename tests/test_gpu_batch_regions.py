@@ -114,3 +114,20 @@ def test_calls_of_few_and_many_instances(k, sizes):
         assert job.stats()["count_by_regions"] == (len(p) > 100)
     assert node_table(job.counts()) == want
     job.close()
+
+
+def test_small_table_takes_batches_after_a_fused_count():
+    """Asked to fuse the filter, a table of fewer than 2^22 slots counted by
+    regions still takes a further batch (its count is not fused)."""
+    _, reads = random_reads(4, 60000, 6000, 150, 0.01)
+    b, off = pack(reads)
+    job = bruno_amd.GraphJob(31, thresholds_L(2), capacity=1 << 21)
+    job.set_fused_filter(True)
+    for part in (reads[:4000], reads[4000:]):
+        job.parse_count(*pack(part))
+        assert job.stats()["count_by_regions"] == 1 and job.stats()["filter_fused"] == 0
+    want = run_oracle(31, thresholds_L(2), b, off)
+    assert node_table(job.counts()) == oracle_node_table(want.unfiltered())
+    job.run()
+    assert job.unitigs() == want.chain_fasta()
+    job.close()
