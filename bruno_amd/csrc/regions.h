@@ -174,8 +174,12 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   };
   /* append every bucket's whole lines (last: everything) to its open chunk,
    * the rest to a new one: fl_n records, of which fl_n1 go to chunk fl_c1
-   * from place fl_f1 and the others to the front of chunk ch_id */
-  auto flush = [&](bool last) {
+   * from place fl_f1 and the others to the front of chunk ch_id.  Returns
+   * the parked records, read between the two barriers, where no record is
+   * put: what follows it in barriers hangs on that number, and a wave that
+   * read it behind the second one could find what a faster wave had already
+   * parked. */
+  auto flush = [&](bool last) -> uint32_t {
     if (tid < nb_) {
       const uint32_t c = cnt[tid], n = c < S ? c : S;
       const uint32_t m = last ? n : n & ~(LINE - 1);
@@ -207,6 +211,7 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       }
     }
     lds_barrier();
+    const uint32_t parked = n_park;
     /* numbers for the next append, while the other waves copy: those left
      * (fewer than nb_, so all of the later range), then nb_ more */
     if (tid == REC_BS - 1 && pl_n - pl_used < nb_) {
@@ -233,13 +238,13 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       if (gl < cnt[b]) stg[b * S + gl] = stg[b * S + m + gl];
     }
     lds_barrier();
+    return parked;
   };
-  /* stage the parked records again until none is left (every bucket has
-   * room for S - LINE of its own each time) */
-  auto unpark = [&]() {
-    for (;;) {
-      const uint32_t n = n_park < REC_PARK ? n_park : REC_PARK;
-      if (n == 0) break;
+  /* stage the parked records (as many as the last append found) again until
+   * none is left (every bucket has room for S - LINE of its own each time) */
+  auto unpark = [&](uint32_t parked) {
+    while (parked) {
+      const uint32_t n = parked < REC_PARK ? parked : REC_PARK;
       R rec = rec_zero<R>();
       uint32_t b = 0;
       if (tid < n) {
@@ -251,7 +256,7 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       lds_barrier();
       if (tid < n) put(b, rec);
       lds_barrier();
-      flush(false);
+      parked = flush(false);
     }
   };
   const int sh2 = 2 * (K - 1);
@@ -261,6 +266,7 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   const uint64_t r_job = ra.first[sh.job], n_job = ra.first[sh.job + 1] - r_job;
   const uint64_t lo_r = r_job + n_job * sh.i / sh.n, hi_r = r_job + n_job * (sh.i + 1) / sh.n;
   const uint64_t rounds = (hi_r - lo_r + REC_BS - 1) / REC_BS;
+  uint32_t parked = 0; /* as the last append found it; nothing is put after the last one */
   for (uint64_t round = 0; round < rounds; ++round) {
     const uint64_t ra0 = lo_r + (hi_r - lo_r) * round / rounds, ra1 = lo_r + (hi_r - lo_r) * (round + 1) / rounds;
     const uint64_t r = ra0 + tid;
@@ -332,13 +338,16 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
         }
         if (q % PF == PF - 1 && (often || q == 15)) {
           lds_barrier();
-          flush(false);
-          if (n_park > REC_PARK / 2) unpark();
+          parked = flush(false);
+          if (parked > REC_PARK / 2) {
+            unpark(parked);
+            parked = 0;
+          }
         }
       }
     }
   }
-  unpark();
+  unpark(parked);
   flush(true);
   for (uint32_t u = pl_used + tid; u < pl_n; u += REC_BS) {
     const uint32_t nid = u < pl_n0 ? pl_b0 + u : pl_b1 + (u - pl_n0);
