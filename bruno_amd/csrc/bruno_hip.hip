@@ -448,12 +448,12 @@ __device__ void resolve_pair(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, u
 
 /* to_simple_biedge (debruijn_chain_node.hpp:84-141): one neighbour per side
  * at dist 1, else term_mask; an end at a branch that answers it is terminal
- * at once (k_termini writes the same).  So every chain end is known here,
- * and the rulers of the list ranking (chain ends and sampled nodes) are
- * marked in a bitmap, a word per wave, instead of by a pass over the 32-byte
- * records (0.85 ms for 40 M chain nodes).  The node's k-mer goes into its
- * mailboxes, beside the pointers, for the placing walk (chains.h); the
- * round-by-round ranking empties them first. */
+ * at once (k_termini writes the same).  So every chain end of a well-formed
+ * graph is known here, and the rulers of the list ranking (chain ends and
+ * sampled nodes) are marked in a bitmap, a word per wave, instead of by a pass
+ * over the 32-byte records (0.85 ms for 40 M chain nodes).  The node's k-mer
+ * goes into its mailboxes, beside the pointers, for the placing walk
+ * (chains.h); the round-by-round ranking empties them first. */
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_t cap, uint32_t rbits, int K,
                                                       const uint64_t* chain_slot,
@@ -516,14 +516,20 @@ __global__ __launch_bounds__(BLOCK) void k_chain_init(const Slot<KT>* T, uint64_
 }
 
 /* setup_chain_termini: each branch node marks the facing end of its chain
- * neighbours as pointing to a branch (dist 0). */
+ * neighbours as pointing to a branch (dist 0).  k_chain_init has done so
+ * where the chain node's own edge leads there.  An end whose edge leads to
+ * another chain node (the thresholds kept the branch's edge and dropped the
+ * chain node's share of it) becomes terminal only here, with that neighbour
+ * still pointing at it: the chain nodes are then no disjoint paths, and the
+ * end counts as ill-formed for the list ranking. */
 template <typename KT>
 __global__ __launch_bounds__(BLOCK) void k_termini(const Slot<KT>* T, uint64_t cap, uint32_t rbits, int K,
                                                    const uint64_t* branch_slot,
                                                    const uint32_t* branch_job, const JobLayout* lay, uint32_t n_jobs,
-                                                   uint64_t n_branch, LRNode* lr, KT* bkmer) {
+                                                   uint64_t n_branch, LRNode* lr, KT* bkmer, Counters* ctr) {
   kops<KT> ops(K);
   const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+  unsigned long long ill = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n_branch; i += stride) {
     const Slot<KT>* p = T + branch_slot[i];
     uint64_t tbase = 0, tcap = cap;
@@ -553,9 +559,12 @@ __global__ __launch_bounds__(BLOCK) void k_termini(const Slot<KT>* T, uint64_t c
         if (q->cls != CLS_CHAIN) continue;
         int orient_in = (side == 0);  /* IN for out neighbours */
         if (flipped) orient_in = !orient_in;
-        lr[q->idx].d[orient_in ? 0 : 1] = 0;
+        uint32_t* d = &lr[q->idx].d[orient_in ? 0 : 1];
+        ill += !is_terminal(*d);
+        *d = 0;
       }
   }
+  block_add(ill, &ctr->lr_ill);
 }
 
 /* ================================================================== */
@@ -2450,7 +2459,7 @@ bruno_status chains_t(bruno_job* j) {
                        j->ruler_base, j->ruler_node, j->ctr);
   hipLaunchKernelGGL((k_termini<KT>), dim3(grid_for(j->n_branch)), dim3(BLOCK), 0, j->stream,
                      (const Slot<KT>*)j->table, probe_span(j), j->rbits, j->K, j->branch_slot, j->branch_job,
-                     j->d_lay, j->n_jobs, j->n_branch, j->lr, (KT*)j->bkmer);
+                     j->d_lay, j->n_jobs, j->n_branch, j->lr, (KT*)j->bkmer, j->ctr);
   TRY(sync_counters(j));
   j->n_virt = j->hctr->n_virt;
   j->n_rulers = j->hctr->lr_next;
@@ -2493,7 +2502,7 @@ bruno_status list_rank_fast(bruno_job* j, bool* used) {
   *used = false;
   const uint64_t nc = j->n_chain, nr = j->n_rulers;
   if (nc == 0) return BRUNO_OK;
-  /* k_chain_init counted the ill-formed ends */
+  /* k_chain_init and k_termini counted the ill-formed ends */
   if (j->hctr->lr_ill != 0) return BRUNO_OK;
   const uint32_t nj = j->n_jobs;
   const uint32_t* cjob = nj > 1 ? j->chain_job : nullptr;
