@@ -1986,6 +1986,15 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   uint32_t* rcount = (uint32_t*)get(nreg * 4);
   uint32_t* first = (uint32_t*)get((n_sb + 1) * 4);
   ParseShare* d_share = (ParseShare*)get(share.size() * sizeof(ParseShare));
+  /* a parser workgroup's records of one interval, at most 16 per read, that
+   * its park has no room for */
+  uint64_t lanes = 0;
+  for (uint32_t q = ja; q < jb; ++q)
+    if (wgs[q - ja]) lanes = std::max(lanes, (h_first[q + 1] - h_first[q] + wgs[q - ja] - 1) / wgs[q - ja]);
+  const uint64_t interval = std::min<uint64_t>(rec_interval<R>(), 16 * lanes);
+  const uint32_t over_cap = (uint32_t)(interval > REC_PARK ? interval - REC_PARK : 0);
+  void* over = get(share.size() * over_cap * RB);
+  uint32_t* over_at = (uint32_t*)get(share.size() * over_cap * 4);
   /* zeroed: chunks taken in all and overflow flag, statistics, per bucket
    * chunks taken and listed */
   const uint64_t n_zero = 1 + 2 * (uint64_t)nj + (n_sb + 1) / 2 + n_sb * (LISTED_STRIDE / 2);
@@ -2008,7 +2017,7 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   ChunkPool pool{recs, clog, (uint32_t)n_chunks, next, taken - b_lo, owner, overflow};
   if (!share.empty()) {
     HIP_CHECK(hipMemcpyAsync(d_share, share.data(), share.size() * sizeof(ParseShare), hipMemcpyHostToDevice, j->stream));
-    RecArgs ra{pool, j->d_lay, d_first, d_share, stat};
+    RecArgs ra{pool, j->d_lay, d_first, d_share, over, over_at, over_cap, stat};
     constexpr int PF = RB == 8 ? 8 : 4;
     const dim3 g((unsigned)share.size());
     if (beta_max <= 8)

@@ -45,9 +45,12 @@ constexpr uint32_t REGION_WIDE_SLOTS = 1280;
 constexpr uint32_t REGION_WIDE_SMALL_SLOTS = 640;
 constexpr uint64_t REGION_BUILD_CU_SLOTS = 512; /* build workgroups resident on the device (x2 for small) */
 /* record parser: workgroup size, staged records of all its buckets (128 KB),
- * records parked while their bucket's stage is full */
-constexpr int REC_BS = 1024, REC_PARK = 512;
+ * records parked in LDS that found their bucket's stage full */
+constexpr int REC_BS = 1024, REC_PARK = 256;
 constexpr uint32_t REC_STAGE_BYTES = 128 << 10;
+/* most records between two appends: a workgroup appends every PF positions,
+ * or every 16 when its reads have at most so many records in them */
+template <typename R> constexpr uint32_t rec_interval() { return REC_STAGE_BYTES / sizeof(R) / 4 * 3; }
 constexpr int REGION_ITEMS = 8;              /* records per thread loaded at once by the build */
 
 /* A parser workgroup's share: reads of job `job`, part i of n of them. */
@@ -60,6 +63,9 @@ struct RecArgs {
   const JobLayout* jobs;
   const uint64_t* first;     /* job q holds reads [first[q], first[q + 1]) */
   const ParseShare* share;   /* per workgroup */
+  void* over;                /* per workgroup over_cap records (RecOf<KT>::T) that found the park full, */
+  uint32_t* over_at;         /* and their places */
+  uint32_t over_cap;
   unsigned long long* stat;  /* per job: instances, dropped reads */
 };
 
@@ -95,6 +101,35 @@ template <typename R> __device__ __forceinline__ R rec_filler();
 template <> __device__ __forceinline__ uint64_t rec_filler<uint64_t>() { return REC_CODE_FILL; }
 template <> __device__ __forceinline__ ulonglong2 rec_filler<ulonglong2>() { return make_ulonglong2(REC_CODE_FILL, 0); }
 
+/* `more` consecutive chunks of the pool for a bucket at once (more than one
+ * for a crowded bucket only, so out of line: inlined, these parts cost the
+ * parser registers); NO_CHUNK and the overflow flag if there are none. */
+__device__ __noinline__ uint32_t take_chunks(uint32_t* next, uint32_t* taken, uint32_t* owner, uint32_t n_max,
+                                             uint32_t* overflow, uint32_t bucket, uint32_t more) {
+  const uint32_t nid = atomicAdd(next, more);
+  atomicAdd(taken, more);
+  if (nid > n_max || more > n_max - nid) {
+    *overflow = 1;
+    return NO_CHUNK;
+  }
+  for (uint32_t q = 0; q < more; ++q) owner[nid + q] = bucket;
+  return nid;
+}
+
+/* the parked records that are in HBM to their chunks (see flush) */
+template <typename R>
+__device__ __noinline__ void place_over(const R* over, const uint32_t* over_at, uint32_t n, R* recs, uint32_t clog,
+                                        const uint32_t* fl_n, const uint32_t* fl_n1, const uint32_t* fl_c1,
+                                        const uint32_t* fl_f1, const uint32_t* fl_c2) {
+  for (uint32_t p = threadIdx.x; p < n; p += REC_BS) {
+    const uint32_t b = over_at[p] & 511u, i = over_at[p] >> 9, m1 = fl_n1[b];
+    if (fl_n[b] == 0) continue;
+    R* d = i < m1 ? recs + ((uint64_t)fl_c1[b] << clog) + fl_f1[b] + i
+                  : recs + ((uint64_t)fl_c2[b] << clog) + (i - m1);
+    *d = over[p];
+  }
+}
+
 /* Parse into bucketed instance records, one read per lane.  A lane rolls
  * its read's k-mer and reverse complement along the read one base at a
  * time (a shift and an or each), so an instance costs its hash and its
@@ -109,16 +144,22 @@ template <> __device__ __forceinline__ ulonglong2 rec_filler<ulonglong2>() { ret
  * positions the workgroup appends each bucket's whole 128-byte lines to the
  * bucket's open chunk (the rest moves to the front of its stage), so chunks
  * are written in full lines whatever their number.  A record that finds its
- * stage full is parked and staged again when the park is half full; one that
- * finds the park full too gives the count up (the caller counts with
- * atomics), which takes one bucket getting a fifteenth of all records.
+ * stage full is parked, in LDS and past REC_PARK of them in HBM, with its
+ * number in the bucket, which is its place in the append: the append takes a
+ * crowded bucket's records all, staged and parked (reads of low complexity
+ * or of one locus side by side put a whole interval's into one bucket).  The
+ * count of 1 M reads of 150 bases, 2.7 ms, takes 3.6 with 2,000 poly-A reads
+ * among them in one place and 10.2 with 20 times 1,000; when a record that
+ * found a park of 512 full gave the count up, to HBM atomics, 13.3 and 43.  An
+ * append without crowded buckets pays for it with 2% of the kernel (917 for
+ * 900 us, 2.46 for 2.42 ms of 16-byte records).
  *
  * One 1,024-thread workgroup per CU with 256 buckets (512 for the largest
  * tables).  Bound by instruction issue.  The appends to 256 buckets cost
  * 5-15% over 32 and the split after it needs one pass instead of two; the
  * bases tested and coded four at a time and read four blocks at a time give
- * it back (1.6 G instances 7.4 ms with 32 buckets, 7.8 with 256, now 7.2; 184
- * M 0.84, 0.96, 0.91; 301 M of k = 63 2.48, 2.59, 2.42).  With the split the
+ * it back (1.6 G instances 7.4 ms with 32 buckets, 7.8 with 256, now 7.3; 184
+ * M 0.84, 0.96, 0.92; 301 M of k = 63 2.48, 2.59, 2.46).  With the split the
  * count phase as a whole 35.9 -> 30.1, 4.5 -> 3.8, 13.2 -> 10.7 and 1.39 ->
  * 0.81 ms.  A batch of 16 jobs of 0.05 to 2 Mbp (243 M instances), which HBM
  * atomics counted in 18.6 ms, takes 5.9. */
@@ -130,14 +171,24 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   __shared__ R stg[STAGE];
   __shared__ uint32_t cnt[MAXB];
   __shared__ uint32_t ch_id[MAXB], ch_fill[MAXB];     /* open chunk (NO_CHUNK: none) */
-  __shared__ uint32_t fl_n1[MAXB], fl_n[MAXB], fl_c1[MAXB], fl_f1[MAXB]; /* an append: see flush */
-  __shared__ R park[REC_PARK];
-  __shared__ uint16_t park_b[REC_PARK];
+  __shared__ uint32_t fl_n1[MAXB], fl_n[MAXB], fl_c1[MAXB], fl_f1[MAXB], fl_c2[MAXB]; /* an append: see flush */
+  /* Parked records are numbered through the whole launch, n_park of them so
+   * far, `parked` of them before the last append.  An interval's first
+   * REC_PARK are here, by their number, beside as many of the interval
+   * before, which are placed meanwhile. */
+  __shared__ R park[2 * REC_PARK];
+  __shared__ uint32_t park_at[2 * REC_PARK]; /* number in the bucket << 9 | bucket */
   __shared__ uint32_t n_park, blocks_max;
+  /* (kept here for the rare path that uses them, not in registers) */
+  __shared__ R* over;
+  __shared__ uint32_t* over_at;
+  __shared__ uint32_t over_cap;
   /* chunk numbers in hand, at least one per bucket before an append: pl_n0
    * from pl_b0, then up to pl_n from pl_b1; pl_used are given out */
   __shared__ uint32_t pl_b0, pl_n0, pl_b1, pl_n, pl_used;
   static_assert(16 % PF == 0, "flush points split a block evenly");
+  static_assert(REC_BS * PF <= rec_interval<R>(), "an interval's records");
+  static_assert(MAXB <= 512 && rec_interval<R>() + STAGE < (1u << 23), "park_at");
   const uint32_t tid = threadIdx.x;
   const ParseShare sh = ra.share[blockIdx.x];
   const JobLayout* jb = ra.jobs + sh.job;
@@ -152,66 +203,83 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
     ch_fill[b] = 0;
   }
   if (tid == 0) {
+    over = (R*)ra.over + (uint64_t)blockIdx.x * ra.over_cap;
+    over_at = ra.over_at + (uint64_t)blockIdx.x * ra.over_cap;
+    over_cap = ra.over_cap;
     n_park = pl_b0 = pl_n0 = pl_used = 0;
     pl_b1 = atomicAdd(ra.pool.next, nb_);
     pl_n = nb_;
   }
   __syncthreads();
   R* const recs = (R*)ra.pool.recs;
+  uint32_t parked = 0;
   auto put = [&](uint32_t b, const R& rec) {
     const uint32_t pos = atomicAdd(&cnt[b], 1u);
     if (pos < S) {
       stg[b * S + pos] = rec;
     } else {
-      const uint32_t p = atomicAdd(&n_park, 1u);
-      if (p < REC_PARK) {
-        park[p] = rec;
-        park_b[p] = (uint16_t)b;
+      const uint32_t p = atomicAdd(&n_park, 1u), i = p - parked, at = pos << 9 | b;
+      if (i < REC_PARK) {
+        park[p & (2 * REC_PARK - 1)] = rec;
+        park_at[p & (2 * REC_PARK - 1)] = at;
+      } else if (i - REC_PARK < over_cap) {
+        over[i - REC_PARK] = rec;
+        over_at[i - REC_PARK] = at;
       } else {
-        *ra.pool.overflow = 1;
+        *ra.pool.overflow = 1; /* no interval has so many */
       }
     }
   };
-  /* append every bucket's whole lines (last: everything) to its open chunk,
-   * the rest to a new one: fl_n records, of which fl_n1 go to chunk fl_c1
-   * from place fl_f1 and the others to the front of chunk ch_id.  Returns
-   * the parked records, read between the two barriers, where no record is
-   * put: what follows it in barriers hangs on that number, and a wave that
-   * read it behind the second one could find what a faster wave had already
-   * parked. */
-  auto flush = [&](bool last) -> uint32_t {
+  /* append every bucket's whole lines, up to a line's end in its chunk (last,
+   * or some of them parked: everything), to its open chunk, the rest to new
+   * ones: the first fl_n1 of them to chunk fl_c1 from place fl_f1, the others
+   * to the chunks from fl_c2 on, consecutive ones, the last of which is open
+   * then; fl_n are staged, the rest is parked.  The number of parked records is read between the two
+   * barriers, where nothing is put, so that every wave finds the same. */
+  auto flush = [&](bool last) {
     if (tid < nb_) {
-      const uint32_t c = cnt[tid], n = c < S ? c : S;
-      const uint32_t m = last ? n : n & ~(LINE - 1);
-      const uint32_t id = ch_id[tid], fill = ch_fill[tid];
+      const uint32_t c = cnt[tid];
+      const uint32_t id = ch_id[tid], fill = ch_fill[tid], end = (fill + c) & ~(LINE - 1);
+      const uint32_t m = last || c > S ? c : end > fill ? end - fill : 0u;
       const uint32_t room = id == NO_CHUNK ? 0u : C - fill;
-      const uint32_t m1 = m < room ? m : room, m2 = m - m1;
-      fl_n[tid] = m;
+      const uint32_t m1 = m < room ? m : room, m2 = m - m1, more = (m2 + C - 1) >> clog;
+      fl_n[tid] = m < S ? m : S;
       fl_n1[tid] = m1;
       fl_c1[tid] = id;
       fl_f1[tid] = fill;
-      cnt[tid] = n - m;
-      ch_fill[tid] = m2 ? m2 : fill + m1;
+      cnt[tid] = c - m;
+      ch_fill[tid] = m2 ? m2 - ((more - 1) << clog) : fill + m1;
       /* One chunk number per bucket that needs one, from those in hand (an
        * atomic in HBM here would hold up the whole workgroup at the next
        * barrier: 2 of 9 ms). */
-      const uint64_t need = __ballot(m2 != 0);
+      const uint64_t need = __ballot(more == 1);
       if (need) {
         const uint32_t lane = tid & 63;
         uint32_t u = 0;
         if (lane == 0) u = atomicAdd(&pl_used, (uint32_t)__popcll(need));
         u = (uint32_t)__builtin_amdgcn_readfirstlane((int)u) + (uint32_t)__popcll(need & ((1ULL << lane) - 1));
-        if (m2) {
+        if (more == 1) {
           const uint32_t nid = u < pl_n0 ? pl_b0 + u : pl_b1 + (u - pl_n0);
           atomicAdd(&ra.pool.taken[bucket0 + tid], 1u);
           if (nid < ra.pool.n_max) ra.pool.owner[nid] = bucket0 + tid;
           else *ra.pool.overflow = 1;
-          ch_id[tid] = nid < ra.pool.n_max ? nid : ra.pool.n_max - 1;
+          fl_c2[tid] = ch_id[tid] = nid < ra.pool.n_max ? nid : ra.pool.n_max - 1;
+        }
+      }
+      if (more > 1) {
+        const uint32_t nid = take_chunks(ra.pool.next, ra.pool.taken + bucket0 + tid, ra.pool.owner, ra.pool.n_max,
+                                         ra.pool.overflow, bucket0 + tid, more);
+        if (nid == NO_CHUNK) { /* nothing will be counted, so nothing is written */
+          fl_n[tid] = 0;
+          ch_id[tid] = ra.pool.n_max - 1;
+        } else {
+          fl_c2[tid] = nid;
+          ch_id[tid] = nid + more - 1;
         }
       }
     }
     lds_barrier();
-    const uint32_t parked = n_park;
+    const uint32_t n_parked = n_park;
     /* numbers for the next append, while the other waves copy: those left
      * (fewer than nb_, so all of the later range), then nb_ more */
     if (tid == REC_BS - 1 && pl_n - pl_used < nb_) {
@@ -229,7 +297,7 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       if (m == 0) continue;
       const uint32_t m1 = fl_n1[b];
       R* d1 = recs + ((uint64_t)fl_c1[b] << clog) + fl_f1[b];
-      R* d2 = recs + ((uint64_t)ch_id[b] << clog);
+      R* d2 = recs + ((uint64_t)fl_c2[b] << clog);
       for (uint32_t i = gl; i < m; i += LINE) {
         R* d = i < m1 ? d1 + i : d2 + (i - m1);
         *d = stg[b * S + i];
@@ -237,27 +305,28 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       /* fewer than LINE records are left; the lanes read before they write */
       if (gl < cnt[b]) stg[b * S + gl] = stg[b * S + m + gl];
     }
-    lds_barrier();
-    return parked;
-  };
-  /* stage the parked records (as many as the last append found) again until
-   * none is left (every bucket has room for S - LINE of its own each time) */
-  auto unpark = [&](uint32_t parked) {
-    while (parked) {
-      const uint32_t n = parked < REC_PARK ? parked : REC_PARK;
-      R rec = rec_zero<R>();
-      uint32_t b = 0;
-      if (tid < n) {
-        rec = park[tid];
-        b = park_b[tid];
-      }
-      lds_barrier();
-      if (tid == 0) n_park = 0;
-      lds_barrier();
-      if (tid < n) put(b, rec);
-      lds_barrier();
-      parked = flush(false);
+    const uint32_t p0 = parked;
+    parked = (uint32_t)__builtin_amdgcn_readfirstlane((int)n_parked);
+    const uint32_t np = parked - p0;
+    if (np > REC_PARK) {
+      __syncthreads(); /* the records in HBM are there */
+      place_over<R>(over, over_at, np - REC_PARK < over_cap ? np - REC_PARK : over_cap, recs, clog, fl_n, fl_n1, fl_c1,
+                    fl_f1, fl_c2);
     }
+    /* The parked records in LDS: behind the barrier, since their reads one
+     * after the other would hold up the whole workgroup; fl_* stay as they
+     * are until all waves have come to the next append.  (More than the LDS
+     * holds: the next interval's may take the same places.) */
+    if (np <= REC_PARK) lds_barrier();
+    if (np && tid < (np < REC_PARK ? np : (uint32_t)REC_PARK)) {
+      const uint32_t q = (p0 + tid) & (2 * REC_PARK - 1), b = park_at[q] & 511u, i = park_at[q] >> 9, m1 = fl_n1[b];
+      if (fl_n[b] != 0) {
+        R* d = i < m1 ? recs + ((uint64_t)fl_c1[b] << clog) + fl_f1[b] + i
+                      : recs + ((uint64_t)fl_c2[b] << clog) + (i - m1);
+        *d = park[q];
+      }
+    }
+    if (np > REC_PARK) lds_barrier();
   };
   const int sh2 = 2 * (K - 1);
   const KT kmask = ops.mask;
@@ -266,7 +335,6 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   const uint64_t r_job = ra.first[sh.job], n_job = ra.first[sh.job + 1] - r_job;
   const uint64_t lo_r = r_job + n_job * sh.i / sh.n, hi_r = r_job + n_job * (sh.i + 1) / sh.n;
   const uint64_t rounds = (hi_r - lo_r + REC_BS - 1) / REC_BS;
-  uint32_t parked = 0; /* as the last append found it; nothing is put after the last one */
   for (uint64_t round = 0; round < rounds; ++round) {
     const uint64_t ra0 = lo_r + (hi_r - lo_r) * round / rounds, ra1 = lo_r + (hi_r - lo_r) * (round + 1) / rounds;
     const uint64_t r = ra0 + tid;
@@ -300,7 +368,7 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
     /* a round of few reads fills its stages more slowly: an append at every
      * PF-th position, or once a block when a bucket's share of the block's
      * records leaves a quarter of its stage to chance and what stays behind */
-    const bool often = (ra1 - ra0) * 16 > (uint64_t)(STAGE - STAGE / 4 - nb_ * (LINE / 2));
+    const bool often = (ra1 - ra0) * 16 > (uint64_t)(rec_interval<R>() - nb_ * (LINE / 2));
     uint4 v[4] = {};
     for (uint32_t t = 0; t < nbw; ++t) {
       if (t % 4 == 0) rd.four(t, v);
@@ -338,16 +406,12 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
         }
         if (q % PF == PF - 1 && (often || q == 15)) {
           lds_barrier();
-          parked = flush(false);
-          if (parked > REC_PARK / 2) {
-            unpark(parked);
-            parked = 0;
-          }
+          flush(false);
         }
       }
     }
   }
-  unpark(parked);
+  lds_barrier(); /* the last append's parked records are placed */
   flush(true);
   for (uint32_t u = pl_used + tid; u < pl_n; u += REC_BS) {
     const uint32_t nid = u < pl_n0 ? pl_b0 + u : pl_b1 + (u - pl_n0);
