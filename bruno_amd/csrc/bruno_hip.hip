@@ -1555,6 +1555,14 @@ double ev_ms(bruno_job* j, int a, int b) {
  * dozen launches (180 us, against 40 for the atomic kernel's one) outweigh
  * the atomics of any call it has room for keeps one probe window. */
 constexpr uint64_t REGION_MIN_CAP = 1ULL << 19;
+/* A table whose jobs are so small that their buckets (32 for a job at least)
+ * have fewer slots than this on average keeps probe windows: every bucket of
+ * a job is a round of the split and every job a parser workgroup, whatever
+ * they hold, and its regions' room for the spread of the hash is a multiple of
+ * its slots.  Measured on 4,096 equal jobs in one batch, count to unitigs, ms,
+ * atomics / regions, k = 31: 286 slots a bucket 4.6 / 9.3, 655 9.6 / 10.9, 1,710
+ * 25.6 / 16.6; 1,024 jobs: 1,183 5.8 / 3.9; k = 63: 354 5.5 / 8.8, 883 13.6 / 11.3. */
+constexpr uint64_t REGION_MIN_BUCKET_SLOTS = 768;
 /* Below this a plain job's regions get room for the spread of the hash
  * (region_layout), so that a tight table takes what one probe window takes. */
 constexpr uint64_t REGION_TIGHT_CAP = 1ULL << 22;
@@ -1620,8 +1628,8 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
       n_buck += 1ULL << l.beta;
       max_span = std::max(max_span, l.span);
     }
-    /* regions and buckets are numbered in 32 bits */
-    if (n_reg >= (1ULL << 31) || n_buck >= (1ULL << 31)) j->regions = false;
+    /* (regions and buckets are numbered in 32 bits) */
+    if (total < n_buck * REGION_MIN_BUCKET_SLOTS || n_reg >= (1ULL << 31) || n_buck >= (1ULL << 31)) j->regions = false;
   }
   j->seg.assign(nj + 1, 0);
   for (uint32_t i = 0; i < nj; ++i) {
@@ -1875,9 +1883,10 @@ bruno_status autosize(bruno_job* j, const char* d_bases, const uint64_t* d_offse
   return BRUNO_OK;
 }
 
-/* Records of a region count's pass over several jobs of a batch: at most
- * this many bytes of them (a job with more is a pass of its own), so the record
- * buffers of a batch stay small beside its table. */
+/* A region count's pass over several jobs of a batch: at most this many bytes
+ * of records and of the chunks that the jobs' buckets leave partly filled (a
+ * job with more is a pass of its own), so the record buffers of a batch stay
+ * small beside its table. */
 constexpr uint64_t REC_PASS_BYTES = 1ULL << 32;
 
 /* Jobs [ja, jb) counted by regions: the reads of these jobs into bucketed
@@ -1898,11 +1907,10 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   const uint32_t q_lo = j->lay[ja].region0, q_hi = jb < nj ? j->lay[jb].region0 : (uint32_t)j->n_regions;
   const uint64_t n_sb = b_hi - b_lo;
   uint64_t n_inst = 0;
-  uint32_t beta_min = MAX_BUCKET_BITS, beta_max = 0;
+  uint32_t beta_max = 0;
   int b2_max = 0;
   for (uint32_t q = ja; q < jb; ++q) {
     n_inst += inst[q];
-    beta_min = std::min(beta_min, j->lay[q].beta);
     beta_max = std::max(beta_max, j->lay[q].beta);
     b2_max = std::max(b2_max, (int)(j->lay[q].rbits - j->lay[q].beta));
   }
@@ -1933,10 +1941,11 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
     for (uint32_t i = 0; i < w; ++i) share.push_back(ParseShare{q, i, w, 0});
   }
   /* chunks of up to 1024 records, smaller for small inputs so padding stays
-   * under ~1/8 of the records; an append holds at most a bucket's stage */
-  const uint64_t stage = (REC_STAGE_BYTES / RB) >> beta_min;
-  uint32_t clog = 10;
-  while (clog > 6 && (1ULL << (clog - 1)) >= stage && (open << clog) * 4 > n_inst) --clog;
+   * under ~1/8 of the records.  (Chunks smaller than a bucket's stage are
+   * taken several at once; a floor at the stage of the job with the fewest
+   * buckets, 512 records, gave every other job's open chunks that size too.) */
+  uint32_t clog = REC_CHUNK_LOG;
+  while (clog > REC_CHUNK_LOG_MIN && (open << clog) * 4 > n_inst) --clog;
   /* every record's chunk, the partly filled ones, and at most two per
    * (workgroup, bucket) taken ahead and not used */
   const uint64_t n_chunks = (n_inst >> clog) + 3 * open + 1;
@@ -2231,9 +2240,13 @@ bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, const uint64_t* 
   }
   if (!sbits) cbits = nullptr;
   bool all = true;
+  /* records a job takes room for: its instances, and per bucket an open chunk
+   * and two in hand (of one workgroup: a pass of many jobs has no more) */
+  auto room_of = [&](uint32_t q) { return inst[q] + ((uint64_t)3 << j->lay[q].beta << REC_CHUNK_LOG_MIN); };
   for (uint32_t ja = 0, jb; ja < nj; ja = jb) {
-    uint64_t n = inst[ja];
-    for (jb = ja + 1; jb < nj && n + inst[jb] <= REC_PASS_BYTES / sizeof(typename RecOf<KT>::T); ++jb) n += inst[jb];
+    uint64_t n = room_of(ja);
+    for (jb = ja + 1; jb < nj && n + room_of(jb) <= REC_PASS_BYTES / sizeof(typename RecOf<KT>::T); ++jb)
+      n += room_of(jb);
     bool done = false;
     TRY(count_regions_pass<KT>(j, a, d_first, h_first, ja, jb, inst, valid, cbits, sbits, &done));
     if (done) continue;

@@ -45,6 +45,7 @@ constexpr int SPLIT_BS = 1024;
 constexpr int SPLIT_BITS = 11, SPLIT_MAX_BITS = 12; /* region bits a bucket is split by: usual, more than 2^19 regions */
 constexpr uint32_t REC_CODE_FILL = 31; /* chunk padding, never a biedge index (0..24) */
 constexpr uint32_t NO_CHUNK = ~0u;
+constexpr int REC_CHUNK_LOG = 10, REC_CHUNK_LOG_MIN = 6; /* log2 records per chunk: at most SPLIT_BS, at least a piece */
 
 /* A record: one word (k <= 31) or the key word and the k-mer's high word
  * (k <= 63).  The key word, (hash << 5) | biedge index, is what the split
