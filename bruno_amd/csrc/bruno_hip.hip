@@ -1561,8 +1561,9 @@ constexpr uint64_t REGION_MIN_CAP = 1ULL << 19;
  * they hold, and its regions' room for the spread of the hash is a multiple of
  * its slots.  Measured on 4,096 equal jobs in one batch, count to unitigs, ms,
  * atomics / regions, k = 31: 286 slots a bucket 4.6 / 9.3, 655 9.6 / 10.9, 1,710
- * 25.6 / 16.6; 1,024 jobs: 1,183 5.8 / 3.9; k = 63: 354 5.5 / 8.8, 883 13.6 / 11.3. */
-constexpr uint64_t REGION_MIN_BUCKET_SLOTS = 768;
+ * 25.6 / 16.6; 1,024 jobs: 1,183 5.8 / 3.9; the 4,096 of 286 slots and one of 63 M,
+ * 800 on average, 10.9 / 12.5; k = 63: 354 5.5 / 8.8, 883 13.6 / 11.4, 17.0 / 14.0. */
+constexpr uint64_t REGION_MIN_BUCKET_SLOTS = 1024, REGION_MIN_BUCKET_WIDE_SLOTS = 768;
 /* Below this a plain job's regions get room for the spread of the hash
  * (region_layout), so that a tight table takes what one probe window takes. */
 constexpr uint64_t REGION_TIGHT_CAP = 1ULL << 22;
@@ -1629,7 +1630,8 @@ bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
       max_span = std::max(max_span, l.span);
     }
     /* (regions and buckets are numbered in 32 bits) */
-    if (total < n_buck * REGION_MIN_BUCKET_SLOTS || n_reg >= (1ULL << 31) || n_buck >= (1ULL << 31)) j->regions = false;
+    const uint64_t least = j->words == 1 ? REGION_MIN_BUCKET_SLOTS : REGION_MIN_BUCKET_WIDE_SLOTS;
+    if (total < n_buck * least || n_reg >= (1ULL << 31) || n_buck >= (1ULL << 31)) j->regions = false;
   }
   j->seg.assign(nj + 1, 0);
   for (uint32_t i = 0; i < nj; ++i) {
@@ -1915,9 +1917,12 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
     b2_max = std::max(b2_max, (int)(j->lay[q].rbits - j->lay[q].beta));
   }
   if (b2_max > SPLIT_MAX_BITS) return BRUNO_OK;
-  /* parser workgroups: one per CU and at least one per job with reads, each
-   * next one to the job whose workgroups have the most instances (a wave's
-   * reads or more per workgroup) */
+  /* Parser workgroups: at least one per job with reads, and each next one to
+   * the job whose workgroups have the most instances (a wave's reads or more
+   * per workgroup), up to one per CU and then while one has more than half as
+   * much again as a CU's even share: of more jobs than CUs the large ones would
+   * else get one each (4,096 jobs of 7,200 instances and one of 96 M: 106 ms,
+   * now 11).  Then the longest start first. */
   std::vector<uint32_t> wgs(jb - ja, 0);
   std::priority_queue<std::pair<double, uint32_t>> most;
   uint64_t given = 0;
@@ -1928,7 +1933,8 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   };
   for (uint32_t q = ja; q < jb; ++q)
     if (h_first[q + 1] > h_first[q]) give(q);
-  while (given < cus && !most.empty()) {
+  const double even = (double)n_inst / (double)cus;
+  while (!most.empty() && (given < cus || most.top().first > 1.5 * even)) {
     const uint32_t q = most.top().second;
     most.pop();
     give(q);
@@ -1940,12 +1946,20 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
     open += (uint64_t)w << j->lay[q].beta;
     for (uint32_t i = 0; i < w; ++i) share.push_back(ParseShare{q, i, w, 0});
   }
+  if (given > cus)
+    std::stable_sort(share.begin(), share.end(), [&](const ParseShare& a, const ParseShare& b) {
+      return (double)inst[a.job] / a.n > (double)inst[b.job] / b.n;
+    });
   /* chunks of up to 1024 records, smaller for small inputs so padding stays
-   * under ~1/8 of the records.  (Chunks smaller than a bucket's stage are
-   * taken several at once; a floor at the stage of the job with the fewest
-   * buckets, 512 records, gave every other job's open chunks that size too.) */
+   * under ~1/8 of the records, but not below an average record's stage.  (A
+   * bucket whose stage is larger takes several chunks at once, an atomic in
+   * HBM; a floor at the largest stage, of the job with the fewest buckets, 512
+   * records, gave every other job's open chunks that size too.) */
+  double stage = 0;
+  for (uint32_t q = ja; q < jb; ++q) stage += (double)inst[q] * (double)((REC_STAGE_BYTES / RB) >> j->lay[q].beta);
+  stage /= (double)std::max<uint64_t>(1, n_inst);
   uint32_t clog = REC_CHUNK_LOG;
-  while (clog > REC_CHUNK_LOG_MIN && (open << clog) * 4 > n_inst) --clog;
+  while (clog > REC_CHUNK_LOG_MIN && (double)(1u << (clog - 1)) >= stage && (open << clog) * 4 > n_inst) --clog;
   /* every record's chunk, the partly filled ones, and at most two per
    * (workgroup, bucket) taken ahead and not used */
   const uint64_t n_chunks = (n_inst >> clog) + 3 * open + 1;

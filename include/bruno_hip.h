@@ -377,7 +377,7 @@ typedef struct {
                               fewer): the walk length between rulers and the size of the
                               contracted list                                               */
   uint32_t count_regions;  /* 1 or 2: tables (k <= 63) of >= 2^19 slots, all jobs of a batch
-                              together (but not of very small jobs, of some 24,000 slots and
+                              together (but not of very small jobs, of some 30,000 slots and
                               fewer on average), are laid out in LDS-sized regions and count by
                               writing instance records grouped by region, then building each
                               region on chip (1: the calls with enough instances for that to

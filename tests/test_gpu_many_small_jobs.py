@@ -50,3 +50,25 @@ def test_one_small_job_beside_others(k):
             assert node_table(bt.job(i).counts()) == oracle_node_table(want.unfiltered()), i
         bt.close()
     assert peak[1] < 1.05 * peak[0]
+
+
+def test_more_jobs_than_workgroups():
+    """300 jobs, one of them with most of the reads: it gets more than one
+    workgroup of the record parser, and every job its own counts."""
+    k, n = 31, 300
+    rng = np.random.default_rng(8)
+    g = "".join(rng.choice(list("ACGT"), 30_000))
+
+    def reads(m):
+        return [g[i:i + 150] for i in rng.integers(0, len(g) - 150, m)]
+
+    jobs = [reads(int(m)) for m in rng.integers(0, 60, n)]
+    jobs[170] = reads(60_000)
+    bt = bruno_amd.GraphBatch(k, None, [45_000] * n)
+    bt.parse_count(*pack_jobs(jobs))
+    assert bt.stats()["count_by_regions"] == 1
+    for i in list(range(0, n, 23)) + [170]:
+        want = run_oracle(k, None, *pack(jobs[i]))
+        assert node_table(bt.job(i).counts()) == oracle_node_table(want.unfiltered()), i
+        assert bt.job(i).stats()["n_reads"] == len(jobs[i])
+    bt.close()
