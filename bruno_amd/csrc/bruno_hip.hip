@@ -2005,8 +2005,8 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   uint32_t* pieces = (uint32_t*)get(n_pieces * 4);
   uint32_t* owner = (uint32_t*)get(n_chunks * 4);
   uint32_t* list = (uint32_t*)get(n_chunks * 4);
-  uint32_t* rstart = (uint32_t*)get(nreg * 4);
-  uint32_t* rcount = (uint32_t*)get(nreg * 4);
+  uint32_t* rstart = (uint32_t*)get(nreg * 8);
+  uint32_t* rcount = rstart + nreg;
   uint32_t* first = (uint32_t*)get((n_sb + 1) * 4);
   ParseShare* d_share = (ParseShare*)get(share.size() * sizeof(ParseShare));
   /* a parser workgroup's records of one interval, at most 16 per read, that
@@ -2016,8 +2016,8 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
     if (wgs[q - ja]) lanes = std::max(lanes, (h_first[q + 1] - h_first[q] + wgs[q - ja] - 1) / wgs[q - ja]);
   const uint64_t interval = std::min<uint64_t>(rec_interval<R>(), 16 * lanes);
   const uint32_t over_cap = (uint32_t)(interval > REC_PARK ? interval - REC_PARK : 0);
-  void* over = get(share.size() * over_cap * RB);
-  uint32_t* over_at = (uint32_t*)get(share.size() * over_cap * 4);
+  void* over = get(share.size() * over_cap * (RB + 4));
+  uint32_t* over_at = (uint32_t*)((char*)over + share.size() * over_cap * RB);
   /* zeroed: chunks taken in all and overflow flag, statistics, per bucket
    * chunks taken and listed */
   const uint64_t n_zero = 1 + 2 * (uint64_t)nj + (n_sb + 1) / 2 + n_sb * (LISTED_STRIDE / 2);
