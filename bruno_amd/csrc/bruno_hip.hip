@@ -1922,14 +1922,15 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
    * per workgroup), up to one per CU and then while one has more than half as
    * much again as a CU's even share: of more jobs than CUs the large ones would
    * else get one each (4,096 jobs of 7,200 instances and one of 96 M: 106 ms,
-   * now 11).  Then the longest start first. */
+   * now 11).  Then the longest start first.  (Reads whose instances make a
+   * wave's work each may have a workgroup each.) */
   std::vector<uint32_t> wgs(jb - ja, 0);
   std::priority_queue<std::pair<double, uint32_t>> most;
   uint64_t given = 0;
   auto give = [&](uint32_t q) {
     const uint64_t nr = h_first[q + 1] - h_first[q], w = ++wgs[q - ja];
     ++given;
-    if (w * 64 < nr) most.push({(double)inst[q] / (double)w, q});
+    if (w * 64 < nr || (w < nr && inst[q] / w >= REC_WG_INSTANCES)) most.push({(double)inst[q] / (double)w, q});
   };
   for (uint32_t q = ja; q < jb; ++q)
     if (h_first[q + 1] > h_first[q]) give(q);
@@ -1951,7 +1952,7 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
       return (double)inst[a.job] / a.n > (double)inst[b.job] / b.n;
     });
   /* chunks of up to 1024 records, smaller for small inputs so padding stays
-   * under ~1/8 of the records, but not below an average record's stage.  (A
+   * under ~1/8 of the records, but not far below an average record's stage.  (A
    * bucket whose stage is larger takes several chunks at once, an atomic in
    * HBM; a floor at the largest stage, of the job with the fewest buckets, 512
    * records, gave every other job's open chunks that size too.) */
@@ -1959,7 +1960,7 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   for (uint32_t q = ja; q < jb; ++q) stage += (double)inst[q] * (double)((REC_STAGE_BYTES / RB) >> j->lay[q].beta);
   stage /= (double)std::max<uint64_t>(1, n_inst);
   uint32_t clog = REC_CHUNK_LOG;
-  while (clog > REC_CHUNK_LOG_MIN && (double)(1u << (clog - 1)) >= stage && (open << clog) * 4 > n_inst) --clog;
+  while (clog > REC_CHUNK_LOG_MIN && (1u << (clog - 1)) >= 0.75 * stage && (open << clog) * 4 > n_inst) --clog;
   /* every record's chunk, the partly filled ones, and at most two per
    * (workgroup, bucket) taken ahead and not used */
   const uint64_t n_chunks = (n_inst >> clog) + 3 * open + 1;
@@ -2009,11 +2010,14 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   uint32_t* rcount = rstart + nreg;
   uint32_t* first = (uint32_t*)get((n_sb + 1) * 4);
   ParseShare* d_share = (ParseShare*)get(share.size() * sizeof(ParseShare));
-  /* a parser workgroup's records of one interval, at most 16 per read, that
-   * its park has no room for */
-  uint64_t lanes = 0;
+  /* A parser workgroup's lanes: one per read, or for reads taken by all lanes
+   * one per 64 instances; and its records of one interval, at most 16 per
+   * lane, that its park has no room for. */
+  uint64_t lanes = 1;
   for (uint32_t q = ja; q < jb; ++q)
-    if (wgs[q - ja]) lanes = std::max(lanes, (h_first[q + 1] - h_first[q] + wgs[q - ja] - 1) / wgs[q - ja]);
+    if (const uint64_t w = wgs[q - ja])
+      lanes = std::max<uint64_t>(lanes, std::max<uint64_t>((h_first[q + 1] - h_first[q] + w - 1) / w, inst[q] / w / 64));
+  lanes = std::min<uint64_t>(lanes, REC_BS);
   const uint64_t interval = std::min<uint64_t>(rec_interval<R>(), 16 * lanes);
   const uint32_t over_cap = (uint32_t)(interval > REC_PARK ? interval - REC_PARK : 0);
   void* over = get(share.size() * over_cap * (RB + 4));
@@ -2040,7 +2044,7 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   ChunkPool pool{recs, clog, (uint32_t)n_chunks, next, taken - b_lo, owner, overflow};
   if (!share.empty()) {
     HIP_CHECK(hipMemcpyAsync(d_share, share.data(), share.size() * sizeof(ParseShare), hipMemcpyHostToDevice, j->stream));
-    RecArgs ra{pool, j->d_lay, d_first, d_share, over, over_at, over_cap, stat};
+    RecArgs ra{pool, j->d_lay, d_first, d_share, over, over_at, over_cap, (uint32_t)lanes, stat};
     constexpr int PF = RB == 8 ? 8 : 4;
     const dim3 g((unsigned)share.size());
     if (beta_max <= 8)

@@ -48,6 +48,7 @@ constexpr uint64_t REGION_BUILD_CU_SLOTS = 512; /* build workgroups resident on 
  * records parked in LDS that found their bucket's stage full */
 constexpr int REC_BS = 1024, REC_PARK = 256;
 constexpr uint32_t REC_STAGE_BYTES = 128 << 10;
+constexpr uint64_t REC_WG_INSTANCES = 1 << 15; /* enough instances for a parser workgroup */
 /* most records between two appends: a workgroup appends every PF positions,
  * or every 16 when its reads have at most so many records in them */
 template <typename R> constexpr uint32_t rec_interval() { return REC_STAGE_BYTES / sizeof(R) / 4 * 3; }
@@ -66,6 +67,7 @@ struct RecArgs {
   void* over;                /* per workgroup over_cap records (RecOf<KT>::T) that found the park full, */
   uint32_t* over_at;         /* and their places */
   uint32_t over_cap;
+  uint32_t lanes;            /* most lanes that take part in one round */
   unsigned long long* stat;  /* per job: instances, dropped reads */
 };
 
@@ -140,6 +142,14 @@ __device__ __noinline__ void place_over(const R* over, const uint32_t* over_at, 
  * (NFilterSequencesIterator, compact_dbg_freq_construct_clean.cpp:210-213),
  * found by a first pass over its blocks.
  *
+ * Long reads: a round lasts as long as its longest read, so reads that the
+ * others would wait for are left out of it and then taken one by one, each
+ * by all lanes, a piece of its instances per lane; where the line lies
+ * depends on the round (long_line).  A read of 1 M bases among 50,000 of 150: 266
+ * ms by one lane, 78 by atomics (a wave per read), now 1.5; 3,000 reads of 5,000
+ * to 15,000: 5.5, 2.3, now 1.1; 60,000 of log-normal length (median 490, up to
+ * 20,000) 4.5, 2.8, now 1.9.
+ *
  * Staging: the LDS stage is divided among the job's buckets; every PF
  * positions the workgroup appends each bucket's whole 128-byte lines to the
  * bucket's open chunk (the rest moves to the front of its stage), so chunks
@@ -163,6 +173,26 @@ __device__ __noinline__ void place_over(const R* over, const uint32_t* over_at, 
  * count phase as a whole 35.9 -> 30.1, 4.5 -> 3.8, 13.2 -> 10.7 and 1.39 ->
  * 0.81 ms.  A batch of 16 jobs of 0.05 to 2 Mbp (243 M instances), which HBM
  * atomics counted in 18.6 ms, takes 5.9. */
+constexpr int LONG_BINS = 40, LONG_LOG = 8; /* bin b: reads of 2^(LONG_LOG + b) + 1 .. 2^(LONG_LOG + b + 1) bases */
+constexpr uint64_t LANE_READ_MAX = 1ULL << 30; /* a lane's positions are 32-bit numbers */
+
+/* The length from which a round's reads are taken by all lanes: the power
+ * of two 2^b >= 2^LONG_LOG with the fewest steps in all, 2^b for the reads up to
+ * it and for every longer one a lane's piece and the k bases before it (~0: none). */
+__device__ __noinline__ uint64_t long_line(const uint32_t* hist, uint32_t lanes, int K) {
+  uint64_t line = ~0ULL, least = 0, longer = 0;
+  for (int b = LONG_BINS - 1; b >= 0; --b) {
+    const uint64_t n = hist[b], at = 1ULL << (LONG_LOG + b);
+    if (n && least == 0) least = 2 * at;
+    longer += n * (2 * at / lanes + (uint64_t)K + 48);
+    if (longer && at + longer < least) {
+      least = at + longer;
+      line = at;
+    }
+  }
+  return line < LANE_READ_MAX ? line : least < LANE_READ_MAX ? line : LANE_READ_MAX;
+}
+
 template <typename KT, int MAXB, int PF>
 __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs ra) {
   typedef typename RecOf<KT>::T R;
@@ -179,6 +209,10 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
   __shared__ R park[2 * REC_PARK];
   __shared__ uint32_t park_at[2 * REC_PARK]; /* number in the bucket << 9 | bucket */
   __shared__ uint32_t n_park, blocks_max;
+  /* the round's reads of more than 2^LONG_LOG bases by length, those left for all
+   * lanes, whether one of these has a byte that is no base */
+  __shared__ uint32_t len_hist[LONG_BINS], long_bad;
+  __shared__ unsigned long long long_mask[REC_BS / 64];
   /* (kept here for the rare path that uses them, not in registers) */
   __shared__ R* over;
   __shared__ uint32_t* over_at;
@@ -343,72 +377,120 @@ __global__ __launch_bounds__(REC_BS) void k_parse_records(ParseArgs a, RecArgs r
       lo = a.starts ? a.starts[r] : a.offsets[r];
       L = (a.starts ? a.ends[r] : a.offsets[r + 1]) - lo;
     }
-    const LaneRead rd(a.bases + lo, L);
-    const int64_t mis = rd.mis;
-    const bool bad = rd.bad(L);
-    if (bad) ++my_drop;
-    /* reads shorter than the parser window k + 2 give nothing
-     * (debruijn_biedge_loader.hpp:464-465) */
-    const uint64_t Lp = (bad || L < (uint64_t)K + 2) ? 0 : L;
-    const uint64_t nb = Lp ? (uint64_t)(mis + (int64_t)Lp + 16) / 16 : 0; /* through position Lp */
-    /* every thread has read the last round's maximum before it is reset */
+    /* (every thread is past the last round's use of these) */
     __syncthreads();
+    if (tid < LONG_BINS) len_hist[tid] = 0;
+    if (tid < REC_BS / 64) long_mask[tid] = 0;
     if (tid == 0) blocks_max = 0;
     __syncthreads();
-    if (nb) atomicMax(&blocks_max, (uint32_t)nb);
+    if (L > (1u << LONG_LOG)) {
+      const int b = 63 - __clzll(L - 1) - LONG_LOG;
+      atomicAdd(&len_hist[b < LONG_BINS ? b : LONG_BINS - 1], 1u);
+      blocks_max = 1;
+    }
     __syncthreads();
-    const uint32_t nbw = blocks_max;
-    /* fw: the last k bases read, rv its reverse complement; gone: the base
-     * that left fw at the previous step.  At position j >= k the instance
-     * starting at j - k is complete: its out base is base j (none at
-     * j == L) and its in base the one that left at step j - 1 (none for
-     * the first instance). */
-    KT fw = 0, rv = 0;
-    uint32_t gone = 0;
-    /* a round of few reads fills its stages more slowly: an append at every
-     * PF-th position, or once a block when a bucket's share of the block's
-     * records leaves a quarter of its stage to chance and what stays behind */
-    const bool often = (ra1 - ra0) * 16 > (uint64_t)(rec_interval<R>() - nb_ * (LINE / 2));
-    uint4 v[4] = {};
-    for (uint32_t t = 0; t < nbw; ++t) {
-      if (t % 4 == 0) rd.four(t, v);
-      const uint4 cur = v[0];
-      v[0] = v[1];
-      v[1] = v[2];
-      v[2] = v[3];
-      const uint32_t cw[4] = {codes4(cur.x), codes4(cur.y), codes4(cur.z), codes4(cur.w)};
+    uint32_t long_w = REC_BS / 64; /* words of long_mask gone through */
+    unsigned long long long_m = 0;
+    if (blocks_max) {
+      const bool left = L > long_line(len_hist, ra.lanes, K);
+      const uint64_t m = __ballot(left);
+      if ((tid & 63) == 0) long_mask[tid >> 6] = m;
+      if (left) L = 0;
+      long_w = 0;
+    }
+    /* the instances at j_lo .. j_hi of this lane's bases [lo, lo + L) */
+    int j_lo = K, j_hi = (int)L;
+    uint32_t lanes = (uint32_t)(ra1 - ra0);
+    bool piece = false; /* of a read that all lanes share */
+    for (;;) {
+      const LaneRead rd(a.bases + lo, L);
+      const int mis = rd.mis;
+      const bool bad = rd.bad(L);
+      __syncthreads();
+      if (tid == 0) blocks_max = long_bad = 0;
+      __syncthreads();
+      /* reads shorter than the parser window k + 2 give nothing
+       * (debruijn_biedge_loader.hpp:464-465) */
+      int Lp = bad || L < (uint64_t)K + 1 + !piece ? 0 : (int)L;
+      if (!piece && bad) ++my_drop;
+      if (piece && bad) long_bad = 1;
+      if (Lp) atomicMax(&blocks_max, (uint32_t)(mis + Lp + 16) / 16); /* through position Lp */
+      __syncthreads();
+      uint32_t nbw = blocks_max;
+      if (piece && long_bad) {
+        if (tid == 0) ++my_drop;
+        nbw = 0;
+      }
+      if (Lp == 0) j_hi = -1;
+      /* fw: the last k bases read, rv its reverse complement; gone: the base
+       * that left fw at the previous step.  At position j >= k the instance
+       * starting at j - k is complete: its out base is base j (none at
+       * j == L) and its in base the one that left at step j - 1 (none for
+       * the first instance). */
+      KT fw = 0, rv = 0;
+      uint32_t gone = 0;
+      /* a round of few reads fills its stages more slowly: an append at every
+       * PF-th position, or once a block when a bucket's share of the block's
+       * records leaves a quarter of its stage to chance and what stays behind */
+      const bool often = lanes * 16 > rec_interval<R>() - nb_ * (LINE / 2);
+      uint4 v[4] = {};
+      for (uint32_t t = 0; t < nbw; ++t) {
+        if (t % 4 == 0) rd.four(t, v);
+        const uint4 cur = v[0];
+        v[0] = v[1];
+        v[1] = v[2];
+        v[2] = v[3];
+        const uint32_t cw[4] = {codes4(cur.x), codes4(cur.y), codes4(cur.z), codes4(cur.w)};
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int64_t j = (int64_t)(16 * t) + q - mis;
-        if (j >= 0 && j <= (int64_t)Lp) {
-          const uint32_t c = (cw[q >> 2] >> (8 * (q & 3))) & 3u;
-          const bool in_read = j < (int64_t)Lp;
-          if (j >= K) {
-            const bool flip = !(fw < rv);
-            const KT km = flip ? rv : fw;
-            const uint32_t has_in = j > K, has_out = in_read;
-            const uint32_t il = !has_in ? 0u : flip ? 0u : 1u + gone;
-            const uint32_t ir = !has_out ? 0u : flip ? 0u : 1u + c;
-            /* biedge_rc: the in side becomes the complement of the out
-             * base and the other way round */
-            const uint32_t il2 = flip && has_out ? 4u - c : il;
-            const uint32_t ir2 = flip && has_in ? 4u - gone : ir;
-            const uint64_t h = kmer_hash(km);
-            const uint64_t key = (h << REC_BUCKET_BITS) | (il2 * 5u + ir2);
-            put((uint32_t)(h >> (64 - beta)), make_rec<KT>(key, km));
-            ++my_inst;
+        for (int q = 0; q < 16; ++q) {
+          const int j = (int)(16 * t) + q - mis;
+          if (j >= 0 && j <= j_hi) {
+            const uint32_t c = (cw[q >> 2] >> (8 * (q & 3))) & 3u;
+            const bool in_read = j < Lp;
+            if (j >= j_lo) {
+              const bool flip = !(fw < rv);
+              const KT km = flip ? rv : fw;
+              const uint32_t has_in = j > K, has_out = in_read;
+              const uint32_t il = !has_in ? 0u : flip ? 0u : 1u + gone;
+              const uint32_t ir = !has_out ? 0u : flip ? 0u : 1u + c;
+              /* biedge_rc: the in side becomes the complement of the out
+               * base and the other way round */
+              const uint32_t il2 = flip && has_out ? 4u - c : il;
+              const uint32_t ir2 = flip && has_in ? 4u - gone : ir;
+              const uint64_t h = kmer_hash(km);
+              const uint64_t key = (h << REC_BUCKET_BITS) | (il2 * 5u + ir2);
+              put((uint32_t)(h >> (64 - beta)), make_rec<KT>(key, km));
+              ++my_inst;
+            }
+            if (in_read) {
+              gone = (uint32_t)(fw >> sh2) & 3u;
+              fw = ((fw << 2) | (KT)c) & kmask;
+              rv = (rv >> 2) | ((KT)(3u - c) << sh2);
+            }
           }
-          if (in_read) {
-            gone = (uint32_t)(fw >> sh2) & 3u;
-            fw = ((fw << 2) | (KT)c) & kmask;
-            rv = (rv >> 2) | ((KT)(3u - c) << sh2);
+          if (q % PF == PF - 1 && (often || q == 15)) {
+            lds_barrier();
+            flush(false);
           }
-        }
-        if (q % PF == PF - 1 && (often || q == 15)) {
-          lds_barrier();
-          flush(false);
         }
       }
+      /* the next read left for all lanes */
+      while (long_m == 0 && long_w < REC_BS / 64) long_m = long_mask[long_w++];
+      if (long_m == 0) break;
+      const uint64_t rl = ra0 + 64 * (long_w - 1) + __builtin_ctzll(long_m);
+      long_m &= long_m - 1;
+      const uint64_t l0 = a.starts ? a.starts[rl] : a.offsets[rl], ll = (a.starts ? a.ends[rl] : a.offsets[rl + 1]) - l0;
+      /* a piece's instances begin at bases [i0, i1) of the read; its own bases
+       * are those and the one on either side */
+      piece = true;
+      lanes = ra.lanes;
+      const uint64_t n = ll - K + 1, per = (n + lanes - 1) / lanes;
+      const uint64_t i0 = tid < lanes ? tid * per : n, i1 = i0 + per < n ? i0 + per : n;
+      const uint64_t from = i0 ? i0 - 1 : 0, to = i1 + K < ll ? i1 + K : ll;
+      lo = l0 + from;
+      L = i0 < n ? to - from : 0;
+      j_lo = K + (i0 ? 1 : 0);
+      j_hi = (int)(i1 == n ? L : L - 1);
     }
   }
   lds_barrier(); /* the last append's parked records are placed */
