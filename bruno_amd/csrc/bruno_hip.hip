@@ -1316,6 +1316,8 @@ struct bruno_job {
    * segment).  lay: per job (d_lay on the device); rbits, rspan: a plain
    * job's. */
   bool regions = false;
+  bool no_regions = false;           /* asked for without */
+  uint64_t scratch_limit = ~0ULL;    /* bytes that a region count may take for its pass */
   std::vector<JobLayout> lay;
   JobLayout* d_lay = nullptr;
   uint32_t rbits = 0;
@@ -1606,51 +1608,66 @@ void region_layout(uint64_t cap, uint64_t most, bool spread, uint32_t* rbits, ui
   }
 }
 
-/* One table for all jobs: job i gets caps[i] slots (with the region layout,
- * a whole number of regions) from seg[i].  A region table's slots are
- * written by the first count, not filled here. */
-bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
-  const uint32_t nj = j->n_jobs;
-  const uint32_t cr = tuning().count_regions;
-  uint64_t total = 0, n_reg = 0, n_buck = 0, max_span = 0;
+/* The layout of one table for jobs of caps[i] slots each, regions or (not
+ * allowed, or no gain) a probe window per job. */
+struct TableLayout {
+  bool regions;
+  std::vector<JobLayout> lay;
+  uint64_t n_regions = 0, n_buckets = 0, max_span = 0, slots = 0;
+};
+TableLayout table_layout(int words, uint32_t nj, const uint64_t* caps, bool allowed) {
+  TableLayout t;
+  uint64_t total = 0;
   for (uint32_t i = 0; i < nj; ++i) total += caps[i];
-  j->regions = cr && total >= REGION_MIN_CAP;
-  j->fusable = nj == 1 && caps[0] >= REGION_TIGHT_CAP;
+  t.regions = allowed && tuning().count_regions && total >= REGION_MIN_CAP;
   /* the knob counts 32-byte slots: a 64-byte-slot region holds half */
-  const uint64_t most = j->words == 1 ? tuning().region_slots : tuning().region_slots / 2;
-  j->lay.assign(nj, JobLayout{});
-  if (j->regions) {
+  const uint64_t most = words == 1 ? tuning().region_slots : tuning().region_slots / 2;
+  t.lay.assign(nj, JobLayout{});
+  if (t.regions) {
     for (uint32_t i = 0; i < nj; ++i) {
-      JobLayout& l = j->lay[i];
+      JobLayout& l = t.lay[i];
       region_layout(caps[i], most, nj > 1 || caps[i] < REGION_TIGHT_CAP, &l.rbits, &l.span);
       /* buckets: one per CU, 512 when one split pass would have more than
        * SPLIT_MAX_BITS region bits left (2^20 regions, 4.0 G instances:
        * parser 17.2 and split 32.1 ms with 256 buckets and 12 bits, 26.3 and
        * 27.5 with 512 and 11) */
       l.beta = std::min<uint32_t>(l.rbits, l.rbits > 8 + SPLIT_MAX_BITS ? MAX_BUCKET_BITS : 8);
-      l.region0 = (uint32_t)n_reg;
-      l.bucket0 = (uint32_t)n_buck;
-      n_reg += 1ULL << l.rbits;
-      n_buck += 1ULL << l.beta;
-      max_span = std::max(max_span, l.span);
+      l.region0 = (uint32_t)t.n_regions;
+      l.bucket0 = (uint32_t)t.n_buckets;
+      t.n_regions += 1ULL << l.rbits;
+      t.n_buckets += 1ULL << l.beta;
+      t.max_span = std::max(t.max_span, l.span);
     }
     /* (regions and buckets are numbered in 32 bits) */
-    const uint64_t least = j->words == 1 ? REGION_MIN_BUCKET_SLOTS : REGION_MIN_BUCKET_WIDE_SLOTS;
-    if (total < n_buck * least || n_reg >= (1ULL << 31) || n_buck >= (1ULL << 31)) j->regions = false;
+    const uint64_t least = words == 1 ? REGION_MIN_BUCKET_SLOTS : REGION_MIN_BUCKET_WIDE_SLOTS;
+    if (total < t.n_buckets * least || t.n_regions >= (1ULL << 31) || t.n_buckets >= (1ULL << 31)) t.regions = false;
   }
-  j->seg.assign(nj + 1, 0);
   for (uint32_t i = 0; i < nj; ++i) {
-    JobLayout& l = j->lay[i];
-    if (!j->regions) {
+    JobLayout& l = t.lay[i];
+    if (!t.regions) {
       l = JobLayout{};
       l.span = caps[i];
     }
-    l.slot0 = j->seg[i];
-    j->seg[i + 1] = j->seg[i] + (l.span << l.rbits);
+    l.slot0 = t.slots;
+    t.slots += l.span << l.rbits;
   }
-  j->n_regions = n_reg;
-  j->n_buckets = n_buck;
-  j->bit_stride = (max_span + 63) / 64;
+  return t;
+}
+
+/* One table for all jobs: job i gets caps[i] slots (with the region layout,
+ * a whole number of regions) from seg[i].  A region table's slots are
+ * written by the first count, not filled here. */
+bruno_status alloc_table(bruno_job* j, const uint64_t* caps) {
+  const uint32_t nj = j->n_jobs;
+  TableLayout t = table_layout(j->words, nj, caps, !j->no_regions);
+  j->regions = t.regions;
+  j->fusable = nj == 1 && caps[0] >= REGION_TIGHT_CAP;
+  j->lay = std::move(t.lay);
+  j->seg.assign(nj + 1, t.slots);
+  for (uint32_t i = 0; i < nj; ++i) j->seg[i] = j->lay[i].slot0;
+  j->n_regions = t.n_regions;
+  j->n_buckets = t.n_buckets;
+  j->bit_stride = (t.max_span + 63) / 64;
   j->rbits = nj == 1 ? j->lay[0].rbits : 0;
   j->rspan = nj == 1 && j->regions ? j->lay[0].span : 0;
   const uint64_t cap = j->seg[nj];
@@ -1965,7 +1982,9 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   for (uint32_t q = ja; q < jb; ++q) stage += (double)inst[q] * (double)((REC_STAGE_BYTES / RB) >> j->lay[q].beta);
   stage /= (double)std::max<uint64_t>(1, n_inst);
   uint32_t clog = REC_CHUNK_LOG;
-  while (clog > REC_CHUNK_LOG_MIN && (1u << (clog - 1)) >= 0.75 * stage && (open << clog) * 4 > n_inst) --clog;
+  while (clog > REC_CHUNK_LOG_MIN && (open << clog) * 4 > n_inst &&
+         ((1u << (clog - 1)) >= 0.75 * stage || 2 * RB * (n_inst + (3 * open << clog)) > j->scratch_limit / 8 * 7))
+    --clog;
   /* every record's chunk, the partly filled ones, and at most two per
    * (workgroup, bucket) taken ahead and not used */
   const uint64_t n_chunks = (n_inst >> clog) + 3 * open + 1;
@@ -1992,9 +2011,11 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
   };
   std::vector<Buf> bufs;
   bool room = true;
+  uint64_t scratch = 0;
   auto get = [&](uint64_t bytes) -> void* {
     void* p = nullptr;
-    if (!room || dev_alloc(j, &p, std::max<uint64_t>(16, bytes)) != BRUNO_OK) {
+    scratch += bytes;
+    if (!room || scratch > j->scratch_limit || dev_alloc(j, &p, std::max<uint64_t>(16, bytes)) != BRUNO_OK) {
       room = false;
       return nullptr;
     }
@@ -2037,7 +2058,9 @@ bruno_status count_regions_pass(bruno_job* j, const ParseArgs& a, const uint64_t
     return BRUNO_OK;
   }
   uint64_t* spq = nullptr;
-  if (dev_alloc(j, (void**)&spq, n_waves * spq_cap * 8) == BRUNO_OK) bufs.push_back(Buf{spq, n_waves * spq_cap * 8});
+  if (scratch + n_waves * spq_cap * 8 <= j->scratch_limit &&
+      dev_alloc(j, (void**)&spq, n_waves * spq_cap * 8) == BRUNO_OK)
+    bufs.push_back(Buf{spq, n_waves * spq_cap * 8});
   else spq_cap = 0;
   uint32_t* next = (uint32_t*)zero;
   uint32_t* overflow = next + 1;
@@ -2266,10 +2289,10 @@ bruno_status count_by_regions(bruno_job* j, const ParseArgs& a, const uint64_t* 
   /* records a job takes room for: its instances, and per bucket an open chunk
    * and two in hand (of one workgroup: a pass of many jobs has no more) */
   auto room_of = [&](uint32_t q) { return inst[q] + ((uint64_t)3 << j->lay[q].beta << REC_CHUNK_LOG_MIN); };
+  const uint64_t pass_bytes = std::min(REC_PASS_BYTES, j->scratch_limit / 7 * 2);
   for (uint32_t ja = 0, jb; ja < nj; ja = jb) {
     uint64_t n = room_of(ja);
-    for (jb = ja + 1; jb < nj && n + room_of(jb) <= REC_PASS_BYTES / sizeof(typename RecOf<KT>::T); ++jb)
-      n += room_of(jb);
+    for (jb = ja + 1; jb < nj && n + room_of(jb) <= pass_bytes / sizeof(typename RecOf<KT>::T); ++jb) n += room_of(jb);
     bool done = false;
     TRY(count_regions_pass<KT>(j, a, d_first, h_first, ja, jb, inst, valid, cbits, sbits, &done));
     if (done) continue;
@@ -3114,7 +3137,8 @@ const char* bruno_status_string(bruno_status s) {
   return "unknown";
 }
 
-static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, const uint64_t* caps, bruno_job** out) {
+static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, const uint64_t* caps, bruno_job** out,
+                                  bool regions = true, uint64_t scratch_limit = ~0ULL) {
   if (!d || !out) return BRUNO_BAD_INPUT;
   *out = nullptr;
   if (d->k < 3 || d->k > 63 || n_jobs == 0 || d->thresholding < 0 || d->thresholding > 2) return BRUNO_BAD_INPUT;
@@ -3133,6 +3157,8 @@ static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, cons
   j->load_factor = (d->load_factor > 0 && d->load_factor < 1) ? d->load_factor : 0.5;
   j->stream = (hipStream_t)d->stream;
   j->n_jobs = n_jobs;
+  j->no_regions = !regions;
+  j->scratch_limit = scratch_limit;
   j->job_reads.assign(n_jobs, 0);
   if (pool_alloc((void**)&j->ctr, sizeof(Counters)) != hipSuccess ||
       hipHostMalloc((void**)&j->hctr, sizeof(Counters), hipHostMallocDefault) != hipSuccess) {
@@ -3185,6 +3211,46 @@ bruno_status bruno_batch_create(const bruno_job_desc* d, uint32_t n_jobs, const 
 __attribute__((visibility("hidden"))) uint64_t br_region_count_min_slots() {
   const uint32_t cr = tuning().count_regions;
   return cr == 0 ? 0 : REGION_MIN_CAP;
+}
+
+/* For the request server, not exported.  Bytes that a batch of n_jobs (of
+ * caps[i] slots and at most inst[i] instances) takes with the region layout,
+ * beyond the slots asked for: *table the regions' room and the filter's bits,
+ * *scratch what a count's pass takes while it runs (an upper bound, see
+ * count_regions_pass).  Both 0 if it keeps probe windows. */
+__attribute__((visibility("hidden"))) void br_region_bytes(int k, uint32_t n_jobs, const uint64_t* caps,
+                                                           const uint64_t* inst, uint64_t n_reads, uint64_t* table,
+                                                           uint64_t* scratch) {
+  const int words = k <= 31 ? 1 : 2;
+  const TableLayout t = table_layout(words, n_jobs, caps, true);
+  *table = *scratch = 0;
+  if (!t.regions) return;
+  uint64_t asked = 0, n = 0, largest = 0;
+  for (uint32_t i = 0; i < n_jobs; ++i) {
+    asked += caps[i];
+    n += inst[i];
+    largest = std::max(largest, inst[i]);
+  }
+  const uint64_t slot = words == 1 ? sizeof(Slot<uint64_t>) : sizeof(Slot<u128>), rb = words == 1 ? 8 : 16;
+  *table = (t.slots - std::min(asked, t.slots)) * (slot + sizeof(Spill) / 32) +
+           2 * 8 * t.n_regions * ((t.max_span + 63) / 64);
+  n = std::min(n, std::max(REC_PASS_BYTES / rb, largest));
+  uint32_t beta = 0;
+  for (const JobLayout& l : t.lay) beta = std::max(beta, l.beta);
+  const uint64_t wgs = std::min<uint64_t>(device_cus() + n_jobs, n_reads / 64 + n / REC_WG_INSTANCES + 2 * n_jobs);
+  const uint64_t open = std::max<uint64_t>(REC_STAGE_BYTES / rb * 9 / 2, (uint64_t)3 << beta << REC_CHUNK_LOG_MIN);
+  const uint64_t recs = n + std::max<uint64_t>(n * 3 / 4, wgs * open);
+  *scratch = (2 * recs + (t.n_regions << PIECE_LOG)) * rb + (recs / PIECE + t.n_regions) * 16 +
+             wgs * rec_interval<uint64_t>() * 12 + t.n_buckets * 4 * (LISTED_STRIDE + 2) +
+             std::max<uint64_t>(64 << 20, n / 16) + (1 << 20) + 64 * (uint64_t)n_jobs;
+}
+/* ... and a batch without the region layout, or whose counts take at most
+ * scratch_limit bytes for a pass (they count with atomics where that is too
+ * little). */
+__attribute__((visibility("hidden"))) bruno_status br_batch_create(const bruno_job_desc* d, uint32_t n_jobs,
+                                                                   const uint64_t* caps, int regions,
+                                                                   uint64_t scratch_limit, bruno_job** out) {
+  return create_common(d, n_jobs, caps, out, regions != 0, scratch_limit);
 }
 
 bruno_status bruno_job_destroy(bruno_job* j) {

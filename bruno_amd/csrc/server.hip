@@ -37,8 +37,13 @@
 #include "../../include/bruno_hip.h"
 #include "pool.h"
 
-/* bruno_hip.hip: slots from which a one-job table counts by regions */
+/* bruno_hip.hip: slots from which a one-job table counts by regions; what the
+ * region layout and a count's pass take; a batch without or within that */
 extern "C" uint64_t br_region_count_min_slots();
+extern "C" void br_region_bytes(int k, uint32_t n_jobs, const uint64_t* caps, const uint64_t* inst, uint64_t n_reads,
+                                uint64_t* table, uint64_t* scratch);
+extern "C" bruno_status br_batch_create(const bruno_job_desc* d, uint32_t n_jobs, const uint64_t* caps, int regions,
+                                        uint64_t scratch_limit, bruno_job** out);
 
 namespace {
 
@@ -104,11 +109,36 @@ constexpr uint64_t SOLO_MIN_SLOTS = 1ULL << 26;
 /* Estimated peak HBM of one job: table and side table, the present list
  * (8 B per distinct k-mer, at most one per slot), the chain, list-ranking
  * and output arrays (a quarter of the table for reads of one genome), the
- * reads themselves and a fixed allowance for small buffers. */
+ * reads themselves and a fixed allowance for small buffers.  Requests are
+ * admitted by this; a batch then gets of the budget's rest what the region
+ * count takes beyond it (region_grant), or counts with atomics. */
 uint64_t footprint(const bruno_job_desc& j, uint64_t cap, uint64_t n_reads, uint64_t n_bases) {
   const uint64_t slot = j.k <= 31 ? 32 : 64;
   const uint64_t table = cap * slot + std::max<uint64_t>(1024, cap / 32) * 64;
   return table + table / 4 + cap * 8 + n_bases + 8 * (n_reads + 1) + (16ULL << 20);
+}
+
+/* What a batch with `left` bytes of the budget beyond its footprint may do: the
+ * region layout (its room in the table for the whole batch) and a count's pass
+ * buffers, until the count is done. */
+struct Grant {
+  bool regions = false;
+  uint64_t table = 0, scratch = 0;
+};
+Grant region_grant(const std::vector<std::shared_ptr<Request>>& batch, uint64_t left) {
+  std::vector<uint64_t> caps, inst;
+  uint64_t n_reads = 0;
+  for (auto& r : batch) {
+    caps.push_back(r->capacity);
+    inst.push_back(r->n_bases);
+    n_reads += r->n_reads;
+  }
+  Grant g;
+  br_region_bytes(batch[0]->job.k, (uint32_t)caps.size(), caps.data(), inst.data(), n_reads, &g.table, &g.scratch);
+  if (g.table > left) return Grant{};
+  g.regions = true;
+  g.scratch = std::min(g.scratch, left - g.table);
+  return g;
 }
 
 void finish(bruno_server* S, const std::shared_ptr<Request>& r, const bruno_result_info& info, std::string&& u,
@@ -123,8 +153,9 @@ void finish(bruno_server* S, const std::shared_ptr<Request>& r, const bruno_resu
 }
 
 /* Run one batch on stream st.  Returns the batch status; per-job results in
- * out (only when the status is OK). */
-bruno_status run_batch(bruno_server* S, hipStream_t st, const std::vector<std::shared_ptr<Request>>& batch,
+ * out (only when the status is OK).  The grant's scratch is given back (and
+ * set to 0) once the count is done. */
+bruno_status run_batch(bruno_server* S, hipStream_t st, const std::vector<std::shared_ptr<Request>>& batch, Grant& grant,
                        std::vector<bruno_result_info>& info, std::vector<std::string>& uni,
                        std::vector<std::string>& bra) {
   const uint32_t n = (uint32_t)batch.size();
@@ -179,9 +210,15 @@ bruno_status run_batch(bruno_server* S, hipStream_t st, const std::vector<std::s
     jd.capacity = 0;
     std::vector<uint64_t> caps(n);
     for (uint32_t i = 0; i < n; ++i) caps[i] = batch[i]->capacity;
-    status = bruno_batch_create(&jd, n, caps.data(), &job);
+    status = br_batch_create(&jd, n, caps.data(), grant.regions, grant.scratch, &job);
   }
   if (status == BRUNO_OK) status = bruno_batch_parse_count(job, d_bases, d_offs, nr, first.data());
+  if (grant.scratch) {
+    std::lock_guard<std::mutex> lk(S->mu);
+    S->reserved -= grant.scratch;
+    grant.scratch = 0;
+    S->cv_work.notify_all();
+  }
   if (status == BRUNO_OK) status = bruno_run_pipeline(job, S->d.variant);
   info.assign(n, bruno_result_info{});
   uni.assign(n, std::string());
@@ -227,6 +264,7 @@ void worker(bruno_server* S) {
   for (;;) {
     std::vector<std::shared_ptr<Request>> batch;
     uint64_t fp = 0, bid = 0;
+    Grant grant;
     {
       std::unique_lock<std::mutex> lk(S->mu);
       for (;;) {
@@ -272,6 +310,8 @@ void worker(bruno_server* S) {
         }
       }
       S->reserved += fp;
+      grant = region_grant(batch, S->d.hbm_budget - std::min(S->d.hbm_budget, S->reserved));
+      S->reserved += grant.table + grant.scratch;
       bid = S->next_batch++;
       ++S->st.batches;
       S->st.max_batch_jobs = std::max<uint64_t>(S->st.max_batch_jobs, batch.size());
@@ -280,11 +320,11 @@ void worker(bruno_server* S) {
     const double t_start = S->now();
     std::vector<bruno_result_info> info;
     std::vector<std::string> uni, bra;
-    bruno_status s = run_batch(S, st, batch, info, uni, bra);
+    bruno_status s = run_batch(S, st, batch, grant, info, uni, bra);
     const double t_end = S->now();
     {
       std::lock_guard<std::mutex> lk(S->mu);
-      S->reserved -= fp;
+      S->reserved -= fp + grant.table + grant.scratch;
       if (s == BRUNO_OK) {
         for (size_t i = 0; i < batch.size(); ++i) {
           info[i].status = BRUNO_OK;
