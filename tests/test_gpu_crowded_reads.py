@@ -86,6 +86,23 @@ def test_crowded_run(k, n, length, run, poly, what):
         check(k, *reads_with(n + k, n, length, slice(0, 0), 1, at))
 
 
+def test_one_bucket_of_all_records_falls_back():
+    """A tenth of all records in one bucket would be one workgroup's split: the
+    call is counted with atomics, alone and after one counted by regions."""
+    k, n = 31, 60_000
+    skew = reads_with(3, n, 150, slice(0, n, 4), 100)
+    even = reads_with(3, n, 150, slice(0, 0), 1)
+    for calls in ((skew,), (even, skew)):
+        job = bruno_amd.GraphJob(k, None, capacity=1 << 20)
+        for b, off in calls:
+            job.parse_count(b, off)
+        assert job.stats()["count_by_regions"] == 0
+        want = run_oracle(k, None, np.concatenate([b for b, _ in calls]),
+                          np.concatenate([calls[0][1]] + [o[1:] + calls[0][1][-1] for _, o in calls[1:]]))
+        assert node_table(job.counts()) == oracle_node_table(want.unfiltered())
+        job.close()
+
+
 def test_crowded_run_of_512_buckets():
     set_tuning(region_slots=1280)
     check(31, *reads_with(5, 300_000, 150, slice(100_000, 101_200), 60), capacity=1_400_000_000)
