@@ -1317,6 +1317,7 @@ struct bruno_job {
    * job's. */
   bool regions = false;
   bool no_regions = false;           /* asked for without */
+  int device = 0;                    /* current when the job was made */
   uint64_t scratch_limit = ~0ULL;    /* bytes that a region count may take for its pass */
   std::vector<JobLayout> lay;
   JobLayout* d_lay = nullptr;
@@ -3157,6 +3158,7 @@ static bruno_status create_common(const bruno_job_desc* d, uint32_t n_jobs, cons
   j->load_factor = (d->load_factor > 0 && d->load_factor < 1) ? d->load_factor : 0.5;
   j->stream = (hipStream_t)d->stream;
   j->n_jobs = n_jobs;
+  if (hipGetDevice(&j->device) != hipSuccess) (void)hipGetLastError();
   j->no_regions = !regions;
   j->scratch_limit = scratch_limit;
   j->job_reads.assign(n_jobs, 0);
@@ -3964,7 +3966,11 @@ constexpr uint64_t COPY_THREADS_MIN = 2 << 20;
 static hipError_t copy_out(bruno_job* j, void* dst, const void* src, uint64_t bytes) {
   if (!bytes) return hipStreamSynchronize(j->stream);
   DevicePool& pool = DevicePool::current();
-  PinnedRing* r = pool.take_ring();
+  /* (a ring's events belong to its device: from a thread that has another one
+   * current than the job was made on, the copy goes without) */
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) (void)hipGetLastError();
+  PinnedRing* r = dev == j->device ? pool.take_ring() : nullptr;
   hipError_t e;
   if (!r) {
     e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, j->stream);

@@ -64,3 +64,22 @@ def test_jobs_at_once():
     for t in ts:
         t.join()
     assert got == {s: [want[s]] * 5 for s in want}
+
+
+def test_another_device_current():
+    """Results fetched by a thread whose current device is not the job's."""
+    import torch
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two devices")
+    job = compacted(genome_reads(1, 60_000))
+    want, got = job.unitigs(), []
+
+    def fetch():
+        torch.cuda.set_device(1)
+        got.append(job.unitigs())
+
+    t = threading.Thread(target=fetch)
+    t.start()
+    t.join()
+    assert got == [want]
+    job.close()
