@@ -343,37 +343,13 @@ __global__ __launch_bounds__(BLOCK) void k_filter_spilled(Slot<KT>* T, const Spi
 /* ================================================================== */
 /* chain extraction                                                     */
 /* ================================================================== */
-/* Resolve neighbour k-mer n (on the pointing node's strand) to a chain
- * pointer.  facing_if_canonical: which end of n faces the pointing node
- * when n is itself canonical.  Non-chain targets get a virtual index
- * holding the canonical k-mer (updates to them are dropped, as
- * map.update(..., false, ...) drops keys absent from the chain map). */
-template <typename KT>
-__device__ uint32_t resolve(const Slot<KT>* T, uint64_t tbase, uint64_t tcap, uint32_t rbits, const kops<KT>& ops,
-                            KT n, uint32_t facing_if_canonical, uint64_t n_chain, KT* vkmer, uint64_t vcap,
-                            Counters* ctr) {
-  KT rn = ops.rc(n);
-  bool flipped = !(n < rn);
-  KT cn = flipped ? rn : n;
-  uint32_t end = flipped ? (facing_if_canonical ^ END_OUT) : facing_if_canonical;
-  uint64_t s = SlotOps<KT>::find(T + tbase, tcap, rbits, cn, true);
-  if (s != ~0ULL) {
-    const NodeRec* nr = (const NodeRec*)&T[tbase + s].sub[0];
-    if (nr->cls == CLS_CHAIN) return end | nr->idx;
-  }
-  unsigned long long v = atomicAdd(&ctr->n_virt, 1ULL);
-  if (v >= vcap) {
-    atomicOr(&ctr->err, ERR_LIST_FULL);
-    return end | IDX_MASK;
-  }
-  vkmer[v] = cn;
-  return end | (uint32_t)(n_chain + v);
-}
-
-/* resolve() of a chain node's in neighbour (its OUT end faces the node when
- * canonical) and out neighbour (its IN end) at once: the two probe
+/* A chain node's in neighbour (its OUT end faces the node when canonical) and
+ * out neighbour (its IN end) resolved to chain pointers at once: the two probe
  * sequences advance in lockstep, so their table reads are in flight
- * together.  Each pointer is written only when its neighbour exists.
+ * together.  A neighbour that is no chain node gets a virtual index holding
+ * the canonical k-mer (updates to it are dropped, as map.update(..., false,
+ * ...) drops keys absent from the chain map).  Each pointer is written only
+ * when its neighbour exists.
  *
  * It also tests, from the neighbours' records it has read, that the chain
  * graph is well formed for list ranking: every edge of the node (k, chain
