@@ -161,15 +161,15 @@ __device__ __noinline__ void place_over(const R* over, const uint32_t* over_at, 
  * count of 1 M reads of 150 bases, 2.7 ms, takes 3.6 with 2,000 poly-A reads
  * among them in one place and 10.2 with 20 times 1,000; when a record that
  * found a park of 512 full gave the count up, to HBM atomics, 13.3 and 43.  An
- * append without crowded buckets pays for it with 2% of the kernel (917 for
- * 900 us, 2.46 for 2.42 ms of 16-byte records).
+ * append without crowded buckets pays for it with 1 to 2% of the kernel (910 for
+ * 900 us, 2.47 for 2.42 ms of 16-byte records).
  *
  * One 1,024-thread workgroup per CU with 256 buckets (512 for the largest
  * tables).  Bound by instruction issue.  The appends to 256 buckets cost
  * 5-15% over 32 and the split after it needs one pass instead of two; the
  * bases tested and coded four at a time and read four blocks at a time give
  * it back (1.6 G instances 7.4 ms with 32 buckets, 7.8 with 256, now 7.3; 184
- * M 0.84, 0.96, 0.92; 301 M of k = 63 2.48, 2.59, 2.46).  With the split the
+ * M 0.84, 0.96, 0.91; 301 M of k = 63 2.48, 2.59, 2.47).  With the split the
  * count phase as a whole 35.9 -> 30.1, 4.5 -> 3.8, 13.2 -> 10.7 and 1.39 ->
  * 0.81 ms.  A batch of 16 jobs of 0.05 to 2 Mbp (243 M instances), which HBM
  * atomics counted in 18.6 ms, takes 5.9. */
